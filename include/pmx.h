@@ -177,8 +177,9 @@ int pmx_sys_timing_end(pmx_sys *sys, float *avg_ms, int *ncalls);
  * the forces of the last evaluation are kept. */
 int pmx_sys_time_pair(pmx_sys *sys, int reps, float *ms_per_launch);
 /* Launch shapes for the autotuner (no counterpart in the reference):
- * PMX_TUNE_FFT_LINES     most lines per FFT block (1..64, default 16; the
- *                        LDS limit of 24 KiB per block also applies);
+ * PMX_TUNE_FFT_LINES     most lines per FFT block of the x and y transforms
+ *                        (1..64, default 16; a block also holds at most 2,048
+ *                        points);
  * PMX_TUNE_PAIR_BLOCKS_PER_CU  pair-kernel blocks per CU (0: as many as fit,
  *                        -k: k fewer than fit, at least 1; fewer leave room
  *                        for the PME chain beside it);
@@ -189,9 +190,11 @@ int pmx_sys_time_pair(pmx_sys *sys, int reps, float *ms_per_launch);
  *                        static, later ones come one at a time from a
  *                        device-wide counter (better when fewer waves are
  *                        resident than the default launch's 4,096);
- * PMX_TUNE_SPREAD_STREAM 0 (default): the PME charge spread runs on the main
- *                        stream before the pair kernel; 1: it runs first on
- *                        the second stream, beside the pair kernel;
+ * PMX_TUNE_SPREAD_STREAM 0 (default below 10,000 atoms): the PME charge spread
+ *                        (with the z transform) runs on the main stream before
+ *                        the pair kernel; 1 (default from 10,000 atoms): it
+ *                        runs first on the second stream, beside the pair
+ *                        kernel;
  * PMX_TUNE_LIST_PRUNE    1 (default): the first pair pass after each list
  *                        build drops, for the later passes, the cluster pairs
  *                        with no candidate pair inside the list radius;
@@ -202,11 +205,11 @@ int pmx_sys_time_pair(pmx_sys *sys, int reps, float *ms_per_launch);
  *                        atoms): on the main stream, in one launch with the
  *                        boundary pairs after the pair kernel (better where
  *                        the PME chain is the longer branch);
- * PMX_TUNE_FUSED_SPREAD  1 (default): inside an MD chunk the PME charge spread
- *                        of the next force pass runs in the launch that kicks
- *                        and drifts the atoms; 0: in a launch of its own.
+ * PMX_TUNE_FUSED_SPREAD  0 or 1, no effect: the charge spread is one launch
+ *                        with the z transform (kept for callers that set it);
  * PMX_TUNE_FFT_PLANES    1 (default): on PME grids whose x-y planes have at
- *                        most 1,024 points, the y transform, the x transform
+ *                        most 4,096 points (mixed form, 2,048 in FP64), the y
+ *                        transform, the x transform
  *                        with the convolution and the inverse y transform run
  *                        as one launch with a block per plane; 0: three
  *                        launches over lines (also the only form on larger

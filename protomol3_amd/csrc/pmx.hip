@@ -89,7 +89,7 @@ struct Sys {
   BinParams bin{};
   PairParams pp{};
   ListParams lp{};
-  PmeParams pme{};
+  PmeParams pme{}, pme_g{};  // the same but for the tiles: spread, gather
   FftPlan plx{}, ply{}, plz{};
   bool pme_on = false;
   int cap = 0, maxmaskwork = 0, ntiles_cap = 0;
@@ -100,7 +100,6 @@ struct Sys {
   int tune_spread_stream2 = 0; // 1: the PME spread runs on the second stream, beside the pair kernel
   int tune_fixup_main = 0;     // 1: exclusion correction and bonded terms on the main stream after the pair kernel
                                // (default 1 below kFixupMainBelow atoms)
-  int tune_fused_spread = 1;   // 1: inside an MD chunk the next pass's spread joins the kick-drift
   int tune_fft_planes = 1;     // 1: y, x and convolution passes in one launch per plane on small planes
   bool fft_plane = false;      // the plane launch is in use
   int border_blocks = 4;       // blocks of the boundary-pair pass
@@ -110,13 +109,14 @@ struct Sys {
   long long nbins = 0;
   int nscanblocks = 0;
   int recip_blocks = 0, corr_blocks = 0;
-  int zl = 1, tky = 1, tkx = 1;
+  int xlog = 0, ylog = 0;              // lines of a block of the x and y passes (log2)
+  size_t lds_z = 0, lds_g = 0, lds_y = 0, lds_x = 0, lds_p = 0;  // dynamic LDS of the PME launches
+  int thr_z = 256, thr_g = 256, thr_y = 256, thr_x = 256, thr_p = 256;  // and their block sizes
   // device buffers
   std::vector<DevBuf *> all;
   DevBuf xorig, xwrap, q_d, type_d, key, hist, start, cursor, scansum, perm, permp, slot, refcell, xs, xs64, ts,
       perm2, sc_info, sc_col, colsc, sctr, shalf, sorg, ctr, half, entries, count, ecost, lcost, tep, tcp, tpos, tposS, wstart, maskwork, nmaskwork, masks, overflow, tiles, ntiles, tilectr, ljtab, ljt32, facc, fout,
-      pair_e, npairs, hash, eptr_d, elist_d, etab_d, corr_e, recip_e, eout, np_out, hash_out, grid64, gridfx, spec, spec2,
-      greal, theta, twx, twy, twz, border, nborder, border_acc;
+      pair_e, npairs, hash, eptr_d, elist_d, etab_d, corr_e, recip_e, eout, np_out, hash_out, pmw, pmb, tcol, spec, theta, twx, twy, twz, border, nborder, border_acc;
   int maxborder = 65536;
   // results
   long long last_np = 0;
@@ -130,8 +130,7 @@ struct Sys {
   bool have_positions = false;
   bool cached = false;
   bool list_valid = false;             // entries, counts and work of a built list are in place
-  bool acc_clean = false;              // force accumulators, PME grid and pass counters are zero
-  bool spread_ready = false;           // the grid holds the next pass's spread (fused into the last kick-drift)
+  bool acc_clean = false;              // force accumulators and pass counters are zero
   bool dry = false;                    // size only: allocations are counted, nothing runs
   unsigned long long dry_bytes = 0;
   double eout_h[4] = {0, 0, 0, 0};
@@ -160,6 +159,9 @@ struct Sys {
 };
 constexpr int kMaxChunk = 128;
 constexpr int kFixupMainBelow = 100000;  // atoms; default of PMX_TUNE_FIXUP_STREAM
+// Atoms from which the charge spread runs beside the pair kernel by default
+// (PMX_TUNE_SPREAD_STREAM): below, the PME chain is the longer branch.
+constexpr int kSpread2From = 10000;
 constexpr double kInvTimeFactor = 0.02045482828087295;  // protomol/base/PMConstants.cpp:54
 constexpr double kBoltzmann = 0.001987191;              // protomol/base/PMConstants.cpp:70
 
@@ -270,20 +272,41 @@ double choose_alpha(double rc, double acc) {
   return a;
 }
 
+// The transform of length n as a product of the kernels' radices: the fewest
+// passes (each costs two block barriers and a trip through LDS), and among
+// those the smallest largest radix.
 bool make_plan(int n, FftPlan &pl) {
-  pl.n = n;
-  pl.nrad = 0;
-  int m = n;
-  while (m % 4 == 0 && pl.nrad < 16) {
-    pl.rad[pl.nrad++] = 4;
-    m /= 4;
-  }
-  for (int r : {2, 3, 5})
-    while (m % r == 0 && pl.nrad < 16) {
-      pl.rad[pl.nrad++] = r;
-      m /= r;
+  static const int kRad[] = {10, 9, 8, 6, 5, 4, 3, 2};
+  int best[12], cur[12], nbest = 0;
+  auto search = [&](auto &self, int m, int depth) -> void {
+    if (m == 1) {
+      const int big = *std::max_element(cur, cur + depth), was = nbest ? *std::max_element(best, best + nbest) : 0;
+      if (!nbest || depth < nbest || (depth == nbest && big < was)) {
+        nbest = depth;
+        std::copy(cur, cur + depth, best);
+      }
+      return;
     }
-  return m == 1;
+    if (depth >= 12 || (nbest && depth >= nbest)) return;
+    for (int r : kRad)
+      if (m % r == 0 && (depth == 0 || r <= cur[depth - 1])) {
+        cur[depth] = r;
+        self(self, m / r, depth + 1);
+      }
+  };
+  pl = FftPlan{};
+  pl.n = n;
+  if (n < 2) return false;
+  search(search, n, 0);
+  pl.nrad = nbest;
+  pl.magic_n = div_magic((unsigned)n);
+  unsigned ns = 1;
+  for (int s = 0; s < nbest; ++s) {
+    pl.rad[s] = best[s];
+    pl.magic[s] = ns > 1 ? div_magic(ns) : 0u;
+    ns *= (unsigned)best[s];
+  }
+  return nbest > 0;
 }
 
 void bspline_host(int order, double w, double *th, double *dth) {
@@ -364,22 +387,97 @@ int validate(pmx_ctx *c, const pmx_sys_desc *d) {
   return PMX_OK;
 }
 
-// FFT blocking: lines per block, two LDS buffers of lines * n complex
-// within 24 KiB (so that FFT blocks fit beside the pair kernel's blocks,
-// which leave about that much LDS free on each CU), at most
-// tune_fft_lines lines (the transposed segments); one energy partial per
-// x-pass block.
+// Launch shapes of the PME passes.  Beside the pair kernel's four blocks a
+// CU has room for one more block of 256 threads (64 VGPRs a lane are left on
+// each SIMD) and about 38 KB of LDS, so the passes that run there stay within
+// that; a block of 512 threads would wait for the pair kernel's last blocks
+// (the y pass of a 216 x 240 x 240 grid took 0.70 ms that way, 0.1 ms so).
+//  - Tiles of the spread and gather passes: tx x ty lines along z.  Wider
+//    tiles repeat less of an atom's work (each tile that an atom's stencil
+//    touches visits it: (tx + p - 1)(ty + p - 1) / (tx ty) tiles) and write
+//    longer segments; the spread takes 8 x 4 where it has the device to
+//    itself and that still gives at least 4 tiles per CU.
+//  - y pass: 8 neighbouring lines (64- or 128-byte segments), x pass: 8
+//    (contiguous anyway), fewer while that leaves fewer than two blocks per
+//    CU; at most tune_fft_lines.
 int fft_blocking(Sys *s) {
-  const PmeParams &pm = s->pme;
-  const int cpx = s->mixed ? 8 : 16;
-  const int budget = 24576 / (2 * cpx);
-  const int lines = s->tune_fft_lines;
-  s->zl = std::max(1, std::min(lines, budget / pm.nz));
-  s->tky = std::max(1, std::min(lines, budget / pm.ny));
-  s->tkx = std::max(1, std::min(lines, budget / pm.nx));
-  s->fft_plane = s->tune_fft_planes && pm.nx * pm.ny <= kFftPlanePoints;
-  s->recip_blocks = s->fft_plane ? pm.nzh : pm.nzh * ((pm.ny + s->tkx - 1) / s->tkx);
-  return dalloc(s, s->recip_e, 8 * (size_t)s->recip_blocks);
+  PmeParams &pm = s->pme, &pg = s->pme_g;
+  const size_t cx = s->mixed ? 8 : 16;
+  const int small = 256 * kFftPerThread;  // points of a block of 256 threads
+  // the larger of the charge sums (16 bytes a point of two lines) and the
+  // transforms (a complex number), and the twiddles
+  auto lds = [&](const PmeParams &q, size_t per_point) {
+    return per_point * (size_t)(q.tx * q.ty / 2) * pme_line(q.nz, q.order) + cx * (q.nz + 1);
+  };
+  auto tiles = [&](PmeParams &q, int tx, size_t per_point, size_t most) {
+    q.tx = tx;
+    q.ty = 4;
+    while (q.tx * q.ty > 2 && lds(q, per_point) > most) {
+      if (q.tx > 4)
+        q.tx /= 2;
+      else if (q.ty > 1)
+        q.ty /= 2;
+      else
+        q.tx /= 2;
+    }
+    q.ntx = (q.nx + q.tx - 1) / q.tx;
+    q.nty = (q.ny + q.ty - 1) / q.ty;
+  };
+  pg = pm;
+  const bool wide = (long long)pm.nx * pm.ny >= 32ll * 4 * s->ctx->cus;
+  const bool alone = !s->tune_spread_stream2;
+  tiles(pg, wide ? 8 : 4, cx, 36864);
+  tiles(pm, wide ? 8 : 4, 16, alone ? 73728 : 36864);
+  s->lds_z = lds(pm, 16);
+  s->lds_g = lds(pg, cx);
+  auto lines = [&](int n, int other) {
+    int l = 0;
+    while (l < 3 && (2 << l) <= s->tune_fft_lines && ((long long)n << (l + 1)) <= small) ++l;
+    while (l > 0 && (1 << l) >= 2 * other) --l;
+    while (l > 2 && (long long)pm.nzh * ((other + (1 << l) - 1) >> l) < 2 * s->ctx->cus) --l;
+    return l;
+  };
+  s->ylog = lines(pm.ny, pm.nx);
+  s->xlog = lines(pm.nx, pm.ny);
+  s->lds_y = cx * (((size_t)(pm.ny | 1) << s->ylog) + pm.ny);
+  s->lds_x = cx * (((size_t)(pm.nx | 1) << s->xlog) + pm.nx);
+  s->lds_p = cx * ((size_t)(pm.nx | 1) * pm.ny + pm.nx + pm.ny);
+  // threads: a line needs n / kFftPerThread; the tiles and planes transform
+  // as many lines at a time as the block has threads for
+  auto threads = [&](int n, int l) { return ((long long)n << l) > small ? 512 : 256; };
+  s->thr_z = alone && wide ? 512 : threads(pm.nz, 0);
+  s->thr_g = threads(pm.nz, 0);
+  s->thr_y = threads(pm.ny, s->ylog);
+  s->thr_x = threads(pm.nx, s->xlog);
+  s->thr_p = threads(std::max(pm.nx, pm.ny), 0);
+  s->fft_plane = s->tune_fft_planes && pm.nx * pm.ny <= kFftPlanePoints && s->lds_p <= 36864;
+  s->recip_blocks = s->fft_plane ? pm.nzh : pm.nzh * ((pm.ny + (1 << s->xlog) - 1) >> s->xlog);
+  // the columns of the sort that can hold atoms whose stencils touch a row or
+  // column of tiles: places from the first base's to the last base's cell,
+  // widened by half the skin (an atom's way since the sort)
+  std::vector<int2> tc;
+  const double m = 0.5 * s->md.skin + 1e-3;
+  auto window = [&](int nt, int tl, int K, double L, int ncol) {
+    const int p = pm.order, back = (p - 1) / 2;
+    const double h = L / K, w = L / ncol;
+    for (int t = 0; t < nt; ++t) {
+      const double lo = (t * tl - p + 1 + back) * h - m, hi = (t * tl + tl + back) * h + m;
+      const long long a = (long long)std::floor(lo / w), b = (long long)std::floor(hi / w);
+      if (b - a + 1 >= ncol)
+        tc.push_back(make_int2(0, ncol));
+      else
+        tc.push_back(make_int2((int)(((a % ncol) + ncol) % ncol), (int)(b - a + 1)));
+    }
+  };
+  for (const PmeParams *q : {&pm, &pg}) {
+    window(q->ntx, q->tx, q->nx, s->box.L[0], q->ncx);
+    window(q->nty, q->ty, q->ny, s->box.L[1], q->ncy);
+  }
+  if (int rc = dalloc(s, s->tcol, 8 * tc.size())) return rc;
+  if (int rc = dalloc(s, s->recip_e, 8 * (size_t)s->recip_blocks)) return rc;
+  HIPCHK(hipMemcpyAsync(s->tcol.p, tc.data(), 8 * tc.size(), hipMemcpyHostToDevice, s->ctx->stream));
+  HIPCHK(hipStreamSynchronize(s->ctx->stream));
+  return PMX_OK;
 }
 
 template <bool MIXED>
@@ -599,13 +697,13 @@ int setup(Sys *s) {
   s->border_blocks = std::min(128, std::max(4, (int)(s->nsuper / 16)));
   if ((rc = A(s->corr_e, 8 * (size_t)s->corr_blocks))) return rc;
   if (s->dry) {
-    // PME buffers as allocated below (grid, half spectrum, real potential,
-    // influence table, twiddles, energy partials bounded by ny * nzh)
+    // PME buffers as allocated below (grid records, tile windows, half
+    // spectrum, influence table, twiddles, energy partials bounded by ny * nzh)
     if (s->pme_on) {
       const size_t nx = d.pme_grid[0], ny = d.pme_grid[1], nz = d.pme_grid[2], nzh = nz / 2 + 1;
-      const size_t G = nx * ny * nz, GH = nx * ny * nzh, cxb = s->mixed ? 8 : 16, rb = s->mixed ? 4 : 8;
-      for (size_t b : {8 * G, cxb * GH, cxb * GH, rb * G, rb * GH, cxb * nx, cxb * ny, cxb * nz, 8 * ny * nzh, (size_t)8,
-                       (size_t)8, (size_t)8, (size_t)8, (size_t)8})
+      const size_t GH = nx * ny * nzh, cxb = s->mixed ? 8 : 16, rb = s->mixed ? 4 : 8;
+      for (size_t b : {(s->mixed ? 16 : 32) * NP, 8 * NP, 4 * (nx + ny + 4), cxb * GH, rb * GH, cxb * nx, cxb * ny,
+                       cxb * nz, 8 * ny * nzh})
         s->dry_bytes += size_class(b);
     }
     return PMX_OK;
@@ -648,10 +746,13 @@ int setup(Sys *s) {
     pm.offz = -(pm.order - 1) / 2 + pm.nz;
     if (!make_plan(pm.nx, s->plx) || !make_plan(pm.ny, s->ply) || !make_plan(pm.nz, s->plz))
       return fail(s->ctx, PMX_ERR_UNSUPPORTED, "PME grid sizes must be products of 2, 3 and 5");
-    const size_t G = (size_t)pm.nx * pm.ny * pm.nz, GH = (size_t)pm.nx * pm.ny * pm.nzh;
+    if (std::max(pm.nx, std::max(pm.ny, pm.nz)) > kFftMax)
+      return fail(s->ctx, PMX_ERR_UNSUPPORTED, "PME grid axes have at most 4096 points");
+    pm.ncx = bp.ncx;
+    pm.ncy = bp.ncy;
+    const size_t GH = (size_t)pm.nx * pm.ny * pm.nzh;
     const size_t cxb = s->mixed ? 8 : 16;
-    if ((rc = A(s->grid64, s->mixed ? 8 : 8 * G)) || (rc = A(s->gridfx, s->mixed ? 8 * G : 8)) ||
-        (rc = A(s->spec, cxb * GH)) || (rc = A(s->spec2, cxb * GH)) || (rc = A(s->greal, (s->mixed ? 4 : 8) * G)) ||
+    if ((rc = A(s->pmw, (s->mixed ? 16 : 32) * NP)) || (rc = A(s->pmb, 8 * NP)) || (rc = A(s->spec, cxb * GH)) ||
         (rc = A(s->theta, (s->mixed ? 4 : 8) * GH)) || (rc = A(s->twx, cxb * pm.nx)) ||
         (rc = A(s->twy, cxb * pm.ny)) || (rc = A(s->twz, cxb * pm.nz)))
       return rc;
@@ -703,7 +804,7 @@ int setup(Sys *s) {
             double mk = k * Hr, m2 = mij + mk * mk;
             v = bxy * bzm[k] * exy * ez[k] / m2;
           }
-          th[((size_t)k * pm.ny + j) * pm.nx + i] = v;  // the x pass's layout [k][j][i]
+          th[((size_t)k * pm.ny + j) * pm.nx + i] = v;  // the spectrum's layout [k][j][i]
         }
       }
     }
@@ -894,109 +995,64 @@ void run_pair_phase(Sys *s, bool stats, int phase) {
   }
 }
 
-// Spreading and gathering for the stencil order ORDER (validated: even, 2..8).
-template <bool MIXED, int ORDER>
-void launch_spread(Sys *s, hipStream_t st) {
-  if (ORDER >= 4) {
-    hipLaunchKernelGGL((k_spread_patch<MIXED, ORDER>), dim3(nblk(s->npad, kSpreadSlots)), dim3(256), 0, st, s->npad,
-                       s->pme, P<double>(s->xorig), P<int>(s->permp), P<double>(s->q_d), P<double>(s->grid64),
-                       P<unsigned long long>(s->gridfx));
-    return;
-  }
-  constexpr int P3 = ORDER * ORDER * ORDER;
-  constexpr int apw = P3 >= 64 ? 1 : 64 / P3;
-  const int waves = (int)nblk(s->npad, apw);
-  hipLaunchKernelGGL((k_spread<MIXED, ORDER>), dim3(nblk((long long)waves * 64, 256)), dim3(256), 0, st, s->npad,
-                     s->pme, P<double>(s->xorig), P<int>(s->permp), P<double>(s->q_d), P<double>(s->grid64),
-                     P<unsigned long long>(s->gridfx));
+// The atoms' grid records, for the kernels that write them (null without PME).
+template <class R>
+PmeSlots<R> pme_slots(Sys *s) {
+  if (!s->pme_on || !(s->d.pme_terms & PMX_PME_RECIP)) return PmeSlots<R>{nullptr, nullptr};
+  return PmeSlots<R>{P<typename Real4<R>::type>(s->pmw), P<int2>(s->pmb)};
 }
 
-template <bool MIXED, int ORDER>
-void launch_gather(Sys *s, hipStream_t st) {
-  using T = typename std::conditional<MIXED, float, double>::type;
-  if (ORDER >= 4) {
-    hipLaunchKernelGGL((k_gather_patch<MIXED, ORDER>), dim3(nblk(s->npad, kSpreadSlots)), dim3(256), 0, st, s->npad,
-                       s->pme, P<double>(s->xorig), P<int>(s->permp), P<double>(s->q_d), P<T>(s->greal),
-                       P<typename AccT<MIXED>::type>(s->facc));
-    return;
-  }
-  const int waves = (int)nblk(s->npad, 64 / pme_tpa(ORDER));
-  hipLaunchKernelGGL((k_gather<MIXED, ORDER>), dim3(nblk((long long)waves * 64, 256)), dim3(256), 0, st, s->npad,
-                     waves,
-                     s->pme, P<double>(s->xorig), P<int>(s->permp), P<double>(s->q_d), P<T>(s->greal),
-                     P<typename AccT<MIXED>::type>(s->facc));
-}
-
-// The fused unsort + kick + drift + next spread (orders 4 to 8).
-template <bool MIXED>
-void launch_unsort_kick_drift_spread(Sys *s, const Kick &kk, unsigned *dmax) {
-  using R = typename std::conditional<MIXED, float, double>::type;
-  using R4 = typename Real4<R>::type;
-  hipStream_t st = s->ctx->stream;
-#define PMX_UKDS(ORD)                                                                                              \
-  hipLaunchKernelGGL((k_unsort_kick_drift_spread<MIXED, R, ORD>), dim3(nblk(s->npad, kSpreadSlots)), dim3(256), 0, \
-                     st, s->npad, kk, s->md.h, P<int>(s->permp), P<typename AccT<MIXED>::type>(s->facc),           \
-                     P<double>(s->fout), P<int>(s->tilectr), P<int>(s->nborder), P<double>(s->md.minv),             \
-                     P<double>(s->md.v), P<double>(s->xorig), P<double>(s->md.xbuild), P<R4>(s->xs),                \
-                     P<double4>(s->xs64), P<float4>(s->sorg), dmax, s->pme, P<double>(s->q_d),                      \
-                     P<double>(s->grid64), P<unsigned long long>(s->gridfx))
-  switch (s->pme.order) {
-    case 4: PMX_UKDS(4); break;
-    case 6: PMX_UKDS(6); break;
-    default: PMX_UKDS(8); break;
-  }
-#undef PMX_UKDS
-}
-
-// Charge spreading on the main stream (before the pair kernel: alone it
-// runs at full rate, next to the pair kernel its many small waves would
-// not); the charge grid was zeroed by the k_zero launch of the pass.
+// Charge spread with the z transform (order: even, 2..8).
 template <bool MIXED>
 void run_spread(Sys *s, hipStream_t st) {
+  using T = typename std::conditional<MIXED, float, double>::type;
+  using T4 = typename Real4<T>::type;
+#define PMX_SPREAD(ORD)                                                                                              \
+  hipLaunchKernelGGL((k_pme_spread_z<MIXED, ORD>), dim3(s->pme.ntx * s->pme.nty), dim3(s->thr_z), s->lds_z, st,      \
+                     s->pme, s->plz, P<int2>(s->tcol), P<int>(s->colsc), P<T4>(s->pmw), P<int2>(s->pmb),              \
+                     P<Cx<T>>(s->twz), P<Cx<T>>(s->spec))
   switch (s->pme.order) {
-    case 2: launch_spread<MIXED, 2>(s, st); break;
-    case 4: launch_spread<MIXED, 4>(s, st); break;
-    case 6: launch_spread<MIXED, 6>(s, st); break;
-    default: launch_spread<MIXED, 8>(s, st); break;
+    case 2: PMX_SPREAD(2); break;
+    case 4: PMX_SPREAD(4); break;
+    case 6: PMX_SPREAD(6); break;
+    default: PMX_SPREAD(8); break;
   }
+#undef PMX_SPREAD
 }
 
-// FFT convolution and force gather on the second stream.
+// The transforms and the force gather on the second stream.
 template <bool MIXED>
 int run_pme(Sys *s, bool timing) {
   using T = typename std::conditional<MIXED, float, double>::type;
+  using T4 = typename Real4<T>::type;
+  using Acc = typename AccT<MIXED>::type;
   hipStream_t st = s->ctx->stream2;
-  const PmeParams &pm = s->pme;
+  const PmeParams &pm = s->pme, &pg = s->pme_g;
   if (s->d.pme_terms & PMX_PME_RECIP) {
-    const size_t cx = sizeof(Cx<T>);
-    // z pass per (i, TY lines of j), y passes per (k, TI lines of i), x pass
-    // per (k, TJ lines of j)
-    const int zb = pm.nx * ((pm.ny + s->zl - 1) / s->zl);
-    const int yb = pm.nzh * ((pm.nx + s->tky - 1) / s->tky);
-    hipLaunchKernelGGL((k_fft_z_r2c<T, MIXED>), dim3(zb), dim3(256), 2 * s->zl * pm.nz * cx, st, pm, s->plz, s->zl,
-                       P<double>(s->grid64), P<unsigned long long>(s->gridfx), P<Cx<T>>(s->twz), P<Cx<T>>(s->spec));
     if (s->fft_plane) {
-      hipLaunchKernelGGL((k_fft_plane_conv<T>), dim3(pm.nzh), dim3(256), 2 * (size_t)pm.nx * pm.ny * cx, st, pm,
-                         s->ply, s->plx, P<Cx<T>>(s->twy), P<Cx<T>>(s->twx), P<T>(s->theta), P<Cx<T>>(s->spec),
-                         P<double>(s->recip_e));
+      hipLaunchKernelGGL((k_fft_plane_conv<T>), dim3(pm.nzh), dim3(s->thr_p), s->lds_p, st, pm, s->ply, s->plx,
+                         P<Cx<T>>(s->twy), P<Cx<T>>(s->twx), P<T>(s->theta), P<Cx<T>>(s->spec), P<double>(s->recip_e));
     } else {
-      hipLaunchKernelGGL((k_fft_y<T>), dim3(yb), dim3(256), 2 * s->tky * pm.ny * cx, st, pm, s->ply, s->tky, false,
-                         P<Cx<T>>(s->twy), P<Cx<T>>(s->spec), P<Cx<T>>(s->spec2));
-      hipLaunchKernelGGL((k_fft_x_conv<T>), dim3(s->recip_blocks), dim3(256), 2 * s->tkx * pm.nx * cx, st, pm,
-                         s->plx, s->tkx, P<Cx<T>>(s->twx), P<T>(s->theta), P<Cx<T>>(s->spec2),
-                         P<double>(s->recip_e));
-      hipLaunchKernelGGL((k_fft_y<T>), dim3(yb), dim3(256), 2 * s->tky * pm.ny * cx, st, pm, s->ply, s->tky, true,
-                         P<Cx<T>>(s->twy), P<Cx<T>>(s->spec2), P<Cx<T>>(s->spec));
+      const int yb = pm.nzh * ((pm.nx + (1 << s->ylog) - 1) >> s->ylog);
+      hipLaunchKernelGGL((k_fft_y<T>), dim3(yb), dim3(s->thr_y), s->lds_y, st, pm, s->ply, s->ylog, false,
+                         P<Cx<T>>(s->twy), P<Cx<T>>(s->spec));
+      hipLaunchKernelGGL((k_fft_x_conv<T>), dim3(s->recip_blocks), dim3(s->thr_x), s->lds_x, st, pm, s->plx, s->xlog,
+                         P<Cx<T>>(s->twx), P<T>(s->theta), P<Cx<T>>(s->spec), P<double>(s->recip_e));
+      hipLaunchKernelGGL((k_fft_y<T>), dim3(yb), dim3(s->thr_y), s->lds_y, st, pm, s->ply, s->ylog, true,
+                         P<Cx<T>>(s->twy), P<Cx<T>>(s->spec));
     }
-    hipLaunchKernelGGL((k_fft_z_c2r<T>), dim3(zb), dim3(256), 2 * s->zl * pm.nz * cx, st, pm, s->plz, s->zl,
-                       P<Cx<T>>(s->twz), P<Cx<T>>(s->spec), P<T>(s->greal));
     if (timing) hipEventRecord(s->ev[5], st);
+#define PMX_GATHER(ORD)                                                                                              \
+  hipLaunchKernelGGL((k_pme_z_gather<MIXED, ORD>), dim3(pg.ntx * pg.nty), dim3(s->thr_g), s->lds_g, st, pg, s->plz, \
+                     P<int2>(s->tcol) + pm.ntx + pm.nty, P<int>(s->colsc), P<T4>(s->pmw), P<int2>(s->pmb), P<Cx<T>>(s->twz),           \
+                     P<Cx<T>>(s->spec), P<Acc>(s->facc))
     switch (pm.order) {
-      case 2: launch_gather<MIXED, 2>(s, st); break;
-      case 4: launch_gather<MIXED, 4>(s, st); break;
-      case 6: launch_gather<MIXED, 6>(s, st); break;
-      default: launch_gather<MIXED, 8>(s, st); break;
+      case 2: PMX_GATHER(2); break;
+      case 4: PMX_GATHER(4); break;
+      case 6: PMX_GATHER(6); break;
+      default: PMX_GATHER(8); break;
     }
+#undef PMX_GATHER
   } else if (timing) {
     hipEventRecord(s->ev[5], st);
   }
@@ -1069,13 +1125,13 @@ int rebuild(Sys *s, bool timing) {
                        P<int2>(s->sc_info), P<int>(s->perm2), P<double>(s->xwrap), P<int>(s->permp), P<int>(s->slot),
                        P<double>(s->q_d), P<int>(s->type_d), P<float4>(s->xs), P<double4>(s->xs64), P<int>(s->ts),
                        P<double>(s->xorig), xbuild, P<float4>(s->sorg), P<float4>(s->ctr), P<float4>(s->half),
-                       P<float4>(s->sctr), P<float4>(s->shalf), P<int>(s->nmaskwork), s->qpair);
+                       P<float4>(s->sctr), P<float4>(s->shalf), P<int>(s->nmaskwork), s->qpair, s->pme, pme_slots<float>(s));
   else
     hipLaunchKernelGGL(k_split_fill<double>, dim3(nblk((long long)s->nsuper * 64, 256)), dim3(256), 0, st, s->nsuper,
                        P<int2>(s->sc_info), P<int>(s->perm2), P<double>(s->xwrap), P<int>(s->permp), P<int>(s->slot),
                        P<double>(s->q_d), P<int>(s->type_d), P<double4>(s->xs), P<double4>(s->xs64), P<int>(s->ts),
                        P<double>(s->xorig), xbuild, P<float4>(s->sorg), P<float4>(s->ctr), P<float4>(s->half),
-                       P<float4>(s->sctr), P<float4>(s->shalf), P<int>(s->nmaskwork), s->qpair);
+                       P<float4>(s->sctr), P<float4>(s->shalf), P<int>(s->nmaskwork), s->qpair, s->pme, pme_slots<double>(s));
   if (timing) hipEventRecord(s->ev[1], st);
   hipLaunchKernelGGL(k_build_list, dim3(s->nsuper), dim3(kListBlock), 0, st, s->lp, P<int>(s->sc_col),
                      P<int>(s->colsc), P<float4>(s->sctr), P<float4>(s->shalf), P<float4>(s->ctr),
@@ -1106,7 +1162,7 @@ int rebuild(Sys *s, bool timing) {
 // next: the following MD step's kick (with next_dmax, its displacement
 // record): the pass ends with that step's kick and drift fused into the
 // force unsort.
-// Clears the force accumulators, the pass counters and the PME charge grid.
+// Clears the force accumulators and the pass counters.
 void launch_zero(Sys *s) {
   const int npad = s->npad;
   ZeroRanges z{};
@@ -1119,27 +1175,17 @@ void launch_zero(Sys *s) {
   z.n[nr++] = 1;
   z.p[nr] = P<unsigned long long>(s->border_acc);
   z.n[nr++] = 4;
-  if (s->pme_on && (s->d.pme_terms & PMX_PME_RECIP)) {
-    const long long G = (long long)s->pme.nx * s->pme.ny * s->pme.nz;
-    z.p[nr] = s->mixed ? P<unsigned long long>(s->gridfx) : P<unsigned long long>(s->grid64);
-    z.n[nr++] = G;
-  }
   hipLaunchKernelGGL(k_zero, dim3(std::max(1u, nblk(3ll * npad, 256)), nr), dim3(256), 0, s->ctx->stream, z);
 }
 
-int forces(Sys *s, unsigned flags, bool energies, const Kick *next = nullptr, unsigned *next_dmax = nullptr,
-           bool spread_done = false) {
+int forces(Sys *s, unsigned flags, bool energies, const Kick *next = nullptr, unsigned *next_dmax = nullptr) {
   hipStream_t st = s->ctx->stream;
   const bool timing = flags & PMX_EVAL_TIMING;
   const bool stats = flags & PMX_EVAL_PAIRSTATS;
   const int n = s->n, npad = s->npad;
-  // A completed pass leaves the accumulators, the PME grid and the counters
-  // cleared (k_unsort_forces, k_fft_z_r2c, k_pair); only the first pass after
-  // (re)allocation or after an interrupted pass clears them here.  A spread
-  // fused into the previous kick-drift is this pass's only when the caller
-  // says so; otherwise it belongs to other positions and is cleared.
-  if (s->spread_ready && !spread_done) s->acc_clean = false;
-  s->spread_ready = false;
+  // A completed pass leaves the accumulators and the counters cleared
+  // (k_unsort_forces, k_pair); only the first pass after (re)allocation or
+  // after an interrupted pass clears them here.
   if (!s->acc_clean) launch_zero(s);
   s->acc_clean = false;
   if (timing) hipEventRecord(s->ev[2], st);
@@ -1151,7 +1197,7 @@ int forces(Sys *s, unsigned flags, bool energies, const Kick *next = nullptr, un
   hipStream_t st2 = s->ctx->stream2;
   const bool spread = s->pme_on && (s->d.pme_terms & PMX_PME_RECIP);
   const bool spread2 = spread && s->tune_spread_stream2;
-  if (spread && !spread2 && !spread_done) {
+  if (spread && !spread2) {
     if (s->mixed)
       run_spread<true>(s, st);
     else
@@ -1196,26 +1242,18 @@ int forces(Sys *s, unsigned flags, bool energies, const Kick *next = nullptr, un
   else
     run_pair_phase<false>(s, stats, fix_phase);
   HIPCHK(hipStreamWaitEvent(st, s->join_ev, 0));
-  // inside an MD chunk the next pass's spread joins the kick-drift
-  const bool fuse_spread = next && spread && !spread2 && s->pme.order >= 4 && s->tune_fused_spread;
-  if (fuse_spread) {
-    if (s->mixed)
-      launch_unsort_kick_drift_spread<true>(s, *next, next_dmax);
-    else
-      launch_unsort_kick_drift_spread<false>(s, *next, next_dmax);
-    s->spread_ready = true;
-  } else if (next && s->mixed)
+  if (next && s->mixed)
     hipLaunchKernelGGL((k_unsort_kick_drift<true, float>), dim3(nblk(npad, 256)), dim3(256), 0, st, npad, *next,
                        s->md.h, P<int>(s->permp), P<unsigned long long>(s->facc), P<double>(s->fout),
                        P<int>(s->tilectr), P<int>(s->nborder), P<double>(s->md.minv), P<double>(s->md.v),
                        P<double>(s->xorig), P<double>(s->md.xbuild), P<float4>(s->xs), P<double4>(s->xs64),
-                       P<float4>(s->sorg), next_dmax);
+                       P<float4>(s->sorg), next_dmax, s->pme, pme_slots<float>(s));
   else if (next)
     hipLaunchKernelGGL((k_unsort_kick_drift<false, double>), dim3(nblk(npad, 256)), dim3(256), 0, st, npad, *next,
                        s->md.h, P<int>(s->permp), P<double>(s->facc), P<double>(s->fout), P<int>(s->tilectr),
                        P<int>(s->nborder), P<double>(s->md.minv), P<double>(s->md.v), P<double>(s->xorig),
                        P<double>(s->md.xbuild), P<double4>(s->xs), P<double4>(s->xs64), P<float4>(s->sorg),
-                       next_dmax);
+                       next_dmax, s->pme, pme_slots<double>(s));
   else if (s->mixed)
     hipLaunchKernelGGL(k_unsort_forces<true>, dim3(nblk(n, 256)), dim3(256), 0, st, n, P<int>(s->slot),
                        P<unsigned long long>(s->facc), P<double>(s->fout), P<int>(s->tilectr),
@@ -1368,6 +1406,7 @@ int pmx_sys_create(pmx_ctx *ctx, const pmx_sys_desc *desc, pmx_sys **out) {
   // below this size the PME chain (a fixed number of short dependent
   // launches) is the longer branch of a force pass
   ps->s.tune_fixup_main = desc->n < kFixupMainBelow ? 1 : 0;
+  ps->s.tune_spread_stream2 = desc->n >= kSpread2From ? 1 : 0;
   rc = setup(&ps->s);
   if (rc) {
     pmx_sys_destroy(ps);
@@ -1620,8 +1659,9 @@ int pmx_sys_set_tuning(pmx_sys *sys, int knob, int value) {
       s->tune_fixup_main = value;
       break;
     case PMX_TUNE_FUSED_SPREAD:
+      // kept for callers that set it: the spread has no launch of its own
+      // that could be fused
       if (value < 0 || value > 1) return fail(s->ctx, PMX_ERR_ARG, "fused spread must be 0 or 1");
-      s->tune_fused_spread = value;
       break;
     case PMX_TUNE_FFT_PLANES:
       if (value < 0 || value > 1) return fail(s->ctx, PMX_ERR_ARG, "FFT planes must be 0 or 1");
@@ -1631,7 +1671,7 @@ int pmx_sys_set_tuning(pmx_sys *sys, int knob, int value) {
       return fail(s->ctx, PMX_ERR_ARG, "unknown tuning knob");
   }
   // captured chunks hold the old launch shapes; the energy partials of the
-  // x pass may be reallocated
+  // x pass may be reallocated, and the tile windows change
   hipSetDevice(s->ctx->device);
   HIPCHK(hipStreamSynchronize(s->ctx->stream));
   HIPCHK(hipStreamSynchronize(s->ctx->stream2));
@@ -1832,12 +1872,12 @@ int md_step(Sys *s, double kick, long long step, bool rebuild_here, int dslot,
     hipLaunchKernelGGL(k_kick_drift<float>, dim3(nblk(s->npad, 256)), dim3(256), 0, st, s->npad, kk, m.h,
                        P<int>(s->permp), P<double>(s->fout), P<double>(m.minv), P<double>(m.v), P<double>(s->xorig),
                        P<double>(m.xbuild), P<float4>(s->xs), P<double4>(s->xs64),
-                       P<float4>(s->sorg), P<unsigned>(m.dmax) + dslot);
+                       P<float4>(s->sorg), P<unsigned>(m.dmax) + dslot, s->pme, pme_slots<float>(s));
   else
     hipLaunchKernelGGL(k_kick_drift<double>, dim3(nblk(s->npad, 256)), dim3(256), 0, st, s->npad, kk, m.h,
                        P<int>(s->permp), P<double>(s->fout), P<double>(m.minv), P<double>(m.v), P<double>(s->xorig),
                        P<double>(m.xbuild), P<double4>(s->xs), P<double4>(s->xs64),
-                       P<float4>(s->sorg), P<unsigned>(m.dmax) + dslot);
+                       P<float4>(s->sorg), P<unsigned>(m.dmax) + dslot, s->pme, pme_slots<double>(s));
   if (rebuild_here) {
     int rc = rebuild(s, timing);
     if (rc) return rc;
@@ -1845,10 +1885,7 @@ int md_step(Sys *s, double kick, long long step, bool rebuild_here, int dslot,
     hipEventRecord(s->ev[1], st);
     hipEventRecord(s->ev[2], st);
   }
-  // the previous pass's kick-drift spread these positions when it was fused
-  const bool spread_done = kicked && s->spread_ready;
-  return forces(s, timing ? PMX_EVAL_TIMING : 0u, false, next, next ? P<unsigned>(m.dmax) + next_dslot : nullptr,
-                spread_done);
+  return forces(s, timing ? PMX_EVAL_TIMING : 0u, false, next, next ? P<unsigned>(m.dmax) + next_dslot : nullptr);
 }
 
 // A chunk of K steps from the committed state: its state is backed up in
@@ -2141,6 +2178,7 @@ struct BatchLaunch {
   BatchBuf tab, first, b2s;
   unsigned blocks = 0;
   size_t lds = 0;
+  int threads = 0;  // block size (0: the op's kBlock)
 };
 
 struct Batch {
@@ -2148,7 +2186,7 @@ struct Batch {
   std::vector<Sys *> sys;
   int nsys = 0;
   BatchLaunch bin, scan, scatter, binrank, columns, split, list, excl, masks, rprefix, rcut, rtiles;
-  BatchLaunch kick, spread, pair, zr2c, yfwd, xconv, yinv, plane, zc2r, gather, fixups, ukds, unsort, begin, half;
+  BatchLaunch kick, spread, pair, yfwd, xconv, yinv, plane, gather, fixups, ukd, unsort, begin, half;
   BatchLaunch energy;
   BatchBuf bsys, need, base, flags, rebuilds;
   // slices of the context's pinned staging, and its events
@@ -2162,7 +2200,7 @@ struct Batch {
 // system s; dynamic LDS `lds`).
 template <class Op>
 int batch_table(Batch &b, BatchLaunch &L, const std::vector<typename Op::Args> &args,
-                const std::vector<int> &nblocks, size_t lds = 0) {
+                const std::vector<int> &nblocks, size_t lds = 0, int threads = 0) {
   std::vector<int> first(b.nsys + 1, 0);
   for (int i = 0; i < b.nsys; ++i) first[i + 1] = first[i] + nblocks[i];
   std::vector<int> b2s(std::max(1, first[b.nsys]));
@@ -2170,6 +2208,7 @@ int batch_table(Batch &b, BatchLaunch &L, const std::vector<typename Op::Args> &
     for (int k = first[i]; k < first[i + 1]; ++k) b2s[k] = i;
   L.blocks = (unsigned)first[b.nsys];
   L.lds = lds;
+  L.threads = threads ? threads : Op::kBlock;
   const int dev = b.ctx->device;
   if (!L.tab.get(dev, sizeof(typename Op::Args) * args.size()) || !L.first.get(dev, 4 * first.size()) ||
       !L.b2s.get(dev, 4 * b2s.size()))
@@ -2184,7 +2223,7 @@ int batch_table(Batch &b, BatchLaunch &L, const std::vector<typename Op::Args> &
 template <class Op>
 void batch_go(const BatchLaunch &L, hipStream_t st, const BatchStep &bs) {
   if (!L.blocks) return;
-  hipLaunchKernelGGL(k_batch<Op>, dim3(L.blocks), dim3(Op::kBlock), L.lds, st,
+  hipLaunchKernelGGL(k_batch<Op>, dim3(L.blocks), dim3(L.threads), L.lds, st,
                      reinterpret_cast<const typename Op::Args *>(L.tab.p), reinterpret_cast<const int *>(L.b2s.p),
                      reinterpret_cast<const int *>(L.first.p), bs);
 }
@@ -2258,6 +2297,8 @@ int batch_tables(Batch &b) {
       sp.shalf = P<float4>(s->shalf);
       sp.nmaskwork = P<int>(s->nmaskwork);
       sp.qpair = s->qpair;
+      sp.pme = s->pme;
+      sp.rec = pme_slots<R>(s);
       args_list[i] = {s->lp, P<int>(s->sc_col), P<int>(s->colsc), P<float4>(s->sctr), P<float4>(s->shalf),
                       P<float4>(s->ctr), P<float4>(s->half), P<int4>(s->entries), P<int>(s->count),
                       P<int>(s->ecost), P<int>(s->lcost), P<int>(s->maskwork), P<int>(s->nmaskwork),
@@ -2297,23 +2338,22 @@ int batch_tables(Batch &b) {
   }
   {
     std::vector<typename OpKickDrift<R>::Args> args_kick(ns);
-    std::vector<typename OpSpreadPatch<MIXED, ORDER>::Args> args_spread(ns);
+    std::vector<typename OpPmeSpreadZ<MIXED, ORDER>::Args> args_spread(ns);
     std::vector<typename PairOp<MIXED, C, LJ, CS, BIGLJ, ORDER>::Args> args_pair(ns);
-    std::vector<typename OpFftZr2c<T, MIXED>::Args> args_zr2c(ns);
     std::vector<typename OpFftY<T>::Args> args_yfwd(ns), args_yinv(ns);
     std::vector<typename OpFftXConv<T>::Args> args_xconv(ns);
     std::vector<typename OpFftPlane<T>::Args> args_plane(ns);
-    std::vector<typename OpFftZc2r<T>::Args> args_zc2r(ns);
-    std::vector<typename OpGatherPatch<MIXED, ORDER>::Args> args_gather(ns);
+    std::vector<typename OpPmeZGather<MIXED, ORDER>::Args> args_gather(ns);
     std::vector<FixupArgs<MIXED>> args_fixups(ns);
-    std::vector<typename OpUnsortKickDriftSpread<MIXED, R, ORDER>::Args> args_ukds(ns);
+    std::vector<typename OpUnsortKickDrift<MIXED, R>::Args> args_ukd(ns);
     std::vector<typename OpUnsortForces<MIXED>::Args> args_unsort(ns);
     std::vector<OpChunkBegin::Args> args_begin(ns);
     std::vector<OpHalfKick::Args> args_half(ns);
     std::vector<OpReduceEnergy::Args> args_energy(ns);
     std::vector<int> nfix(ns);
     long long natoms = 0;
-    size_t lds_z = 0, lds_y = 0, lds_x = 0, lds_p = 0;
+    size_t lds_z = 0, lds_g = 0, lds_y = 0, lds_x = 0, lds_p = 0;
+    int thr_z = 256, thr_g = 256, thr_y = 256, thr_x = 256, thr_p = 256;
     for (int i = 0; i < ns; ++i) {
       Sys *s = b.sys[i];
       Sys::Md &m = s->md;
@@ -2322,9 +2362,9 @@ int batch_tables(Batch &b) {
       Acc *facc = P<Acc>(s->facc);
       args_kick[i] = {s->npad, kk, m.h, P<int>(s->permp), P<double>(s->fout), P<double>(m.minv), P<double>(m.xbuild),
                       P<double>(m.v), P<double>(s->xorig), P<R4>(s->xs), P<double4>(s->xs64), P<float4>(s->sorg),
-                      P<unsigned>(m.dmax)};
-      args_spread[i] = {s->npad, s->pme, P<double>(s->xorig), P<double>(s->q_d), P<int>(s->permp),
-                        P<double>(s->grid64), P<unsigned long long>(s->gridfx)};
+                      P<unsigned>(m.dmax), s->pme, pme_slots<R>(s)};
+      args_spread[i] = {s->pme, s->plz, P<int2>(s->tcol), P<int>(s->colsc), P<R4>(s->pmw), P<int2>(s->pmb),
+                        P<Cx<T>>(s->twz), P<Cx<T>>(s->spec)};
       const R4 *ljt = MIXED ? reinterpret_cast<const R4 *>(s->ljt32.p) : reinterpret_cast<const R4 *>(s->ljtab.p);
       args_pair[i] = {s->pp, P<int4>(s->tiles), P<int>(s->ntiles), P<int>(s->wstart), P<int>(s->tilectr),
                       P<int4>(s->entries), s->cap, P<unsigned short>(s->masks), P<R4>(s->xs), P<float4>(s->sorg),
@@ -2333,21 +2373,18 @@ int batch_tables(Batch &b) {
                               P<int2>(s->border), P<int>(s->nborder), s->maxborder, P<int>(s->overflow),
                               P<unsigned long long>(s->border_acc)}};
       const PmeParams &pm = s->pme;
-      args_zr2c[i] = {pm, s->plz, s->zl, P<double>(s->grid64), P<unsigned long long>(s->gridfx), P<Cx<T>>(s->twz),
-                      P<Cx<T>>(s->spec)};
-      args_yfwd[i] = {pm, s->ply, s->tky, false, P<Cx<T>>(s->twy), P<Cx<T>>(s->spec), P<Cx<T>>(s->spec2)};
-      args_xconv[i] = {pm, s->plx, s->tkx, P<Cx<T>>(s->twx), P<T>(s->theta), P<Cx<T>>(s->spec2),
+      args_yfwd[i] = {pm, s->ply, s->ylog, false, P<Cx<T>>(s->twy), P<Cx<T>>(s->spec)};
+      args_xconv[i] = {pm, s->plx, s->xlog, s->thr_x, P<Cx<T>>(s->twx), P<T>(s->theta), P<Cx<T>>(s->spec),
                        P<double>(s->recip_e)};
-      args_yinv[i] = {pm, s->ply, s->tky, true, P<Cx<T>>(s->twy), P<Cx<T>>(s->spec2), P<Cx<T>>(s->spec)};
-      args_plane[i] = {pm, s->ply, s->plx, P<Cx<T>>(s->twy), P<Cx<T>>(s->twx), P<T>(s->theta), P<Cx<T>>(s->spec),
+      args_yinv[i] = {pm, s->ply, s->ylog, true, P<Cx<T>>(s->twy), P<Cx<T>>(s->spec)};
+      args_plane[i] = {pm, s->ply, s->plx, s->thr_p, P<Cx<T>>(s->twy), P<Cx<T>>(s->twx), P<T>(s->theta), P<Cx<T>>(s->spec),
                        P<double>(s->recip_e)};
-      args_zc2r[i] = {pm, s->plz, s->zl, P<Cx<T>>(s->twz), P<Cx<T>>(s->spec), P<T>(s->greal)};
-      args_gather[i] = {s->npad, pm, P<double>(s->xorig), P<double>(s->q_d), P<int>(s->permp), P<T>(s->greal), facc};
+      args_gather[i] = {s->pme_g, s->plz, P<int2>(s->tcol) + pm.ntx + pm.nty, P<int>(s->colsc), P<R4>(s->pmw), P<int2>(s->pmb),
+                        P<Cx<T>>(s->twz), P<Cx<T>>(s->spec), facc};
       args_fixups[i] = fixup_args<MIXED>(s, false, true, true, &nfix[i]);
-      args_ukds[i] = {s->npad, kk, m.h, P<int>(s->permp), facc, P<double>(s->fout), P<int>(s->tilectr),
-                      P<int>(s->nborder), P<double>(m.minv), P<double>(m.xbuild), P<double>(s->q_d), P<double>(m.v),
-                      P<double>(s->xorig), P<R4>(s->xs), P<double4>(s->xs64), P<float4>(s->sorg),
-                      P<unsigned>(m.dmax), pm, P<double>(s->grid64), P<unsigned long long>(s->gridfx)};
+      args_ukd[i] = {s->npad, kk, m.h, P<int>(s->permp), facc, P<double>(s->fout), P<int>(s->tilectr),
+                     P<int>(s->nborder), P<double>(m.minv), P<double>(m.xbuild), P<double>(m.v), P<double>(s->xorig),
+                     P<R4>(s->xs), P<double4>(s->xs64), P<float4>(s->sorg), P<unsigned>(m.dmax), pm, pme_slots<R>(s)};
       args_unsort[i] = {s->n, P<int>(s->slot), facc, P<double>(s->fout), P<int>(s->tilectr), P<int>(s->nborder)};
       args_begin[i] = {3ll * s->n, P<double>(s->xorig), P<double>(m.v), P<double>(s->fout), P<double>(m.xbak),
                        P<double>(m.vbak), P<double>(m.fbak), P<int>(s->overflow), P<unsigned>(m.dmax), kMaxChunk};
@@ -2359,21 +2396,29 @@ int batch_tables(Batch &b) {
                         P<double>(s->corr_e), P<long long>(s->npairs), P<unsigned long long>(s->hash),
                         P<unsigned long long>(s->border_acc), P<unsigned long long>(s->border_acc) + 2,
                         P<double>(s->eout), P<long long>(s->np_out), P<unsigned long long>(s->hash_out)};
-      // dynamic LDS of each launch: the largest of the systems it serves
-      lds_z = std::max(lds_z, 2 * (size_t)s->zl * pm.nz * cx);
+      // dynamic LDS and block size of each launch: the largest of the
+      // systems it serves
+      thr_z = std::max(thr_z, s->thr_z);
+      thr_g = std::max(thr_g, s->thr_g);
+      lds_g = std::max(lds_g, s->lds_g);
+      lds_z = std::max(lds_z, s->lds_z);
       if (s->fft_plane) {
-        lds_p = std::max(lds_p, 2 * (size_t)pm.nx * pm.ny * cx);
+        lds_p = std::max(lds_p, s->lds_p);
+        thr_p = std::max(thr_p, s->thr_p);
       } else {
-        lds_y = std::max(lds_y, 2 * (size_t)s->tky * pm.ny * cx);
-        lds_x = std::max(lds_x, 2 * (size_t)s->tkx * pm.nx * cx);
+        lds_y = std::max(lds_y, s->lds_y);
+        lds_x = std::max(lds_x, s->lds_x);
+        thr_y = std::max(thr_y, s->thr_y);
+        thr_x = std::max(thr_x, s->thr_x);
       }
     }
     for (int i = 0; i < ns; ++i) nb[i] = (int)nblk(b.sys[i]->npad, 256);
     if ((rc = batch_table<OpKickDrift<R>>(b, b.kick, args_kick, nb, 0))) return rc;
-    for (int i = 0; i < ns; ++i) nb[i] = (int)nblk(b.sys[i]->npad, kSpreadSlots);
-    if ((rc = batch_table<OpSpreadPatch<MIXED, ORDER>>(b, b.spread, args_spread, nb, 0))) return rc;
-    if ((rc = batch_table<OpGatherPatch<MIXED, ORDER>>(b, b.gather, args_gather, nb, 0))) return rc;
-    if ((rc = batch_table<OpUnsortKickDriftSpread<MIXED, R, ORDER>>(b, b.ukds, args_ukds, nb, 0))) return rc;
+    if ((rc = batch_table<OpUnsortKickDrift<MIXED, R>>(b, b.ukd, args_ukd, nb, 0))) return rc;
+    for (int i = 0; i < ns; ++i) nb[i] = b.sys[i]->pme.ntx * b.sys[i]->pme.nty;
+    if ((rc = batch_table<OpPmeSpreadZ<MIXED, ORDER>>(b, b.spread, args_spread, nb, lds_z, thr_z))) return rc;
+    for (int i = 0; i < ns; ++i) nb[i] = b.sys[i]->pme_g.ntx * b.sys[i]->pme_g.nty;
+    if ((rc = batch_table<OpPmeZGather<MIXED, ORDER>>(b, b.gather, args_gather, nb, lds_g, thr_g))) return rc;
     // pair-kernel blocks in proportion to the atoms (a run's share of a
     // system's waves changes no result), about the device's resident blocks
     // in all
@@ -2383,24 +2428,18 @@ int batch_tables(Batch &b) {
     for (int i = 0; i < ns; ++i)
       nb[i] = std::max(1, (int)std::lround(pair_blocks * b.sys[i]->n / (double)natoms));
     if ((rc = batch_table<PairOp<MIXED, C, LJ, CS, BIGLJ, ORDER>>(b, b.pair, args_pair, nb, 0))) return rc;
-    for (int i = 0; i < ns; ++i) {
-      const Sys *s = b.sys[i];
-      nb[i] = s->pme.nx * ((s->pme.ny + s->zl - 1) / s->zl);
-    }
-    if ((rc = batch_table<OpFftZr2c<T, MIXED>>(b, b.zr2c, args_zr2c, nb, lds_z))) return rc;
-    if ((rc = batch_table<OpFftZc2r<T>>(b, b.zc2r, args_zc2r, nb, lds_z))) return rc;
     // systems with small planes take the one-launch plane pass, the others
     // the three line passes
     for (int i = 0; i < ns; ++i) {
       const Sys *s = b.sys[i];
-      nb[i] = s->fft_plane ? 0 : s->pme.nzh * ((s->pme.nx + s->tky - 1) / s->tky);
+      nb[i] = s->fft_plane ? 0 : s->pme.nzh * ((s->pme.nx + (1 << s->ylog) - 1) >> s->ylog);
     }
-    if ((rc = batch_table<OpFftY<T>>(b, b.yfwd, args_yfwd, nb, lds_y))) return rc;
-    if ((rc = batch_table<OpFftY<T>>(b, b.yinv, args_yinv, nb, lds_y))) return rc;
+    if ((rc = batch_table<OpFftY<T>>(b, b.yfwd, args_yfwd, nb, lds_y, thr_y))) return rc;
+    if ((rc = batch_table<OpFftY<T>>(b, b.yinv, args_yinv, nb, lds_y, thr_y))) return rc;
     for (int i = 0; i < ns; ++i) nb[i] = b.sys[i]->fft_plane ? 0 : b.sys[i]->recip_blocks;
-    if ((rc = batch_table<OpFftXConv<T>>(b, b.xconv, args_xconv, nb, lds_x))) return rc;
+    if ((rc = batch_table<OpFftXConv<T>>(b, b.xconv, args_xconv, nb, lds_x, thr_x))) return rc;
     for (int i = 0; i < ns; ++i) nb[i] = b.sys[i]->fft_plane ? b.sys[i]->pme.nzh : 0;
-    if ((rc = batch_table<OpFftPlane<T>>(b, b.plane, args_plane, nb, lds_p))) return rc;
+    if ((rc = batch_table<OpFftPlane<T>>(b, b.plane, args_plane, nb, lds_p, thr_p))) return rc;
     if ((rc = batch_table<OpFixups<MIXED, C, LJ, CS>>(b, b.fixups, args_fixups, nfix, 0))) return rc;
     for (int i = 0; i < ns; ++i) nb[i] = (int)nblk(b.sys[i]->n, 256);
     if ((rc = batch_table<OpUnsortForces<MIXED>>(b, b.unsort, args_unsort, nb, 0))) return rc;
@@ -2455,25 +2494,26 @@ int batch_chunk(Batch &b, int K, bool opening) {
     batch_go<OpRunsPrefix>(b.rprefix, st, bk);
     batch_go<OpRunsCut>(b.rcut, st, bk);
     batch_go<OpRunsTiles>(b.rtiles, st, bk);
-    if (k == 0) batch_go<OpSpreadPatch<MIXED, ORDER>>(b.spread, st, bk);
-    // fork: the PME chain beside the pair kernel
+    // the spread has the device to itself (beside the pair kernel a CU has
+    // room for one of its blocks at a time: 0.51 ms instead of 0.1 for 64
+    // systems of 331,000 atoms); fork: the rest of the PME chain beside the
+    // pair kernel
+    batch_go<OpPmeSpreadZ<MIXED, ORDER>>(b.spread, st, bk);
     BHIPCHK(hipEventRecord(b.fork, st));
     BHIPCHK(hipStreamWaitEvent(st2, b.fork, 0));
     batch_go<PairOp<MIXED, C, LJ, CS, BIGLJ, ORDER>>(b.pair, st, bk);
-    batch_go<OpFftZr2c<T, MIXED>>(b.zr2c, st2, bk);
     batch_go<OpFftPlane<T>>(b.plane, st2, bk);
     batch_go<OpFftY<T>>(b.yfwd, st2, bk);
     batch_go<OpFftXConv<T>>(b.xconv, st2, bk);
     batch_go<OpFftY<T>>(b.yinv, st2, bk);
-    batch_go<OpFftZc2r<T>>(b.zc2r, st2, bk);
-    batch_go<OpGatherPatch<MIXED, ORDER>>(b.gather, st2, bk);
+    batch_go<OpPmeZGather<MIXED, ORDER>>(b.gather, st2, bk);
     BHIPCHK(hipEventRecord(b.join, st2));
     // boundary pairs, exclusion correction and bonded terms after the pair
     // kernel, then the join
     batch_go<OpFixups<MIXED, C, LJ, CS>>(b.fixups, st, bk);
     BHIPCHK(hipStreamWaitEvent(st, b.join, 0));
     if (k + 1 < K)
-      batch_go<OpUnsortKickDriftSpread<MIXED, R, ORDER>>(b.ukds, st, bk);
+      batch_go<OpUnsortKickDrift<MIXED, R>>(b.ukd, st, bk);
     else
       batch_go<OpUnsortForces<MIXED>>(b.unsort, st, bk);
   }
@@ -2497,8 +2537,7 @@ int batch_forces(Batch &b) {
   int rc = batch_tables<MIXED, C, LJ, CS, BIGLJ, ORDER>(b);
   if (rc) return rc;
   for (Sys *s : b.sys) {
-    if (!s->acc_clean || s->spread_ready) launch_zero(s);
-    s->spread_ready = false;
+    if (!s->acc_clean) launch_zero(s);
     hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, P<int>(s->overflow), 0, 2ll);
   }
   std::vector<unsigned char> all(ns, 1);
@@ -2517,17 +2556,15 @@ int batch_forces(Batch &b) {
   batch_go<OpRunsPrefix>(b.rprefix, st, bk);
   batch_go<OpRunsCut>(b.rcut, st, bk);
   batch_go<OpRunsTiles>(b.rtiles, st, bk);
-  batch_go<OpSpreadPatch<MIXED, ORDER>>(b.spread, st, bk);
+  batch_go<OpPmeSpreadZ<MIXED, ORDER>>(b.spread, st, bk);
   BHIPCHK(hipEventRecord(b.fork, st));
   BHIPCHK(hipStreamWaitEvent(st2, b.fork, 0));
   batch_go<PairOp<MIXED, C, LJ, CS, BIGLJ, ORDER>>(b.pair, st, bk);
-  batch_go<OpFftZr2c<T, MIXED>>(b.zr2c, st2, bk);
   batch_go<OpFftPlane<T>>(b.plane, st2, bk);
   batch_go<OpFftY<T>>(b.yfwd, st2, bk);
   batch_go<OpFftXConv<T>>(b.xconv, st2, bk);
   batch_go<OpFftY<T>>(b.yinv, st2, bk);
-  batch_go<OpFftZc2r<T>>(b.zc2r, st2, bk);
-  batch_go<OpGatherPatch<MIXED, ORDER>>(b.gather, st2, bk);
+  batch_go<OpPmeZGather<MIXED, ORDER>>(b.gather, st2, bk);
   BHIPCHK(hipEventRecord(b.join, st2));
   batch_go<OpFixups<MIXED, C, LJ, CS>>(b.fixups, st, bk);
   BHIPCHK(hipStreamWaitEvent(st, b.join, 0));
@@ -2607,7 +2644,6 @@ int batch_run(Batch &b, int nsteps) {
     s->md.rebuilds += nreb[i];
     s->list_valid = true;
     s->prune_pending = false;
-    s->spread_ready = false;
     s->acc_clean = true;
   }
   return PMX_OK;
@@ -2767,8 +2803,7 @@ int batch_entry(pmx_sys *const *systems, int nsys, int nsteps) {
       if (int rc = setup(s)) return rc;
     if (md) {
       if (int rc = md_ensure_forces(s)) return rc;
-      if (!s->acc_clean || s->spread_ready) {
-        s->spread_ready = false;
+      if (!s->acc_clean) {
         launch_zero(s);
         s->acc_clean = true;
       }

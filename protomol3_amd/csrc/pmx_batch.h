@@ -143,12 +143,15 @@ struct OpSplitFill {
     float4 *sorg, *ctr, *half, *sctr, *shalf;
     int *nmaskwork;
     double qpair;
+    PmeParams pme;
+    PmeSlots<R> rec;
   };
   static constexpr int kBlock = 256, kMinBlocks = 1;
   static constexpr bool kGated = true;
   __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &) {
     split_fill_body<R>(bid, nbk, a.nsuper, a.sc_info, a.order, a.xwrap, a.permp, a.slot, a.q, a.type, a.xs, a.xs64,
-                       a.ts, a.xorig, a.xbuild, a.sorg, a.ctr, a.half, a.sctr, a.shalf, a.nmaskwork, a.qpair);
+                       a.ts, a.xorig, a.xbuild, a.sorg, a.ctr, a.half, a.sctr, a.shalf, a.nmaskwork, a.qpair, a.pme,
+                       a.rec);
   }
 };
 
@@ -263,29 +266,34 @@ struct OpKickDrift {
     const double4 *xs64;
     const float4 *sorg;
     unsigned *dmax;  // displacement record of the chunk, one word per step
+    PmeParams pme;
+    PmeSlots<R> rec;
   };
   static constexpr int kBlock = 256, kMinBlocks = 1;
   static constexpr bool kGated = false;
   __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &st) {
     kick_drift_body<R>(bid, nbk, a.n, batch_kick(a.kick, a.h, st.k, st.opening), a.h, a.perm, a.fout, a.minv, a.v,
-                       a.x, a.xbuild, a.xs, a.xs64, a.sorg, a.dmax + st.k);
+                       a.x, a.xbuild, a.xs, a.xs64, a.sorg, a.dmax + st.k, a.pme, a.rec);
   }
 };
 
 template <bool MIXED, int P>
-struct OpSpreadPatch {
+struct OpPmeSpreadZ {
+  using T = typename std::conditional<MIXED, float, double>::type;
   struct Args {
-    int n;
     PmeParams p;
-    const double *xorig, *q;
-    const int *perm;
-    double *grid64;
-    unsigned long long *gridfx;
+    FftPlan pl;
+    const int2 *tcol;
+    const int *colsc;
+    const typename Real4<T>::type *pmw;
+    const int2 *pmb;
+    const Cx<T> *tw;
+    Cx<T> *spec;
   };
-  static constexpr int kBlock = 256, kMinBlocks = 1;
+  static constexpr int kBlock = kPmeBlock, kMinBlocks = kPmeWaves<T>;
   static constexpr bool kGated = false;
   __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &) {
-    spread_patch_body<MIXED, P>(bid, nbk, a.n, a.p, a.xorig, a.perm, a.q, a.grid64, a.gridfx);
+    pme_spread_z_body<MIXED, P>(bid, nbk, a.p, a.pl, a.tcol, a.colsc, a.pmw, a.pmb, a.tw, a.spec);
   }
 };
 
@@ -318,38 +326,20 @@ struct OpPair {
   }
 };
 
-template <class T, bool FIXED>
-struct OpFftZr2c {
-  struct Args {
-    PmeParams p;
-    FftPlan pl;
-    int lines;
-    double *g64;
-    unsigned long long *gfx;
-    const Cx<T> *tw;
-    Cx<T> *sa;
-  };
-  static constexpr int kBlock = 256, kMinBlocks = 1;
-  static constexpr bool kGated = false;
-  __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &) {
-    fft_z_r2c_body<T, FIXED>(bid, nbk, a.p, a.pl, a.lines, a.g64, a.gfx, a.tw, a.sa);
-  }
-};
-
 template <class T>
 struct OpFftY {
   struct Args {
     PmeParams p;
     FftPlan pl;
-    int lines;
+    int llog;
     bool inverse;
-    const Cx<T> *tw, *src;
-    Cx<T> *dst;
+    const Cx<T> *tw;
+    Cx<T> *spec;
   };
-  static constexpr int kBlock = 256, kMinBlocks = 1;
+  static constexpr int kBlock = kPmeBlock, kMinBlocks = kPmeWaves<T>;
   static constexpr bool kGated = false;
   __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &) {
-    fft_y_body<T>(bid, nbk, a.p, a.pl, a.lines, a.inverse, a.tw, a.src, a.dst);
+    fft_y_body<T>(bid, nbk, a.p, a.pl, a.llog, a.inverse, a.tw, a.spec);
   }
 };
 
@@ -358,16 +348,16 @@ struct OpFftXConv {
   struct Args {
     PmeParams p;
     FftPlan pl;
-    int lines;
+    int llog, threads;
     const Cx<T> *tw;
     const T *theta;
-    Cx<T> *sb;
+    Cx<T> *spec;
     double *epart;
   };
-  static constexpr int kBlock = 256, kMinBlocks = 1;
+  static constexpr int kBlock = kPmeBlock, kMinBlocks = kPmeWaves<T>;
   static constexpr bool kGated = false;
   __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &) {
-    fft_x_conv_body<T>(bid, nbk, a.p, a.pl, a.lines, a.tw, a.theta, a.sb, a.epart);
+    fft_x_conv_body<T>(bid, nbk, a.p, a.pl, a.llog, a.threads, a.tw, a.theta, a.spec, a.epart);
   }
 };
 
@@ -376,48 +366,36 @@ struct OpFftPlane {
   struct Args {
     PmeParams p;
     FftPlan ply, plx;
+    int threads;
     const Cx<T> *twy, *twx;
     const T *theta;
-    Cx<T> *sa;
+    Cx<T> *spec;
     double *epart;
   };
-  static constexpr int kBlock = 256, kMinBlocks = 1;
+  static constexpr int kBlock = kPmeBlock, kMinBlocks = kPmeWaves<T>;
   static constexpr bool kGated = false;
   __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &) {
-    fft_plane_conv_body<T>(bid, nbk, a.p, a.ply, a.plx, a.twy, a.twx, a.theta, a.sa, a.epart);
-  }
-};
-
-template <class T>
-struct OpFftZc2r {
-  struct Args {
-    PmeParams p;
-    FftPlan pl;
-    int lines;
-    const Cx<T> *tw, *sa;
-    T *greal;
-  };
-  static constexpr int kBlock = 256, kMinBlocks = 1;
-  static constexpr bool kGated = false;
-  __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &) {
-    fft_z_c2r_body<T>(bid, nbk, a.p, a.pl, a.lines, a.tw, a.sa, a.greal);
+    fft_plane_conv_body<T>(bid, nbk, a.p, a.ply, a.plx, a.threads, a.twy, a.twx, a.theta, a.spec, a.epart);
   }
 };
 
 template <bool MIXED, int P>
-struct OpGatherPatch {
+struct OpPmeZGather {
+  using T = typename std::conditional<MIXED, float, double>::type;
   struct Args {
-    int n;
     PmeParams p;
-    const double *xorig, *q;
-    const int *perm;
-    const typename std::conditional<MIXED, float, double>::type *greal;
+    FftPlan pl;
+    const int2 *tcol;
+    const int *colsc;
+    const typename Real4<T>::type *pmw;
+    const int2 *pmb;
+    const Cx<T> *tw, *spec;
     typename AccT<MIXED>::type *facc;
   };
-  static constexpr int kBlock = 256, kMinBlocks = 1;
+  static constexpr int kBlock = kPmeBlock, kMinBlocks = kPmeWaves<T>;
   static constexpr bool kGated = false;
   __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &) {
-    gather_patch_body<MIXED, P>(bid, nbk, a.n, a.p, a.xorig, a.perm, a.q, a.greal, a.facc);
+    pme_z_gather_body<MIXED, P>(bid, nbk, a.p, a.pl, a.tcol, a.colsc, a.pmw, a.pmb, a.tw, a.spec, a.facc);
   }
 };
 
@@ -431,9 +409,9 @@ struct OpFixups {
   }
 };
 
-// unsort of step k's forces, kick and drift of step k + 1, its charge spread
-template <bool MIXED, class R, int P>
-struct OpUnsortKickDriftSpread {
+// unsort of step k's forces, kick and drift of step k + 1
+template <bool MIXED, class R>
+struct OpUnsortKickDrift {
   struct Args {
     int n;
     Kick kick;
@@ -442,23 +420,21 @@ struct OpUnsortKickDriftSpread {
     typename AccT<MIXED>::type *facc;
     double *fout;
     int *tilectr, *nborder;
-    const double *minv, *xbuild, *q;
+    const double *minv, *xbuild;
     double *v, *x;
     typename Real4<R>::type *xs;
     const double4 *xs64;
     const float4 *sorg;
     unsigned *dmax;
     PmeParams pme;
-    double *grid64;
-    unsigned long long *gridfx;
+    PmeSlots<R> rec;
   };
   static constexpr int kBlock = 256, kMinBlocks = 1;
   static constexpr bool kGated = false;
   __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &st) {
-    unsort_kick_drift_spread_body<MIXED, R, P>(bid, nbk, a.n, batch_kick(a.kick, a.h, st.k + 1, false), a.h, a.perm,
-                                               a.facc, a.fout, a.tilectr, a.nborder, a.minv, a.v, a.x, a.xbuild,
-                                               a.xs, a.xs64, a.sorg, a.dmax + st.k + 1, a.pme, a.q, a.grid64,
-                                               a.gridfx);
+    unsort_kick_drift_body<MIXED, R>(bid, nbk, a.n, batch_kick(a.kick, a.h, st.k + 1, false), a.h, a.perm, a.facc,
+                                     a.fout, a.tilectr, a.nborder, a.minv, a.v, a.x, a.xbuild, a.xs, a.xs64, a.sorg,
+                                     a.dmax + st.k + 1, a.pme, a.rec);
   }
 };
 

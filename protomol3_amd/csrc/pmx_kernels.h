@@ -94,6 +94,59 @@ __device__ inline int wave_max(int v) {
   return v;
 }
 
+struct PmeParams {
+  int nx, ny, nz, nzh, order;
+  double hxr, hyr, hzr;   // K/L per axis (Grid.h:520-522)
+  int offx, offy, offz;   // -(p-1)/2 + K (Grid.h:509-511)
+  int tx, ty;             // lines of a tile along x (even) and y, powers of two
+  int ntx, nty;           // tiles per axis
+  int ncy, ncx;           // x-y columns of the sort
+};
+
+// An atom's place on the grid, per sorted slot: fractional offsets and charge
+// (pmw), base indices x | y << 16 and z (pmb; x = kNoGrid for slots without a
+// charge).  Written by the sort and by every drift.
+constexpr int kNoGrid = -1;
+template <class R>
+struct PmeSlots {
+  typename Real4<R>::type *w;
+  int2 *b;
+};
+
+// Grid index of base + offset for base in [0, K), offset < K.
+__device__ inline int wrap_grid(int v, int K) { return v >= K ? v - K : v; }
+
+// Grid coordinate of one axis: u = x K/L wrapped to [0, K) (Grid.h:111-120);
+// the base is wrapped too.
+__device__ inline void grid_coord(double x, double hr, int K, int off, int &base, double &w) {
+  double u = x * hr;
+  while (u < 0.0) u += K;
+  while (u >= K) u -= K;
+  const int iu = (int)u;
+  base = wrap_grid(iu + off, K);
+  w = u - iu;
+}
+
+// The grid record of slot s for an atom of charge q at x (a < 0: no atom).
+template <class R>
+__device__ inline void pme_record(const PmeParams &p, const PmeSlots<R> &rec, int s, bool atom, const double x[3],
+                                  double q) {
+  int b[3] = {kNoGrid, 0, 0};
+  double w[3] = {0, 0, 0};
+  if (atom && (R)q != (R)0) {
+    grid_coord(x[0], p.hxr, p.nx, p.offx, b[0], w[0]);
+    grid_coord(x[1], p.hyr, p.ny, p.offy, b[1], w[1]);
+    grid_coord(x[2], p.hzr, p.nz, p.offz, b[2], w[2]);
+  }
+  typename Real4<R>::type v;
+  v.x = (R)w[0];
+  v.y = (R)w[1];
+  v.z = (R)w[2];
+  v.w = (R)q;
+  rec.w[s] = v;
+  rec.b[s] = make_int2(b[0] < 0 ? kNoGrid : (b[0] | (b[1] << 16)), b[2]);
+}
+
 // ---------------------------------------------------------------------------
 // 1. Binning: wrapped coordinates, column x z-bin sort key, reference cell.
 struct BinParams {
@@ -403,6 +456,7 @@ constexpr float kScSlack = 1e-3f;
 //    times qpair (0 when the pair pass carries no Coulomb term),
 //    FP64 copy in xs64, LJ type (padding: type -1); xbuild (MD only, else
 //    null) receives the positions the list is built from;
+//  - with PME, the atoms' grid records (rec);
 //  - bounding boxes (FP32, list building only): per cluster (8-lane groups;
 //    ctr.w = real atoms, empty clusters get negative half extents), and per
 //    supercluster (the whole wave, widened by kScSlack).
@@ -417,7 +471,8 @@ __device__ __forceinline__ void split_fill_body(const int bid_, const int nbk_, 
                                                 const double *__restrict__ xorig, double *__restrict__ xbuild,
                                                 float4 *__restrict__ sorg, float4 *__restrict__ ctr,
                                                 float4 *__restrict__ half, float4 *__restrict__ sctr,
-                                                float4 *__restrict__ shalf, int *__restrict__ nmaskwork, double qpair) {
+                                                float4 *__restrict__ shalf, int *__restrict__ nmaskwork, double qpair,
+                                                const PmeParams &pme, PmeSlots<R> rec) {
   const int sc = (bid_ * blockDim.x + threadIdx.x) >> 6;
   const int lane = threadIdx.x & 63;
   if (bid_ == 0 && threadIdx.x == 0) *nmaskwork = 0;
@@ -466,6 +521,7 @@ __device__ __forceinline__ void split_fill_body(const int bid_, const int nbk_, 
     xs64[s] = make_double4(0, 0, 0, 0);
   }
   xs[s] = v;
+  if (rec.w) pme_record<R>(pme, rec, s, a >= 0, p, a >= 0 ? q[a] : 0.0);
   // boxes: clusters (8-lane groups), then the supercluster (the wave)
   double lo[3], hi[3];
 #pragma unroll
@@ -529,9 +585,9 @@ __global__ void __launch_bounds__(256) k_split_fill(int nsuper_max, const int2 *
                                                     float4 *__restrict__ sorg, float4 *__restrict__ ctr,
                                                     float4 *__restrict__ half, float4 *__restrict__ sctr,
                                                     float4 *__restrict__ shalf, int *__restrict__ nmaskwork,
-                                                    double qpair) {
+                                                    double qpair, PmeParams pme, PmeSlots<R> rec) {
   split_fill_body<R>(blockIdx.x, gridDim.x, nsuper_max, sc_info, order, xwrap, permp, slot, q, type, xs, xs64, ts,
-                     xorig, xbuild, sorg, ctr, half, sctr, shalf, nmaskwork, qpair);
+                     xorig, xbuild, sorg, ctr, half, sctr, shalf, nmaskwork, qpair, pme, rec);
 }
 
 
@@ -1942,14 +1998,24 @@ __device__ void border_pairs(int blk, int nblocks, const PairParams &pp, int sta
 }
 
 // ---------------------------------------------------------------------------
-// 4. PME: B-spline spreading, LDS FFT passes with the influence function,
-//    force gather.  Grid [nx][ny][nz], z fastest (Grid.h:70).
-
-struct PmeParams {
-  int nx, ny, nz, nzh, order;
-  double hxr, hyr, hzr;   // K/L per axis (Grid.h:520-522)
-  int offx, offy, offz;   // -(p-1)/2 + K (Grid.h:509-511)
-};
+// 4. PME (Grid.h:107-341): charge spread with the z transform, y and x
+//    transforms with the influence function, inverse z transform with the
+//    force gather.  The half spectrum is [k][j][i] (i fastest) throughout.
+//
+// The charge grid and the real potential never exist in memory: a block owns
+// a tile of grid lines along z (tx x ty neighbouring (i, j)), sums every
+// stencil contribution to them in LDS and transforms them there; the inverse
+// pass transforms the tile's lines back and interpolates the forces from
+// LDS.  A tile finds the atoms whose stencils touch it in the x-y columns of
+// the sort (the window of the tile widened by the stencil and by half the
+// skin the atoms may have moved since the sort).  With the grid in memory
+// (atomics from an LDS patch per 32 atoms, a transform that read and cleared
+// it, a gather that loaded patches of the potential) the reciprocal part of a
+// step moved 2.7 GB on a 256^3 grid, the atomics 0.58 GB of it; here each
+// pass reads and writes the half spectrum once.  Million-atom box, 216 x 240 x
+// 240 points, order 6, before and after: spread + z 1.18 -> 0.30 ms alone, x
+// and y 0.91 -> 0.25 ms, inverse z + gather 0.46 -> 0.35 ms (the last two
+// beside the pair kernel).
 
 // BSpline::set (mdl/interface/force/nonbonded/BSpline.cpp:55-105) for a
 // compile-time order P (2..8): weights th[0..P-1] and derivatives dth.
@@ -1977,264 +2043,8 @@ __device__ inline void bspline_w(R w, R *th, R *dth) {
   th[0] = div * ((R)1 - w) * th[0];
 }
 
-// Element m of a register array as a sum of 0/1-weighted terms.  A select
-// chain would be folded into a dynamically indexed load, which moves the
-// array out of registers into LDS or scratch.
-template <int P, class R>
-__device__ inline R pick(const R *v, int m) {
-  R r = (R)0;
-#pragma unroll
-  for (int t = 0; t < P; ++t) r += (R)(m == t) * v[t];
-  return r;
-}
-
-// Threads per atom in spreading and gathering: one per (i, j) stencil row,
-// rounded up to a power of two (order 2: 4, order 4: 16, orders 6 and 8: 64).
-__host__ __device__ constexpr int pme_tpa(int order) {
-  return order * order <= 4 ? 4 : order * order <= 16 ? 16 : 64;
-}
-
-// Grid index (base + offset) mod K for base + offset in [0, 3K).
-__device__ inline int wrap_grid(int v, int K) {
-  v -= v >= K ? K : 0;
-  v -= v >= K ? K : 0;
-  return v;
-}
-
-// Grid coordinate of one axis: u = x K/L wrapped to [0, K) (Grid.h:111-120).
-__device__ inline void grid_coord(double x, double hr, int K, int off, int &base, double &w) {
-  double u = x * hr;
-  while (u < 0.0) u += K;
-  while (u >= K) u -= K;
-  int iu = (int)u;
-  base = iu + off;
-  w = u - iu;
-}
-
-// Charge spreading through an LDS patch (Grid::anterpolateCharge,
-// Grid.h:107-154).  One block takes kSpreadSlots consecutive sorted slots
-// (half a supercluster: a compact group of atoms).  Wave 0 computes each
-// atom's grid base and fractional offsets and the box of grid points the
-// group's stencils cover (bases taken relative to the first atom's, on the
-// periodic grid); the block accumulates every stencil contribution into an
-// LDS copy of that box with LDS atomics, then adds the box's nonzero points
-// to the grid with one global atomic each.  The accumulator type is the
-// grid's (int64 fixed point 2^-40 in the mixed form, so the result does not
-// depend on the order of the adds; double in the FP64 form).  A group whose
-// box exceeds the patch capacity, or wraps onto itself, adds to the grid
-// directly.
-constexpr int kSpreadSlots = 32;
-template <int P>
-__host__ __device__ constexpr int spread_patch_max() {
-  return P <= 4 ? 2048 : 4096;
-}
-
-// The spread of one group (the block's kSpreadSlots slots from s0): lane t
-// of wave 0 brings atom a (-1: none) of slot s0 + t at position xa; the
-// other threads' a and xa are not read.
-template <bool MIXED, int P>
-__device__ void spread_patch_group(int s0, const PmeParams &p, int a, const double xa[3],
-                                   const double *__restrict__ q, double *__restrict__ grid64,
-                                   unsigned long long *__restrict__ gridfx) {
-  using R = typename std::conditional<MIXED, float, double>::type;
-  using G = typename std::conditional<MIXED, unsigned long long, double>::type;
-  constexpr int P3 = P * P * P;
-  constexpr int PMAX = spread_patch_max<P>();
-  __shared__ G s_patch[PMAX];
-  __shared__ int s_rb[kSpreadSlots][3];  // base relative to the patch origin
-  __shared__ R s_w[kSpreadSlots][3];
-  __shared__ R s_q[kSpreadSlots];
-  __shared__ int s_org[3], s_ext[3], s_direct, s_any;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int K[3] = {p.nx, p.ny, p.nz};
-  if (wv == 0) {
-    const int t = lane;
-    int b[3] = {0, 0, 0};
-    double w[3] = {0, 0, 0};
-    if (a >= 0) {
-      grid_coord(xa[0], p.hxr, p.nx, p.offx, b[0], w[0]);
-      grid_coord(xa[1], p.hyr, p.ny, p.offy, b[1], w[1]);
-      grid_coord(xa[2], p.hzr, p.nz, p.offz, b[2], w[2]);
-    }
-    const unsigned long long ok = __ballot(a >= 0);
-    if (ok) {
-      const int first = __builtin_ctzll(ok);
-      int lo[3], hi[3], db[3], ref[3];
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        ref[k] = __shfl(b[k], first);
-        int d = b[k] - ref[k];  // on the periodic grid, nearest to the reference
-        d -= K[k] * (int)floorf(((float)d + 0.5f * (float)K[k]) / (float)K[k]);
-        db[k] = d;
-        lo[k] = a >= 0 ? d : 0x3fffffff;
-        hi[k] = a >= 0 ? d : -0x3fffffff;
-      }
-#pragma unroll
-      for (int m = 32; m >= 1; m >>= 1)
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-          lo[k] = min(lo[k], __shfl_xor(lo[k], m));
-          hi[k] = max(hi[k], __shfl_xor(hi[k], m));
-        }
-      const int ex = hi[0] - lo[0] + P, ey = hi[1] - lo[1] + P, ez = hi[2] - lo[2] + P;
-      const bool direct = ex > K[0] || ey > K[1] || ez > K[2] || (long long)ex * ey * ez > PMAX;
-      if (t < kSpreadSlots) {
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-          // direct adds use the plain base; patch adds the base within the box
-          s_rb[t][k] = direct ? b[k] : db[k] - lo[k];
-          s_w[t][k] = (R)w[k];
-        }
-        s_q[t] = a >= 0 ? (R)q[a] : (R)0;
-      }
-      if (lane == 0) {
-#pragma unroll
-        for (int k = 0; k < 3; ++k) s_org[k] = ref[k] + lo[k];
-        s_ext[0] = ex;
-        s_ext[1] = ey;
-        s_ext[2] = ez;
-        s_direct = direct ? 1 : 0;
-        s_any = 1;
-      }
-    } else if (lane == 0) {
-      s_any = 0;
-    }
-  }
-  __syncthreads();
-  if (!s_any) return;  // block-uniform: no atoms in this group
-  const bool direct = s_direct;
-  const int ex = s_ext[0], ey = s_ext[1], ez = s_ext[2];
-  const int vol = ex * ey * ez;
-  if (!direct)
-    for (int i = tid; i < vol; i += blockDim.x) s_patch[i] = (G)0;
-  __syncthreads();
-  for (int t = wv; t < kSpreadSlots; t += blockDim.x / kWave) {
-    const R qa = s_q[t];
-    if (qa == (R)0) continue;  // padding slot or uncharged atom: no contribution
-    R tx[P], ty[P], tz[P], dd[P];
-    bspline_w<P, R>(s_w[t][0], tx, dd);
-    bspline_w<P, R>(s_w[t][1], ty, dd);
-    bspline_w<P, R>(s_w[t][2], tz, dd);
-    const int rb0 = s_rb[t][0], rb1 = s_rb[t][1], rb2 = s_rb[t][2];
-#pragma unroll
-    for (int pt0 = 0; pt0 < P3; pt0 += kWave) {
-      const int pt = pt0 + lane;
-      if (P3 % kWave != 0 && pt >= P3) break;
-      const int i = pt / (P * P), j = (pt / P) % P, kk = pt % P;
-      const R v = ((qa * pick<P>(tx, i)) * pick<P>(ty, j)) * pick<P>(tz, kk);
-      G add;
-      if (MIXED)
-        add = (G)(unsigned long long)__double2ll_rn((double)v * kGridScale);
-      else
-        add = (G)v;
-      if (!direct) {
-        atomicAdd(&s_patch[((rb0 + i) * ey + (rb1 + j)) * ez + (rb2 + kk)], add);
-      } else {
-        const size_t g = ((size_t)wrap_grid(i + rb0, p.nx) * p.ny + wrap_grid(j + rb1, p.ny)) * p.nz +
-                         wrap_grid(kk + rb2, p.nz);
-        if (MIXED)
-          atomicAdd(&gridfx[g], (unsigned long long)add);
-        else
-          unsafeAtomicAdd(&grid64[g], (double)add);
-      }
-    }
-  }
-  if (direct) return;
-  __syncthreads();
-  const int ox = s_org[0], oy = s_org[1], oz = s_org[2];
-  for (int i = tid; i < vol; i += blockDim.x) {
-    const G v = s_patch[i];
-    if (v == (G)0) continue;
-    const int iz = i % ez, iy = (i / ez) % ey, ix = i / (ez * ey);
-    const int gx = (ox + ix) % p.nx, gy = (oy + iy) % p.ny, gz = (oz + iz) % p.nz;
-    const size_t g = ((size_t)(gx < 0 ? gx + p.nx : gx) * p.ny + (gy < 0 ? gy + p.ny : gy)) * p.nz +
-                     (gz < 0 ? gz + p.nz : gz);
-    if (MIXED)
-      atomicAdd(&gridfx[g], (unsigned long long)v);
-    else
-      unsafeAtomicAdd(&grid64[g], (double)v);
-  }
-}
-
-template <bool MIXED, int P>
-__device__ __forceinline__ void spread_patch_body(const int bid_, const int nbk_, int n, PmeParams p,
-                                                  const double *__restrict__ xorig, const int *__restrict__ perm,
-                                                  const double *__restrict__ q, double *__restrict__ grid64,
-                                                  unsigned long long *__restrict__ gridfx) {
-  const int s0 = bid_ * kSpreadSlots;
-  const int t = threadIdx.x, s = s0 + t;
-  int a = -1;
-  double xa[3] = {0, 0, 0};
-  if (t < kSpreadSlots && s < n) {
-    a = perm[s];
-    if (a >= 0) {
-      xa[0] = xorig[3 * a];
-      xa[1] = xorig[3 * a + 1];
-      xa[2] = xorig[3 * a + 2];
-    }
-  }
-  spread_patch_group<MIXED, P>(s0, p, a, xa, q, grid64, gridfx);
-}
-
-template <bool MIXED, int P>
-__global__ void __launch_bounds__(256) k_spread_patch(int n, PmeParams p, const double *__restrict__ xorig,
-                                                      const int *__restrict__ perm, const double *__restrict__ q,
-                                                      double *__restrict__ grid64,
-                                                      unsigned long long *__restrict__ gridfx) {
-  // the blocks of one XCD take a contiguous range of slots (one region of
-  // the grid)
-  spread_patch_body<MIXED, P>(xcd_block(blockIdx.x, gridDim.x), gridDim.x, n, p, xorig, perm, q, grid64, gridfx);
-}
-
-// Charge spreading (Grid::anterpolateCharge, Grid.h:107-154).  The P^3
-// stencil points of one atom go to consecutive lanes (z fastest), so each
-// atomic instruction of a wave updates P^2 short contiguous rows of one
-// atom's stencil; orders 2 (8 points) pack 8 atoms into a wave, orders 6 and
-// 8 loop over their points in steps of 64.  Slots run in sorted order; n
-// counts slots (padding slots return at once).
-template <bool MIXED, int P>
-__global__ void __launch_bounds__(256) k_spread(int n, PmeParams p, const double *__restrict__ xorig,
-                                                const int *__restrict__ perm, const double *__restrict__ q,
-                                                double *__restrict__ grid64, unsigned long long *__restrict__ gridfx) {
-  using R = typename std::conditional<MIXED, float, double>::type;
-  constexpr int P3 = P * P * P;
-  constexpr int LPA = P3 >= kWave ? kWave : P3;  // lanes per atom
-  constexpr int APW = kWave / LPA;               // atoms per wave
-  const int gt = blockIdx.x * blockDim.x + threadIdx.x;
-  const int wave = gt >> 6, lane = gt & 63;
-  const int s = wave * APW + lane / LPA;
-  if (s >= n) return;
-  const int a = perm[s];
-  if (a < 0) return;  // padding slot
-  const int l0 = lane % LPA;
-  int b[3];
-  double w[3];
-  grid_coord(xorig[3 * a], p.hxr, p.nx, p.offx, b[0], w[0]);
-  grid_coord(xorig[3 * a + 1], p.hyr, p.ny, p.offy, b[1], w[1]);
-  grid_coord(xorig[3 * a + 2], p.hzr, p.nz, p.offz, b[2], w[2]);
-  R tx[P], ty[P], tz[P], d[P];
-  bspline_w<P, R>((R)w[0], tx, d);
-  bspline_w<P, R>((R)w[1], ty, d);
-  bspline_w<P, R>((R)w[2], tz, d);
-  const R qa = (R)q[a];
-#pragma unroll
-  for (int pt0 = 0; pt0 < P3; pt0 += LPA) {
-    const int pt = pt0 + l0;
-    const int i = pt / (P * P), j = (pt / P) % P, kk = pt % P;
-    const R v = ((qa * pick<P>(tx, i)) * pick<P>(ty, j)) * pick<P>(tz, kk);
-    const size_t g = ((size_t)wrap_grid(i + b[0], p.nx) * p.ny + wrap_grid(j + b[1], p.ny)) * p.nz +
-                     wrap_grid(kk + b[2], p.nz);
-    if (MIXED) {
-      long long fx = __double2ll_rn((double)v * kGridScale);
-      atomicAdd(&gridfx[g], (unsigned long long)fx);
-    } else {
-      unsafeAtomicAdd(&grid64[g], (double)v);
-    }
-  }
-}
-
 template <class T>
-struct Cx {
+struct alignas(2 * sizeof(T)) Cx {
   T x, y;
 };
 
@@ -2242,577 +2052,667 @@ template <class T>
 __device__ inline Cx<T> cmul(Cx<T> a, Cx<T> b) {
   return Cx<T>{a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x};
 }
+template <class T>
+__device__ inline Cx<T> cadd(Cx<T> a, Cx<T> b) {
+  return Cx<T>{a.x + b.x, a.y + b.y};
+}
+template <class T>
+__device__ inline Cx<T> csub(Cx<T> a, Cx<T> b) {
+  return Cx<T>{a.x - b.x, a.y - b.y};
+}
 
-// Forward DFT of small radix R in registers, e^{-2 pi i rk/R}.
+// Forward DFT of small radix R in registers, e^{-2 pi i rk/R}.  6 and 10 are
+// prime-factor products (no twiddles), 8 and 9 two steps.
 template <int R, class T>
-__device__ inline void dft_small(Cx<T> *v) {
+__device__ __forceinline__ void dft_small(Cx<T> *v) {
   if constexpr (R == 2) {
-    Cx<T> a = v[0], b = v[1];
-    v[0] = Cx<T>{a.x + b.x, a.y + b.y};
-    v[1] = Cx<T>{a.x - b.x, a.y - b.y};
+    const Cx<T> a = v[0], b = v[1];
+    v[0] = cadd(a, b);
+    v[1] = csub(a, b);
   } else if constexpr (R == 4) {
-    Cx<T> a = v[0], b = v[1], c = v[2], d = v[3];
-    Cx<T> s0{a.x + c.x, a.y + c.y}, s1{a.x - c.x, a.y - c.y};
-    Cx<T> s2{b.x + d.x, b.y + d.y}, s3{b.x - d.x, b.y - d.y};
-    v[0] = Cx<T>{s0.x + s2.x, s0.y + s2.y};
-    v[2] = Cx<T>{s0.x - s2.x, s0.y - s2.y};
+    const Cx<T> s0 = cadd(v[0], v[2]), s1 = csub(v[0], v[2]);
+    const Cx<T> s2 = cadd(v[1], v[3]), s3 = csub(v[1], v[3]);
+    v[0] = cadd(s0, s2);
+    v[2] = csub(s0, s2);
     // -i * s3 = (s3.y, -s3.x)
     v[1] = Cx<T>{s1.x + s3.y, s1.y - s3.x};
     v[3] = Cx<T>{s1.x - s3.y, s1.y + s3.x};
   } else if constexpr (R == 3) {
     const T c = (T)-0.5, s = (T)0.86602540378443864676;
-    Cx<T> a = v[0], b = v[1], d = v[2];
-    Cx<T> t{b.x + d.x, b.y + d.y}, u{b.x - d.x, b.y - d.y};
-    v[0] = Cx<T>{a.x + t.x, a.y + t.y};
-    Cx<T> m{a.x + c * t.x, a.y + c * t.y};
+    const Cx<T> a = v[0], t = cadd(v[1], v[2]), u = csub(v[1], v[2]);
+    v[0] = cadd(a, t);
+    const Cx<T> m{a.x + c * t.x, a.y + c * t.y};
     // -i s u = (s u.y, -s u.x)
     v[1] = Cx<T>{m.x + s * u.y, m.y - s * u.x};
     v[2] = Cx<T>{m.x - s * u.y, m.y + s * u.x};
-  } else {
-    static_assert(R == 5, "radix 2, 3, 4 or 5");
+  } else if constexpr (R == 5) {
     const T c1 = (T)0.30901699437494742410, c2 = (T)-0.80901699437494742410;
     const T s1 = (T)0.95105651629515357212, s2 = (T)0.58778525229247312917;
-    Cx<T> a = v[0];
-    Cx<T> t1{v[1].x + v[4].x, v[1].y + v[4].y}, u1{v[1].x - v[4].x, v[1].y - v[4].y};
-    Cx<T> t2{v[2].x + v[3].x, v[2].y + v[3].y}, u2{v[2].x - v[3].x, v[2].y - v[3].y};
+    const Cx<T> a = v[0], t1 = cadd(v[1], v[4]), u1 = csub(v[1], v[4]), t2 = cadd(v[2], v[3]), u2 = csub(v[2], v[3]);
     v[0] = Cx<T>{a.x + t1.x + t2.x, a.y + t1.y + t2.y};
-    Cx<T> m1{a.x + c1 * t1.x + c2 * t2.x, a.y + c1 * t1.y + c2 * t2.y};
-    Cx<T> m2{a.x + c2 * t1.x + c1 * t2.x, a.y + c2 * t1.y + c1 * t2.y};
+    const Cx<T> m1{a.x + c1 * t1.x + c2 * t2.x, a.y + c1 * t1.y + c2 * t2.y};
+    const Cx<T> m2{a.x + c2 * t1.x + c1 * t2.x, a.y + c2 * t1.y + c1 * t2.y};
     // y1 = m1 - i(s1 u1 + s2 u2); y4 = m1 + i(...); y2 = m2 - i(s2 u1 - s1 u2); y3 = m2 + i(...)
-    Cx<T> n1{s1 * u1.x + s2 * u2.x, s1 * u1.y + s2 * u2.y};
-    Cx<T> n2{s2 * u1.x - s1 * u2.x, s2 * u1.y - s1 * u2.y};
+    const Cx<T> n1{s1 * u1.x + s2 * u2.x, s1 * u1.y + s2 * u2.y};
+    const Cx<T> n2{s2 * u1.x - s1 * u2.x, s2 * u1.y - s1 * u2.y};
     v[1] = Cx<T>{m1.x + n1.y, m1.y - n1.x};
     v[4] = Cx<T>{m1.x - n1.y, m1.y + n1.x};
     v[2] = Cx<T>{m2.x + n2.y, m2.y - n2.x};
     v[3] = Cx<T>{m2.x - n2.y, m2.y + n2.x};
+  } else if constexpr (R == 6 || R == 10) {
+    // element (n1, n2) is input (H n1 + 2 n2) mod R; output k has k1 = k mod 2, k2 = k mod H
+    constexpr int H = R / 2;
+    Cx<T> e[H], o[H];
+#pragma unroll
+    for (int m = 0; m < H; ++m) {
+      const Cx<T> a = v[(2 * m) % R], b = v[(H + 2 * m) % R];
+      e[m] = cadd(a, b);
+      o[m] = csub(a, b);
+    }
+    dft_small<H, T>(e);
+    dft_small<H, T>(o);
+#pragma unroll
+    for (int k = 0; k < R; ++k) v[k] = (k & 1) ? o[k % H] : e[k % H];
+  } else if constexpr (R == 8) {
+    const T h = (T)0.70710678118654752440;
+    Cx<T> e[4] = {v[0], v[2], v[4], v[6]}, o[4] = {v[1], v[3], v[5], v[7]};
+    dft_small<4, T>(e);
+    dft_small<4, T>(o);
+    // o[k] e^{-2 pi i k/8}
+    o[1] = Cx<T>{h * (o[1].x + o[1].y), h * (o[1].y - o[1].x)};
+    o[2] = Cx<T>{o[2].y, -o[2].x};
+    o[3] = Cx<T>{h * (o[3].y - o[3].x), -h * (o[3].x + o[3].y)};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      v[k] = cadd(e[k], o[k]);
+      v[k + 4] = csub(e[k], o[k]);
+    }
+  } else {
+    static_assert(R == 9, "radix 2, 3, 4, 5, 6, 8, 9 or 10");
+    const Cx<T> w1{(T)0.76604444311897803520, (T)-0.64278760968653932632};
+    const Cx<T> w2{(T)0.17364817766693034885, (T)-0.98480775301220805937};
+    const Cx<T> w4{(T)-0.93969262078590838405, (T)-0.34202014332566873304};
+    Cx<T> a[3][3];
+#pragma unroll
+    for (int n2 = 0; n2 < 3; ++n2) {
+#pragma unroll
+      for (int n1 = 0; n1 < 3; ++n1) a[n2][n1] = v[3 * n1 + n2];
+      dft_small<3, T>(a[n2]);
+    }
+    a[1][1] = cmul(a[1][1], w1);
+    a[1][2] = cmul(a[1][2], w2);
+    a[2][1] = cmul(a[2][1], w2);
+    a[2][2] = cmul(a[2][2], w4);
+#pragma unroll
+    for (int k1 = 0; k1 < 3; ++k1) {
+      Cx<T> b[3] = {a[0][k1], a[1][k1], a[2][k1]};
+      dft_small<3, T>(b);
+#pragma unroll
+      for (int k2 = 0; k2 < 3; ++k2) v[k1 + 3 * k2] = b[k2];
+    }
   }
 }
 
+// Division of t < 2^16 by a constant d: (t * magic) >> 32, magic =
+// floor(2^32 / d) + 1 (exact for t d < 2^32; d = 1 has none).
+__host__ __device__ inline unsigned div_magic(unsigned d) { return (unsigned)(0x100000000ull / d) + 1u; }
+__device__ inline int div_by(int t, unsigned magic) { return (int)__umulhi((unsigned)t, magic); }
+
+constexpr int kFftMax = 4096;       // longest transform (points), and most points of a block
+constexpr int kFftPerThread = 8;    // points a thread holds in a pass, at least (8 keeps a pass within 64 VGPRs,
+                                    // so that these kernels fit on a SIMD beside four pair-kernel waves)
+constexpr int kPmeBlock = kFftMax / kFftPerThread;  // threads of a PME block, at most
+template <class T>
+constexpr int kPmeWaves = sizeof(T) == 4 ? 8 : 4;   // resident waves per SIMD to compile for
 struct FftPlan {
   int n;
   int nrad;
-  int rad[16];
+  int rad[12];
+  unsigned magic[12];  // div_magic of the product of the radices before this one
+  unsigned magic_n;    // div_magic(n)
 };
 
-// One Stockham pass of radix R over `nb` lines of length n (src -> dst):
-// butterfly j reads src[j + r n/R], twiddles by tw[k r n/(Ns R)] (k = j mod
-// Ns; the index stays below n), writes dst[(j - k) R + k + r Ns].
+// `lines` transforms in LDS: element e of line l at l ls + e es.  Threads
+// take the lines fastest (1 << llog of them, a power of two of at least
+// `lines`), so that with an odd ls (or es = 1 across odd rows) neighbouring
+// lanes fall on different banks and no thread index is divided by a length.
+struct FftLines {
+  int llog, lines, ls, es;
+};
+
+// One Stockham pass of radix R in place: every thread holds its butterflies
+// (up to kFftPerThread points or the next multiple of R) in registers between the two
+// barriers.  Butterfly j reads elements j + r n/R, twiddles by
+// tw[k r n/(Ns R)] (k = j mod Ns), writes (j - k) R + k + r Ns.
 template <int R, class T>
-__device__ inline void fft_pass(const Cx<T> *__restrict__ src, Cx<T> *__restrict__ dst, int nb, int n, int Ns,
-                                const Cx<T> *__restrict__ tw) {
-  const int nbut = n / R;
-  const int tstep = n / (Ns * R);
-  for (int t = threadIdx.x; t < nbut * nb; t += blockDim.x) {
-    const int line = t / nbut, j = t - line * nbut;
-    const int k = j % Ns;
-    const Cx<T> *s = src + line * n;
-    Cx<T> *d = dst + line * n;
-    Cx<T> v[R];
+__device__ __forceinline__ void fft_pass(Cx<T> *buf, const FftLines &f, int n, int Ns, unsigned magic,
+                                         const Cx<T> *tw) {
+  constexpr int NB = (kFftPerThread + R - 1) / R;
+  const int line = threadIdx.x & ((1 << f.llog) - 1), tb = threadIdx.x >> f.llog, step = blockDim.x >> f.llog;
+  const int nbut = n / R, tstep = n / (Ns * R);
+  Cx<T> v[NB][R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      v[r] = s[j + r * nbut];
-      if (r > 0 && k > 0) v[r] = cmul(v[r], tw[k * r * tstep]);
+  for (int m = 0; m < NB; ++m) {
+    const int j = tb + m * step;
+    if (line < f.lines && j < nbut) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[m][r] = buf[line * f.ls + (j + r * nbut) * f.es];
+      if (Ns > 1) {
+        const int k = (j - div_by(j, magic) * Ns) * tstep;
+#pragma unroll
+        for (int r = 1; r < R; ++r) v[m][r] = cmul(v[m][r], tw[k * r]);
+      }
+      dft_small<R, T>(v[m]);
     }
-    dft_small<R, T>(v);
-    const int idxD = (j - k) * R + k;
-#pragma unroll
-    for (int r = 0; r < R; ++r) d[idxD + r * Ns] = v[r];
   }
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < NB; ++m) {
+    const int j = tb + m * step;
+    if (line < f.lines && j < nbut) {
+      const int k = Ns > 1 ? j - div_by(j, magic) * Ns : 0;
+      Cx<T> *d = buf + line * f.ls + ((j - k) * R + k) * f.es;
+#pragma unroll
+      for (int r = 0; r < R; ++r) d[r * Ns * f.es] = v[m][r];
+    }
+  }
+  __syncthreads();
 }
 
-// Batched forward Stockham FFT of `nb` lines of length plan.n in LDS
-// (a -> b ping-pong); twiddle table tw[m] = e^{-2 pi i m/n}.  Returns the
-// buffer holding the result.  All threads of the block participate.
+// Forward transforms of the lines in place (blockDim.x >> f.llog threads per
+// line, at least n / kFftPerThread; tw in LDS).  All threads of the block take part;
+// the data are in place before the call and after it.
 template <class T>
-__device__ Cx<T> *lds_fft(Cx<T> *a, Cx<T> *b, int nb, const FftPlan &pl, const Cx<T> *__restrict__ tw) {
-  const int n = pl.n;
+__device__ __forceinline__ void lds_fft(Cx<T> *buf, const FftLines &f, const FftPlan &pl, const Cx<T> *tw) {
   int Ns = 1;
   for (int s = 0; s < pl.nrad; ++s) {
-    const int R = pl.rad[s];
-    if (R == 4)
-      fft_pass<4, T>(a, b, nb, n, Ns, tw);
-    else if (R == 2)
-      fft_pass<2, T>(a, b, nb, n, Ns, tw);
-    else if (R == 3)
-      fft_pass<3, T>(a, b, nb, n, Ns, tw);
-    else
-      fft_pass<5, T>(a, b, nb, n, Ns, tw);
-    __syncthreads();
-    Cx<T> *tmp = a;
-    a = b;
-    b = tmp;
+    const unsigned mg = pl.magic[s];
+    const int R = __builtin_amdgcn_readfirstlane(pl.rad[s]);
+    switch (R) {
+      case 2: fft_pass<2, T>(buf, f, pl.n, Ns, mg, tw); break;
+      case 3: fft_pass<3, T>(buf, f, pl.n, Ns, mg, tw); break;
+      case 4: fft_pass<4, T>(buf, f, pl.n, Ns, mg, tw); break;
+      case 5: fft_pass<5, T>(buf, f, pl.n, Ns, mg, tw); break;
+      case 6: fft_pass<6, T>(buf, f, pl.n, Ns, mg, tw); break;
+      case 8: fft_pass<8, T>(buf, f, pl.n, Ns, mg, tw); break;
+      case 9: fft_pass<9, T>(buf, f, pl.n, Ns, mg, tw); break;
+      default: fft_pass<10, T>(buf, f, pl.n, Ns, mg, tw); break;
+    }
     Ns *= R;
   }
-  return a;
 }
 
-// The 3-D FFT passes move the data between three layouts so that every pass
-// reads and writes whole lines: the charge grid and the real potential are
-// [i][j][k] (k fastest); the half spectrum is SA = [i][k][j] after the z pass
-// and SB = [k][j][i] after the y pass.  A block takes a few consecutive lines
-// (TY, TI or TJ), so the transposing reads and writes move segments of that
-// many consecutive elements.
+template <class T>
+__device__ __forceinline__ void lds_twiddles(Cx<T> *s_tw, const Cx<T> *__restrict__ tw, int n) {
+  for (int t = threadIdx.x; t < n; t += blockDim.x) s_tw[t] = tw[t];
+}
 
-// z pass, real -> half complex, for the TY lines (i, j0 .. j0 + TY - 1):
-// the grid points are read once and cleared for the next spread; out: SA.
-template <class T, bool FIXED>
-__device__ __forceinline__ void fft_z_r2c_body(const int bid_, const int nbk_, const PmeParams &p, const FftPlan &pl,
-                                               int TY, double *__restrict__ g64, unsigned long long *__restrict__ gfx,
-                                               const Cx<T> *__restrict__ tw, Cx<T> *__restrict__ sa) {
-  extern __shared__ unsigned char smem_raw[];
-  Cx<T> *a = reinterpret_cast<Cx<T> *>(smem_raw);
-  Cx<T> *b = a + TY * p.nz;
-  const int jt = (p.ny + TY - 1) / TY;
-  const int i = bid_ / jt, j0 = (bid_ - i * jt) * TY;
-  const int nb = min(TY, p.ny - j0);
-  const size_t base = ((size_t)i * p.ny + j0) * p.nz;
-  for (int t = threadIdx.x; t < nb * p.nz; t += blockDim.x) {
-    T v;
-    if (FIXED) {
-      v = (T)((double)(long long)gfx[base + t] * (1.0 / kGridScale));
-      gfx[base + t] = 0ull;
-    } else {
-      v = (T)g64[base + t];
-      g64[base + t] = 0.0;
+// Calls work(cnt, slot) for the atoms whose stencils touch the tile (i0, j0),
+// up to 64 of them at a time on one wave (lanes below cnt hold a slot).
+// Waves take the superclusters of the tile's columns in turn.
+template <int P, class WORK>
+__device__ __forceinline__ void pme_tile_atoms(const PmeParams &p, const int2 *__restrict__ tcol, int tix, int tjy,
+                                               const int *__restrict__ colsc, const int2 *__restrict__ pmb,
+                                               int (*s_q)[128], WORK work) {
+  const int lane = threadIdx.x & 63, nw = blockDim.x >> 6;
+  const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int i0 = tix * p.tx, j0 = tjy * p.ty;
+  const int2 cx = tcol[tix], cy = tcol[p.ntx + tjy];  // first column and column count
+  int *const q = s_q[wv];
+  int qn = 0;                   // queued slots
+  int r = -1;                   // range of superclusters: column a = r / 2 of the x window, part r & 1 in y
+  int sc = 0, s1 = 0;           // the range's next supercluster and its end
+  int turn = wv;                // superclusters until this wave's next
+  bool more = true;
+  while (true) {
+    while (more && qn < kWave) {
+      while (sc + turn >= s1) {
+        turn -= s1 - sc;
+        sc = s1 = 0;
+        if (++r >= 2 * cx.y) {
+          more = false;
+          break;
+        }
+        const int col = wrap_grid(cx.x + (r >> 1), p.ncx) * p.ncy;
+        const int y0 = (r & 1) ? 0 : cy.x, y1 = (r & 1) ? cy.x + cy.y - p.ncy : min(cy.x + cy.y, p.ncy);
+        if (y1 <= y0) continue;
+        sc = __builtin_amdgcn_readfirstlane(colsc[col + y0]);
+        s1 = __builtin_amdgcn_readfirstlane(colsc[col + y1]);
+      }
+      if (!more) break;
+      const int s = (sc + turn) * kSuperSize + lane;
+      sc += nw;
+      const int b = pmb[s].x;
+      int ex = (b & 0xffff) - (i0 - P + 1), ey = (b >> 16) - (j0 - P + 1);
+      ex -= ex >= p.nx ? p.nx : 0;
+      ex += ex < 0 ? p.nx : 0;
+      ey -= ey >= p.ny ? p.ny : 0;
+      ey += ey < 0 ? p.ny : 0;
+      const bool hit = b != kNoGrid && ex < p.tx + P - 1 && ey < p.ty + P - 1;
+      const unsigned long long m = __ballot(hit);
+      if (hit) q[qn + __popcll(m & ((1ull << lane) - 1ull))] = s;
+      qn += __popcll(m);
     }
-    a[t] = Cx<T>{v, (T)0};
+    if (qn == 0) break;
+    const int cnt = min(qn, kWave);
+    __builtin_amdgcn_wave_barrier();
+    const int mine = q[lane < cnt ? lane : 0], rest = q[kWave + (lane < qn - cnt ? lane : 0)];
+    __builtin_amdgcn_wave_barrier();
+    if (lane < qn - cnt) q[lane] = rest;
+    qn -= cnt;
+    work(cnt, mine);
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+// Line stride of a tile in LDS: nz points, and the p - 1 points after the
+// last that the stencils of the last cells reach (copies of the first points:
+// a stencil's z points then lie at fixed offsets from its first), made odd.
+__host__ __device__ constexpr int pme_line(int nz, int order) { return (nz + order - 1) | 1; }
+
+// Transforms of all of a tile's np line pairs, as many at a time as the block
+// holds points for.
+template <class T>
+__device__ __forceinline__ void pme_tile_fft(Cx<T> *buf, int np, int n, int ls, const FftPlan &pl, const Cx<T> *tw) {
+  const int need = n > kFftPerThread ? 32 - __clz((n - 1) / kFftPerThread) : 0;  // log2 of a line's threads
+  const int llog = min(31 - __clz(np), 31 - __clz((int)blockDim.x) - need);
+  for (int l0 = 0; l0 < np; l0 += 1 << llog)
+    lds_fft<T>(buf + l0 * ls, FftLines{llog, min(1 << llog, np - l0), ls, 1}, pl, tw);
+}
+
+// Fixed-point charge sums: a double holding a multiple of 2^-40 below 2^12
+// in size adds exactly, so sums of charges rounded to that grid do not depend
+// on the order of the adds (an LDS ds_add_f64 instead of the conversions to
+// and from int64).
+constexpr double kGridRound = 6144.0;  // 1.5 2^12: its last bit is 2^-40
+
+// Spread and z transform of one tile (see above).  Bound by VALU and LDS
+// atomics: each lane takes one atom and walks the stencil rows inside the
+// tile.  Two real lines share one complex transform.  On small grids the
+// block's own latency bounds it: 9.5 us at 30^3 points and 1,500 atoms, where
+// the spread (in the kick-drift launch) and the z transform took 7 + 5.6 us
+// and a launch gap.
+template <bool MIXED, int P>
+__device__ __forceinline__ void pme_spread_z_body(
+    const int bid_, const int nbk_, const PmeParams &p, const FftPlan &pl, const int2 *__restrict__ tcol,
+    const int *__restrict__ colsc,
+    const typename Real4<typename std::conditional<MIXED, float, double>::type>::type *__restrict__ pmw,
+    const int2 *__restrict__ pmb, const Cx<typename std::conditional<MIXED, float, double>::type> *__restrict__ tw,
+    Cx<typename std::conditional<MIXED, float, double>::type> *__restrict__ spec) {
+  using T = typename std::conditional<MIXED, float, double>::type;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  __shared__ int s_q[kPmeBlock / kWave][128];
+  Cx<T> *const s_tw = reinterpret_cast<Cx<T> *>(smem_raw);
+  // sums of lines 2 l and 2 l + 1 interleaved at l, in the order of the
+  // complex lines they become
+  double *const acc = reinterpret_cast<double *>(s_tw + ((p.nz + 1) & ~1));
+  Cx<T> *const buf = reinterpret_cast<Cx<T> *>(acc);
+  const int nzs = pme_line(p.nz, P), lines = p.tx * p.ty;
+  const int tjy = bid_ / p.ntx, tix = bid_ - tjy * p.ntx;
+  const int i0 = tix * p.tx, j0 = tjy * p.ty;
+  lds_twiddles(s_tw, tw, p.nz);
+  for (int t = threadIdx.x; t < lines * nzs; t += blockDim.x) acc[t] = 0.0;
+  __syncthreads();
+  pme_tile_atoms<P>(p, tcol, tix, tjy, colsc, pmb, s_q, [&](int cnt, int slot) {
+    if ((int)(threadIdx.x & 63) >= cnt) return;
+    const auto a = pmw[slot];
+    const int2 b = pmb[slot];
+    T wx[P], wy[P], wz[P], dd[P];
+    bspline_w<P, T>(a.x, wx, dd);
+    bspline_w<P, T>(a.y, wy, dd);
+    bspline_w<P, T>(a.z, wz, dd);
+    const int bx = (b.x & 0xffff), by = b.x >> 16;
+#pragma unroll
+    for (int i = 0; i < P; ++i) {
+      const int li = wrap_grid(bx + i, p.nx) - i0;
+      if ((unsigned)li >= (unsigned)p.tx) continue;
+      const T qx = a.w * wx[i];
+#pragma unroll
+      for (int j = 0; j < P; ++j) {
+        const int lj = wrap_grid(by + j, p.ny) - j0;
+        if ((unsigned)lj >= (unsigned)p.ty) continue;
+        const T qxy = qx * wy[j];
+        const int line = lj * p.tx + li;
+        double *const row = acc + ((line >> 1) * nzs + b.y) * 2 + (line & 1);
+#pragma unroll
+        for (int k = 0; k < P; ++k) {
+          double v = (double)(qxy * wz[k]);
+          if (MIXED) v = (v + kGridRound) - kGridRound;
+          unsafeAtomicAdd(&row[2 * k], v);
+        }
+      }
+    }
+  });
+  __syncthreads();
+  // the points past the end belong to the first ones
+  for (int t = threadIdx.x; t < lines * (P - 1); t += blockDim.x) {
+    const int k = t / lines, line = t - k * lines, z = (line >> 1) * nzs * 2 + (line & 1);
+    int g = k;  // nz may be smaller than p - 1
+    while (g >= p.nz) g -= p.nz;
+    unsafeAtomicAdd(&acc[z + 2 * g], acc[z + 2 * (p.nz + k)]);
   }
   __syncthreads();
-  const Cx<T> *r = lds_fft<T>(a, b, nb, pl, tw);
-  for (int t = threadIdx.x; t < nb * p.nzh; t += blockDim.x) {
-    const int k = t / nb, jj = t - k * nb;
-    sa[((size_t)i * p.nzh + k) * p.ny + j0 + jj] = r[jj * p.nz + k];
+  // lines 2 l and 2 l + 1 are the real and imaginary part of transform l
+  const int np = lines >> 1, nplog = 31 - __clz(np);
+  if (MIXED) {
+    // to FP32 in place, through registers; what a round writes lies below
+    // what later rounds read
+    const double2 *const a2 = reinterpret_cast<const double2 *>(acc);
+    for (int e0 = threadIdx.x; e0 - (int)threadIdx.x < np * nzs; e0 += 4 * blockDim.x) {
+      Cx<T> v[4];
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        const int e = e0 + m * blockDim.x;
+        if (e < np * nzs) v[m] = Cx<T>{(T)a2[e].x, (T)a2[e].y};
+      }
+      __syncthreads();
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        const int e = e0 + m * blockDim.x;
+        if (e < np * nzs) buf[e] = v[m];
+      }
+    }
+    __syncthreads();
+  }
+  pme_tile_fft<T>(buf, np, p.nz, nzs, pl, s_tw);
+  const int hlog = 31 - __clz(p.tx) - 1;  // line pairs per row of the tile: tx / 2
+  for (int t = threadIdx.x; t < p.nzh << nplog; t += blockDim.x) {
+    const int l = t & (np - 1), k = t >> nplog;
+    const int i = i0 + 2 * (l & ((1 << hlog) - 1)), j = j0 + (l >> hlog);
+    if (i >= p.nx || j >= p.ny) continue;
+    const Cx<T> u = buf[l * nzs + k], v = buf[l * nzs + (k ? p.nz - k : 0)];
+    Cx<T> *o = spec + ((size_t)k * p.ny + j) * p.nx + i;
+    o[0] = Cx<T>{(T)0.5 * (u.x + v.x), (T)0.5 * (u.y - v.y)};
+    if (i + 1 < p.nx) o[1] = Cx<T>{(T)0.5 * (u.y + v.y), (T)0.5 * (v.x - u.x)};
   }
 }
 
-template <class T, bool FIXED>
-__global__ void k_fft_z_r2c(PmeParams p, FftPlan pl, int TY, double *__restrict__ g64,
-                            unsigned long long *__restrict__ gfx, const Cx<T> *__restrict__ tw, Cx<T> *__restrict__ sa) {
-  fft_z_r2c_body<T, FIXED>(blockIdx.x, gridDim.x, p, pl, TY, g64, gfx, tw, sa);
+template <bool MIXED, int P>
+__global__ void __launch_bounds__(kPmeBlock, MIXED ? 8 : 4) k_pme_spread_z(
+    PmeParams p, FftPlan pl, const int2 *__restrict__ tcol, const int *__restrict__ colsc,
+    const typename Real4<typename std::conditional<MIXED, float, double>::type>::type *__restrict__ pmw,
+    const int2 *__restrict__ pmb, const Cx<typename std::conditional<MIXED, float, double>::type> *__restrict__ tw,
+    Cx<typename std::conditional<MIXED, float, double>::type> *__restrict__ spec) {
+  // the blocks of one XCD take a contiguous range of tiles
+  pme_spread_z_body<MIXED, P>(xcd_block(blockIdx.x, gridDim.x), gridDim.x, p, pl, tcol, colsc, pmw, pmb, tw, spec);
 }
 
-// y pass for the TI lines (i0 .. i0 + TI - 1, k): forward SA -> SB; inverse
-// (conj-in / conj-out around the forward transform) SB -> SA.
+// y pass of the lines (k, i0 .. i0 + (1 << llog) - 1), in place: forward, or
+// inverse (conj-in / conj-out around the forward transform).  Bound by memory
+// on large grids: 0.21 -> 0.058 ms for 2 x 50 MB (216 x 240 x 240, beside the
+// pair kernel).
 template <class T>
 __device__ __forceinline__ void fft_y_body(const int bid_, const int nbk_, const PmeParams &p, const FftPlan &pl,
-                                           int TI, bool inverse, const Cx<T> *__restrict__ tw,
-                                           const Cx<T> *__restrict__ src, Cx<T> *__restrict__ dst) {
-  extern __shared__ unsigned char smem_raw[];
-  Cx<T> *a = reinterpret_cast<Cx<T> *>(smem_raw);
-  Cx<T> *b = a + TI * p.ny;
-  const int it = (p.nx + TI - 1) / TI;
-  const int k = bid_ / it, i0 = (bid_ - k * it) * TI;
-  const int nb = min(TI, p.nx - i0);
-  if (!inverse) {
-    for (int t = threadIdx.x; t < nb * p.ny; t += blockDim.x) {
-      const int ii = t / p.ny, j = t - ii * p.ny;
-      a[t] = src[((size_t)(i0 + ii) * p.nzh + k) * p.ny + j];
+                                           int llog, bool inverse, const Cx<T> *__restrict__ tw,
+                                           Cx<T> *__restrict__ spec) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  Cx<T> *const s_tw = reinterpret_cast<Cx<T> *>(smem_raw);
+  Cx<T> *const buf = s_tw + p.ny;
+  const int it = (p.nx + (1 << llog) - 1) >> llog;
+  const int k = bid_ / it, i0 = (bid_ - k * it) << llog;
+  const FftLines f{llog, min(1 << llog, p.nx - i0), p.ny | 1, 1};
+  Cx<T> *const g = spec + (size_t)k * p.ny * p.nx + i0;
+  lds_twiddles(s_tw, tw, p.ny);
+  const int l = threadIdx.x & ((1 << llog) - 1);
+  if (l < f.lines)
+    for (int j = threadIdx.x >> llog; j < p.ny; j += blockDim.x >> llog) {
+      Cx<T> v = g[(size_t)j * p.nx + l];
+      if (inverse) v.y = -v.y;
+      buf[l * f.ls + j] = v;
     }
-  } else {
-    for (int t = threadIdx.x; t < nb * p.ny; t += blockDim.x) {
-      const int j = t / nb, ii = t - j * nb;
-      Cx<T> v = src[((size_t)k * p.ny + j) * p.nx + i0 + ii];
-      v.y = -v.y;
-      a[ii * p.ny + j] = v;
-    }
-  }
   __syncthreads();
-  const Cx<T> *r = lds_fft<T>(a, b, nb, pl, tw);
-  if (!inverse) {
-    for (int t = threadIdx.x; t < nb * p.ny; t += blockDim.x) {
-      const int j = t / nb, ii = t - j * nb;
-      dst[((size_t)k * p.ny + j) * p.nx + i0 + ii] = r[ii * p.ny + j];
+  lds_fft<T>(buf, f, pl, s_tw);
+  if (l < f.lines)
+    for (int j = threadIdx.x >> llog; j < p.ny; j += blockDim.x >> llog) {
+      Cx<T> v = buf[l * f.ls + j];
+      if (inverse) v.y = -v.y;
+      g[(size_t)j * p.nx + l] = v;
     }
-  } else {
-    for (int t = threadIdx.x; t < nb * p.ny; t += blockDim.x) {
-      const int ii = t / p.ny, j = t - ii * p.ny;
-      Cx<T> v = r[t];
-      v.y = -v.y;
-      dst[((size_t)(i0 + ii) * p.nzh + k) * p.ny + j] = v;
-    }
-  }
 }
 
 template <class T>
-__global__ void k_fft_y(PmeParams p, FftPlan pl, int TI, bool inverse, const Cx<T> *__restrict__ tw,
-                        const Cx<T> *__restrict__ src, Cx<T> *__restrict__ dst) {
-  fft_y_body<T>(blockIdx.x, gridDim.x, p, pl, TI, inverse, tw, src, dst);
+__global__ void __launch_bounds__(kPmeBlock, kPmeWaves<T>) k_fft_y(PmeParams p, FftPlan pl, int llog, bool inverse,
+                                                     const Cx<T> *__restrict__ tw, Cx<T> *__restrict__ spec) {
+  fft_y_body<T>(xcd_block(blockIdx.x, gridDim.x), gridDim.x, p, pl, llog, inverse, tw, spec);
 }
 
-// x pass for the TJ lines (k, j0 .. j0 + TJ - 1) of SB, in place: forward
-// FFT, influence function multiply with the energy (Grid.h:237-341; theta in
-// the SB layout), inverse FFT.
+// Weight of plane k of the half spectrum in the energy.
+__device__ inline double plane_weight(const PmeParams &p, int k) {
+  return (k > 0 && ((k != p.nz / 2) || (p.nz & 1))) ? 2.0 : 1.0;
+}
+
+// The block's energy sum into epart[bid].
+__device__ __forceinline__ void block_energy(double e, double *epart) {
+  __shared__ double s_e[1024 / kWave];
+  e = wave_sum(e);
+  if ((threadIdx.x & 63) == 0) s_e[threadIdx.x >> 6] = e;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double tot = 0;
+    for (int w = 0; w < (int)(blockDim.x / kWave); ++w) tot += s_e[w];
+    *epart = tot;
+  }
+}
+
+// Influence function on one element (Grid.h:237-341; theta [k][j][i]): the
+// energy term, and the product conjugated for the inverse transform.
+template <class T>
+__device__ inline double convolve(Cx<T> &v, T th) {
+  const double e = (double)th * ((double)v.x * (double)v.x + (double)v.y * (double)v.y);
+  v = Cx<T>{v.x * th, -(v.y * th)};
+  return e;
+}
+
+// x pass of the lines (k, j0 .. j0 + (1 << llog) - 1), in place: forward
+// transform, influence function with the energy, inverse transform.  The
+// energy is summed over `threads` threads (the block may be larger in a
+// batched launch), so it does not depend on the batch.  0.49 -> 0.11 ms for
+// 125 MB on that grid: radices up to 10 in registers (three passes of LDS
+// instead of five), no division by a length, odd line strides.
 template <class T>
 __device__ __forceinline__ void fft_x_conv_body(const int bid_, const int nbk_, const PmeParams &p, const FftPlan &pl,
-                                                int TJ, const Cx<T> *__restrict__ tw, const T *__restrict__ theta,
-                                                Cx<T> *__restrict__ sb, double *__restrict__ epart) {
-  extern __shared__ unsigned char smem_raw[];
-  Cx<T> *a = reinterpret_cast<Cx<T> *>(smem_raw);
-  Cx<T> *b = a + TJ * p.nx;
-  __shared__ double s_e[1024 / kWave];
-  const int jt = (p.ny + TJ - 1) / TJ;
-  const int k = bid_ / jt, j0 = (bid_ - k * jt) * TJ;
-  const int nb = min(TJ, p.ny - j0);
+                                                int llog, int threads, const Cx<T> *__restrict__ tw,
+                                                const T *__restrict__ theta, Cx<T> *__restrict__ spec,
+                                                double *__restrict__ epart) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  Cx<T> *const s_tw = reinterpret_cast<Cx<T> *>(smem_raw);
+  Cx<T> *const buf = s_tw + p.nx;
+  const int jt = (p.ny + (1 << llog) - 1) >> llog;
+  const int k = bid_ / jt, j0 = (bid_ - k * jt) << llog;
+  const FftLines f{llog, min(1 << llog, p.ny - j0), p.nx | 1, 1};
+  const int pad = f.ls - p.nx;
   const size_t base = ((size_t)k * p.ny + j0) * p.nx;
-  for (int t = threadIdx.x; t < nb * p.nx; t += blockDim.x) a[t] = sb[base + t];
+  lds_twiddles(s_tw, tw, p.nx);
+  for (int t = threadIdx.x; t < f.lines * p.nx; t += blockDim.x)
+    buf[t + pad * div_by(t, pl.magic_n)] = spec[base + t];
   __syncthreads();
-  Cx<T> *r = lds_fft<T>(a, b, nb, pl, tw);
-  const double wgt = (k > 0 && ((k != p.nz / 2) || (p.nz & 1))) ? 2.0 : 1.0;
   double e = 0.0;
-  for (int t = threadIdx.x; t < nb * p.nx; t += blockDim.x) {
-    const T th = theta[base + t];
-    const Cx<T> v = r[t];
-    e += (double)th * ((double)v.x * (double)v.x + (double)v.y * (double)v.y);
-    // conj for the inverse transform (conj-in / conj-out)
-    r[t] = Cx<T>{v.x * th, -(v.y * th)};
+  for (int back = 0; back < 2; ++back) {
+    lds_fft<T>(buf, f, pl, s_tw);
+    if (back) break;
+    for (int t = threadIdx.x; (int)threadIdx.x < threads && t < f.lines * p.nx; t += threads)
+      e += convolve<T>(buf[t + pad * div_by(t, pl.magic_n)], theta[base + t]);
+    __syncthreads();
   }
-  __syncthreads();
-  Cx<T> *o = (r == a) ? b : a;
-  const Cx<T> *r2 = lds_fft<T>(r, o, nb, pl, tw);
-  for (int t = threadIdx.x; t < nb * p.nx; t += blockDim.x) {
-    Cx<T> v = r2[t];
+  for (int t = threadIdx.x; t < f.lines * p.nx; t += blockDim.x) {
+    Cx<T> v = buf[t + pad * div_by(t, pl.magic_n)];
     v.y = -v.y;
-    sb[base + t] = v;
+    spec[base + t] = v;
   }
-  e = wave_sum(wgt * e);
-  if ((threadIdx.x & 63) == 0) s_e[threadIdx.x >> 6] = e;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double tot = 0;
-    for (int w = 0; w < (int)(blockDim.x / kWave); ++w) tot += s_e[w];
-    epart[bid_] = tot;
-  }
+  block_energy(plane_weight(p, k) * e, &epart[bid_]);
 }
 
 template <class T>
-__global__ void k_fft_x_conv(PmeParams p, FftPlan pl, int TJ, const Cx<T> *__restrict__ tw,
-                             const T *__restrict__ theta, Cx<T> *__restrict__ sb, double *__restrict__ epart) {
-  fft_x_conv_body<T>(blockIdx.x, gridDim.x, p, pl, TJ, tw, theta, sb, epart);
+__global__ void __launch_bounds__(kPmeBlock, kPmeWaves<T>) k_fft_x_conv(PmeParams p, FftPlan pl, int llog,
+                                                          const Cx<T> *__restrict__ tw, const T *__restrict__ theta,
+                                                          Cx<T> *__restrict__ spec, double *__restrict__ epart) {
+  fft_x_conv_body<T>(xcd_block(blockIdx.x, gridDim.x), gridDim.x, p, pl, llog, blockDim.x, tw, theta, spec, epart);
 }
-
-// Largest plane (nx ny points) that k_fft_plane_conv takes: two LDS copies
-// of 1,024 points take 16 KiB (mixed) or 32 KiB (FP64).  On larger planes
-// the three line launches, with many more blocks, are faster (measured on
-// 45 x 48 and 60 x 60 planes).
-constexpr int kFftPlanePoints = 1024;
 
 // The y pass, the x pass with the convolution and the inverse y pass of one
-// plane k of the half spectrum in one block (the work of k_fft_y, k_fft_x_conv
-// and k_fft_y in one launch, for small planes): SA plane k
-// is read as nx lines along y, transformed, transposed in LDS to ny lines
-// along x, transformed, multiplied by the influence function (energy summed
-// as in k_fft_x_conv), transformed back along x and, transposed, along y, and
-// written back to SA.  The conj-out of the inverse x transform and the
+// plane k in one block (for planes of at most kFftPlanePoints): the plane
+// stays in LDS, rows of odd length, so both directions are transformed in
+// place without a transpose.  18 -> 13 us at 30 x 30 points alone.  The conj-out of the inverse x transform and the
 // conj-in of the inverse y transform cancel, so only the last conj remains.
+constexpr int kFftPlanePoints = kFftMax;
 template <class T>
 __device__ __forceinline__ void fft_plane_conv_body(const int bid_, const int nbk_, const PmeParams &p,
-                                                    const FftPlan &ply, const FftPlan &plx,
+                                                    const FftPlan &ply, const FftPlan &plx, int threads,
                                                     const Cx<T> *__restrict__ twy, const Cx<T> *__restrict__ twx,
-                                                    const T *__restrict__ theta, Cx<T> *__restrict__ sa,
+                                                    const T *__restrict__ theta, Cx<T> *__restrict__ spec,
                                                     double *__restrict__ epart) {
-  extern __shared__ unsigned char smem_raw[];
-  const int nx = p.nx, ny = p.ny, nxy = nx * ny;
-  Cx<T> *const a = reinterpret_cast<Cx<T> *>(smem_raw);
-  Cx<T> *const b = a + nxy;
-  __shared__ double s_e[256 / kWave];
-  const int k = bid_;
-  for (int t = threadIdx.x; t < nxy; t += blockDim.x) {
-    const int i = t / ny, j = t - i * ny;
-    a[t] = sa[((size_t)i * p.nzh + k) * ny + j];
-  }
-  __syncthreads();
-  // forward y: lines i, layout [i][j]
-  Cx<T> *r = lds_fft<T>(a, b, nx, ply, twy);
-  Cx<T> *o = (r == a) ? b : a;
-  for (int t = threadIdx.x; t < nxy; t += blockDim.x) {
-    const int j = t / nx, i = t - j * nx;
-    o[t] = r[i * ny + j];
-  }
-  __syncthreads();
-  // forward x: lines j, layout [j][i] (the SB order of theta)
-  r = lds_fft<T>(o, r, ny, plx, twx);
-  const double wgt = (k > 0 && ((k != p.nz / 2) || (p.nz & 1))) ? 2.0 : 1.0;
-  const T *th_k = theta + (size_t)k * nxy;
-  double e = 0.0;
-  for (int t = threadIdx.x; t < nxy; t += blockDim.x) {
-    const T th = th_k[t];
-    const Cx<T> v = r[t];
-    e += (double)th * ((double)v.x * (double)v.x + (double)v.y * (double)v.y);
-    r[t] = Cx<T>{v.x * th, -(v.y * th)};  // conj-in of the inverse x transform
-  }
-  __syncthreads();
-  o = (r == a) ? b : a;
-  r = lds_fft<T>(r, o, ny, plx, twx);
-  o = (r == a) ? b : a;
-  for (int t = threadIdx.x; t < nxy; t += blockDim.x) {
-    const int i = t / ny, j = t - i * ny;
-    o[t] = r[j * nx + i];
-  }
-  __syncthreads();
-  // inverse y (forward transform of the conjugate), conj-out into SA
-  r = lds_fft<T>(o, r, nx, ply, twy);
-  for (int t = threadIdx.x; t < nxy; t += blockDim.x) {
-    const int i = t / ny, j = t - i * ny;
-    Cx<T> v = r[t];
-    v.y = -v.y;
-    sa[((size_t)i * p.nzh + k) * ny + j] = v;
-  }
-  e = wave_sum(wgt * e);
-  if ((threadIdx.x & 63) == 0) s_e[threadIdx.x >> 6] = e;
-  __syncthreads();
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  Cx<T> *const s_twx = reinterpret_cast<Cx<T> *>(smem_raw);
+  Cx<T> *const s_twy = s_twx + p.nx;
+  Cx<T> *const buf = s_twy + p.ny;
+  const int k = bid_, nxy = p.nx * p.ny, row = p.nx | 1, pad = row - p.nx;
+  const size_t base = (size_t)k * nxy;
+  lds_twiddles(s_twx, twx, p.nx);
+  lds_twiddles(s_twy, twy, p.ny);
+  for (int t = threadIdx.x; t < nxy; t += blockDim.x) buf[t + pad * div_by(t, plx.magic_n)] = spec[base + t];
+  __shared__ FftPlan s_pl[2];  // read by index: y, x
   if (threadIdx.x == 0) {
-    double tot = 0;
-    for (int w = 0; w < (int)(blockDim.x / kWave); ++w) tot += s_e[w];
-    epart[k] = tot;
-  }
-}
-
-template <class T>
-__global__ void __launch_bounds__(256) k_fft_plane_conv(PmeParams p, FftPlan ply, FftPlan plx,
-                                                        const Cx<T> *__restrict__ twy, const Cx<T> *__restrict__ twx,
-                                                        const T *__restrict__ theta, Cx<T> *__restrict__ sa,
-                                                        double *__restrict__ epart) {
-  fft_plane_conv_body<T>(blockIdx.x, gridDim.x, p, ply, plx, twy, twx, theta, sa, epart);
-}
-
-// z pass, half complex -> real for the TY lines (i, j0 .. j0 + TY - 1) of SA
-// (Hermitian completion along z, inverse sign); out: the real potential.
-template <class T>
-__device__ __forceinline__ void fft_z_c2r_body(const int bid_, const int nbk_, const PmeParams &p, const FftPlan &pl,
-                                               int TY, const Cx<T> *__restrict__ tw, const Cx<T> *__restrict__ sa,
-                                               T *__restrict__ greal) {
-  extern __shared__ unsigned char smem_raw[];
-  Cx<T> *a = reinterpret_cast<Cx<T> *>(smem_raw);
-  Cx<T> *b = a + TY * p.nz;
-  const int jt = (p.ny + TY - 1) / TY;
-  const int i = bid_ / jt, j0 = (bid_ - i * jt) * TY;
-  const int nb = min(TY, p.ny - j0);
-  for (int t = threadIdx.x; t < nb * p.nz; t += blockDim.x) {
-    const int k = t / nb, jj = t - k * nb;
-    Cx<T> v;
-    if (k < p.nzh) {
-      v = sa[((size_t)i * p.nzh + k) * p.ny + j0 + jj];
-      v.y = -v.y;  // conj-in
-    } else {
-      v = sa[((size_t)i * p.nzh + (p.nz - k)) * p.ny + j0 + jj];  // conj(conj(X[nz-k]))
-    }
-    a[jj * p.nz + k] = v;
+    s_pl[0] = ply;
+    s_pl[1] = plx;
   }
   __syncthreads();
-  const Cx<T> *r = lds_fft<T>(a, b, nb, pl, tw);
-  const size_t base = ((size_t)i * p.ny + j0) * p.nz;
-  for (int t = threadIdx.x; t < nb * p.nz; t += blockDim.x) greal[base + t] = r[t].x;
+  const int blog = 31 - __clz((int)blockDim.x);
+  double e = 0.0;
+  // y, x, (influence function) x, y
+  for (int turn = 0; turn < 4; ++turn) {
+    const bool y = turn == 0 || turn == 3;
+    const FftPlan &pl = s_pl[y ? 0 : 1];
+    const int n = y ? p.ny : p.nx, nlines = y ? p.nx : p.ny;
+    // as many lines at a time as leave n / kFftPerThread threads or more for each
+    const int nlog = nlines > 1 ? 32 - __clz(nlines - 1) : 0;
+    const int need = n > kFftPerThread ? 32 - __clz((n - 1) / kFftPerThread) : 0;
+    const int llog = min(nlog, blog - need);
+    if (turn == 2) {
+      for (int t = threadIdx.x; (int)threadIdx.x < threads && t < nxy; t += threads)
+        e += convolve<T>(buf[t + pad * div_by(t, plx.magic_n)], theta[base + t]);
+      __syncthreads();
+    }
+    for (int l0 = 0; l0 < nlines; l0 += 1 << llog)
+      lds_fft<T>(buf + l0 * (y ? 1 : row), FftLines{llog, min(1 << llog, nlines - l0), y ? 1 : row, y ? row : 1}, pl,
+                 y ? s_twy : s_twx);
+  }
+  for (int t = threadIdx.x; t < nxy; t += blockDim.x) {
+    Cx<T> v = buf[t + pad * div_by(t, plx.magic_n)];
+    v.y = -v.y;
+    spec[base + t] = v;
+  }
+  block_energy(plane_weight(p, k) * e, &epart[k]);
 }
 
 template <class T>
-__global__ void k_fft_z_c2r(PmeParams p, FftPlan pl, int TY, const Cx<T> *__restrict__ tw,
-                            const Cx<T> *__restrict__ sa, T *__restrict__ greal) {
-  fft_z_c2r_body<T>(blockIdx.x, gridDim.x, p, pl, TY, tw, sa, greal);
+__global__ void __launch_bounds__(kPmeBlock, kPmeWaves<T>) k_fft_plane_conv(
+    PmeParams p, FftPlan ply, FftPlan plx, const Cx<T> *__restrict__ twy, const Cx<T> *__restrict__ twx,
+    const T *__restrict__ theta, Cx<T> *__restrict__ spec, double *__restrict__ epart) {
+  fft_plane_conv_body<T>(blockIdx.x, gridDim.x, p, ply, plx, blockDim.x, twy, twx, theta, spec, epart);
 }
 
-// Force interpolation (Grid.h:159-189) into the sorted accumulators.  Lane
-// groups as in k_spread: each lane sums one (i, j) stencil row, the group
-// reduces with cross-lane adds and its first lane adds the atom's force.
+// Inverse z transform and force gather of one tile (Grid.h:159-189): the
+// potential of lines 2 l and 2 l + 1 is the real and the (negated) imaginary
+// part of transform l; each lane takes one atom, sums the stencil rows
+// inside the tile and adds the atom's force.
 template <bool MIXED, int P>
-__global__ void __launch_bounds__(256) k_gather(int n, int waves, PmeParams p, const double *__restrict__ xorig,
-                                                const int *__restrict__ perm, const double *__restrict__ q,
-                                                const typename std::conditional<MIXED, float, double>::type *__restrict__ greal,
-                                                typename AccT<MIXED>::type *__restrict__ facc) {
-  using R = typename std::conditional<MIXED, float, double>::type;
-  constexpr int TPA = pme_tpa(P);
-  const int gt = blockIdx.x * blockDim.x + threadIdx.x;
-  const int wave = gt >> 6, lane = gt & 63;
-  if (wave >= waves) return;  // whole waves only: the group reduction below needs every lane
-  const int r = lane % TPA;
-  const int s = (lane / TPA) * waves + wave;
-  R fx = 0, fy = 0, fz = 0;
-  int a = -1;
-  if (s < n) a = perm[s];  // n counts slots; padding slots have a < 0
-  if (a >= 0 && r < P * P) {
-    const int i = r / P, j = r - (r / P) * P;
-    int b[3];
-    double w[3];
-    grid_coord(xorig[3 * a], p.hxr, p.nx, p.offx, b[0], w[0]);
-    grid_coord(xorig[3 * a + 1], p.hyr, p.ny, p.offy, b[1], w[1]);
-    grid_coord(xorig[3 * a + 2], p.hzr, p.nz, p.offz, b[2], w[2]);
-    R tx[P], ty[P], tz[P], dx[P], dy[P], dz[P];
-    bspline_w<P, R>((R)w[0], tx, dx);
-    bspline_w<P, R>((R)w[1], ty, dy);
-    bspline_w<P, R>((R)w[2], tz, dz);
-    const R txi = pick<P>(tx, i), tyj = pick<P>(ty, j);
-    const R xij = pick<P>(dx, i) * tyj, yij = txi * pick<P>(dy, j), zij = txi * tyj;
-    const int i1 = wrap_grid(i + b[0], p.nx), j1 = wrap_grid(j + b[1], p.ny);
-    const size_t row = ((size_t)i1 * p.ny + j1) * p.nz;
-#pragma unroll
-    for (int kk = 0; kk < P; kk++) {
-      const int k1 = wrap_grid(kk + b[2], p.nz);
-      const R term = greal[row + k1];
-      fx -= term * xij * tz[kk];
-      fy -= term * yij * tz[kk];
-      fz -= term * zij * dz[kk];
-    }
-  }
-#pragma unroll
-  for (int m = 1; m < TPA; m <<= 1) {
-    fx += __shfl_xor(fx, m);
-    fy += __shfl_xor(fy, m);
-    fz += __shfl_xor(fz, m);
-  }
-  if (r == 0 && a >= 0) {
-    const R qa = (R)q[a];
-    AccT<MIXED>::add(&facc[3 * s], fx * (R)p.hxr * qa);
-    AccT<MIXED>::add(&facc[3 * s + 1], fy * (R)p.hyr * qa);
-    AccT<MIXED>::add(&facc[3 * s + 2], fz * (R)p.hzr * qa);
-  }
-}
-
-// Force interpolation through an LDS patch of the real potential: one block
-// takes kSpreadSlots consecutive sorted slots (a compact group of atoms, as
-// k_spread_patch); wave 0 finds their grid bases and the box of grid points
-// their stencils cover; the block loads that box once, then 8 lanes per atom
-// sum its P^2 stencil rows from LDS (row r on lane r mod 8), reduce across
-// the 8 lanes and add the force.  A group whose box exceeds the patch reads
-// the potential from the grid directly.  The grid is read about once per
-// block instead of once per atom's stencil row.
-template <bool MIXED, int P>
-__device__ __forceinline__ void gather_patch_body(const int bid_, const int nbk_, int n, PmeParams p,
-    const double *__restrict__ xorig, const int *__restrict__ perm, const double *__restrict__ q,
-    const typename std::conditional<MIXED, float, double>::type *__restrict__ greal,
+__device__ __forceinline__ void pme_z_gather_body(
+    const int bid_, const int nbk_, const PmeParams &p, const FftPlan &pl, const int2 *__restrict__ tcol,
+    const int *__restrict__ colsc,
+    const typename Real4<typename std::conditional<MIXED, float, double>::type>::type *__restrict__ pmw,
+    const int2 *__restrict__ pmb, const Cx<typename std::conditional<MIXED, float, double>::type> *__restrict__ tw,
+    const Cx<typename std::conditional<MIXED, float, double>::type> *__restrict__ spec,
     typename AccT<MIXED>::type *__restrict__ facc) {
-  using R = typename std::conditional<MIXED, float, double>::type;
-  constexpr int PMAX = spread_patch_max<P>();
-  constexpr int LPA = 8;  // lanes per atom
-  static_assert(kSpreadSlots * LPA == 256, "one block of 256 threads per group");
-  __shared__ R s_patch[PMAX];
-  __shared__ int s_rb[kSpreadSlots][3];  // base relative to the patch origin (direct: the plain base)
-  __shared__ R s_w[kSpreadSlots][3];
-  __shared__ int s_org[3], s_ext[3], s_direct, s_any;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int s0 = bid_ * kSpreadSlots;
-  const int K[3] = {p.nx, p.ny, p.nz};
-  if (wv == 0) {
-    const int t = lane;
-    const int sl = s0 + t;
-    const int a = (t < kSpreadSlots && sl < n) ? perm[sl] : -1;
-    int b[3] = {0, 0, 0};
-    double w[3] = {0, 0, 0};
-    if (a >= 0) {
-      grid_coord(xorig[3 * a], p.hxr, p.nx, p.offx, b[0], w[0]);
-      grid_coord(xorig[3 * a + 1], p.hyr, p.ny, p.offy, b[1], w[1]);
-      grid_coord(xorig[3 * a + 2], p.hzr, p.nz, p.offz, b[2], w[2]);
+  using T = typename std::conditional<MIXED, float, double>::type;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  __shared__ int s_q[kPmeBlock / kWave][128];
+  Cx<T> *const s_tw = reinterpret_cast<Cx<T> *>(smem_raw);
+  Cx<T> *const buf = s_tw + p.nz;
+  const int nzs = pme_line(p.nz, P), lines = p.tx * p.ty;
+  const int tjy = bid_ / p.ntx, tix = bid_ - tjy * p.ntx;
+  const int i0 = tix * p.tx, j0 = tjy * p.ty;
+  lds_twiddles(s_tw, tw, p.nz);
+  const int np = lines >> 1, nplog = 31 - __clz(np), hlog = 31 - __clz(p.tx) - 1;
+  for (int t = threadIdx.x; t < p.nzh << nplog; t += blockDim.x) {
+    const int l = t & (np - 1), k = t >> nplog;
+    const int i = i0 + 2 * (l & ((1 << hlog) - 1)), j = j0 + (l >> hlog);
+    Cx<T> a{(T)0, (T)0}, b{(T)0, (T)0};
+    if (i < p.nx && j < p.ny) {
+      const Cx<T> *o = spec + ((size_t)k * p.ny + j) * p.nx + i;
+      a = o[0];
+      if (i + 1 < p.nx) b = o[1];
     }
-    const unsigned long long ok = __ballot(a >= 0);
-    if (ok) {
-      const int first = __builtin_ctzll(ok);
-      int lo[3], hi[3], db[3], ref[3];
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        ref[k] = __shfl(b[k], first);
-        int d = b[k] - ref[k];  // on the periodic grid, nearest to the reference
-        d -= K[k] * (int)floorf(((float)d + 0.5f * (float)K[k]) / (float)K[k]);
-        db[k] = d;
-        lo[k] = a >= 0 ? d : 0x3fffffff;
-        hi[k] = a >= 0 ? d : -0x3fffffff;
-      }
-#pragma unroll
-      for (int m = 32; m >= 1; m >>= 1)
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-          lo[k] = min(lo[k], __shfl_xor(lo[k], m));
-          hi[k] = max(hi[k], __shfl_xor(hi[k], m));
-        }
-      const int ex = hi[0] - lo[0] + P, ey = hi[1] - lo[1] + P, ez = hi[2] - lo[2] + P;
-      const bool direct = ex > K[0] || ey > K[1] || ez > K[2] || (long long)ex * ey * ez > PMAX;
-      if (t < kSpreadSlots) {
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-          s_rb[t][k] = a < 0 ? -1 : (direct ? b[k] : db[k] - lo[k]);
-          s_w[t][k] = (R)w[k];
-        }
-      }
-      if (lane == 0) {
-#pragma unroll
-        for (int k = 0; k < 3; ++k) s_org[k] = ref[k] + lo[k];
-        s_ext[0] = ex;
-        s_ext[1] = ey;
-        s_ext[2] = ez;
-        s_direct = direct ? 1 : 0;
-        s_any = 1;
-      }
-    } else if (lane == 0) {
-      s_any = 0;
-    }
+    // the lines are real: k = 0 and the middle of an even line have no
+    // imaginary part
+    const bool self = k == 0 || 2 * k == p.nz;
+    if (self) a.y = b.y = (T)0;
+    // conj-in of a + i b, and of its Hermitian completion at nz - k
+    buf[l * nzs + k] = Cx<T>{a.x - b.y, -(a.y + b.x)};
+    if (!self) buf[l * nzs + p.nz - k] = Cx<T>{a.x + b.y, a.y - b.x};
   }
   __syncthreads();
-  if (!s_any) return;  // block-uniform: no atoms in this group
-  const bool direct = s_direct;
-  const int ex = s_ext[0], ey = s_ext[1], ez = s_ext[2];
-  if (!direct) {
-    const int vol = ex * ey * ez;
-    const int o0 = s_org[0], o1 = s_org[1], o2 = s_org[2];
-    for (int i = tid; i < vol; i += blockDim.x) {
-      const int x = i / (ey * ez), rem = i - x * (ey * ez), y = rem / ez, z = rem - y * ez;
-      s_patch[i] = greal[((size_t)wrap_grid(o0 + x, p.nx) * p.ny + wrap_grid(o1 + y, p.ny)) * p.nz +
-                         wrap_grid(o2 + z, p.nz)];
-    }
+  pme_tile_fft<T>(buf, np, p.nz, nzs, pl, s_tw);
+  for (int t = threadIdx.x; t < np * (P - 1); t += blockDim.x) {
+    const int l = t & (np - 1), k = t >> nplog;
+    int g = k;
+    while (g >= p.nz) g -= p.nz;
+    buf[l * nzs + p.nz + k] = buf[l * nzs + g];
   }
   __syncthreads();
-  const int t = tid / LPA, r0 = tid % LPA;  // atom t of the group, lane r0 of its 8
-  R fx = 0, fy = 0, fz = 0;
-  const int rb0 = s_rb[t][0], rb1 = s_rb[t][1], rb2 = s_rb[t][2];
-  if (rb0 >= 0) {
-    R tx[P], ty[P], tz[P], dx[P], dy[P], dz[P];
-    bspline_w<P, R>(s_w[t][0], tx, dx);
-    bspline_w<P, R>(s_w[t][1], ty, dy);
-    bspline_w<P, R>(s_w[t][2], tz, dz);
-    for (int rr = r0; rr < P * P; rr += LPA) {
-      const int i = rr / P, j = rr - (rr / P) * P;
-      const R txi = pick<P>(tx, i), tyj = pick<P>(ty, j);
-      const R xij = pick<P>(dx, i) * tyj, yij = txi * pick<P>(dy, j), zij = txi * tyj;
-      if (!direct) {
-        const R *row = s_patch + ((rb0 + i) * ey + (rb1 + j)) * ez + rb2;
+  const T *const pot = reinterpret_cast<const T *>(buf);
+  pme_tile_atoms<P>(p, tcol, tix, tjy, colsc, pmb, s_q, [&](int cnt, int slot) {
+    if ((int)(threadIdx.x & 63) >= cnt) return;
+    const auto a = pmw[slot];
+    const int2 b = pmb[slot];
+    T wx[P], wy[P], wz[P], dx[P], dy[P], dz[P];
+    bspline_w<P, T>(a.x, wx, dx);
+    bspline_w<P, T>(a.y, wy, dy);
+    bspline_w<P, T>(a.z, wz, dz);
+    const int bx = (b.x & 0xffff), by = b.x >> 16;
+    T fx = 0, fy = 0, fz = 0;
 #pragma unroll
-        for (int kk = 0; kk < P; kk++) {
-          const R term = row[kk];
-          fx -= term * xij * tz[kk];
-          fy -= term * yij * tz[kk];
-          fz -= term * zij * dz[kk];
-        }
-      } else {
-        const int i1 = wrap_grid(i + rb0, p.nx), j1 = wrap_grid(j + rb1, p.ny);
-        const size_t row = ((size_t)i1 * p.ny + j1) * p.nz;
+    for (int i = 0; i < P; ++i) {
+      const int li = wrap_grid(bx + i, p.nx) - i0;
+      if ((unsigned)li >= (unsigned)p.tx) continue;
+      T gx = 0, gy = 0, gz = 0;  // this x row of the stencil, without its x weights
 #pragma unroll
-        for (int kk = 0; kk < P; kk++) {
-          const R term = greal[row + wrap_grid(kk + rb2, p.nz)];
-          fx -= term * xij * tz[kk];
-          fy -= term * yij * tz[kk];
-          fz -= term * zij * dz[kk];
+      for (int j = 0; j < P; ++j) {
+        const int lj = wrap_grid(by + j, p.ny) - j0;
+        if ((unsigned)lj >= (unsigned)p.ty) continue;
+        const int line = lj * p.tx + li;
+        const T *const r = pot + ((line >> 1) * nzs + b.y) * 2 + (line & 1);
+        T s = 0, d = 0;
+#pragma unroll
+        for (int k = 0; k < P; ++k) {
+          const T v = r[2 * k];
+          s += v * wz[k];
+          d += v * dz[k];
         }
+        gx += wy[j] * s;
+        gy += dy[j] * s;
+        gz += wy[j] * d;
       }
+      // odd lines hold the negated potential
+      const T w = (li & 1) ? -wx[i] : wx[i], v = (li & 1) ? -dx[i] : dx[i];
+      fx -= v * gx;
+      fy -= w * gy;
+      fz -= w * gz;
     }
-  }
-#pragma unroll
-  for (int m = 1; m < LPA; m <<= 1) {
-    fx += __shfl_xor(fx, m);
-    fy += __shfl_xor(fy, m);
-    fz += __shfl_xor(fz, m);
-  }
-  const int sl = s0 + t;
-  if (r0 == 0 && rb0 >= 0) {
-    const R qa = (R)q[perm[sl]];
-    AccT<MIXED>::add(&facc[3 * sl], fx * (R)p.hxr * qa);
-    AccT<MIXED>::add(&facc[3 * sl + 1], fy * (R)p.hyr * qa);
-    AccT<MIXED>::add(&facc[3 * sl + 2], fz * (R)p.hzr * qa);
-  }
+    AccT<MIXED>::add(&facc[3 * slot], fx * (T)p.hxr * a.w);
+    AccT<MIXED>::add(&facc[3 * slot + 1], fy * (T)p.hyr * a.w);
+    AccT<MIXED>::add(&facc[3 * slot + 2], fz * (T)p.hzr * a.w);
+  });
 }
 
 template <bool MIXED, int P>
-__global__ void __launch_bounds__(256) k_gather_patch(int n, PmeParams p, const double *__restrict__ xorig,
-                                                      const int *__restrict__ perm, const double *__restrict__ q,
-                                                      const typename std::conditional<MIXED, float, double>::type
-                                                          *__restrict__ greal,
-                                                      typename AccT<MIXED>::type *__restrict__ facc) {
-  gather_patch_body<MIXED, P>(xcd_block(blockIdx.x, gridDim.x), gridDim.x, n, p, xorig, perm, q, greal, facc);
+__global__ void __launch_bounds__(kPmeBlock, MIXED ? 8 : 4) k_pme_z_gather(
+    PmeParams p, FftPlan pl, const int2 *__restrict__ tcol, const int *__restrict__ colsc,
+    const typename Real4<typename std::conditional<MIXED, float, double>::type>::type *__restrict__ pmw,
+    const int2 *__restrict__ pmb, const Cx<typename std::conditional<MIXED, float, double>::type> *__restrict__ tw,
+    const Cx<typename std::conditional<MIXED, float, double>::type> *__restrict__ spec,
+    typename AccT<MIXED>::type *__restrict__ facc) {
+  pme_z_gather_body<MIXED, P>(xcd_block(blockIdx.x, gridDim.x), gridDim.x, p, pl, tcol, colsc, pmw, pmb, tw, spec,
+                              facc);
 }
 
 // ---------------------------------------------------------------------------
@@ -3200,19 +3100,20 @@ __device__ __forceinline__ void kick_drift_body(const int bid_, const int nbk_, 
                                                 double *__restrict__ x, const double *__restrict__ xbuild,
                                                 typename Real4<R>::type *__restrict__ xs,
                                                 const double4 *__restrict__ xs64, const float4 *__restrict__ sorg,
-                                                unsigned int *__restrict__ dmax) {
+                                                unsigned int *__restrict__ dmax, const PmeParams &pme,
+                                                PmeSlots<R> rec) {
   const int s = bid_ * blockDim.x + threadIdx.x;
   float d2f = 0.f;
   const int a = s < n ? perm[s] : -1;  // n counts slots; padding slots have a < 0
   if (a >= 0) {
-    double dd[3], vv[3] = {v[3 * a], v[3 * a + 1], v[3 * a + 2]};
+    double dd[3], xn[3], vv[3] = {v[3 * a], v[3 * a + 1], v[3 * a + 2]};
     const double ff[3] = {fout[3 * a], fout[3 * a + 1], fout[3 * a + 2]};
     apply_kick(kk, a, ff, minv[a], vv);
     double d2 = 0;
     for (int k = 0; k < 3; ++k) {
       v[3 * a + k] = vv[k];
       const double xk = x[3 * a + k] + vv[k] * h;
-      x[3 * a + k] = xk;
+      x[3 * a + k] = xn[k] = xk;
       dd[k] = xk - xbuild[3 * a + k];
       d2 += dd[k] * dd[k];
     }
@@ -3224,6 +3125,7 @@ __device__ __forceinline__ void kick_drift_body(const int bid_, const int nbk_, 
     r.y = (R)((b.y + dd[1]) - (double)o.y);
     r.z = (R)((b.z + dd[2]) - (double)o.z);
     xs[s] = r;
+    if (rec.w) pme_record<R>(pme, rec, s, true, xn, b.w);
   }
   // wave max, one atomic per wave
   for (int m = 32; m >= 1; m >>= 1) d2f = fmaxf(d2f, __shfl_xor(d2f, m));
@@ -3235,8 +3137,10 @@ __global__ void k_kick_drift(int n, Kick kk, double h, const int *__restrict__ p
                              const double *__restrict__ fout, const double *__restrict__ minv, double *__restrict__ v,
                              double *__restrict__ x, const double *__restrict__ xbuild,
                              typename Real4<R>::type *__restrict__ xs, const double4 *__restrict__ xs64,
-                             const float4 *__restrict__ sorg, unsigned int *__restrict__ dmax) {
-  kick_drift_body<R>(blockIdx.x, gridDim.x, n, kk, h, perm, fout, minv, v, x, xbuild, xs, xs64, sorg, dmax);
+                             const float4 *__restrict__ sorg, unsigned int *__restrict__ dmax, PmeParams pme,
+                             PmeSlots<R> rec) {
+  kick_drift_body<R>(blockIdx.x, gridDim.x, n, kk, h, perm, fout, minv, v, x, xbuild, xs, xs64, sorg, dmax, pme,
+                     rec);
 }
 
 // The end of one MD step and the start of the next in one pass over the
@@ -3244,14 +3148,19 @@ __global__ void k_kick_drift(int n, Kick kk, double h, const int *__restrict__ p
 // pass counters) for the caller's atom order, and the next step's kick and
 // drift use them at once (k_unsort_forces followed by k_kick_drift).
 template <bool MIXED, class R>
-__global__ void k_unsort_kick_drift(int n, Kick kk, double h, const int *__restrict__ perm,
-                                    typename AccT<MIXED>::type *__restrict__ facc, double *__restrict__ fout,
-                                    int *__restrict__ tilectr, int *__restrict__ nborder,
-                                    const double *__restrict__ minv, double *__restrict__ v,
-                                    double *__restrict__ x, const double *__restrict__ xbuild,
-                                    typename Real4<R>::type *__restrict__ xs, const double4 *__restrict__ xs64,
-                                    const float4 *__restrict__ sorg, unsigned int *__restrict__ dmax) {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void unsort_kick_drift_body(const int bid_, const int nbk_, int n, const Kick &kk, double h,
+                                                       const int *__restrict__ perm,
+                                                       typename AccT<MIXED>::type *__restrict__ facc,
+                                                       double *__restrict__ fout, int *__restrict__ tilectr,
+                                                       int *__restrict__ nborder, const double *__restrict__ minv,
+                                                       double *__restrict__ v, double *__restrict__ x,
+                                                       const double *__restrict__ xbuild,
+                                                       typename Real4<R>::type *__restrict__ xs,
+                                                       const double4 *__restrict__ xs64,
+                                                       const float4 *__restrict__ sorg,
+                                                       unsigned int *__restrict__ dmax, const PmeParams &pme,
+                                                       PmeSlots<R> rec) {
+  const int s = bid_ * blockDim.x + threadIdx.x;
   if (s == 0) {
     *tilectr = 0;
     *nborder = 0;
@@ -3269,13 +3178,13 @@ __global__ void k_unsort_kick_drift(int n, Kick kk, double h, const int *__restr
       facc[3 * s + k] = 0;
       fout[3 * a + k] = ff[k];
     }
-    double dd[3], vv[3] = {v[3 * a], v[3 * a + 1], v[3 * a + 2]};
+    double dd[3], xn[3], vv[3] = {v[3 * a], v[3 * a + 1], v[3 * a + 2]};
     apply_kick(kk, a, ff, minv[a], vv);
     double d2 = 0;
     for (int k = 0; k < 3; ++k) {
       v[3 * a + k] = vv[k];
       const double xk = x[3 * a + k] + vv[k] * h;
-      x[3 * a + k] = xk;
+      x[3 * a + k] = xn[k] = xk;
       dd[k] = xk - xbuild[3 * a + k];
       d2 += dd[k] * dd[k];
     }
@@ -3287,91 +3196,23 @@ __global__ void k_unsort_kick_drift(int n, Kick kk, double h, const int *__restr
     r.y = (R)((b.y + dd[1]) - (double)o.y);
     r.z = (R)((b.z + dd[2]) - (double)o.z);
     xs[s] = r;
+    if (rec.w) pme_record<R>(pme, rec, s, true, xn, b.w);
   }
   for (int m = 32; m >= 1; m >>= 1) d2f = fmaxf(d2f, __shfl_xor(d2f, m));
   if ((threadIdx.x & 63) == 0) atomicMax(dmax, __float_as_uint(d2f));
 }
 
-// k_unsort_kick_drift and the charge spread of the next force pass in one
-// launch: block b takes the kSpreadSlots slots from 32 b; lanes 0..31 of wave
-// 0 unsort their slot's force, kick and drift its atom as k_unsort_kick_drift
-// does, and bring the new position to the group's spread (the grid was left
-// cleared by the previous pass).  Used inside an MD chunk, where the next
-// pass spreads these positions.
-template <bool MIXED, class R, int P>
-__device__ __forceinline__ void unsort_kick_drift_spread_body(const int bid_, const int nbk_, int n, Kick kk, double h,
-                                                              const int *__restrict__ perm,
-                                                              typename AccT<MIXED>::type *__restrict__ facc,
-                                                              double *__restrict__ fout, int *__restrict__ tilectr,
-                                                              int *__restrict__ nborder,
-                                                              const double *__restrict__ minv, double *__restrict__ v,
-                                                              double *__restrict__ x, const double *__restrict__ xbuild,
-                                                              typename Real4<R>::type *__restrict__ xs,
-                                                              const double4 *__restrict__ xs64,
-                                                              const float4 *__restrict__ sorg,
-                                                              unsigned int *__restrict__ dmax, PmeParams pme,
-                                                              const double *__restrict__ q, double *__restrict__ grid64,
-                                                              unsigned long long *__restrict__ gridfx) {
-  const int s0 = bid_ * kSpreadSlots;
-  const int t = threadIdx.x, s = s0 + t;
-  if (bid_ == 0 && t == 0) {
-    *tilectr = 0;
-    *nborder = 0;
-  }
-  int a = -1;
-  double xa[3] = {0, 0, 0};
-  if (t < kWave) {
-    float d2f = 0.f;
-    if (t < kSpreadSlots && s < n) a = perm[s];
-    if (a >= 0) {
-      double ff[3];
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        if (MIXED)
-          ff[k] = (double)(long long)facc[3 * s + k] * (1.0 / kForceScale);
-        else
-          ff[k] = ((const double *)facc)[3 * s + k];
-        facc[3 * s + k] = 0;
-        fout[3 * a + k] = ff[k];
-      }
-      double dd[3], vv[3] = {v[3 * a], v[3 * a + 1], v[3 * a + 2]};
-      apply_kick(kk, a, ff, minv[a], vv);
-      double d2 = 0;
-      for (int k = 0; k < 3; ++k) {
-        v[3 * a + k] = vv[k];
-        const double xk = x[3 * a + k] + vv[k] * h;
-        x[3 * a + k] = xk;
-        xa[k] = xk;
-        dd[k] = xk - xbuild[3 * a + k];
-        d2 += dd[k] * dd[k];
-      }
-      d2f = (float)d2;
-      const double4 b = xs64[s];
-      const float4 o = sorg[s / kSuperSize];
-      typename Real4<R>::type r = xs[s];
-      r.x = (R)((b.x + dd[0]) - (double)o.x);
-      r.y = (R)((b.y + dd[1]) - (double)o.y);
-      r.z = (R)((b.z + dd[2]) - (double)o.z);
-      xs[s] = r;
-    }
-    for (int m = 32; m >= 1; m >>= 1) d2f = fmaxf(d2f, __shfl_xor(d2f, m));
-    if (t == 0) atomicMax(dmax, __float_as_uint(d2f));
-  }
-  spread_patch_group<MIXED, P>(s0, pme, a, xa, q, grid64, gridfx);
-}
-
-template <bool MIXED, class R, int P>
-__global__ void __launch_bounds__(256) k_unsort_kick_drift_spread(
-    int n, Kick kk, double h, const int *__restrict__ perm, typename AccT<MIXED>::type *__restrict__ facc,
-    double *__restrict__ fout, int *__restrict__ tilectr, int *__restrict__ nborder, const double *__restrict__ minv,
-    double *__restrict__ v, double *__restrict__ x, const double *__restrict__ xbuild,
-    typename Real4<R>::type *__restrict__ xs, const double4 *__restrict__ xs64, const float4 *__restrict__ sorg,
-    unsigned int *__restrict__ dmax, PmeParams pme, const double *__restrict__ q, double *__restrict__ grid64,
-    unsigned long long *__restrict__ gridfx) {
-  // the blocks of one XCD take a contiguous range of slots
-  unsort_kick_drift_spread_body<MIXED, R, P>(xcd_block(blockIdx.x, gridDim.x), gridDim.x, n, kk, h, perm, facc, fout,
-                                             tilectr, nborder, minv, v, x, xbuild, xs, xs64, sorg, dmax, pme, q,
-                                             grid64, gridfx);
+template <bool MIXED, class R>
+__global__ void k_unsort_kick_drift(int n, Kick kk, double h, const int *__restrict__ perm,
+                                    typename AccT<MIXED>::type *__restrict__ facc, double *__restrict__ fout,
+                                    int *__restrict__ tilectr, int *__restrict__ nborder,
+                                    const double *__restrict__ minv, double *__restrict__ v,
+                                    double *__restrict__ x, const double *__restrict__ xbuild,
+                                    typename Real4<R>::type *__restrict__ xs, const double4 *__restrict__ xs64,
+                                    const float4 *__restrict__ sorg, unsigned int *__restrict__ dmax, PmeParams pme,
+                                    PmeSlots<R> rec) {
+  unsort_kick_drift_body<MIXED, R>(blockIdx.x, gridDim.x, n, kk, h, perm, facc, fout, tilectr, nborder, minv, v, x,
+                                   xbuild, xs, xs64, sorg, dmax, pme, rec);
 }
 
 // Start of an MD chunk in one launch: the committed state (x, v, f: m3 =
