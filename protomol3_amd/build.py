@@ -7,10 +7,16 @@ import subprocess
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 LIB = os.path.join(HERE, "lib", "libpmx.so")
-SOURCES = [os.path.join(HERE, "csrc", f) for f in ("pmx.hip", "pmx_kernels.h", "pmx_batch.h", "pmx_common.h")]
+SOURCES = [os.path.join(HERE, "csrc", f) for f in ("pmx.hip", "pmx_pair.hip", "pmx_pair.h", "pmx_kernels.h",
+                                                   "pmx_batch.h", "pmx_common.h")]
+# options of single files
+FILE_FLAGS = {
+    # see the head of the file
+    "pmx_pair.hip": ["-mllvm", "-structurizecfg-skip-uniform-regions"],
+}
 
 HIPCC_FLAGS = [
-    "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
+    "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
     "-munsafe-fp-atomics",
     # packed FP32 arithmetic is kept off (only scalar/FMA FP32 VALU forms)
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
@@ -20,9 +26,19 @@ HIPCC_FLAGS = [
 
 def build_lib(verbose: bool = False) -> str:
     os.makedirs(os.path.dirname(LIB), exist_ok=True)
-    cmd = ["hipcc", *HIPCC_FLAGS, "-I" + os.path.join(ROOT, "include"),
-           os.path.join(HERE, "csrc", "pmx.hip"), "-o", LIB + ".tmp"]
-    r = subprocess.run(cmd, capture_output=True, text=True)
+    jobs = []
+    for src in (s for s in SOURCES if s.endswith(".hip")):
+        obj = os.path.join(os.path.dirname(LIB), os.path.basename(src) + ".o")
+        cmd = ["hipcc", *HIPCC_FLAGS, *FILE_FLAGS.get(os.path.basename(src), []), "-I" + os.path.join(ROOT, "include"),
+               "-c", src, "-o", obj]
+        jobs.append((obj, subprocess.Popen(cmd, stdout=subprocess.DEVNULL, stderr=subprocess.PIPE, text=True)))
+    failed = [err for err in (p.communicate()[1] for _, p in jobs) if err and "error" in err]
+    if any(p.returncode for _, p in jobs):
+        raise RuntimeError("hipcc failed:\n" + "\n".join(failed)[-4000:])
+    r = subprocess.run(["hipcc", "--offload-arch=gfx950", "-fPIC", "-shared", *(obj for obj, _ in jobs),
+                        "-o", LIB + ".tmp"], capture_output=True, text=True)
+    for obj, _ in jobs:
+        os.remove(obj)
     if r.returncode != 0:
         raise RuntimeError("hipcc failed:\n" + r.stderr[-4000:])
     os.replace(LIB + ".tmp", LIB)

@@ -19,7 +19,7 @@
 
 #include "../../include/pmx.h"
 #include "pmx_kernels.h"
-#include "pmx_batch.h"
+#include "pmx_pair.h"
 
 using namespace pmx;
 
@@ -633,6 +633,28 @@ int setup(Sys *s) {
   lp.skin = (float)s->md.skin;
   lp.rlist2 = (float)((rcmax + margin + s->md.skin) * (rcmax + margin + s->md.skin));
   s->pp.prune_r2 = (double)lp.rlist2 * (1.0 + 1e-5);
+  {
+    DirectC &c = s->pp.dc;
+    c = DirectC{};
+    c.lj.load(pp.lj);
+    c.co.load(pp.co);
+    c.ljkind = pp.lj.kind;
+    c.cokind = pp.co.kind;
+    c.rmax2 = !pp.has_lj ? c.co.rc2 : (pp.coul == COUL_NONE ? c.lj.rc2 : std::max(c.lj.rc2, c.co.rc2));
+    c.guard = (float)pp.guard;
+    c.near2 = std::nextafter(c.rmax2 + c.guard, INFINITY);
+    c.in2 = std::nextafter(c.rmax2 - c.guard, 0.f);
+    c.pa = (float)(0.3275911 * pp.alpha);
+    c.ke = (float)(-1.4426950408889634 * pp.alpha * pp.alpha);
+    c.a2pi = (float)pp.a2pi;
+    c.csf = (float)pp.csf;
+    c.prune_r2 = (float)pp.prune_r2;
+    for (int k = 0; k < 3; ++k) {
+      c.hi[k] = (float)pp.Lhi[k];
+      c.lo[k] = (float)pp.Llo[k];
+      c.inv[k] = (float)bx.Linv[k];
+    }
+  }
   lp.rc = (float)rcmax;
   lp.ncl = s->ncl;
   lp.nsuper = s->nsuper;
@@ -854,14 +876,16 @@ int setup(Sys *s) {
 template <bool MIXED>
 FixupArgs<MIXED> fixup_args(Sys *s, bool stats, bool border_here, bool rest_here, int *nblocks);
 
-// Resident blocks per CU of a pair-kernel launch (at least 1, at most the
-// kernel's wave budget per CU); each caller keeps its kernel's value in a
-// function-local static, initialized once even under concurrent first calls.
+// Resident blocks per CU of a pair-kernel launch: at least 1, at most those
+// of kMinRuns waves on the device (the static schedule's runs are cut for
+// them; more would also leave the PME chain no room beside).  Each caller keeps its
+// kernel's value in a function-local static, initialized once even under
+// concurrent first calls.
 int pair_blocks_per_cu(const void *kernel) {
   int per_cu = 0;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kPairBlock, 0) != hipSuccess || per_cu < 1)
     per_cu = 1;
-  return std::min(per_cu, kMaxPairWavesPerCu / (kPairBlock / kWave));
+  return std::min(per_cu, kMinRuns / (kPairBlock / kWave) / 256);
 }
 
 template <bool MIXED, int C, int LJ, int CS, bool BIGLJ = false>

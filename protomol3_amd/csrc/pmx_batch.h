@@ -320,9 +320,14 @@ struct OpPair {
   static constexpr bool kGated = false;
   // the runs in contiguous shares per wave (schedule 0)
   __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &) {
-    pair_body<MIXED, COUL, LJSW, CSW, BIGLJ, kPairPlain>(bid, nbk, a.pp, 0, a.tiles, a.ntiles, a.wstart, a.tilectr,
-                                                         a.entries, a.entries, a.cap, a.masks, a.xs, a.sorg, a.ts,
-                                                         a.perm, a.ljtab, a.ljt, a.facc, a.out);
+    if constexpr (MIXED)
+      pair_direct_body<COUL, LJSW, CSW, BIGLJ, kPairPlain>(bid, nbk, a.pp, 0, a.tiles, a.ntiles, a.wstart, a.tilectr,
+                                                           a.entries, a.entries, a.cap, a.masks, a.xs, a.sorg, a.ts,
+                                                           a.perm, a.ljtab, a.ljt, a.facc, a.out);
+    else
+      pair_body<MIXED, COUL, LJSW, CSW, BIGLJ, kPairPlain>(bid, nbk, a.pp, 0, a.tiles, a.ntiles, a.wstart, a.tilectr,
+                                                           a.entries, a.entries, a.cap, a.masks, a.xs, a.sorg, a.ts,
+                                                           a.perm, a.ljtab, a.ljt, a.facc, a.out);
   }
 };
 
@@ -526,7 +531,7 @@ struct BatchSys {
 
 // need[s]: system s rebuilds its list at step k (first thread of each
 // system); the count of builds goes up.
-__global__ void k_batch_need(int nsys, const BatchSys *__restrict__ bs, int k, unsigned char *__restrict__ need) {
+static __global__ void k_batch_need(int nsys, const BatchSys *__restrict__ bs, int k, unsigned char *__restrict__ need) {
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= nsys) return;
   const BatchSys b = bs[s];
@@ -538,12 +543,12 @@ __global__ void k_batch_need(int nsys, const BatchSys *__restrict__ bs, int k, u
 
 // The chunk's first step index of every system (base[s]) and the overflow
 // flags of the last chunk gathered into one array for the host.
-__global__ void k_batch_steps(int nsys, const BatchSys *__restrict__ bs, const unsigned long long *__restrict__ base) {
+static __global__ void k_batch_steps(int nsys, const BatchSys *__restrict__ bs, const unsigned long long *__restrict__ base) {
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s < nsys) *bs[s].step_dev = base[s];
 }
 
-__global__ void k_batch_flags(int nsys, const BatchSys *__restrict__ bs, int *__restrict__ out) {
+static __global__ void k_batch_flags(int nsys, const BatchSys *__restrict__ bs, int *__restrict__ out) {
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s < nsys) out[s] = *bs[s].overflow;
 }

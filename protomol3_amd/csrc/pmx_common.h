@@ -9,7 +9,6 @@ namespace pmx {
 constexpr int kClusterSize = 8;    // atoms per cluster (one 8-lane group of a wave)
 constexpr int kSuperSize = 64;     // atoms per supercluster (8 clusters, one wave)
 constexpr int kTileEntries = 16;   // granularity of the per-supercluster list capacity
-constexpr int kMaxPairWavesPerCu = 32;  // resident pair-kernel waves per CU, at most
 // Work runs of the pair kernel: the list is cut into runs of equal estimated
 // work whose number depends only on the list (never on the device or the
 // launch shape): kMinRuns k, k = ceil(total work / (kMinRuns kRunCost)),
@@ -45,7 +44,44 @@ struct SwitchC {
   double rc2, on2, s1, s2, s3, c15_1, c05_3, c15_3;
 };
 
+// Switch constants in the arithmetic type of a kernel.
+template <class R>
+struct SwR {
+  R rc2, on2, s1, s2, s3, c15_1, c05_3, c15_3;
+  __host__ __device__ void load(const SwitchC &s) {
+    rc2 = (R)s.rc2;
+    on2 = (R)s.on2;
+    s1 = (R)s.s1;
+    s2 = (R)s.s2;
+    s3 = (R)s.s3;
+    c15_1 = (R)s.c15_1;
+    c05_3 = (R)s.c05_3;
+    c15_3 = (R)s.c15_3;
+  }
+};
+
+// Constants of the mixed pair kernel, in FP32 from the host: kernel arguments
+// stay in scalar registers (conversions in the kernel would hold thirty
+// vector registers).
+struct DirectC {
+  SwR<float> lj, co;
+  int ljkind, cokind;
+  // membership radius^2, guard band; with one cutoff a candidate below in2 is a
+  // member and one from in2 to near2 a boundary pair (rounded outwards: a pair
+  // that is in doubt is re-tested)
+  float rmax2, guard, in2, near2;
+  float pa, ke, a2pi, csf;        // 0.3275911 alpha, -alpha^2 log2(e), 2 alpha/sqrt(pi), 1-4 scaling
+  float prune_r2;
+  float hi[3], lo[3], inv[3];     // box edges (see PairParams::Lhi) and their reciprocals
+  // image k of a difference: d - k (hi + lo), hi exact
+  __device__ float image(float d, int ax) const {
+    const float k = rintf(d * inv[ax]);
+    return (d - k * hi[ax]) - k * lo[ax];
+  }
+};
+
 struct PairParams {
+  DirectC dc;
   Box box;
   SwitchC lj, co;
   double rc2max;     // membership radius^2 (max of the two cutoffs)

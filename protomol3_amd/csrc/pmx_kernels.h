@@ -212,7 +212,7 @@ __device__ __forceinline__ void bin_body(const int bid_, const int nbk_, int n, 
   refcell[a] = (c[0] * p.rc_n[1] + c[1]) * p.rc_n[2] + c[2];
 }
 
-__global__ void k_bin(int n, const double *__restrict__ xorig, BinParams p, uint32_t *__restrict__ key,
+static __global__ void k_bin(int n, const double *__restrict__ xorig, BinParams p, uint32_t *__restrict__ key,
                       double *__restrict__ xwrap, int *__restrict__ refcell, uint32_t *__restrict__ hist) {
   bin_body(blockIdx.x, gridDim.x, n, xorig, p, key, xwrap, refcell, hist);
 }
@@ -220,19 +220,19 @@ __global__ void k_bin(int n, const double *__restrict__ xorig, BinParams p, uint
 // Counting sort by key (one radix digit spanning the key range): histogram,
 // exclusive scan, scatter, then order each bin by atom index so the result is
 // deterministic and stable.
-__global__ void k_fill_u32(uint32_t *p, uint32_t v, long long n) {
+static __global__ void k_fill_u32(uint32_t *p, uint32_t v, long long n) {
   long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
 }
-__global__ void k_fill_i32(int *p, int v, long long n) {
+static __global__ void k_fill_i32(int *p, int v, long long n) {
   long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
 }
-__global__ void k_fill_u64(unsigned long long *p, unsigned long long v, long long n) {
+static __global__ void k_fill_u64(unsigned long long *p, unsigned long long v, long long n) {
   long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
 }
-__global__ void k_fill_f64(double *p, double v, long long n) {
+static __global__ void k_fill_f64(double *p, double v, long long n) {
   long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
 }
@@ -240,7 +240,7 @@ __global__ void k_fill_f64(double *p, double v, long long n) {
 // Exclusive scan of m uint32 in 3 launches: per-block sums, scan of sums in
 // one block, then per-block rescan with the block offset.
 constexpr int kScanBlock = 1024;
-__global__ void k_scan_blocksums(const uint32_t *__restrict__ in, long long m, uint32_t *__restrict__ sums) {
+static __global__ void k_scan_blocksums(const uint32_t *__restrict__ in, long long m, uint32_t *__restrict__ sums) {
   __shared__ uint32_t s[kScanBlock / kWave];
   long long i = (long long)blockIdx.x * kScanBlock + threadIdx.x;
   uint32_t v = i < m ? in[i] : 0u;
@@ -253,7 +253,7 @@ __global__ void k_scan_blocksums(const uint32_t *__restrict__ in, long long m, u
     sums[blockIdx.x] = t;
   }
 }
-__global__ void k_scan_sums(uint32_t *sums, int nb) {
+static __global__ void k_scan_sums(uint32_t *sums, int nb) {
   // single block: serial over chunks of 1024 with a block-wide scan
   __shared__ uint32_t s[kScanBlock];
   uint32_t carry = 0;
@@ -275,7 +275,7 @@ __global__ void k_scan_sums(uint32_t *sums, int nb) {
   }
 }
 // Exclusive scan result to out and to out2 (the scatter cursors).
-__global__ void k_scan_final(uint32_t *__restrict__ in, long long m, const uint32_t *__restrict__ sums,
+static __global__ void k_scan_final(uint32_t *__restrict__ in, long long m, const uint32_t *__restrict__ sums,
                              uint32_t *__restrict__ out, uint32_t *__restrict__ out2) {
   __shared__ uint32_t s[kScanBlock];
   long long i = (long long)blockIdx.x * kScanBlock + threadIdx.x;
@@ -334,7 +334,7 @@ __device__ __forceinline__ void scan_single_body(const int bid_, const int nbk_,
   }
 }
 
-__global__ void k_scan_single(uint32_t *__restrict__ in, long long m, uint32_t *__restrict__ out,
+static __global__ void k_scan_single(uint32_t *__restrict__ in, long long m, uint32_t *__restrict__ out,
                               uint32_t *__restrict__ out2) {
   scan_single_body(blockIdx.x, gridDim.x, in, m, out, out2);
 }
@@ -345,7 +345,7 @@ __device__ __forceinline__ void scatter_body(const int bid_, const int nbk_, int
   if (a < n) perm[atomicAdd(&cursor[key[a]], 1u)] = a;
 }
 
-__global__ void k_scatter(int n, const uint32_t *__restrict__ key, uint32_t *__restrict__ cursor,
+static __global__ void k_scatter(int n, const uint32_t *__restrict__ key, uint32_t *__restrict__ cursor,
                           int *__restrict__ perm) {
   scatter_body(blockIdx.x, gridDim.x, n, key, cursor, perm);
 }
@@ -366,7 +366,7 @@ __device__ __forceinline__ void binrank_body(const int bid_, const int nbk_, int
   out[s0 + rank] = a;
 }
 
-__global__ void k_binrank(int n, long long nbins, const uint32_t *__restrict__ key,
+static __global__ void k_binrank(int n, long long nbins, const uint32_t *__restrict__ key,
                           const uint32_t *__restrict__ start, const int *__restrict__ in, int *__restrict__ out) {
   binrank_body(blockIdx.x, gridDim.x, n, nbins, key, start, in, out);
 }
@@ -415,7 +415,7 @@ __device__ __forceinline__ void columns_body(const int bid_, const int nbk_, int
   }
 }
 
-__global__ void k_columns(int ncols, int nzb, int n, const uint32_t *__restrict__ start, int nsuper_max,
+static __global__ void k_columns(int ncols, int nzb, int n, const uint32_t *__restrict__ start, int nsuper_max,
                           int2 *__restrict__ sc_info, int *__restrict__ sc_col, int *__restrict__ colsc) {
   columns_body(blockIdx.x, gridDim.x, ncols, nzb, n, start, nsuper_max, sc_info, sc_col, colsc);
 }
@@ -913,7 +913,7 @@ __device__ __forceinline__ void build_list_body(const int bid_, const int nbk_, 
   }
 }
 
-__global__ void __launch_bounds__(kListBlock) k_build_list(ListParams q, const int *__restrict__ sc_col,
+static __global__ void __launch_bounds__(kListBlock) k_build_list(ListParams q, const int *__restrict__ sc_col,
                                                            const int *__restrict__ colsc,
                                                            const float4 *__restrict__ sctr,
                                                            const float4 *__restrict__ shalf,
@@ -978,7 +978,7 @@ __device__ __forceinline__ void mark_exclusions_body(const int bid_, const int n
   }
 }
 
-__global__ void k_mark_exclusions(int ne, const int4 *__restrict__ etab, const int *__restrict__ slot,
+static __global__ void k_mark_exclusions(int ne, const int4 *__restrict__ etab, const int *__restrict__ slot,
                                   int4 *__restrict__ entries, const int *__restrict__ count, int cap,
                                   int *__restrict__ maskwork, int *__restrict__ nmaskwork, int maxmaskwork,
                                   int *__restrict__ overflow) {
@@ -1068,7 +1068,7 @@ __device__ __forceinline__ void build_masks_body(const int bid_, const int nbk_,
   }
 }
 
-__global__ void __launch_bounds__(256) k_build_masks(const int *__restrict__ maskwork, const int *__restrict__ nmaskwork,
+static __global__ void __launch_bounds__(256) k_build_masks(const int *__restrict__ maskwork, const int *__restrict__ nmaskwork,
                                                      int maxmaskwork, int4 *__restrict__ entries, int cap,
                                                      const int *__restrict__ perm, const int *__restrict__ eptr,
                                                      const int2 *__restrict__ elist,
@@ -1168,7 +1168,7 @@ __device__ __forceinline__ void runs_prefix_body(const int bid_, const int nbk_,
   }
 }
 
-__global__ void k_runs_prefix(int nsuper, const int *__restrict__ count, const int *__restrict__ cost,
+static __global__ void k_runs_prefix(int nsuper, const int *__restrict__ count, const int *__restrict__ cost,
                               int *__restrict__ nruns_p, int *__restrict__ ep, long long *__restrict__ cp,
                               int *__restrict__ pos, int *__restrict__ posS) {
   runs_prefix_body(blockIdx.x, gridDim.x, nsuper, count, cost, nruns_p, ep, cp, pos, posS);
@@ -1197,7 +1197,7 @@ __device__ __forceinline__ void runs_cut_body(const int bid_, const int nbk_, in
   }
 }
 
-__global__ void k_runs_cut(int nsuper, const int *__restrict__ count, const int *__restrict__ ecost, int cap,
+static __global__ void k_runs_cut(int nsuper, const int *__restrict__ count, const int *__restrict__ ecost, int cap,
                            const int *__restrict__ nruns_p, const int *__restrict__ ep,
                            const long long *__restrict__ cp, int *__restrict__ pos, int *__restrict__ posS) {
   runs_cut_body(blockIdx.x, gridDim.x, nsuper, count, ecost, cap, nruns_p, ep, cp, pos, posS);
@@ -1248,7 +1248,7 @@ __device__ __forceinline__ void runs_tiles_body(const int bid_, const int nbk_, 
   }
 }
 
-__global__ void k_runs_tiles(const int *__restrict__ count, const int *__restrict__ ep, const int *__restrict__ pos,
+static __global__ void k_runs_tiles(const int *__restrict__ count, const int *__restrict__ ep, const int *__restrict__ pos,
                              const int *__restrict__ posS, int *__restrict__ wstart, int4 *__restrict__ tiles,
                              int *__restrict__ ntiles, int ntiles_cap) {
   runs_tiles_body(blockIdx.x, gridDim.x, count, ep, pos, posS, wstart, tiles, ntiles, ntiles_cap);
@@ -1304,22 +1304,6 @@ struct AccT<true> {
   __device__ static void add(unsigned long long *p, double v) {
     long long q = __double2ll_rn(v * kForceScale);
     atomicAdd(p, (unsigned long long)q);
-  }
-};
-
-// Switch constants in the arithmetic type of the kernel.
-template <class R>
-struct SwR {
-  R rc2, on2, s1, s2, s3, c15_1, c05_3, c15_3;
-  __device__ void load(const SwitchC &s) {
-    rc2 = (R)s.rc2;
-    on2 = (R)s.on2;
-    s1 = (R)s.s1;
-    s2 = (R)s.s2;
-    s3 = (R)s.s3;
-    c15_1 = (R)s.c15_1;
-    c05_3 = (R)s.c05_3;
-    c15_3 = (R)s.c15_3;
   }
 };
 
@@ -1914,6 +1898,350 @@ __device__ __forceinline__ void pair_body(const int bid_, const int nbk_, PairPa
   }
 }
 
+// ---- mixed form: direct evaluation --------------------------------------
+//
+// The mixed kernel evaluates the member lanes of a cluster pair where they
+// stand: no queue, no force slots.  Its FP32 math is short (about 60 issue
+// slots a cluster pair), so packing members first (about two fifths of the
+// lanes) cost as much issue time as it saved, and LDS round trips and scalar
+// work on top; FP64 math is several times longer and keeps the queue
+// (pair_body).  i-atoms sit in LDS, i-forces in registers for a whole tile,
+// constants in scalar registers.  Bound by VALU issue.
+// One launch alone, before (the queue) and after, skin 1.5 / 1.0 / 1.2 A:
+// 26,000 atoms 78.8 -> 60.1 us (VALU instructions 29.0 -> 25.1 M, scalar 16.0
+// -> 6.5 M, LDS 3.0 -> 0.8 M), 9,400 atoms 31.0 -> 27.3, 1,000,000 atoms 1.63
+// -> 1.07 ms; unequal cutoffs, 46,000 atoms 126 -> 97 us.
+// 72 VGPRs and 8 KB of LDS a block would take six blocks per CU (55.7 us and
+// 0.93 ms alone), but then the PME passes beside it starve and a step takes
+// longer (26,000 atoms 124 -> 136 us): four, which leave them half the
+// registers.
+
+// Energies and scalar force (F = f d) of one member pair; il, ic: in range of
+// the LJ and the Coulomb cutoff.
+template <int COUL, int LJSW, int CSW>
+__device__ __forceinline__ void direct_eval(const DirectC &k, float r2, float qq, float A, float B, float &elj,
+                                            float &eco, float &flj, float &fco) {
+  const float rinv = fast_rsqrt(r2);
+  const float rinv2 = rinv * rinv;
+  if (LJSW != SW_NONE) {
+    // LennardJonesForce.h:28-60
+    const float r6 = rinv2 * rinv2 * rinv2;
+    const float t = A * r6 - B;
+    float e = t * r6;                               // A r^-12 - B r^-6
+    float f = (A * r6 + t) * (r6 * (6.f * rinv2));  // (12 A r^-12 - 6 B r^-6) / r^2
+    if (LJSW == SW_C2) {
+      // C2SwitchingFunction.h:42-53: 1 below r_on, the polynomial up to rc
+      const bool on = r2 >= k.lj.on2;
+      if (__builtin_amdgcn_ballot_w64(on)) {
+        const float c2 = k.lj.rc2 - r2, c4 = c2 * (k.lj.s2 + 2.f * r2);
+        const float sv = k.lj.s1 * (c2 * c4);
+        const float fs = f * sv - e * (k.lj.s3 * (c2 * c2 - c4)), es = e * sv;
+        f = on ? fs : f;
+        e = on ? es : e;
+      }
+    } else {
+      float sv, sd;
+      switch_val<LJSW, float>(k.ljkind, k.lj, r2, rinv, sv, sd);
+      f = f * sv - e * sd;
+      e = e * sv;
+    }
+    flj = f;
+    elj = e;
+  }
+  if (COUL != COUL_NONE) {
+    float e, f;
+    if (COUL == COUL_CUTOFF) {
+      // CoulombForce.h:29-40
+      e = qq * rinv;
+      f = e * rinv2;
+    } else {
+      // NonbondedPMEwaldSystemForce.h:657-683 (poly5 form)
+      const float t = fast_rcp(1.f + k.pa * (r2 * rinv));
+      const float ex = qq * __builtin_amdgcn_exp2f(k.ke * r2);
+      const float p = t * (0.254829592f +
+                           t * (-0.284496736f + t * (1.421413741f + t * (-1.453152027f + t * 1.061405429f))));
+      e = p * ex * rinv;
+      f = (e + k.a2pi * ex) * rinv2;
+    }
+    if constexpr (CSW != SW_CUTOFF) {
+      float sv, sd;
+      switch_val<CSW, float>(k.cokind, k.co, r2, rinv, sv, sd);
+      f = f * sv - e * sd;
+      e = e * sv;
+    }
+    fco = f;
+    eco = e;
+  }
+}
+
+// a over lane l and lane l ^ 32 in the lower half wave, b in the upper.
+__device__ inline float swap32_sum(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+// The same over lane l ^ 16: a in even rows of 16 lanes, b in odd ones.
+__device__ inline float swap16_sum(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+// The same over lane l ^ 8: a in lanes with bit 3 clear, b in the others.
+__device__ inline float swap8_sum(float a, float b, bool hi) {
+  const float keep = hi ? b : a, give = hi ? a : b;
+  return keep + __uint_as_float((unsigned)__builtin_amdgcn_update_dpp(0, __float_as_int(give), 0x128, 0xF, 0xF, true));
+}
+
+template <int COUL, int LJSW, int CSW, bool BIGLJ, int MODE>
+__device__ __forceinline__ void pair_direct_body(
+    const int bid_, const int nbk_, const PairParams &pp, int dynamic, const int4 *__restrict__ tiles,
+    const int *__restrict__ ntiles_p, const int *__restrict__ wstart, int *__restrict__ tile_counter,
+    const int4 *__restrict__ entries, int4 *entries_w, int cap, const unsigned short *__restrict__ masks,
+    const float4 *__restrict__ xs, const float4 *__restrict__ sorg, const int *__restrict__ ts,
+    const int *__restrict__ perm, const double *__restrict__ ljtab, const float4 *__restrict__ ljt,
+    unsigned long long *__restrict__ facc, PairOut out) {
+  using WA = WaveAcc<true>;
+  constexpr int W = kPairBlock / kWave;
+  constexpr bool PRUNE = MODE == kPairPrune, STATS = MODE == kPairStats;
+  constexpr bool LJ = LJSW != SW_NONE;
+  // {A, B} of the plain and of the 1-4 pairs
+  __shared__ float2 s_lj[2][kMaxTypes * kMaxTypes];
+  __shared__ float4 s_i[W][kSuperSize];  // the tile's i-atoms
+  const int nt = pp.ntypes;
+  for (int k = threadIdx.x; LJ && !BIGLJ && k < nt * nt; k += blockDim.x) {
+    s_lj[0][k] = make_float2((float)ljtab[4 * k], (float)ljtab[4 * k + 1]);
+    s_lj[1][k] = make_float2((float)ljtab[4 * k + 2], (float)ljtab[4 * k + 3]);
+  }
+  __syncthreads();
+
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int ti = lane & 7, tj = lane >> 3;
+  const DirectC &kc = pp.dc;
+  const bool same_cut = !LJ || COUL == COUL_NONE || kc.lj.rc2 == kc.co.rc2;
+  // the boundary-pair sums are filled after this kernel (same stream)
+  if (bid_ == 0 && threadIdx.x < 4) out.border_acc[threadIdx.x] = 0ull;
+
+  // Runs: see pair_body.
+  const int nwaves = nbk_ * W;
+  const int gw = bid_ * W + wv;
+  const int nruns = ntiles_p[2];
+  const int r0 = dynamic ? gw : (int)((long long)gw * nruns / nwaves);
+  const int r1 = dynamic ? min(gw + 1, nruns) : (int)((long long)(gw + 1) * nruns / nwaves);
+  int t = r0 < r1 ? wstart[r0] : 0, tstop = r0 < r1 ? wstart[r1] : 0;
+  while (true) {
+    if (t >= tstop) {
+      if (!dynamic) break;
+      int rn = 0;
+      if (lane == 0) rn = nwaves + atomicAdd(tile_counter, 1);
+      const int r = __builtin_amdgcn_readfirstlane(__shfl(rn, 0));
+      if (r >= nruns) break;
+      t = wstart[r];
+      tstop = wstart[r + 1];
+      continue;
+    }
+    const int4 tile = tiles[t];
+    const int S = __builtin_amdgcn_readfirstlane(tile.x);
+    const int e0 = __builtin_amdgcn_readfirstlane(tile.y), e1 = __builtin_amdgcn_readfirstlane(tile.z);
+    const float4 oS = sorg[S];
+    // i-atoms, and the rows of the LJ table of this lane's (8 c + ti), 8 bits each
+    __builtin_amdgcn_wave_barrier();
+    s_i[wv][lane] = xs[S * kSuperSize + lane];
+    __builtin_amdgcn_wave_barrier();
+    unsigned irow[2] = {0, 0};
+#pragma unroll
+    for (int c = 0; LJ && !BIGLJ && c < 8; ++c)
+      irow[c >> 2] |= (unsigned)(max(0, ts[S * kSuperSize + c * kClusterSize + ti]) * nt) << (8 * (c & 3));
+    float fi[8][3];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) fi[c][0] = fi[c][1] = fi[c][2] = 0.f;
+    float elT = 0.f, ecT = 0.f;  // this lane's pair energies over the tile
+    int npair = 0;
+    unsigned long long hsum = 0;
+
+    const int4 *const ep = entries + (size_t)S * cap;
+    // the next entry is read while the current one is evaluated
+    auto entry = [&](int e) {
+      int4 v = ep[max(0, min(e, e1 - 1))];  // (an empty tile has e1 = 0)
+      v.x = __builtin_amdgcn_readfirstlane(v.x);
+      v.y = __builtin_amdgcn_readfirstlane(v.y);
+      v.z = __builtin_amdgcn_readfirstlane(v.z);
+      v.w = __builtin_amdgcn_readfirstlane(v.w);
+      return v;
+    };
+    auto mask_of = [&](const int4 &v) {
+      return v.z >= 0 ? (unsigned)masks[(size_t)v.z * kWave + lane] : 0xffu;
+    };
+    int4 nent = entry(e0);
+    for (int e = e0; e < e1; ++e) {
+      const int4 ent = nent;
+      const int sj = ent.x * kClusterSize + tj;
+      const unsigned em = ent.y & 0xff;
+      const int sh = ent.w, masked = ent.z >= 0;
+      float4 xj = xs[sj];
+      const int tyj = ts[sj];
+      const float4 oJ = sorg[ent.x / (kSuperSize / kClusterSize)];
+      const unsigned mb = mask_of(ent);
+      nent = entry(e + 1);
+      // j-cluster into the frame of S: origin difference (exact) plus the
+      // entry's image shift (hi part exact, lo part rounded once)
+      {
+        float ox = oJ.x - oS.x, oy = oJ.y - oS.y, oz = oJ.z - oS.z;
+        if (!(sh & kShiftPerPair) && sh != 21) {  // 21: no shift
+          const float sx = (float)((sh & 3) - 1), sy = (float)(((sh >> 2) & 3) - 1), sz = (float)(((sh >> 4) & 3) - 1);
+          ox = (ox + sx * kc.hi[0]) + sx * kc.lo[0];
+          oy = (oy + sy * kc.hi[1]) + sy * kc.lo[1];
+          oz = (oz + sz * kc.hi[2]) + sz * kc.lo[2];
+        }
+        xj.x += ox;
+        xj.y += oy;
+        xj.z += oz;
+      }
+      const int tyc = max(0, tyj);
+      if (LJ && !BIGLJ) asm volatile("" : "+v"(irow[0]), "+v"(irow[1]));  // unpacked where used, not ahead of the loop
+      float fj0 = 0.f, fj1 = 0.f, fj2 = 0.f;
+      unsigned used = 0, kept = 0;  // cluster pairs with a member; with a candidate within the list radius
+
+      // GENERAL: the entry carries an exclusion mask or takes the per-pair
+      // image; SAME: one cutoff for both kinds.
+      auto scan = [&](auto same, auto general) {
+        constexpr bool SAME = decltype(same)::value, GENERAL = decltype(general)::value;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+          if (!(em & (1u << c))) continue;
+          const float4 xi = s_i[wv][c * kClusterSize + ti];
+          float dx = xj.x - xi.x, dy = xj.y - xi.y, dz = xj.z - xi.z;
+          if (GENERAL && (sh & kShiftPerPair)) {
+            dx = kc.image(dx, 0);
+            dy = kc.image(dy, 1);
+            dz = kc.image(dz, 2);
+          }
+          float r2 = dx * dx + dy * dy + dz * dz;
+          if (GENERAL && !(mb & (1u << c))) r2 = kFarR2<float>;
+          if (PRUNE && __builtin_amdgcn_ballot_w64(r2 <= kc.prune_r2)) kept |= 1u << c;
+          const bool near = r2 <= kc.near2;
+          const unsigned long long nm = __builtin_amdgcn_ballot_w64(near);
+          if (!nm) continue;
+          // a pair within the guard band of a cutoff is left to the FP64
+          // boundary pass; a member is in range of a cutoff and outside
+          // every band
+          bool in, border;
+          if (SAME) {
+            in = r2 < kc.in2;
+            border = near && !in;
+          } else {
+            const float d = fminf(fabsf(r2 - kc.lj.rc2), fabsf(r2 - kc.co.rc2));
+            in = r2 <= kc.rmax2 && d > kc.guard;
+            border = near && d <= kc.guard;
+          }
+          if (__builtin_expect(
+                  SAME ? nm != __builtin_amdgcn_ballot_w64(in) : __builtin_amdgcn_ballot_w64(border) != 0, 0)) {
+            if (border) {
+              const int b = atomicAdd(out.nborder, 1);
+              int si = ti;
+              asm volatile("" : "+v"(si));  // rare: nothing of it is worth a register outside
+              if (b < out.maxborder)
+                out.border[b] = make_int2(S * kSuperSize + c * kClusterSize + si, sj);
+              else
+                atomicExch(out.overflow, 1);
+            }
+          }
+          if (STATS && in) {
+            const int ai = perm[S * kSuperSize + c * kClusterSize + ti], aj = perm[sj];
+            ++npair;
+            hsum += pair_hash(ai < aj ? ai : aj, ai < aj ? aj : ai);
+          }
+          // lanes without a member are evaluated too and selected away
+          const bool mod = GENERAL && ((mb >> (8 + c)) & 1u);
+          float A = 0.f, B = 0.f;
+          if (LJ && BIGLJ) {
+            const int tyi = max(0, ts[S * kSuperSize + c * kClusterSize + ti]);
+            const float4 v = ljt[(size_t)tyi * nt + tyc];
+            A = mod ? v.z : v.x;
+            B = mod ? v.w : v.y;
+          } else if (LJ) {
+            const float2 v = s_lj[GENERAL ? (mod ? 1 : 0) : 0][((irow[c >> 2] >> (8 * (c & 3))) & 255u) + tyc];
+            A = v.x;
+            B = v.y;
+          }
+          float qq = xi.w * xj.w;
+          if (GENERAL && mod) qq *= kc.csf;
+          float el = 0.f, ec = 0.f, fl = 0.f, fc = 0.f, f;
+          direct_eval<COUL, LJSW, CSW>(kc, r2, qq, A, B, el, ec, fl, fc);
+          if (SAME) {
+            f = in ? fl + fc : 0.f;
+            elT += in ? el : 0.f;
+            ecT += in ? ec : 0.f;
+          } else {
+            const bool il = in && r2 <= kc.lj.rc2, ic = in && r2 <= kc.co.rc2;
+            f = (il ? fl : 0.f) + (ic ? fc : 0.f);
+            elT += il ? el : 0.f;
+            ecT += ic ? ec : 0.f;
+          }
+          fi[c][0] += f * dx;  // of the opposite sign
+          fi[c][1] += f * dy;
+          fi[c][2] += f * dz;
+          fj0 += f * dx;
+          fj1 += f * dy;
+          fj2 += f * dz;
+          used = 1;
+        }
+      };
+      const bool general = masked || (sh & kShiftPerPair);
+      if (__builtin_expect(same_cut && !general, 1))
+        scan(std::true_type{}, std::false_type{});
+      else if (same_cut)
+        scan(std::true_type{}, std::true_type{});
+      else if (!general)
+        scan(std::false_type{}, std::false_type{});
+      else
+        scan(std::false_type{}, std::true_type{});
+      // prune pass: cluster pairs without a candidate pair inside the list
+      // radius cannot have a member before the next list build (every atom
+      // stays within half the skin of its build position); later passes skip
+      // them.  They have no member now either, so no result changes.
+      if (PRUNE && lane == 0 && kept != em) entries_w[(size_t)S * cap + e].y = (int)kept;
+      if (used) {
+        fj0 = group8_sum(fj0);
+        fj1 = group8_sum(fj1);
+        fj2 = group8_sum(fj2);
+        if (ti < 3 && tyj >= 0) {
+          const float v = ti == 0 ? fj0 : (ti == 1 ? fj1 : fj2);
+          AccT<true>::add(&facc[3 * sj + ti], v);
+        }
+      }
+    }
+    // tile end: lane 8 c + ti sums the eight partials of its i-atom
+    {
+      const int s = S * kSuperSize + lane;
+      const bool real = ts[s] >= 0, hi8 = lane & 8;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        float a[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) a[c] = swap32_sum(fi[c][k], fi[c + 4][k]);
+        const float b0 = swap16_sum(a[0], a[2]), b1 = swap16_sum(a[1], a[3]);
+        const float v = swap8_sum(b0, b1, hi8);
+        if (real) WA::add(&facc[3 * s + k], WA::of(-v));
+      }
+    }
+    const long long eljA = wave_sum(WA::of(elT));
+    const long long ecoA = wave_sum(WA::of(ecT));
+    long long np = 0;
+    if (STATS) {
+      np = wave_sum((long long)npair);
+      hsum = wave_sum(hsum);
+    }
+    if (lane == 0) {
+      out.energy[2 * t] = WA::energy_bits(ecoA);
+      out.energy[2 * t + 1] = WA::energy_bits(eljA);
+      if (STATS) {
+        out.npairs[t] = np;
+        out.hash[t] = hsum;
+      }
+    }
+    ++t;
+  }
+}
+
 template <bool MIXED, int COUL, int LJSW, int CSW, bool BIGLJ, int MODE>
 __global__ void __launch_bounds__(kPairBlock, 4) k_pair(
     PairParams pp, int dynamic, const int4 *__restrict__ tiles, const int *__restrict__ ntiles_p,
@@ -1926,9 +2254,15 @@ __global__ void __launch_bounds__(kPairBlock, 4) k_pair(
     const typename Real4<typename std::conditional<MIXED, float, double>::type>::type *__restrict__ ljt,
     typename AccT<MIXED>::type *__restrict__ facc, PairOut out) {
   // the blocks of one XCD take a contiguous range of runs
-  pair_body<MIXED, COUL, LJSW, CSW, BIGLJ, MODE>(xcd_block(blockIdx.x, gridDim.x), gridDim.x, pp, dynamic, tiles,
-                                                 ntiles_p, wstart, tile_counter, entries, entries_w, cap, masks, xs,
-                                                 sorg, ts, perm, ljtab, ljt, facc, out);
+  const int bid = xcd_block(blockIdx.x, gridDim.x);
+  if constexpr (MIXED)
+    pair_direct_body<COUL, LJSW, CSW, BIGLJ, MODE>(bid, gridDim.x, pp, dynamic, tiles, ntiles_p, wstart, tile_counter,
+                                                   entries, entries_w, cap, masks, xs, sorg, ts, perm, ljtab, ljt,
+                                                   facc, out);
+  else
+    pair_body<MIXED, COUL, LJSW, CSW, BIGLJ, MODE>(bid, gridDim.x, pp, dynamic, tiles, ntiles_p, wstart, tile_counter,
+                                                   entries, entries_w, cap, masks, xs, sorg, ts, perm, ljtab, ljt,
+                                                   facc, out);
 }
 
 // Boundary pairs: exact FP64 membership on the original coordinates
@@ -2879,7 +3213,7 @@ __device__ __forceinline__ void reduce_energy_body(const int bid_, const int nbk
   }
 }
 
-__global__ void k_reduce_energy(int ntiles_cap, const int *__restrict__ ntiles_p, const double *__restrict__ pair_e,
+static __global__ void k_reduce_energy(int ntiles_cap, const int *__restrict__ ntiles_p, const double *__restrict__ pair_e,
                                 int pair_fixed, int nrecip, const double *__restrict__ recip_e, int ncorr,
                                 const double *__restrict__ corr_e, const long long *__restrict__ npairs,
                                 const unsigned long long *__restrict__ hash, int stats,
@@ -2898,7 +3232,7 @@ struct ZeroRanges {
   unsigned long long *p[8];
   long long n[8];
 };
-__global__ void k_zero(ZeroRanges z) {
+static __global__ void k_zero(ZeroRanges z) {
   const int r = blockIdx.y;
   unsigned long long *p = z.p[r];
   const long long n = z.n[r];
@@ -3233,14 +3567,14 @@ __device__ __forceinline__ void chunk_begin_body(const int bid_, const int nbk_,
   if (i < nrec) dmax[i] = 0u;
 }
 
-__global__ void k_chunk_begin(long long m3, const double *__restrict__ x, const double *__restrict__ v,
+static __global__ void k_chunk_begin(long long m3, const double *__restrict__ x, const double *__restrict__ v,
                               const double *__restrict__ f, double *__restrict__ xbak, double *__restrict__ vbak,
                               double *__restrict__ fbak, int *__restrict__ overflow, unsigned *__restrict__ dmax,
                               int nrec) {
   chunk_begin_body(blockIdx.x, gridDim.x, m3, x, v, f, xbak, vbak, fbak, overflow, dmax, nrec);
 }
 
-__global__ void k_set_u64(unsigned long long *p, unsigned long long v) { *p = v; }
+static __global__ void k_set_u64(unsigned long long *p, unsigned long long v) { *p = v; }
 
 __device__ __forceinline__ void half_kick_body(const int bid_, const int nbk_, int n, Kick kk,
                                                const double *__restrict__ fout, const double *__restrict__ minv,
@@ -3253,13 +3587,13 @@ __device__ __forceinline__ void half_kick_body(const int bid_, const int nbk_, i
   for (int k = 0; k < 3; ++k) v[3 * a + k] = vv[k];
 }
 
-__global__ void k_half_kick(int n, Kick kk, const double *__restrict__ fout, const double *__restrict__ minv,
+static __global__ void k_half_kick(int n, Kick kk, const double *__restrict__ fout, const double *__restrict__ minv,
                             double *__restrict__ v) {
   half_kick_body(blockIdx.x, gridDim.x, n, kk, fout, minv, v);
 }
 
 // Kinetic energy 0.5 sum m v^2 into per-block partials.
-__global__ void k_kinetic(int n, const double *__restrict__ v, const double *__restrict__ minv,
+static __global__ void k_kinetic(int n, const double *__restrict__ v, const double *__restrict__ minv,
                           double *__restrict__ epart) {
   __shared__ double s_e[kPairBlock / kWave];
   const int a = blockIdx.x * blockDim.x + threadIdx.x;
