@@ -108,7 +108,7 @@ struct Sys {
   int pair_grid = 0;           // blocks of the pair-kernel launch
   long long nbins = 0;
   int nscanblocks = 0;
-  int recip_blocks = 0, corr_blocks = 0;
+  int recip_blocks = 0, term_blocks = 0;  // blocks of the x pass and of the atoms' terms
   int xlog = 0, ylog = 0;              // lines of a block of the x and y passes (log2)
   size_t lds_z = 0, lds_g = 0, lds_y = 0, lds_x = 0, lds_p = 0;  // dynamic LDS of the PME launches
   int thr_z = 256, thr_g = 256, thr_y = 256, thr_x = 256, thr_p = 256;  // and their block sizes
@@ -116,7 +116,7 @@ struct Sys {
   std::vector<DevBuf *> all;
   DevBuf xorig, xwrap, q_d, type_d, key, hist, start, cursor, scansum, perm, permp, slot, refcell, xs, xs64, ts,
       perm2, sc_info, sc_col, colsc, sctr, shalf, sorg, ctr, half, entries, count, ecost, lcost, tep, tcp, tpos, tposS, wstart, maskwork, nmaskwork, masks, overflow, tiles, ntiles, tilectr, ljtab, ljt32, facc, fout,
-      pair_e, npairs, hash, eptr_d, elist_d, etab_d, corr_e, recip_e, eout, np_out, hash_out, pmw, pmb, tcol, spec, theta, twx, twy, twz, border, nborder, border_acc;
+      pair_e, npairs, hash, eptr_d, elist_d, etab_d, cptr_d, clist_d, corr_e, recip_e, eout, np_out, hash_out, pmw, pmb, tcol, spec, theta, twx, twy, twz, border, nborder, border_acc;
   int maxborder = 65536;
   // results
   long long last_np = 0;
@@ -139,7 +139,7 @@ struct Sys {
     bool on = false;
     int nb = 0, na = 0;
     double h = 0, skin = 0;
-    DevBuf bonds, bpar, angles, apar, minv, v, xbuild, xbak, vbak, fbak, dmax, bond_e, ke_e;
+    DevBuf mptr, bonds, bpar, angles, apar, minv, v, xbuild, xbak, vbak, fbak, dmax, bond_e, ke_e;
     int chunk = 16;
     long long steps = 0, rebuilds = 0, rollbacks = 0;
     bool forces_valid = false;
@@ -714,10 +714,28 @@ int setup(Sys *s) {
       (rc = A(s->hash_out, 8)) || (rc = A(s->border, 8 * (size_t)s->maxborder)) ||
       (rc = A(s->nborder, 8)) || (rc = A(s->border_acc, 32)))
     return rc;
-  s->corr_blocks = std::max(1, (int)nblk((long long)s->etab.size(), 256));
+  s->term_blocks = (int)nblk((long long)NP, 256);
+  // the correction table by atom (each entry listed for both of its atoms)
+  std::vector<int> cptr;
+  std::vector<int2> clist;
+  if (!s->dry) {
+    cptr.assign(N + 1, 0);
+    for (const int4 &e : s->etab) {
+      ++cptr[e.x + 1];
+      ++cptr[e.y + 1];
+    }
+    for (size_t a = 0; a < N; ++a) cptr[a + 1] += cptr[a];
+    clist.resize(2 * s->etab.size());
+    std::vector<int> at(cptr.begin(), cptr.end() - 1);
+    for (const int4 &e : s->etab) {
+      clist[at[e.x]++] = make_int2(e.y, e.z);
+      clist[at[e.y]++] = make_int2(e.x, e.z);
+    }
+  }
+  if ((rc = A(s->cptr_d, 4 * (N + 1))) || (rc = A(s->clist_d, 16 * s->etab.size()))) return rc;
   // boundary pairs grow with the pair count: one block per 16 superclusters
   s->border_blocks = std::min(128, std::max(4, (int)(s->nsuper / 16)));
-  if ((rc = A(s->corr_e, 8 * (size_t)s->corr_blocks))) return rc;
+  if ((rc = A(s->corr_e, 8 * (size_t)s->term_blocks))) return rc;
   if (s->dry) {
     // PME buffers as allocated below (grid records, tile windows, half
     // spectrum, influence table, twiddles, energy partials bounded by ny * nzh)
@@ -752,6 +770,9 @@ int setup(Sys *s) {
     HIPCHK(hipMemcpyAsync(s->elist_d.p, s->elist.data(), 8 * s->elist.size(), hipMemcpyHostToDevice, st));
   if (!s->etab.empty())
     HIPCHK(hipMemcpyAsync(s->etab_d.p, s->etab.data(), 16 * s->etab.size(), hipMemcpyHostToDevice, st));
+  HIPCHK(hipMemcpyAsync(s->cptr_d.p, cptr.data(), 4 * cptr.size(), hipMemcpyHostToDevice, st));
+  if (!clist.empty())
+    HIPCHK(hipMemcpyAsync(s->clist_d.p, clist.data(), 8 * clist.size(), hipMemcpyHostToDevice, st));
 
   if (s->pme_on) {
     PmeParams &pm = s->pme;
@@ -963,27 +984,26 @@ FixupArgs<MIXED> fixup_args(Sys *s, bool stats, bool border_here, bool rest_here
   a.border_e = P<unsigned long long>(s->border_acc);
   a.border_stat = P<unsigned long long>(s->border_acc) + 2;
   const bool corr = s->pme_on && (s->d.pme_terms & PMX_PME_CORR) && !s->etab.empty();
-  a.corr_blocks = corr && rest_here ? s->corr_blocks : 0;
-  a.ne = (int)s->etab.size();
-  a.etab = P<int4>(s->etab_d);
+  const bool bonded = s->md.on && s->md.nb + s->md.na > 0;
+  a.npad = s->npad;
   a.q = P<double>(s->q_d);
-  a.slot = P<int>(s->slot);
   a.alpha = s->alpha;
   a.csf = s->d.csf;
   a.corr_e = P<double>(s->corr_e);
-  int bonded_blocks = 0;
-  if (rest_here && s->md.on && s->md.nb + s->md.na > 0) {
-    bonded_blocks = (int)nblk(s->md.nb + s->md.na, 256);
-    a.nbond = s->md.nb;
-    a.nangle = s->md.na;
-    a.bonds = P<int2>(s->md.bonds);
-    a.bpar = P<double2>(s->md.bpar);
-    a.angles = P<int4>(s->md.angles);
-    a.apar = P<double2>(s->md.apar);
+  if (corr) {
+    a.at.eptr = P<int>(s->cptr_d);
+    a.at.excl = P<int2>(s->clist_d);
+  }
+  if (bonded) {
+    a.at.mptr = P<int2>(s->md.mptr);
+    a.at.bond = P<int>(s->md.bonds);
+    a.at.bpar = P<double2>(s->md.bpar);
+    a.at.angle = P<int4>(s->md.angles);
+    a.at.apar = P<double2>(s->md.apar);
     a.bond_e = P<double>(s->md.bond_e);
   }
   a.facc = P<typename AccT<MIXED>::type>(s->facc);
-  *nblocks = a.border_blocks + a.corr_blocks + bonded_blocks;
+  *nblocks = a.border_blocks + (rest_here && (corr || bonded) ? s->term_blocks : 0);
   return a;
 }
 
@@ -1089,7 +1109,7 @@ void reduce_energies(Sys *s, bool stats) {
   const bool corr = s->pme_on && (s->d.pme_terms & PMX_PME_CORR) && !s->etab.empty();
   hipLaunchKernelGGL(k_reduce_energy, dim3(1), dim3(1024), 0, s->ctx->stream, s->ntiles_cap, P<int>(s->ntiles),
                      P<double>(s->pair_e), s->mixed ? 1 : 0, recip ? s->recip_blocks : 0, P<double>(s->recip_e),
-                     corr ? s->corr_blocks : 0, P<double>(s->corr_e), P<long long>(s->npairs),
+                     corr ? s->term_blocks : 0, P<double>(s->corr_e), P<long long>(s->npairs),
                      P<unsigned long long>(s->hash), stats ? 1 : 0, P<unsigned long long>(s->border_acc),
                      P<unsigned long long>(s->border_acc) + 2, P<double>(s->eout), P<long long>(s->np_out),
                      P<unsigned long long>(s->hash_out));
@@ -1771,28 +1791,37 @@ int pmx_md_init(pmx_sys *sys, const pmx_md_desc *d) {
     m.fc = 2.0 * kBoltzmann * d->temperature * g;
   }
   const size_t N = s->n;
-  std::vector<int2> b(m.nb);
-  std::vector<double2> bp(m.nb);
-  for (int i = 0; i < m.nb; ++i) {
-    b[i] = make_int2(d->bonds[2 * i], d->bonds[2 * i + 1]);
-    bp[i] = make_double2(d->bond_par[2 * i], d->bond_par[2 * i + 1]);
-  }
-  std::vector<int4> a(m.na);
-  std::vector<double2> ap(m.na);
-  for (int i = 0; i < m.na; ++i) {
-    a[i] = make_int4(d->angles[3 * i], d->angles[3 * i + 1], d->angles[3 * i + 2], 0);
-    ap[i] = make_double2(d->angle_par[2 * i], d->angle_par[2 * i + 1]);
-  }
+  // bonds and angles by atom, each listed for every atom it acts on
+  std::vector<int2> mp(N + 1, make_int2(0, 0));
+  for (int i = 0; i < 2 * m.nb; ++i) ++mp[d->bonds[i] + 1].x;
+  for (int i = 0; i < 3 * m.na; ++i) ++mp[d->angles[i] + 1].y;
+  for (size_t i = 0; i < N; ++i) mp[i + 1] = make_int2(mp[i + 1].x + mp[i].x, mp[i + 1].y + mp[i].y);
+  std::vector<int> b(2 * (size_t)m.nb);
+  std::vector<double2> bp(2 * (size_t)m.nb);
+  std::vector<int4> a(3 * (size_t)m.na);
+  std::vector<double2> ap(3 * (size_t)m.na);
+  std::vector<int2> at(mp.begin(), mp.end() - 1);
+  for (int i = 0; i < m.nb; ++i)
+    for (int k = 0; k < 2; ++k) {
+      const int t = at[d->bonds[2 * i + k]].x++;
+      b[t] = d->bonds[2 * i + 1 - k];
+      bp[t] = make_double2(d->bond_par[2 * i], d->bond_par[2 * i + 1]);
+    }
+  for (int i = 0; i < m.na; ++i)
+    for (int k = 0; k < 3; ++k) {
+      const int t = at[d->angles[3 * i + k]].y++;
+      a[t] = make_int4(d->angles[3 * i], d->angles[3 * i + 1], d->angles[3 * i + 2], k);
+      ap[t] = make_double2(d->angle_par[2 * i], d->angle_par[2 * i + 1]);
+    }
   std::vector<double> minv(N);
   for (size_t i = 0; i < N; ++i) minv[i] = 1.0 / d->mass[i];
-  const int nbonded_blocks = std::max(1, (int)nblk(m.nb + m.na, 256));
   int rc;
-  if ((rc = dalloc(s, m.bonds, 8 * b.size())) || (rc = dalloc(s, m.bpar, 16 * bp.size())) ||
+  if ((rc = dalloc(s, m.mptr, 8 * mp.size())) || (rc = dalloc(s, m.bonds, 4 * b.size())) || (rc = dalloc(s, m.bpar, 16 * bp.size())) ||
       (rc = dalloc(s, m.angles, 16 * a.size())) || (rc = dalloc(s, m.apar, 16 * ap.size())) ||
       (rc = dalloc(s, m.minv, 8 * N)) || (rc = dalloc(s, m.v, 24 * N)) || (rc = dalloc(s, m.xbuild, 24 * N)) ||
       (rc = dalloc(s, m.xbak, 2 * 24 * N)) || (rc = dalloc(s, m.vbak, 2 * 24 * N)) ||
       (rc = dalloc(s, m.fbak, 2 * 24 * N)) || (rc = dalloc(s, m.dmax, 4 * 2 * kMaxChunk)) ||
-      (rc = dalloc(s, m.step_dev, 8)) || (rc = dalloc(s, m.bond_e, 16 * (size_t)nbonded_blocks)) ||
+      (rc = dalloc(s, m.step_dev, 8)) || (rc = dalloc(s, m.bond_e, 16 * (size_t)s->term_blocks)) ||
       (rc = dalloc(s, m.ke_e, 8 * (size_t)nblk(N, 256))))
     return rc;
   if (!m.host) {
@@ -1801,7 +1830,8 @@ int pmx_md_init(pmx_sys *sys, const pmx_md_desc *d) {
     for (auto &e : m.chunk_ev) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   }
   hipStream_t st = s->ctx->stream;
-  if (m.nb) HIPCHK(hipMemcpyAsync(m.bonds.p, b.data(), 8 * b.size(), hipMemcpyHostToDevice, st));
+  HIPCHK(hipMemcpyAsync(m.mptr.p, mp.data(), 8 * mp.size(), hipMemcpyHostToDevice, st));
+  if (m.nb) HIPCHK(hipMemcpyAsync(m.bonds.p, b.data(), 4 * b.size(), hipMemcpyHostToDevice, st));
   if (m.nb) HIPCHK(hipMemcpyAsync(m.bpar.p, bp.data(), 16 * bp.size(), hipMemcpyHostToDevice, st));
   if (m.na) HIPCHK(hipMemcpyAsync(m.angles.p, a.data(), 16 * a.size(), hipMemcpyHostToDevice, st));
   if (m.na) HIPCHK(hipMemcpyAsync(m.apar.p, ap.data(), 16 * ap.size(), hipMemcpyHostToDevice, st));
@@ -2416,7 +2446,7 @@ int batch_tables(Batch &b) {
       const bool recip = s->pme_on && (s->d.pme_terms & PMX_PME_RECIP);
       const bool corr = s->pme_on && (s->d.pme_terms & PMX_PME_CORR) && !s->etab.empty();
       args_energy[i] = {s->ntiles_cap, P<int>(s->ntiles), P<double>(s->pair_e), s->mixed ? 1 : 0,
-                        recip ? s->recip_blocks : 0, corr ? s->corr_blocks : 0, P<double>(s->recip_e),
+                        recip ? s->recip_blocks : 0, corr ? s->term_blocks : 0, P<double>(s->recip_e),
                         P<double>(s->corr_e), P<long long>(s->npairs), P<unsigned long long>(s->hash),
                         P<unsigned long long>(s->border_acc), P<unsigned long long>(s->border_acc) + 2,
                         P<double>(s->eout), P<long long>(s->np_out), P<unsigned long long>(s->hash_out)};
@@ -2900,7 +2930,7 @@ int pmx_md_get_state(pmx_sys *sys, double *x, double *v, double *energies) {
     reduce_energies(s, false);
     hipLaunchKernelGGL(k_kinetic, dim3(nblk(n, 256)), dim3(256), 0, st, n, P<double>(m.v), P<double>(m.minv),
                        P<double>(m.ke_e));
-    const int nbb = std::max(1, (int)nblk(m.nb + m.na, 256));
+    const int nbb = s->term_blocks;
     std::vector<double> be(2 * nbb, 0.0), ke(nblk(n, 256));
     if (m.nb + m.na > 0) HIPCHK(hipMemcpyAsync(be.data(), m.bond_e.p, 16 * (size_t)nbb, hipMemcpyDeviceToHost, st));
     HIPCHK(hipMemcpyAsync(ke.data(), m.ke_e.p, 8 * ke.size(), hipMemcpyDeviceToHost, st));
@@ -2935,7 +2965,7 @@ unsigned long long pmx_estimate_bytes(const pmx_sys_desc *desc, int kind) {
   // device MD state: velocities, masses, build positions, two chunk backups
   // of x, v and f, bonded tables (bonds and angles about one per atom in the
   // systems served)
-  if (kind == 1) b += 200ull * (unsigned long long)desc->n + 48ull * (unsigned long long)desc->n + 8192;
+  if (kind == 1) b += 200ull * (unsigned long long)desc->n + 132ull * (unsigned long long)desc->n + 8192;
   return b;
 }
 
