@@ -29,7 +29,7 @@ def _molecules(n, seed, star):
         ex.setdefault((min(a, c), max(a, c)), 2)
     return systems.MolSystem(
         name="chain", pos=pos, charge=rng.uniform(-5, 5, n), atype=np.zeros(n, np.int32),
-        molecule=np.arange(n, dtype=np.int32), mass=rng.uniform(1, 16, n),
+        molecule=np.zeros(n, np.int32), mass=rng.uniform(1, 16, n),
         lj=systems.charmm_table([0.1], [0.8], [0.05], [0.7]), box=np.array([box] * 3), origin=np.zeros(3),
         bonds=np.array(bonds, np.int32).reshape(-1, 2), bond_par=rng.uniform(1, 3, (len(bonds), 2)),
         angles=np.array(angles, np.int32).reshape(-1, 3), angle_par=rng.uniform(1, 3, (len(angles), 2)),
