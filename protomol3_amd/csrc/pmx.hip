@@ -115,8 +115,8 @@ struct Sys {
   // device buffers
   std::vector<DevBuf *> all;
   DevBuf xorig, xwrap, q_d, type_d, key, hist, start, cursor, scansum, perm, permp, slot, refcell, xs, xs64, ts,
-      perm2, sc_info, sc_col, colsc, sctr, shalf, sorg, ctr, half, entries, count, ecost, lcost, tep, tcp, tpos, tposS, wstart, maskwork, nmaskwork, masks, overflow, tiles, ntiles, tilectr, ljtab, ljt32, facc, fout,
-      pair_e, npairs, hash, eptr_d, elist_d, etab_d, cptr_d, clist_d, corr_e, recip_e, eout, np_out, hash_out, pmw, pmb, tcol, spec, theta, twx, twy, twz, border, nborder, border_acc;
+      sc_info, sc_col, colsc, sctr, shalf, sorg, ctr, half, entries, count, ecost, lcost, runs, nmaskwork, masks, overflow, ntiles, tilectr, ljtab, ljt32, facc, fout,
+      pair_e, npairs, hash, eptr_d, elist_d, cptr_d, clist_d, corr_e, recip_e, eout, np_out, hash_out, pmw, pmb, tcol, spec, theta, twx, twy, twz, border, nborder, border_acc;
   int maxborder = 65536;
   // results
   long long last_np = 0;
@@ -685,9 +685,9 @@ int setup(Sys *s) {
   auto A = [&](DevBuf &b, size_t bytes) { return dalloc(s, b, bytes); };
   const size_t N = d.n, NP = s->npad;
   if ((rc = A(s->xorig, 24 * N)) || (rc = A(s->xwrap, 24 * N)) || (rc = A(s->q_d, 8 * N)) ||
-      (rc = A(s->type_d, 4 * N)) || (rc = A(s->key, 4 * N)) || (rc = A(s->hist, 4 * s->nbins)) ||
-      (rc = A(s->start, 4 * s->nbins)) || (rc = A(s->cursor, 4 * s->nbins)) ||
-      (rc = A(s->scansum, 4 * (size_t)s->nscanblocks)) || (rc = A(s->perm, 4 * N)) || (rc = A(s->perm2, 4 * N)) ||
+      (rc = A(s->type_d, 4 * N)) || (rc = A(s->key, 4 * N)) || (rc = A(s->hist, 16 * ((s->nbins + 3) / 4))) ||
+      (rc = A(s->start, 16 * ((s->nbins + 3) / 4))) || (rc = A(s->cursor, 16 * ((s->nbins + 3) / 4))) ||
+      (rc = A(s->scansum, 4 * (size_t)s->nscanblocks)) || (rc = A(s->perm, 4 * N)) ||
       (rc = A(s->permp, 4 * NP)) ||
       (rc = A(s->slot, 4 * N)) || (rc = A(s->refcell, 4 * N)) || (rc = A(s->xs, 32 * NP)) ||
       (rc = A(s->xs64, 32 * NP)) || (rc = A(s->ts, 4 * NP)) || (rc = A(s->sc_info, 8 * (size_t)s->nsuper)) ||
@@ -698,19 +698,15 @@ int setup(Sys *s) {
       (rc = A(s->half, 16 * (size_t)s->ncl)) || (rc = A(s->entries, 16 * (size_t)s->nsuper * s->cap)) ||
       (rc = A(s->count, 4 * (size_t)s->nsuper)) || (rc = A(s->lcost, 4 * (size_t)s->nsuper)) ||
       (rc = A(s->ecost, 4 * (size_t)s->nsuper * s->cap)) ||
-      (rc = A(s->tep, 4 * ((size_t)s->nsuper + 1))) || (rc = A(s->tcp, 8 * ((size_t)s->nsuper + 1))) ||
-      (rc = A(s->tpos, 4 * ((size_t)kMaxRuns + 1))) ||
-      (rc = A(s->tposS, 4 * ((size_t)kMaxRuns + 1))) ||
-      (rc = A(s->wstart, 4 * ((size_t)kMaxRuns + 1))) ||
-      (rc = A(s->maskwork, 4 * (size_t)s->maxmaskwork)) ||
+      (rc = A(s->runs, 8 * ((size_t)kMaxRuns + 1))) ||
       (rc = A(s->nmaskwork, 8)) || (rc = A(s->masks, 16 * 8 * (size_t)s->maxmaskwork)) ||
-      (rc = A(s->overflow, 8)) || (rc = A(s->tiles, 16 * (size_t)s->ntiles_cap)) || (rc = A(s->ntiles, 16)) ||
+      (rc = A(s->overflow, 8)) || (rc = A(s->ntiles, 16)) ||
       (rc = A(s->tilectr, 8)) || (rc = A(s->ljtab, 8 * s->lj.size())) ||
       (rc = A(s->ljt32, 4 * s->lj.size())) || (rc = A(s->facc, 24 * NP)) ||
       (rc = A(s->fout, 24 * N)) || (rc = A(s->pair_e, 16 * (size_t)s->ntiles_cap)) ||
       (rc = A(s->npairs, 8 * (size_t)s->ntiles_cap)) || (rc = A(s->hash, 8 * (size_t)s->ntiles_cap)) ||
       (rc = A(s->eptr_d, 4 * (N + 1))) || (rc = A(s->elist_d, 8 * s->elist.size())) ||
-      (rc = A(s->etab_d, 16 * s->etab.size())) || (rc = A(s->eout, 64)) || (rc = A(s->np_out, 8)) ||
+      (rc = A(s->eout, 64)) || (rc = A(s->np_out, 8)) ||
       (rc = A(s->hash_out, 8)) || (rc = A(s->border, 8 * (size_t)s->maxborder)) ||
       (rc = A(s->nborder, 8)) || (rc = A(s->border_acc, 32)))
     return rc;
@@ -751,7 +747,9 @@ int setup(Sys *s) {
 
   hipStream_t st = s->ctx->stream;
   // the cell histogram starts cleared; each rebuild's scan clears it again
-  hipLaunchKernelGGL(k_fill_u32, dim3(nblk(s->nbins, 256)), dim3(256), 0, st, P<uint32_t>(s->hist), 0u, s->nbins);
+  // (with the padding to whole groups of four that the scan reads)
+  hipLaunchKernelGGL(k_fill_u32, dim3(nblk(s->nbins + 3, 256)), dim3(256), 0, st, P<uint32_t>(s->hist), 0u,
+                     (s->nbins + 3) / 4 * 4);
   {
     RtLock lk(g_rt_mu);
     // the fork and join order the two streams of one device only (the host
@@ -768,8 +766,6 @@ int setup(Sys *s) {
   HIPCHK(hipMemcpyAsync(s->eptr_d.p, s->eptr.data(), 4 * (N + 1), hipMemcpyHostToDevice, st));
   if (!s->elist.empty())
     HIPCHK(hipMemcpyAsync(s->elist_d.p, s->elist.data(), 8 * s->elist.size(), hipMemcpyHostToDevice, st));
-  if (!s->etab.empty())
-    HIPCHK(hipMemcpyAsync(s->etab_d.p, s->etab.data(), 16 * s->etab.size(), hipMemcpyHostToDevice, st));
   HIPCHK(hipMemcpyAsync(s->cptr_d.p, cptr.data(), 4 * cptr.size(), hipMemcpyHostToDevice, st));
   if (!clist.empty())
     HIPCHK(hipMemcpyAsync(s->clist_d.p, clist.data(), 8 * clist.size(), hipMemcpyHostToDevice, st));
@@ -939,7 +935,7 @@ void launch_pair_phase(Sys *s, bool stats, int phase) {
     s->prune_pending = false;
     const R4 *ljt = MIXED ? reinterpret_cast<const R4 *>(s->ljt32.p) : reinterpret_cast<const R4 *>(s->ljtab.p);
 #define PMX_PAIR_ARGS                                                                                              \
-  s->pp, s->tune_schedule, P<int4>(s->tiles), P<int>(s->ntiles), P<int>(s->wstart), P<int>(s->tilectr),            \
+  s->pp, s->tune_schedule, P<int2>(s->runs), P<int>(s->ntiles), P<int>(s->count), P<int>(s->tilectr),            \
       P<int4>(s->entries), P<int4>(s->entries), s->cap, P<unsigned short>(s->masks), P<R4>(s->xs),                 \
       P<float4>(s->sorg), P<int>(s->ts), P<int>(s->permp), P<double>(s->ljtab), ljt, facc, out
     if (stats)
@@ -1131,14 +1127,19 @@ void timing_begin_call(Sys *s, bool timing) {
 // (the reference rebuilds its cell lists at every force evaluation,
 // ForceGroup.cpp:57; the MD path rebuilds when the skin requires it).
 // Work tiles of the current list for the current schedule and pair grid.
-void make_tiles(Sys *s, hipStream_t st) {
-  int *const nruns = P<int>(s->ntiles) + 2;
-  hipLaunchKernelGGL(k_runs_prefix, dim3(1), dim3(1024), 0, st, s->nsuper, P<int>(s->count), P<int>(s->lcost), nruns,
-                     P<int>(s->tep), P<long long>(s->tcp), P<int>(s->tpos), P<int>(s->tposS));
-  hipLaunchKernelGGL(k_runs_cut, dim3(s->nsuper), dim3(256), 0, st, s->nsuper, P<int>(s->count), P<int>(s->ecost),
-                     s->cap, nruns, P<int>(s->tep), P<long long>(s->tcp), P<int>(s->tpos), P<int>(s->tposS));
-  hipLaunchKernelGGL(k_runs_tiles, dim3(1), dim3(1024), 0, st, P<int>(s->count), P<int>(s->tep), P<int>(s->tpos),
-                     P<int>(s->tposS), P<int>(s->wstart), P<int4>(s->tiles), P<int>(s->ntiles), s->ntiles_cap);
+unsigned runs_blocks(Sys *s) { return (unsigned)std::min<long long>(256, nblk(s->nsuper, kRunsBlock / kWave)); }
+void make_runs(Sys *s, hipStream_t st) {
+  hipLaunchKernelGGL(k_runs, dim3(runs_blocks(s)), dim3(kRunsBlock), 0, st, s->nsuper, P<int>(s->count),
+                     P<int>(s->lcost), P<int>(s->ecost), s->cap, P<int2>(s->runs), P<int>(s->ntiles));
+}
+
+SortedBins sorted_bins(Sys *s) {
+  return {s->n, s->nbins, P<uint32_t>(s->key), P<uint32_t>(s->start), P<int>(s->perm)};
+}
+
+MaskArgs mask_args(Sys *s) {
+  return {P<int>(s->permp),           P<int>(s->slot), P<int>(s->eptr_d), P<int2>(s->elist_d),
+          P<unsigned short>(s->masks), s->maxmaskwork};
 }
 
 int rebuild(Sys *s, bool timing) {
@@ -1148,52 +1149,39 @@ int rebuild(Sys *s, bool timing) {
   hipLaunchKernelGGL(k_bin, dim3(nblk(n, 256)), dim3(256), 0, st, n, P<double>(s->xorig), s->bin, P<uint32_t>(s->key),
                      P<double>(s->xwrap), P<int>(s->refcell), P<uint32_t>(s->hist));
   if (s->nbins <= kScanSingleMax) {
-    hipLaunchKernelGGL(k_scan_single, dim3(1), dim3(kScanBlock), 0, st, P<uint32_t>(s->hist), s->nbins,
-                       P<uint32_t>(s->start), P<uint32_t>(s->cursor));
+    hipLaunchKernelGGL(k_scan_columns, dim3(1), dim3(kScanBlock), 0, st, P<uint32_t>(s->hist), (int)s->nbins,
+                       P<uint32_t>(s->start), P<uint32_t>(s->cursor), s->ncols, s->bin.nzb, n, s->nsuper,
+                       P<int2>(s->sc_info), P<int>(s->sc_col), P<int>(s->colsc));
   } else {
     hipLaunchKernelGGL(k_scan_blocksums, dim3(s->nscanblocks), dim3(kScanBlock), 0, st, P<uint32_t>(s->hist),
                        s->nbins, P<uint32_t>(s->scansum));
     hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(kScanBlock), 0, st, P<uint32_t>(s->scansum), s->nscanblocks);
     hipLaunchKernelGGL(k_scan_final, dim3(s->nscanblocks), dim3(kScanBlock), 0, st, P<uint32_t>(s->hist), s->nbins,
                        P<uint32_t>(s->scansum), P<uint32_t>(s->start), P<uint32_t>(s->cursor));
+    hipLaunchKernelGGL(k_columns, dim3(1), dim3(kScanBlock), 0, st, s->ncols, s->bin.nzb, n, P<uint32_t>(s->start),
+                       s->nsuper, P<int2>(s->sc_info), P<int>(s->sc_col), P<int>(s->colsc));
   }
   hipLaunchKernelGGL(k_scatter, dim3(nblk(n, 256)), dim3(256), 0, st, n, P<uint32_t>(s->key), P<uint32_t>(s->cursor),
                      P<int>(s->perm));
-  hipLaunchKernelGGL(k_binrank, dim3(nblk(n, 256)), dim3(256), 0, st, n, s->nbins, P<uint32_t>(s->key),
-                     P<uint32_t>(s->start), P<int>(s->perm), P<int>(s->perm2));
-  hipLaunchKernelGGL(k_columns, dim3(1), dim3(1024), 0, st, s->ncols, s->bin.nzb, n, P<uint32_t>(s->start),
-                     s->nsuper, P<int2>(s->sc_info), P<int>(s->sc_col), P<int>(s->colsc));
   double *xbuild = s->md.on ? P<double>(s->md.xbuild) : nullptr;
   if (s->mixed)
     hipLaunchKernelGGL(k_split_fill<float>, dim3(nblk((long long)s->nsuper * 64, 256)), dim3(256), 0, st, s->nsuper,
-                       P<int2>(s->sc_info), P<int>(s->perm2), P<double>(s->xwrap), P<int>(s->permp), P<int>(s->slot),
+                       P<int2>(s->sc_info), sorted_bins(s), P<double>(s->xwrap), P<int>(s->permp), P<int>(s->slot),
                        P<double>(s->q_d), P<int>(s->type_d), P<float4>(s->xs), P<double4>(s->xs64), P<int>(s->ts),
                        P<double>(s->xorig), xbuild, P<float4>(s->sorg), P<float4>(s->ctr), P<float4>(s->half),
                        P<float4>(s->sctr), P<float4>(s->shalf), P<int>(s->nmaskwork), s->qpair, s->pme, pme_slots<float>(s));
   else
     hipLaunchKernelGGL(k_split_fill<double>, dim3(nblk((long long)s->nsuper * 64, 256)), dim3(256), 0, st, s->nsuper,
-                       P<int2>(s->sc_info), P<int>(s->perm2), P<double>(s->xwrap), P<int>(s->permp), P<int>(s->slot),
+                       P<int2>(s->sc_info), sorted_bins(s), P<double>(s->xwrap), P<int>(s->permp), P<int>(s->slot),
                        P<double>(s->q_d), P<int>(s->type_d), P<double4>(s->xs), P<double4>(s->xs64), P<int>(s->ts),
                        P<double>(s->xorig), xbuild, P<float4>(s->sorg), P<float4>(s->ctr), P<float4>(s->half),
                        P<float4>(s->sctr), P<float4>(s->shalf), P<int>(s->nmaskwork), s->qpair, s->pme, pme_slots<double>(s));
   if (timing) hipEventRecord(s->ev[1], st);
-  hipLaunchKernelGGL(k_build_list, dim3(s->nsuper), dim3(kListBlock), 0, st, s->lp, P<int>(s->sc_col),
-                     P<int>(s->colsc), P<float4>(s->sctr), P<float4>(s->shalf), P<float4>(s->ctr),
+  hipLaunchKernelGGL(k_build_list, dim3(s->nsuper), dim3(kListBlock), list_lds_bytes(s->cap), st, s->lp,
+                     P<int>(s->sc_col), P<int>(s->colsc), P<float4>(s->sctr), P<float4>(s->shalf), P<float4>(s->ctr),
                      P<float4>(s->half), P<int4>(s->entries), P<int>(s->count), P<int>(s->ecost), P<int>(s->lcost),
-                     P<int>(s->maskwork), P<int>(s->nmaskwork), s->maxmaskwork, P<int>(s->overflow));
-  if (!s->etab.empty())
-    hipLaunchKernelGGL(k_mark_exclusions, dim3(nblk((long long)s->etab.size(), 256)), dim3(256), 0, st,
-                       (int)s->etab.size(), P<int4>(s->etab_d), P<int>(s->slot), P<int4>(s->entries),
-                       P<int>(s->count), s->cap, P<int>(s->maskwork), P<int>(s->nmaskwork), s->maxmaskwork,
-                       P<int>(s->overflow));
-  // a wave per mask slot, up to 16 blocks per CU (the slots in use are known
-  // on the device only; waves beyond them return at once)
-  hipLaunchKernelGGL(k_build_masks,
-                     dim3((unsigned)std::min<long long>(nblk((long long)s->maxmaskwork, 4), 16ll * s->ctx->cus)),
-                     dim3(256), 0, st, P<int>(s->maskwork),
-                     P<int>(s->nmaskwork), s->maxmaskwork, P<int4>(s->entries), s->cap, P<int>(s->permp),
-                     P<int>(s->eptr_d), P<int2>(s->elist_d), P<unsigned short>(s->masks));
-  make_tiles(s, st);
+                     mask_args(s), P<int>(s->nmaskwork), P<int>(s->overflow));
+  make_runs(s, st);
   s->list_valid = true;
   s->prune_pending = true;
   if (timing) hipEventRecord(s->ev[2], st);
@@ -1367,9 +1355,8 @@ int grow_and_retry(Sys *s) {
   if (int rc0 = dalloc(s, s->border, 8 * (size_t)s->maxborder)) return rc0;
   int rc;
   if ((rc = dalloc(s, s->entries, 16 * (size_t)s->nsuper * s->cap)) || (rc = dalloc(s, s->ecost, 4 * (size_t)s->nsuper * s->cap)) ||
-      (rc = dalloc(s, s->tiles, 16 * (size_t)s->ntiles_cap)) ||
       (rc = dalloc(s, s->pair_e, 16 * (size_t)s->ntiles_cap)) || (rc = dalloc(s, s->npairs, 8 * (size_t)s->ntiles_cap)) ||
-      (rc = dalloc(s, s->hash, 8 * (size_t)s->ntiles_cap)) || (rc = dalloc(s, s->maskwork, 4 * (size_t)s->maxmaskwork)) ||
+      (rc = dalloc(s, s->hash, 8 * (size_t)s->ntiles_cap)) ||
       (rc = dalloc(s, s->masks, 16 * 8 * (size_t)s->maxmaskwork)))
     return rc;
   return PMX_OK;
@@ -1727,10 +1714,10 @@ int pmx_sys_set_tuning(pmx_sys *sys, int knob, int value) {
     run_pair_phase<true>(s, false, -1);
   else
     run_pair_phase<false>(s, false, -1);
-  // the tiles follow the schedule and the grid: cut the current list again
+  // the runs follow the schedule and the grid: cut the current list again
   // (the next MD step may use it without a rebuild)
   if (s->list_valid) {
-    make_tiles(s, s->ctx->stream);
+    make_runs(s, s->ctx->stream);
     HIPCHK(hipStreamSynchronize(s->ctx->stream));
   }
   return s->pme_on ? fft_blocking(s) : PMX_OK;
@@ -2239,7 +2226,7 @@ struct Batch {
   pmx_ctx *ctx = nullptr;
   std::vector<Sys *> sys;
   int nsys = 0;
-  BatchLaunch bin, scan, scatter, binrank, columns, split, list, excl, masks, rprefix, rcut, rtiles;
+  BatchLaunch bin, scan, scatter, split, list, runs;
   BatchLaunch kick, spread, pair, yfwd, xconv, yinv, plane, gather, fixups, ukd, unsort, begin, half;
   BatchLaunch energy;
   BatchBuf bsys, need, base, flags, rebuilds;
@@ -2309,31 +2296,23 @@ int batch_tables(Batch &b) {
   int rc;
   {
     std::vector<OpBin::Args> args_bin(ns);
-    std::vector<OpScanSingle::Args> args_scan(ns);
+    std::vector<OpScanColumns::Args> args_scan(ns);
     std::vector<OpScatter::Args> args_scatter(ns);
-    std::vector<OpBinrank::Args> args_binrank(ns);
-    std::vector<OpColumns::Args> args_columns(ns);
     std::vector<typename OpSplitFill<R>::Args> args_split(ns);
     std::vector<OpBuildList::Args> args_list(ns);
-    std::vector<OpMarkExclusions::Args> args_excl(ns);
-    std::vector<OpBuildMasks::Args> args_masks(ns);
-    std::vector<OpRunsPrefix::Args> args_rprefix(ns);
-    std::vector<OpRunsCut::Args> args_rcut(ns);
-    std::vector<OpRunsTiles::Args> args_rtiles(ns);
+    std::vector<OpRuns::Args> args_runs(ns);
+    size_t list_lds = 0;
     for (int i = 0; i < ns; ++i) {
       Sys *s = b.sys[i];
       args_bin[i] = {s->n, P<double>(s->xorig), s->bin, P<uint32_t>(s->key), P<uint32_t>(s->hist),
                      P<double>(s->xwrap), P<int>(s->refcell)};
-      args_scan[i] = {P<uint32_t>(s->hist), P<uint32_t>(s->start), P<uint32_t>(s->cursor), s->nbins};
+      args_scan[i] = {P<uint32_t>(s->hist), P<uint32_t>(s->start), P<uint32_t>(s->cursor), (int)s->nbins, s->ncols,
+                      s->bin.nzb, s->n, s->nsuper, P<int2>(s->sc_info), P<int>(s->sc_col), P<int>(s->colsc)};
       args_scatter[i] = {s->n, P<uint32_t>(s->key), P<uint32_t>(s->cursor), P<int>(s->perm)};
-      args_binrank[i] = {s->n, s->nbins, P<uint32_t>(s->key), P<uint32_t>(s->start), P<int>(s->perm),
-                         P<int>(s->perm2)};
-      args_columns[i] = {s->ncols, s->bin.nzb, s->n, s->nsuper, P<uint32_t>(s->start), P<int2>(s->sc_info),
-                         P<int>(s->sc_col), P<int>(s->colsc)};
       auto &sp = args_split[i];
       sp.nsuper = s->nsuper;
       sp.sc_info = P<int2>(s->sc_info);
-      sp.order = P<int>(s->perm2);
+      sp.sb = sorted_bins(s);
       sp.xwrap = P<double>(s->xwrap);
       sp.q = P<double>(s->q_d);
       sp.permp = P<int>(s->permp);
@@ -2355,40 +2334,22 @@ int batch_tables(Batch &b) {
       sp.rec = pme_slots<R>(s);
       args_list[i] = {s->lp, P<int>(s->sc_col), P<int>(s->colsc), P<float4>(s->sctr), P<float4>(s->shalf),
                       P<float4>(s->ctr), P<float4>(s->half), P<int4>(s->entries), P<int>(s->count),
-                      P<int>(s->ecost), P<int>(s->lcost), P<int>(s->maskwork), P<int>(s->nmaskwork),
-                      s->maxmaskwork, P<int>(s->overflow)};
-      args_excl[i] = {(int)s->etab.size(), s->cap, s->maxmaskwork, P<int4>(s->etab_d), P<int>(s->slot),
-                      P<int>(s->count), P<int4>(s->entries), P<int>(s->maskwork), P<int>(s->nmaskwork),
-                      P<int>(s->overflow)};
-      args_masks[i] = {P<int>(s->maskwork), P<int>(s->nmaskwork), s->maxmaskwork, s->cap, P<int4>(s->entries),
-                       P<int>(s->permp), P<int>(s->eptr_d), P<int2>(s->elist_d), P<unsigned short>(s->masks)};
-      int *const nruns = P<int>(s->ntiles) + 2;
-      args_rprefix[i] = {s->nsuper, P<int>(s->count), P<int>(s->lcost), nruns, P<int>(s->tep), P<long long>(s->tcp),
-                         P<int>(s->tpos), P<int>(s->tposS), kBatchRunCost};
-      args_rcut[i] = {s->nsuper, s->cap, P<int>(s->count), P<int>(s->ecost), nruns, P<int>(s->tep),
-                      P<long long>(s->tcp), P<int>(s->tpos), P<int>(s->tposS)};
-      args_rtiles[i] = {P<int>(s->count), P<int>(s->tep), P<int>(s->tpos), P<int>(s->tposS), P<int>(s->wstart),
-                        P<int4>(s->tiles), P<int>(s->ntiles), s->ntiles_cap};
+                      P<int>(s->ecost), P<int>(s->lcost), mask_args(s), P<int>(s->nmaskwork), P<int>(s->overflow)};
+      list_lds = std::max(list_lds, list_lds_bytes(s->cap));
+      args_runs[i] = {s->nsuper, s->cap, P<int>(s->count), P<int>(s->lcost), P<int>(s->ecost), kBatchRunCost,
+                      P<int2>(s->runs), P<int>(s->ntiles)};
     }
     for (int i = 0; i < ns; ++i) nb[i] = (int)nblk(b.sys[i]->n, 256);
     if ((rc = batch_table<OpBin>(b, b.bin, args_bin, nb, 0))) return rc;
     if ((rc = batch_table<OpScatter>(b, b.scatter, args_scatter, nb, 0))) return rc;
-    if ((rc = batch_table<OpBinrank>(b, b.binrank, args_binrank, nb, 0))) return rc;
     for (int i = 0; i < ns; ++i) nb[i] = 1;
-    if ((rc = batch_table<OpScanSingle>(b, b.scan, args_scan, nb, 0))) return rc;
-    if ((rc = batch_table<OpColumns>(b, b.columns, args_columns, nb, 0))) return rc;
-    if ((rc = batch_table<OpRunsPrefix>(b, b.rprefix, args_rprefix, nb, 0))) return rc;
-    if ((rc = batch_table<OpRunsTiles>(b, b.rtiles, args_rtiles, nb, 0))) return rc;
+    if ((rc = batch_table<OpScanColumns>(b, b.scan, args_scan, nb, 0))) return rc;
+    for (int i = 0; i < ns; ++i) nb[i] = (int)runs_blocks(b.sys[i]);
+    if ((rc = batch_table<OpRuns>(b, b.runs, args_runs, nb, 0))) return rc;
     for (int i = 0; i < ns; ++i) nb[i] = (int)nblk((long long)b.sys[i]->nsuper * 64, 256);
     if ((rc = batch_table<OpSplitFill<R>>(b, b.split, args_split, nb, 0))) return rc;
     for (int i = 0; i < ns; ++i) nb[i] = b.sys[i]->nsuper;
-    if ((rc = batch_table<OpBuildList>(b, b.list, args_list, nb, 0))) return rc;
-    if ((rc = batch_table<OpRunsCut>(b, b.rcut, args_rcut, nb, 0))) return rc;
-    for (int i = 0; i < ns; ++i) nb[i] = b.sys[i]->etab.empty() ? 0 : (int)nblk((long long)b.sys[i]->etab.size(), 256);
-    if ((rc = batch_table<OpMarkExclusions>(b, b.excl, args_excl, nb, 0))) return rc;
-    // a wave per mask slot in use (known on the device only), up to 64 blocks
-    for (int i = 0; i < ns; ++i) nb[i] = (int)std::min<long long>(nblk((long long)b.sys[i]->maxmaskwork, 4), 64);
-    if ((rc = batch_table<OpBuildMasks>(b, b.masks, args_masks, nb, 0))) return rc;
+    if ((rc = batch_table<OpBuildList>(b, b.list, args_list, nb, list_lds))) return rc;
   }
   {
     std::vector<typename OpKickDrift<R>::Args> args_kick(ns);
@@ -2420,7 +2381,7 @@ int batch_tables(Batch &b) {
       args_spread[i] = {s->pme, s->plz, P<int2>(s->tcol), P<int>(s->colsc), P<R4>(s->pmw), P<int2>(s->pmb),
                         P<Cx<T>>(s->twz), P<Cx<T>>(s->spec)};
       const R4 *ljt = MIXED ? reinterpret_cast<const R4 *>(s->ljt32.p) : reinterpret_cast<const R4 *>(s->ljtab.p);
-      args_pair[i] = {s->pp, P<int4>(s->tiles), P<int>(s->ntiles), P<int>(s->wstart), P<int>(s->tilectr),
+      args_pair[i] = {s->pp, P<int2>(s->runs), P<int>(s->ntiles), P<int>(s->count), P<int>(s->tilectr),
                       P<int4>(s->entries), s->cap, P<unsigned short>(s->masks), P<R4>(s->xs), P<float4>(s->sorg),
                       P<int>(s->ts), P<int>(s->permp), P<double>(s->ljtab), ljt, facc,
                       PairOut{P<double>(s->pair_e), P<long long>(s->npairs), P<unsigned long long>(s->hash),
@@ -2537,17 +2498,11 @@ int batch_chunk(Batch &b, int K, bool opening) {
     if (k == 0) batch_go<OpKickDrift<R>>(b.kick, st, bk);
     hipLaunchKernelGGL(k_batch_need, dim3(nblk(ns, 256)), dim3(256), 0, st, ns, bs, k, need);
     batch_go<OpBin>(b.bin, st, bk);
-    batch_go<OpScanSingle>(b.scan, st, bk);
+    batch_go<OpScanColumns>(b.scan, st, bk);
     batch_go<OpScatter>(b.scatter, st, bk);
-    batch_go<OpBinrank>(b.binrank, st, bk);
-    batch_go<OpColumns>(b.columns, st, bk);
     batch_go<OpSplitFill<R>>(b.split, st, bk);
     batch_go<OpBuildList>(b.list, st, bk);
-    batch_go<OpMarkExclusions>(b.excl, st, bk);
-    batch_go<OpBuildMasks>(b.masks, st, bk);
-    batch_go<OpRunsPrefix>(b.rprefix, st, bk);
-    batch_go<OpRunsCut>(b.rcut, st, bk);
-    batch_go<OpRunsTiles>(b.rtiles, st, bk);
+    batch_go<OpRuns>(b.runs, st, bk);
     // the spread has the device to itself (beside the pair kernel a CU has
     // room for one of its blocks at a time: 0.51 ms instead of 0.1 for 64
     // systems of 331,000 atoms); fork: the rest of the PME chain beside the
@@ -2599,17 +2554,11 @@ int batch_forces(Batch &b) {
   BHIPCHK(hipMemcpyAsync(b.bsys.p, b.bsys_h, sizeof(BatchSys) * ns, hipMemcpyHostToDevice, st));
   const BatchStep bk{0, 0, reinterpret_cast<unsigned char *>(b.need.p)};
   batch_go<OpBin>(b.bin, st, bk);
-  batch_go<OpScanSingle>(b.scan, st, bk);
+  batch_go<OpScanColumns>(b.scan, st, bk);
   batch_go<OpScatter>(b.scatter, st, bk);
-  batch_go<OpBinrank>(b.binrank, st, bk);
-  batch_go<OpColumns>(b.columns, st, bk);
   batch_go<OpSplitFill<R>>(b.split, st, bk);
   batch_go<OpBuildList>(b.list, st, bk);
-  batch_go<OpMarkExclusions>(b.excl, st, bk);
-  batch_go<OpBuildMasks>(b.masks, st, bk);
-  batch_go<OpRunsPrefix>(b.rprefix, st, bk);
-  batch_go<OpRunsCut>(b.rcut, st, bk);
-  batch_go<OpRunsTiles>(b.rtiles, st, bk);
+  batch_go<OpRuns>(b.runs, st, bk);
   batch_go<OpPmeSpreadZ<MIXED, ORDER>>(b.spread, st, bk);
   BHIPCHK(hipEventRecord(b.fork, st));
   BHIPCHK(hipStreamWaitEvent(st2, b.fork, 0));

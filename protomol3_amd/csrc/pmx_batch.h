@@ -71,15 +71,18 @@ struct OpBin {
   }
 };
 
-struct OpScanSingle {
+struct OpScanColumns {
   struct Args {
     uint32_t *hist, *start, *cursor;
-    long long nbins;
+    int nbins, ncols, nzb, n, nsuper;
+    int2 *sc_info;
+    int *sc_col, *colsc;
   };
   static constexpr int kBlock = kScanBlock, kMinBlocks = 1;
   static constexpr bool kGated = true;
   __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &) {
-    scan_single_body(bid, nbk, a.hist, a.nbins, a.start, a.cursor);
+    scan_columns_body(a.hist, a.nbins, a.start, a.cursor, a.ncols, a.nzb, a.n, a.nsuper, a.sc_info, a.sc_col,
+                      a.colsc);
   }
 };
 
@@ -97,41 +100,12 @@ struct OpScatter {
   }
 };
 
-struct OpBinrank {
-  struct Args {
-    int n;
-    long long nbins;
-    const uint32_t *key, *start;
-    const int *in;
-    int *out;
-  };
-  static constexpr int kBlock = 256, kMinBlocks = 1;
-  static constexpr bool kGated = true;
-  __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &) {
-    binrank_body(bid, nbk, a.n, a.nbins, a.key, a.start, a.in, a.out);
-  }
-};
-
-struct OpColumns {
-  struct Args {
-    int ncols, nzb, n, nsuper;
-    const uint32_t *start;
-    int2 *sc_info;
-    int *sc_col, *colsc;
-  };
-  static constexpr int kBlock = 1024, kMinBlocks = 1;
-  static constexpr bool kGated = true;
-  __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &) {
-    columns_body(bid, nbk, a.ncols, a.nzb, a.n, a.start, a.nsuper, a.sc_info, a.sc_col, a.colsc);
-  }
-};
-
 template <class R>
 struct OpSplitFill {
   struct Args {
     int nsuper;
     const int2 *sc_info;
-    const int *order;
+    SortedBins sb;
     const double *xwrap, *q;
     int *permp, *slot;
     const int *type;
@@ -149,7 +123,7 @@ struct OpSplitFill {
   static constexpr int kBlock = 256, kMinBlocks = 1;
   static constexpr bool kGated = true;
   __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &) {
-    split_fill_body<R>(bid, nbk, a.nsuper, a.sc_info, a.order, a.xwrap, a.permp, a.slot, a.q, a.type, a.xs, a.xs64,
+    split_fill_body<R>(bid, nbk, a.nsuper, a.sc_info, a.sb, a.xwrap, a.permp, a.slot, a.q, a.type, a.xs, a.xs64,
                        a.ts, a.xorig, a.xbuild, a.sorg, a.ctr, a.half, a.sctr, a.shalf, a.nmaskwork, a.qpair, a.pme,
                        a.rec);
   }
@@ -161,93 +135,30 @@ struct OpBuildList {
     const int *sc_col, *colsc;
     const float4 *sctr, *shalf, *ctr, *half;
     int4 *entries;
-    int *count, *ecost, *cost_out, *maskwork, *nmaskwork;
-    int maxmaskwork;
-    int *overflow;
+    int *count, *ecost, *cost_out;
+    MaskArgs ma;
+    int *nmaskwork, *overflow;
   };
   static constexpr int kBlock = kListBlock, kMinBlocks = 1;
   static constexpr bool kGated = true;
   __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &) {
     build_list_body(bid, nbk, a.q, a.sc_col, a.colsc, a.sctr, a.shalf, a.ctr, a.half, a.entries, a.count, a.ecost,
-                    a.cost_out, a.maskwork, a.nmaskwork, a.maxmaskwork, a.overflow);
+                    a.cost_out, a.ma, a.nmaskwork, a.overflow);
   }
 };
 
-struct OpMarkExclusions {
-  struct Args {
-    int ne, cap, maxmaskwork;
-    const int4 *etab;
-    const int *slot, *count;
-    int4 *entries;
-    int *maskwork, *nmaskwork, *overflow;
-  };
-  static constexpr int kBlock = 256, kMinBlocks = 1;
-  static constexpr bool kGated = true;
-  __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &) {
-    mark_exclusions_body(bid, nbk, a.ne, a.etab, a.slot, a.entries, a.count, a.cap, a.maskwork, a.nmaskwork,
-                         a.maxmaskwork, a.overflow);
-  }
-};
-
-struct OpBuildMasks {
-  struct Args {
-    const int *maskwork, *nmaskwork;
-    int maxmaskwork, cap;
-    int4 *entries;
-    const int *perm, *eptr;
-    const int2 *elist;
-    unsigned short *masks;
-  };
-  static constexpr int kBlock = 256, kMinBlocks = 1;
-  static constexpr bool kGated = true;
-  __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &) {
-    build_masks_body(bid, nbk, a.maskwork, a.nmaskwork, a.maxmaskwork, a.entries, a.cap, a.perm, a.eptr, a.elist,
-                     a.masks);
-  }
-};
-
-struct OpRunsPrefix {
-  struct Args {
-    int nsuper;
-    const int *count, *cost;
-    int *nruns, *ep;
-    long long *cp;
-    int *pos, *posS;
-    long long min_run_cost;
-  };
-  static constexpr int kBlock = 1024, kMinBlocks = 1;
-  static constexpr bool kGated = true;
-  __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &) {
-    runs_prefix_body(bid, nbk, a.nsuper, a.count, a.cost, a.nruns, a.ep, a.cp, a.pos, a.posS, a.min_run_cost);
-  }
-};
-
-struct OpRunsCut {
+struct OpRuns {
   struct Args {
     int nsuper, cap;
-    const int *count, *ecost, *nruns, *ep;
-    const long long *cp;
-    int *pos, *posS;
-  };
-  static constexpr int kBlock = 256, kMinBlocks = 1;
-  static constexpr bool kGated = true;
-  __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &) {
-    runs_cut_body(bid, nbk, a.nsuper, a.count, a.ecost, a.cap, a.nruns, a.ep, a.cp, a.pos, a.posS);
-  }
-};
-
-struct OpRunsTiles {
-  struct Args {
-    const int *count, *ep, *pos, *posS;
-    int *wstart;
-    int4 *tiles;
+    const int *count, *cost, *ecost;
+    long long min_run_cost;
+    int2 *runs;
     int *ntiles;
-    int ntiles_cap;
   };
-  static constexpr int kBlock = 1024, kMinBlocks = 1;
+  static constexpr int kBlock = kRunsBlock, kMinBlocks = 1;
   static constexpr bool kGated = true;
   __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &) {
-    runs_tiles_body(bid, nbk, a.count, a.ep, a.pos, a.posS, a.wstart, a.tiles, a.ntiles, a.ntiles_cap);
+    runs_body(bid, nbk, a.nsuper, a.count, a.cost, a.ecost, a.cap, a.min_run_cost, a.runs, a.ntiles);
   }
 };
 
@@ -302,8 +213,8 @@ struct OpPair {
   using R4 = typename Real4<typename std::conditional<MIXED, float, double>::type>::type;
   struct Args {
     PairParams pp;
-    const int4 *tiles;
-    const int *ntiles, *wstart;
+    const int2 *runs;
+    const int *ntiles, *count;
     int *tilectr;
     int4 *entries;
     int cap;
@@ -321,11 +232,11 @@ struct OpPair {
   // the runs in contiguous shares per wave (schedule 0)
   __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &) {
     if constexpr (MIXED)
-      pair_direct_body<COUL, LJSW, CSW, BIGLJ, kPairPlain>(bid, nbk, a.pp, 0, a.tiles, a.ntiles, a.wstart, a.tilectr,
+      pair_direct_body<COUL, LJSW, CSW, BIGLJ, kPairPlain>(bid, nbk, a.pp, 0, a.runs, a.ntiles, a.count, a.tilectr,
                                                            a.entries, a.entries, a.cap, a.masks, a.xs, a.sorg, a.ts,
                                                            a.perm, a.ljtab, a.ljt, a.facc, a.out);
     else
-      pair_body<MIXED, COUL, LJSW, CSW, BIGLJ, kPairPlain>(bid, nbk, a.pp, 0, a.tiles, a.ntiles, a.wstart, a.tilectr,
+      pair_body<MIXED, COUL, LJSW, CSW, BIGLJ, kPairPlain>(bid, nbk, a.pp, 0, a.runs, a.ntiles, a.count, a.tilectr,
                                                            a.entries, a.entries, a.cap, a.masks, a.xs, a.sorg, a.ts,
                                                            a.perm, a.ljtab, a.ljt, a.facc, a.out);
   }

@@ -94,6 +94,17 @@ __device__ inline int wave_max(int v) {
   return v;
 }
 
+// inclusive prefix over the wave
+__device__ inline int wave_prefix(int v) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int off = 1; off < kWave; off <<= 1) {
+    const int y = __shfl_up(v, off);
+    if (lane >= off) v += y;
+  }
+  return v;
+}
+
 struct PmeParams {
   int nx, ny, nz, nzh, order;
   double hxr, hyr, hzr;   // K/L per axis (Grid.h:520-522)
@@ -218,8 +229,8 @@ static __global__ void k_bin(int n, const double *__restrict__ xorig, BinParams 
 }
 
 // Counting sort by key (one radix digit spanning the key range): histogram,
-// exclusive scan, scatter, then order each bin by atom index so the result is
-// deterministic and stable.
+// exclusive scan, scatter; the split takes each bin's atoms in index order, so
+// the result is deterministic.
 static __global__ void k_fill_u32(uint32_t *p, uint32_t v, long long n) {
   long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
@@ -296,47 +307,115 @@ static __global__ void k_scan_final(uint32_t *__restrict__ in, long long m, cons
   }
 }
 
-// Exclusive scan of m <= kScanSingleMax counts in one block: each wave owns
-// a contiguous segment and walks it in coalesced 64-count chunks (a wave
-// prefix per chunk, a running offset across chunks); segment totals are
-// combined across the block first.  The counts are cleared for the next
-// histogram.
+// Superclusters of each column: sc_info[sc] = (first sorted position, atom
+// count) and sc_col[sc] = its column for sc < total, (0, 0) and -1 beyond;
+// colsc[col] = first supercluster of column col, colsc[ncols] = total.  One
+// block of 1,024 takes the columns in chunks with a running offset.
+__device__ __forceinline__ void columns_block(int ncols, int nzb, int n, const uint32_t *start, int nsuper_max,
+                                              int2 *__restrict__ sc_info, int *__restrict__ sc_col,
+                                              int *__restrict__ colsc) {
+  __shared__ int s_w[kScanBlock / kWave];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  int carry = 0;
+  for (int base = 0; base < ncols; base += kScanBlock) {
+    const int col = base + threadIdx.x;
+    int cs = 0, cnt = 0;
+    if (col < ncols) {
+      cs = (int)start[(size_t)col * nzb];
+      const int ce = col + 1 < ncols ? (int)start[(size_t)(col + 1) * nzb] : n;
+      cnt = ce - cs;
+    }
+    const int nsc = (cnt + kSuperSize - 1) / kSuperSize;
+    const int incl = wave_prefix(nsc);
+    if (lane == kWave - 1) s_w[wv] = incl;
+    __syncthreads();
+    int before = 0, all = 0;
+    for (int w = 0; w < kScanBlock / kWave; ++w) {
+      const int v = s_w[w];
+      before += w < wv ? v : 0;
+      all += v;
+    }
+    const int first = carry + before + incl - nsc;
+    if (col < ncols) colsc[col] = first;
+    for (int q = 0; q < nsc && first + q < nsuper_max; ++q) {
+      sc_info[first + q] = make_int2(cs + q * kSuperSize, min(kSuperSize, cnt - q * kSuperSize));
+      sc_col[first + q] = col;
+    }
+    carry += all;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) colsc[ncols] = carry;
+  for (int sc = carry + threadIdx.x; sc < nsuper_max; sc += kScanBlock) {
+    sc_info[sc] = make_int2(0, 0);
+    sc_col[sc] = -1;
+  }
+}
+
+static __global__ void __launch_bounds__(kScanBlock) k_columns(int ncols, int nzb, int n, const uint32_t *start,
+                                                               int nsuper_max, int2 *__restrict__ sc_info,
+                                                               int *__restrict__ sc_col, int *__restrict__ colsc) {
+  columns_block(ncols, nzb, n, start, nsuper_max, sc_info, sc_col, colsc);
+}
+
+// Exclusive scan of m <= kScanSingleMax counts and the columns'
+// superclusters, in one block: bound by latency, so each wave owns a
+// contiguous segment, four counts a lane and round, and every round is loaded
+// before the first is summed; segment totals are combined across the block.
+// Counts and starts are padded to whole groups of four.  The counts are cleared for the next histogram.
 constexpr long long kScanSingleMax = 1 << 16;
-__device__ __forceinline__ void scan_single_body(const int bid_, const int nbk_, uint32_t *__restrict__ in, long long m,
-                                                 uint32_t *__restrict__ out, uint32_t *__restrict__ out2) {
-  constexpr int NW = kScanBlock / kWave;
+__device__ __forceinline__ void scan_columns_body(uint32_t *__restrict__ in, int m, uint32_t *out,
+                                                  uint32_t *__restrict__ out2, int ncols, int nzb, int n,
+                                                  int nsuper_max, int2 *__restrict__ sc_info,
+                                                  int *__restrict__ sc_col, int *__restrict__ colsc) {
+  constexpr int NW = kScanBlock / kWave, ROUND = 4 * kWave;
+  constexpr int RMAX = (int)(kScanSingleMax / (NW * ROUND));
   __shared__ uint32_t s_tot[NW];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const long long seg = ((m + NW - 1) / NW + kWave - 1) / kWave * kWave;
-  const long long b = min(m, (long long)w * seg), e = min(m, b + seg);
+  const int seg = ((m + NW - 1) / NW + ROUND - 1) / ROUND * ROUND;  // at most RMAX rounds
+  const int b = w * seg;
+  uint4 v[RMAX];
+#pragma unroll
+  for (int r = 0; r < RMAX; ++r) {
+    v[r] = make_uint4(0, 0, 0, 0);
+    const int i = b + r * ROUND + 4 * lane;
+    if (r * ROUND < seg && i < m) v[r] = *reinterpret_cast<const uint4 *>(in + i);  // (m is padded)
+  }
   uint32_t t = 0;
-  for (long long i = b + lane; i < e; i += kWave) t += in[i];
+#pragma unroll
+  for (int r = 0; r < RMAX; ++r) t += v[r].x + v[r].y + v[r].z + v[r].w;
   t = wave_sum(t);
   if (lane == 0) s_tot[w] = t;
   __syncthreads();
   uint32_t base = 0;
   for (int k = 0; k < w; ++k) base += s_tot[k];
-  for (long long c = b; c < e; c += kWave) {
-    const long long i = c + lane;
-    const uint32_t v = i < e ? in[i] : 0u;
-    uint32_t x = v;
 #pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-      const uint32_t y = __shfl_up(x, off);
-      if (lane >= off) x += y;
+  for (int r = 0; r < RMAX; ++r) {
+    if (r * ROUND >= seg) break;
+    const uint32_t own = v[r].x + v[r].y + v[r].z + v[r].w;
+    const uint32_t incl = (uint32_t)wave_prefix((int)own);
+    const int i = b + r * ROUND + 4 * lane;
+    uint4 at;
+    at.x = base + incl - own;
+    at.y = at.x + v[r].x;
+    at.z = at.y + v[r].y;
+    at.w = at.z + v[r].z;
+    if (i < m) {
+      *reinterpret_cast<uint4 *>(out + i) = at;
+      *reinterpret_cast<uint4 *>(out2 + i) = at;
+      *reinterpret_cast<uint4 *>(in + i) = make_uint4(0, 0, 0, 0);
     }
-    if (i < e) {
-      out[i] = base + x - v;
-      out2[i] = base + x - v;
-      in[i] = 0u;
-    }
-    base += __shfl(x, kWave - 1);
+    base += (uint32_t)__shfl((int)incl, kWave - 1);
   }
+  __syncthreads();
+  columns_block(ncols, nzb, n, out, nsuper_max, sc_info, sc_col, colsc);
 }
 
-static __global__ void k_scan_single(uint32_t *__restrict__ in, long long m, uint32_t *__restrict__ out,
-                              uint32_t *__restrict__ out2) {
-  scan_single_body(blockIdx.x, gridDim.x, in, m, out, out2);
+static __global__ void __launch_bounds__(kScanBlock) k_scan_columns(uint32_t *__restrict__ in, int m, uint32_t *out,
+                                                                    uint32_t *__restrict__ out2, int ncols, int nzb,
+                                                                    int n, int nsuper_max, int2 *__restrict__ sc_info,
+                                                                    int *__restrict__ sc_col,
+                                                                    int *__restrict__ colsc) {
+  scan_columns_body(in, m, out, out2, ncols, nzb, n, nsuper_max, sc_info, sc_col, colsc);
 }
 
 __device__ __forceinline__ void scatter_body(const int bid_, const int nbk_, int n, const uint32_t *__restrict__ key,
@@ -350,74 +429,16 @@ static __global__ void k_scatter(int n, const uint32_t *__restrict__ key, uint32
   scatter_body(blockIdx.x, gridDim.x, n, key, cursor, perm);
 }
 
-// Orders each bin by atom index: position p of the scatter output moves to
-// its bin's start plus the number of smaller atom indices in the bin (bins
-// hold a handful of atoms; the result does not depend on the scatter order).
-__device__ __forceinline__ void binrank_body(const int bid_, const int nbk_, int n, long long nbins,
-                                             const uint32_t *__restrict__ key, const uint32_t *__restrict__ start,
-                                             const int *__restrict__ in, int *__restrict__ out) {
-  const int p = bid_ * blockDim.x + threadIdx.x;
-  if (p >= n) return;
-  const int a = in[p];
-  const uint32_t b = key[a];
-  const int s0 = (int)start[b], s1 = b + 1 < (uint64_t)nbins ? (int)start[b + 1] : n;
-  int rank = 0;
-  for (int q = s0; q < s1; ++q) rank += in[q] < a;
-  out[s0 + rank] = a;
-}
-
-static __global__ void k_binrank(int n, long long nbins, const uint32_t *__restrict__ key,
-                          const uint32_t *__restrict__ start, const int *__restrict__ in, int *__restrict__ out) {
-  binrank_body(blockIdx.x, gridDim.x, n, nbins, key, start, in, out);
-}
-
-// Superclusters of each column: sc_info[sc] = (first sorted position, atom
-// count) and sc_col[sc] = its column for sc < total, (0, 0) and -1 beyond;
-// colsc[col] = first supercluster of column col, colsc[ncols] = total.  One
-// block; columns in chunks of the block size with a running offset.
-__device__ __forceinline__ void columns_body(const int bid_, const int nbk_, int ncols, int nzb, int n,
-                                             const uint32_t *__restrict__ start, int nsuper_max,
-                                             int2 *__restrict__ sc_info, int *__restrict__ sc_col,
-                                             int *__restrict__ colsc) {
-  __shared__ int s[1024];
-  int carry = 0;
-  for (int base = 0; base < ncols; base += blockDim.x) {
-    const int col = base + threadIdx.x;
-    int cs = 0, cnt = 0;
-    if (col < ncols) {
-      cs = (int)start[(size_t)col * nzb];
-      const int ce = col + 1 < ncols ? (int)start[(size_t)(col + 1) * nzb] : n;
-      cnt = ce - cs;
-    }
-    const int nsc = (cnt + kSuperSize - 1) / kSuperSize;
-    s[threadIdx.x] = nsc;
-    __syncthreads();
-    for (int off = 1; off < (int)blockDim.x; off <<= 1) {
-      int v = threadIdx.x >= off ? s[threadIdx.x - off] : 0;
-      __syncthreads();
-      s[threadIdx.x] += v;
-      __syncthreads();
-    }
-    const int first = carry + s[threadIdx.x] - nsc;
-    if (col < ncols) colsc[col] = first;
-    for (int q = 0; q < nsc && first + q < nsuper_max; ++q) {
-      sc_info[first + q] = make_int2(cs + q * kSuperSize, min(kSuperSize, cnt - q * kSuperSize));
-      sc_col[first + q] = col;
-    }
-    __syncthreads();
-    carry += s[blockDim.x - 1];
-    __syncthreads();
+// The atoms of bin [s0, s1) that belong at positions [p0, p1) when the bin is
+// ordered by atom index (the scatter leaves a bin's atoms in any order), one
+// wave; bins hold a handful of atoms.
+__device__ inline void ranked_bin(const int *__restrict__ in, int s0, int s1, int p0, int p1, int *out) {
+  for (int q = s0 + (int)(threadIdx.x & 63); q < s1; q += kWave) {
+    const int a = in[q];
+    int p = s0;
+    for (int r = s0; r < s1; ++r) p += in[r] < a;
+    if (p >= p0 && p < p1) out[p - p0] = a;
   }
-  if (threadIdx.x == 0) colsc[ncols] = carry;
-  for (int sc = carry + threadIdx.x; sc < nsuper_max; sc += blockDim.x) {
-    sc_info[sc] = make_int2(0, 0);
-    sc_col[sc] = -1;
-  }
-}
-
-static __global__ void k_columns(int ncols, int nzb, int n, const uint32_t *__restrict__ start, int nsuper_max,
-                          int2 *__restrict__ sc_info, int *__restrict__ sc_col, int *__restrict__ colsc) {
-  columns_body(blockIdx.x, gridDim.x, ncols, nzb, n, start, nsuper_max, sc_info, sc_col, colsc);
 }
 
 // Ascending bitonic sort of (key, idx) within aligned segments of SEG lanes.
@@ -461,9 +482,18 @@ constexpr float kScSlack = 1e-3f;
 //    ctr.w = real atoms, empty clusters get negative half extents), and per
 //    supercluster (the whole wave, widened by kScSlack).
 // Thread 0 also clears the mask work counter of the list build that follows.
+// The atoms by bin (in any order within a bin) and the bins' first positions.
+struct SortedBins {
+  int n;
+  long long nbins;
+  const uint32_t *key, *start;
+  const int *order;
+  __device__ int end(uint32_t b) const { return (long long)b + 1 < nbins ? (int)start[b + 1] : n; }
+};
+
 template <class R>
 __device__ __forceinline__ void split_fill_body(const int bid_, const int nbk_, int nsuper_max,
-                                                const int2 *__restrict__ sc_info, const int *__restrict__ order,
+                                                const int2 *__restrict__ sc_info, const SortedBins &sb,
                                                 const double *__restrict__ xwrap, int *__restrict__ permp,
                                                 int *__restrict__ slot, const double *__restrict__ q,
                                                 const int *__restrict__ type, typename Real4<R>::type *__restrict__ xs,
@@ -478,7 +508,24 @@ __device__ __forceinline__ void split_fill_body(const int bid_, const int nbk_, 
   if (bid_ == 0 && threadIdx.x == 0) *nmaskwork = 0;
   if (sc >= nsuper_max) return;  // whole waves
   const int2 info = sc_info[sc];
-  int a = lane < info.y ? order[info.x + lane] : -1;
+  // The sort below orders the supercluster's atoms whatever order they come
+  // in; which of a bin's atoms they are matters only for a bin that
+  // continues in the previous or the next supercluster.
+  __shared__ int s_order[256 / kWave][kSuperSize];
+  int *const so = s_order[threadIdx.x >> 6];
+  int a = lane < info.y ? sb.order[info.x + lane] : -1;
+  if (info.y > 0) {
+    const int end = info.x + info.y;
+    const uint32_t b = a >= 0 ? sb.key[a] : 0u;
+    const uint32_t b0 = __shfl(b, 0), b1 = __shfl(b, info.y - 1);
+    so[lane] = a;
+    __builtin_amdgcn_wave_barrier();
+    const int f0 = (int)sb.start[b0], f1 = sb.end(b0), l0 = (int)sb.start[b1], l1 = sb.end(b1);
+    if (f0 < info.x || f1 > end) ranked_bin(sb.order, f0, f1, info.x, end, so);
+    if (b1 != b0 && l1 > end) ranked_bin(sb.order, l0, l1, info.x, end, so);
+    __builtin_amdgcn_wave_barrier();
+    a = so[lane];
+  }
   int idx = a < 0 ? 0x7fffffff : a;
   double key = a < 0 ? 1.0e300 : xwrap[3 * a];
   wave_sort<64>(key, idx);
@@ -576,7 +623,7 @@ __device__ __forceinline__ void split_fill_body(const int bid_, const int nbk_, 
 
 template <class R>
 __global__ void __launch_bounds__(256) k_split_fill(int nsuper_max, const int2 *__restrict__ sc_info,
-                                                    const int *__restrict__ order, const double *__restrict__ xwrap,
+                                                    SortedBins sb, const double *__restrict__ xwrap,
                                                     int *__restrict__ permp, int *__restrict__ slot,
                                                     const double *__restrict__ q, const int *__restrict__ type,
                                                     typename Real4<R>::type *__restrict__ xs,
@@ -586,7 +633,7 @@ __global__ void __launch_bounds__(256) k_split_fill(int nsuper_max, const int2 *
                                                     float4 *__restrict__ half, float4 *__restrict__ sctr,
                                                     float4 *__restrict__ shalf, int *__restrict__ nmaskwork,
                                                     double qpair, PmeParams pme, PmeSlots<R> rec) {
-  split_fill_body<R>(blockIdx.x, gridDim.x, nsuper_max, sc_info, order, xwrap, permp, slot, q, type, xs, xs64, ts,
+  split_fill_body<R>(blockIdx.x, gridDim.x, nsuper_max, sc_info, sb, xwrap, permp, slot, q, type, xs, xs64, ts,
                      xorig, xbuild, sorg, ctr, half, sctr, shalf, nmaskwork, qpair, pme, rec);
 }
 
@@ -689,7 +736,7 @@ __device__ inline int col_runs(int c, int k, int n, int r[2][2]) {
 // appends a list entry when at least one is within the list radius.  Called
 // by every thread of the block with cj ascending over threads; a block-wide
 // prefix count keeps the entries sorted by cj.  Diagonal entries and entries
-// with a partial cluster get a mask work slot (explicit pair masks).
+// with a partial cluster are flagged in s_need (explicit pair masks).
 constexpr int kListBlock = 256;
 // Work estimate of a list entry for cutting the list into runs, in units of
 // about 35 ns of one pair-kernel wave (fitted to per-wave times): kCpCost per
@@ -702,10 +749,9 @@ constexpr int kListBlock = 256;
 // their forces once more).
 constexpr int kCpCost = 8, kMemCost = 9, kEntryCost = 14, kTileCost = 80;
 
-__device__ inline void list_append(const ListParams &q, int S, const float4 (&ic)[8], const float4 (&ih)[8], int cj,
-                                   float4 jc, float4 jh, int4 *__restrict__ entries, int *__restrict__ maskwork,
-                                   int *__restrict__ nmaskwork, int maxmaskwork, int *__restrict__ overflow,
-                                   int *s_cnt, int *s_cost, int *__restrict__ ecost, int &total, int &ctotal) {
+__device__ inline void list_append(const ListParams &q, int S, const float4 *ic, const float4 *ih, int cj,
+                                   float4 jc, float4 jh, int4 *__restrict__ entries, unsigned *s_need,
+                                   int *__restrict__ overflow, int *s_cnt, int *s_cost, int *__restrict__ ecost, int &total, int &ctotal) {
   constexpr int NW = kListBlock / kWave;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   uint32_t imask = 0;
@@ -757,27 +803,10 @@ __device__ inline void list_append(const ListParams &q, int S, const float4 (&ic
   }
   __syncthreads();
   const int e = total + before + __popcll(act & ((1ull << lane) - 1ull));
-  // mask work slots for this wave's entries that need explicit masks, one
-  // atomic per wave
-  const unsigned long long nw = __ballot(imask != 0 && need && e < q.cap);
-  int wbase = 0;
-  if (nw) {
-    if (lane == 0) wbase = atomicAdd(nmaskwork, (int)__popcll(nw));
-    wbase = __builtin_amdgcn_readfirstlane(__shfl(wbase, 0));
-  }
   if (imask != 0) {
     if (e < q.cap) {
-      int moff = -1;
-      if (need) {
-        const int w = wbase + __popcll(nw & ((1ull << lane) - 1ull));
-        if (w < maxmaskwork) {
-          maskwork[w] = S * q.cap + e;
-          moff = -2;
-        } else {
-          atomicExch(overflow, 1);
-        }
-      }
-      entries[(size_t)S * q.cap + e] = make_int4(cj, (int)imask, moff, per_pair ? kShiftPerPair : shift);
+      if (need) atomicOr(&s_need[e >> 5], 1u << (e & 31));
+      entries[(size_t)S * q.cap + e] = make_int4(cj, (int)imask, -1, per_pair ? kShiftPerPair : shift);
       ecost[(size_t)S * q.cap + e] = kTileCost + ctotal + cbefore + wc;  // the tile cost counts from entry 0
     } else {
       atomicExch(overflow, 1);
@@ -786,6 +815,16 @@ __device__ inline void list_append(const ListParams &q, int S, const float4 (&ic
   total += all;
   ctotal += call;
 }
+
+// Masks of one supercluster made together, in LDS.
+constexpr int kMaskBatch = 64;
+struct MaskArgs {
+  const int *perm, *slot, *eptr;
+  const int2 *elist;
+  unsigned short *masks;
+  int maxmaskwork;
+};
+inline size_t list_lds_bytes(int cap) { return 8 * (size_t)((cap + 31) / 32); }
 
 // Cluster-pair list of supercluster S (one block each).  Superclusters are
 // numbered column by column (x-major, then y, then z inside a column), so the
@@ -796,14 +835,31 @@ __device__ inline void list_append(const ListParams &q, int S, const float4 (&ic
 // eight i-clusters of S, and entries are appended in ascending cj.  Only
 // cj >= 8S is listed, so each cluster pair appears once.  The work per S is
 // bounded by the neighbourhood, independent of the system size.
+//
+// The block then gives the entries of S that need them their explicit masks
+// (diagonal entries, entries with a partial cluster or an excluded or scaled
+// pair).  Mask slot w holds one 16-bit word per lane l = tj*8 + ti of the
+// pair kernel: bit c set when i = slot 8ci+ti (ci = 8S + c, c in the entry's
+// mask) and j = slot 8cj+tj are real atoms, i precedes j within a shared
+// cluster, and the pair is not FULL-excluded; bit 8 + c marks MODIFIED.  The
+// entry's mask field becomes w.  The excluded pairs of the supercluster's
+// atoms look up their entry (sorted by j-cluster); a pair whose clusters are
+// not listed is beyond the list radius and never evaluated.
 __device__ __forceinline__ void build_list_body(const int bid_, const int nbk_, const ListParams &q,
                                                 const int *__restrict__ sc_col, const int *__restrict__ colsc,
                                                 const float4 *__restrict__ sctr, const float4 *__restrict__ shalf,
                                                 const float4 *__restrict__ ctr, const float4 *__restrict__ half,
-                                                int4 *__restrict__ entries, int *__restrict__ count,
-                                                int *__restrict__ ecost, int *__restrict__ cost_out,
-                                                int *__restrict__ maskwork, int *__restrict__ nmaskwork,
-                                                int maxmaskwork, int *__restrict__ overflow) {
+                                                int4 *entries, int *__restrict__ count, int *ecost,
+                                                int *__restrict__ cost_out, const MaskArgs &ma,
+                                                int *__restrict__ nmaskwork, int *__restrict__ overflow) {
+  // bit e: entry e needs a mask; flags before each word (list_lds_bytes)
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int words = (q.cap + 31) / 32;
+  unsigned *const s_need = reinterpret_cast<unsigned *>(smem_raw);
+  int *const s_pre = reinterpret_cast<int *>(smem_raw) + words;
+  __shared__ unsigned s_mask[kMaskBatch][kWave / 2];  // two 16-bit words each
+  __shared__ int2 s_ent[kMaskBatch];                  // j-cluster, i-clusters
+  __shared__ int s_wbase, s_nmask;
   constexpr int NW = kListBlock / kWave;
   constexpr int kScPerBatch = kListBlock / kClusterSize;
   __shared__ int s_cnt[NW];
@@ -820,12 +876,10 @@ __device__ __forceinline__ void build_list_body(const int bid_, const int nbk_, 
     }
     return;
   }
-  float4 ic[8], ih[8];
-#pragma unroll
-  for (int c = 0; c < 8; ++c) {
-    ic[c] = ctr[S * 8 + c];
-    ih[c] = half[S * 8 + c];
-  }
+  // the boxes of S in LDS (read by every lane at once): as scalars they spill
+  __shared__ float4 ic[8], ih[8];
+  if (threadIdx.x < 8) ic[threadIdx.x] = ctr[S * 8 + threadIdx.x];
+  if (threadIdx.x >= 64 && threadIdx.x < 72) ih[threadIdx.x - 64] = half[S * 8 + threadIdx.x - 64];
   const float4 Sc = sctr[S], Sh = shalf[S];
   int xr[2][2], yr[2][2];
   const int cx = col / q.ncy, cy = col - cx * q.ncy;
@@ -835,6 +889,7 @@ __device__ __forceinline__ void build_list_body(const int bid_, const int nbk_, 
   // a time) so that each pass of 256 threads tests 256 candidates
   const int nx0 = xr[0][1] - xr[0][0] + 1, nxt = nx0 + (nxr > 1 ? xr[1][1] - xr[1][0] + 1 : 0);
   const int R = nxt * nyr;
+  for (int w = threadIdx.x; w < words; w += kListBlock) s_need[w] = 0u;
   int total = 0;   // block-uniform
   int ctotal = 0;  // block-uniform work of the entries so far
   for (int g0 = 0; g0 < R; g0 += kWave) {
@@ -846,8 +901,8 @@ __device__ __forceinline__ void build_list_body(const int bid_, const int nbk_, 
       if (r < R) {
         const int xi = r / nyr, ry = r - xi * nyr;
         const int x = xi < nx0 ? xr[0][0] + xi : xr[1][0] + (xi - nx0);
-        a = max(S, colsc[x * q.ncy + yr[ry][0]]);
-        len = max(0, colsc[x * q.ncy + yr[ry][1] + 1] - a);
+        a = max(S, colsc[x * q.ncy + (ry ? yr[1][0] : yr[0][0])]);
+        len = max(0, colsc[x * q.ncy + (ry ? yr[1][1] : yr[0][1]) + 1] - a);
       }
       int incl = len;
 #pragma unroll
@@ -900,16 +955,113 @@ __device__ __forceinline__ void build_list_body(const int bid_, const int nbk_, 
           jc = ctr[cj];
           jh = half[cj];
         }
-        list_append(q, S, ic, ih, cj, jc, jh, entries, maskwork, nmaskwork, maxmaskwork, overflow, s_cnt, s_cost,
-                    ecost, total, ctotal);
+        list_append(q, S, ic, ih, cj, jc, jh, entries, s_need, overflow, s_cnt, s_cost, ecost, total, ctotal);
       }
       __syncthreads();  // s_sc and s_cnt are rewritten by the next pass
     }
   }
+  __syncthreads();  // entries, costs and flags of every thread
+  const int n = total < q.cap ? total : q.cap;
+  int4 *const ep = entries + (size_t)S * q.cap;
   if (threadIdx.x == 0) {
-    const int n = total < q.cap ? total : q.cap;
     count[S] = n;
     cost_out[S] = n > 0 ? ecost[(size_t)S * q.cap + n - 1] : 0;
+  }
+  // excluded pairs, four threads an atom: the entry (-1: none, or another
+  // supercluster's pair), the j-slot and the class of the thread's pair k
+  constexpr int TPA = kListBlock / kSuperSize, KEPT = 2;
+  const int si = S * kSuperSize + (int)threadIdx.x / TPA;
+  const int ai = ma.perm[si];
+  const int x0 = (ai >= 0 ? ma.eptr[ai] : 0) + (int)threadIdx.x % TPA, x1 = ai >= 0 ? ma.eptr[ai + 1] : 0;
+  auto excluded = [&](int k) {
+    const int2 x = k < x1 ? ma.elist[k] : make_int2(-1, 0);
+    if (x.x < 0) return make_int3(-1, 0, 0);
+    const int sj = ma.slot[x.x];
+    const int ci = si / kClusterSize, cj = sj / kClusterSize;
+    if (cj < ci || (cj == ci && sj < si)) return make_int3(-1, 0, 0);
+    int lo = 0, hi = n - 1;
+    while (lo <= hi) {
+      const int m = (lo + hi) >> 1;
+      const int v = ep[m].x;
+      if (v == cj) return make_int3(m, sj, x.y);
+      if (v < cj)
+        lo = m + 1;
+      else
+        hi = m - 1;
+    }
+    return make_int3(-1, 0, 0);
+  };
+  int3 kept[KEPT];  // most atoms have no more
+#pragma unroll
+  for (int u = 0; u < KEPT; ++u) kept[u] = excluded(x0 + u * TPA);
+  auto each_excluded = [&](auto f) {
+#pragma unroll
+    for (int u = 0; u < KEPT; ++u)
+      if (kept[u].x >= 0) f(kept[u]);
+    for (int k = x0 + KEPT * TPA; k < x1; k += TPA) {
+      const int3 v = excluded(k);
+      if (v.x >= 0) f(v);
+    }
+  };
+  each_excluded([&](int3 v) { atomicOr(&s_need[v.x >> 5], 1u << (v.x & 31)); });
+  __syncthreads();
+  // mask slots in entry order
+  if (wv == 0) {
+    int carry = 0;
+    for (int w0 = 0; w0 * 32 < n; w0 += kWave) {
+      const int c = (w0 + lane) * 32 < n ? __popc(s_need[w0 + lane]) : 0;
+      const int incl = wave_prefix(c);
+      if (w0 + lane < words) s_pre[w0 + lane] = carry + incl - c;
+      carry += __shfl(incl, kWave - 1);
+    }
+    if (lane == 0) {
+      const int w0 = carry ? atomicAdd(nmaskwork, carry) : 0;
+      const bool fits = w0 + carry <= ma.maxmaskwork;
+      if (!fits) atomicExch(overflow, 1);
+      s_wbase = w0;
+      s_nmask = fits ? carry : 0;
+    }
+  }
+  __syncthreads();
+  const int nmask = s_nmask;
+  auto rank = [&](int e) { return s_pre[e >> 5] + __popc(s_need[e >> 5] & ((1u << (e & 31)) - 1u)); };
+  const int ti = lane & 7, tj = lane >> 3;
+  unsigned ireal = 0;  // i-atoms 8 c + ti
+#pragma unroll
+  for (int c = 0; c < 8; ++c) ireal |= ma.perm[S * kSuperSize + c * kClusterSize + ti] >= 0 ? 1u << c : 0u;
+  for (int m0 = 0; m0 < nmask; m0 += kMaskBatch) {
+    const int mn = min(kMaskBatch, nmask - m0);
+    for (int e = threadIdx.x; e < n; e += kListBlock) {
+      if (!(s_need[e >> 5] >> (e & 31) & 1u)) continue;
+      const int k = rank(e) - m0;
+      if (k < 0 || k >= mn) continue;
+      s_ent[k] = make_int2(ep[e].x, ep[e].y);
+      ep[e].z = s_wbase + m0 + k;
+    }
+    __syncthreads();
+    // without exclusions
+    for (int k = wv; k < mn; k += NW) {
+      const int cj = s_ent[k].x, d = cj - S * 8;  // (only clusters from 8 S on are listed)
+      unsigned bits = s_ent[k].y & ireal;
+      if (ma.perm[cj * kClusterSize + tj] < 0) bits = 0;
+      if (d < 8 && ti >= tj) bits &= ~(1u << d);
+      const unsigned other = __shfl_xor(bits, 1);
+      if (!(lane & 1)) s_mask[k][lane >> 1] = bits | other << 16;
+    }
+    __syncthreads();
+    each_excluded([&](int3 v) {
+      const int k = rank(v.x) - m0;
+      if (k < 0 || k >= mn) return;
+      const int c = (si / kClusterSize) & 7, l = (v.y & 7) * 8 + (si & 7), sh = 16 * (l & 1);
+      if (v.z == 1)
+        atomicAnd(&s_mask[k][l >> 1], ~((1u << c) << sh));
+      else if (v.z == 2 && (s_ent[k].y & (1 << c)))
+        atomicOr(&s_mask[k][l >> 1], (256u << c) << sh);
+    });
+    __syncthreads();
+    unsigned *const out = reinterpret_cast<unsigned *>(ma.masks) + (size_t)(s_wbase + m0) * (kWave / 2);
+    for (int k = threadIdx.x; k < mn * (kWave / 2); k += kListBlock) out[k] = (&s_mask[0][0])[k];
+    __syncthreads();  // the next batch overwrites s_mask and s_ent
   }
 }
 
@@ -918,72 +1070,12 @@ static __global__ void __launch_bounds__(kListBlock) k_build_list(ListParams q, 
                                                            const float4 *__restrict__ sctr,
                                                            const float4 *__restrict__ shalf,
                                                            const float4 *__restrict__ ctr,
-                                                           const float4 *__restrict__ half,
-                                                           int4 *__restrict__ entries, int *__restrict__ count,
-                                                           int *__restrict__ ecost, int *__restrict__ cost_out,
-                                                           int *__restrict__ maskwork, int *__restrict__ nmaskwork,
-                                                           int maxmaskwork, int *__restrict__ overflow) {
+                                                           const float4 *__restrict__ half, int4 *entries,
+                                                           int *__restrict__ count, int *ecost,
+                                                           int *__restrict__ cost_out, MaskArgs ma,
+                                                           int *__restrict__ nmaskwork, int *__restrict__ overflow) {
   build_list_body(blockIdx.x, gridDim.x, q, sc_col, colsc, sctr, shalf, ctr, half, entries, count, ecost, cost_out,
-                  maskwork, nmaskwork, maxmaskwork, overflow);
-}
-
-// Flags the list entry that holds each excluded pair (FULL or MODIFIED) so
-// that k_build_masks gives it explicit pair masks.  Entries of supercluster S
-// are sorted by j-cluster, so the entry is found by binary search; pairs whose
-// clusters are not in the list are beyond the list radius and never evaluated.
-__device__ __forceinline__ void mark_exclusions_body(const int bid_, const int nbk_, int ne,
-                                                     const int4 *__restrict__ etab, const int *__restrict__ slot,
-                                                     int4 *__restrict__ entries, const int *__restrict__ count, int cap,
-                                                     int *__restrict__ maskwork, int *__restrict__ nmaskwork,
-                                                     int maxmaskwork, int *__restrict__ overflow) {
-  const int e = bid_ * blockDim.x + threadIdx.x;
-  const int lane = threadIdx.x & 63;
-  int hit = -1;  // entry index (S * cap + k) this thread claimed
-  if (e < ne) {
-    const int4 t = etab[e];
-    const int c1 = slot[t.x] / kClusterSize, c2 = slot[t.y] / kClusterSize;
-    if (c1 != c2) {  // diagonal entries always carry masks
-      const int ci = c1 < c2 ? c1 : c2, cj = c1 < c2 ? c2 : c1;
-      const int S = ci / 8;
-      int lo = 0, hi = count[S] - 1;
-      while (lo <= hi) {
-        const int mid = (lo + hi) >> 1;
-        const int v = entries[(size_t)S * cap + mid].x;
-        if (v == cj) {
-          if (atomicCAS(&entries[(size_t)S * cap + mid].z, -1, -3) == -1) hit = S * cap + mid;
-          break;
-        }
-        if (v < cj)
-          lo = mid + 1;
-        else
-          hi = mid - 1;
-      }
-    }
-  }
-  // one mask work slot per claimed entry, one counter atomic per wave
-  const unsigned long long got = __ballot(hit >= 0);
-  int wbase = 0;
-  if (got) {
-    if (lane == 0) wbase = atomicAdd(nmaskwork, (int)__popcll(got));
-    wbase = __builtin_amdgcn_readfirstlane(__shfl(wbase, 0));
-  }
-  if (hit >= 0) {
-    const int w = wbase + __popcll(got & ((1ull << lane) - 1ull));
-    if (w < maxmaskwork) {
-      maskwork[w] = hit;
-      atomicExch(&entries[hit].z, -2);
-    } else {
-      atomicExch(overflow, 1);
-    }
-  }
-}
-
-static __global__ void k_mark_exclusions(int ne, const int4 *__restrict__ etab, const int *__restrict__ slot,
-                                  int4 *__restrict__ entries, const int *__restrict__ count, int cap,
-                                  int *__restrict__ maskwork, int *__restrict__ nmaskwork, int maxmaskwork,
-                                  int *__restrict__ overflow) {
-  mark_exclusions_body(blockIdx.x, gridDim.x, ne, etab, slot, entries, count, cap, maskwork, nmaskwork, maxmaskwork,
-                       overflow);
+                  ma, nmaskwork, overflow);
 }
 
 // Binary search of b in the sorted exclusion partners of a (original indices).
@@ -1001,264 +1093,127 @@ __device__ inline int excl_class(const int *__restrict__ eptr, const int2 *__res
   return 0;
 }
 
-// One wave per entry needing explicit masks.  Mask slot w holds one 16-bit
-// word per lane l = tj*8 + ti of the pair kernel: bit c set when i = slot
-// 8ci+ti (ci = 8S + c, c in the entry's mask) and j = slot 8cj+tj are real
-// atoms (perm >= 0), i precedes j within a shared cluster, and the pair is
-// not FULL-excluded; bit 8 + c marks MODIFIED.  Each lane of the pair kernel
-// loads its own word once per entry.  The entry's mask field becomes w.
-__device__ __forceinline__ void build_masks_body(const int bid_, const int nbk_, const int *__restrict__ maskwork,
-                                                 const int *__restrict__ nmaskwork, int maxmaskwork,
-                                                 int4 *__restrict__ entries, int cap, const int *__restrict__ perm,
-                                                 const int *__restrict__ eptr, const int2 *__restrict__ elist,
-                                                 unsigned short *__restrict__ masks) {
-  const int lane = threadIdx.x & 63;
-  int nw = *nmaskwork;
-  if (nw > maxmaskwork) nw = maxmaskwork;
-  const int nwaves = nbk_ * (blockDim.x / kWave);
-  for (int w = bid_ * (blockDim.x / kWave) + (threadIdx.x >> 6); w < nw; w += nwaves) {
-    const int eidx = maskwork[w];
-    const int S = eidx / cap;
-    const int4 ent = entries[eidx];
-    const int cj = ent.x;
-    const int ti = lane & 7, tj = lane >> 3;
-    const int aj = perm[cj * kClusterSize + tj];
-    // the eight i-clusters' exclusion lookups advance together (one
-    // dependent load chain instead of eight)
-    int ai[8], lo[8], hi[8], cls[8];
-    bool ok[8];
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      const int ci = S * 8 + c;
-      ai[c] = (ent.y & (1 << c)) ? perm[ci * kClusterSize + ti] : -1;
-      ok[c] = ai[c] >= 0 && aj >= 0 && (ci != cj || ti < tj);
-      lo[c] = ok[c] ? eptr[ai[c]] : 0;
-      hi[c] = ok[c] ? eptr[ai[c] + 1] - 1 : -1;
-      cls[c] = 0;
-    }
-    bool any = true;
-    while (any) {
-      any = false;
-#pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        if (lo[c] <= hi[c]) {
-          const int mid = (lo[c] + hi[c]) >> 1;
-          const int2 v = elist[mid];
-          if (v.x == aj) {
-            cls[c] = v.y;
-            hi[c] = lo[c] - 1;
-          } else if (v.x < aj) {
-            lo[c] = mid + 1;
-          } else {
-            hi[c] = mid - 1;
-          }
-          any = true;
-        }
-      }
-    }
-    unsigned bits = 0;
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      // ok[c] implies c is in the entry's mask
-      if (ok[c] && cls[c] != 1) bits |= 1u << c;
-      if (ok[c] && cls[c] == 2) bits |= 1u << (8 + c);
-    }
-    masks[(size_t)w * kWave + lane] = (unsigned short)bits;
-    if (lane == 0) entries[eidx].z = w;
-  }
-}
-
-static __global__ void __launch_bounds__(256) k_build_masks(const int *__restrict__ maskwork, const int *__restrict__ nmaskwork,
-                                                     int maxmaskwork, int4 *__restrict__ entries, int cap,
-                                                     const int *__restrict__ perm, const int *__restrict__ eptr,
-                                                     const int2 *__restrict__ elist,
-                                                     unsigned short *__restrict__ masks) {
-  build_masks_body(blockIdx.x, gridDim.x, maskwork, nmaskwork, maxmaskwork, entries, cap, perm, eptr, elist, masks);
-}
-
-// Compact tile list: tiles of up to kTileEntries entries per supercluster.
-template <class T>
-__device__ inline int last_le(const T *__restrict__ a, int n, T v) {
-  int lo = 0, hi = n - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (a[mid] <= v)
-      lo = mid;
-    else
-      hi = mid - 1;
-  }
-  return lo;
-}
-
 // Run schedule: the list entries of all superclusters, in supercluster
 // order, are cut into nruns contiguous runs of equal estimated work (the
 // work estimates of k_build_list: per supercluster, and as an inclusive
 // prefix over its entries); nruns, a multiple of kMinRuns set by C, the
-// total, depends only on the list.  Run w starts at entry
-// position pos[w] (ep[S] + offset, offsets even) in supercluster posS[w],
-// where the global work prefix first exceeds b_w = floor(w C / nruns).  A run
-// is split into one tile per supercluster it touches (at most nruns + nsuper
-// tiles); run r is tiles [wstart[r], wstart[r + 1]).  Three passes, none
-// searching:
-//   k_runs_prefix (one block): prefixes ep (entries) and cp (work) over the
-//     superclusters, the run count, run boundaries preset to the end;
-//   k_runs_cut (a block per supercluster): each entry places the run
-//     boundaries b_w that fall in its work interval;
-//   k_runs_tiles (one block): tiles per run, their prefix, the tiles.
-__device__ __forceinline__ void runs_prefix_body(const int bid_, const int nbk_, int nsuper,
-                                                 const int *__restrict__ count, const int *__restrict__ cost,
-                                                 int *__restrict__ nruns_p, int *__restrict__ ep,
-                                                 long long *__restrict__ cp, int *__restrict__ pos,
-                                                 int *__restrict__ posS, long long min_run_cost = 0) {
-  __shared__ int s_e[1024];
-  __shared__ long long s_c[1024];
-  __shared__ int s_last[1024 / kWave];
-  const int tid = threadIdx.x;
-  int ecarry = 0, last = -1;
-  long long ccarry = 0;
-  for (int base = 0; base < nsuper; base += 1024) {
-    const int S = base + tid;
-    const int c = S < nsuper ? count[S] : 0;
-    const long long w = S < nsuper ? (long long)cost[S] : 0;
+// total, depends only on the list.  Run w starts in supercluster runs[w].x
+// at entry runs[w].y (even: runs hold whole pair-kernel groups), where the
+// global work prefix first exceeds b_w = floor(w C / nruns), and ends where
+// run w + 1 starts; runs[nruns] is the end of the last supercluster with
+// entries.  The tile of run w in supercluster S, which may be empty at the
+// run's end, is number w + S: numbers rise by one from tile to tile, also from a
+// run's last to the next run's first.
+// One launch: each block adds up the work ahead of its superclusters and in
+// total for itself (a table of 4 bytes per supercluster), its waves take one
+// supercluster after the other, and each entry places the run boundaries
+// that fall in its work interval.
+constexpr int kRunsBlock = 1024;
+__device__ __forceinline__ void runs_body(const int bid_, const int nbk_, int nsuper, const int *__restrict__ count,
+                                          const int *__restrict__ cost, const int *__restrict__ ecost, int cap,
+                                          long long min_run_cost, int2 *__restrict__ runs,
+                                          int *__restrict__ ntiles) {
+  constexpr int NW = kRunsBlock / kWave;
+  __shared__ long long s_c[2][NW];
+  __shared__ int s_last[NW];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int c0 = (int)((long long)bid_ * nsuper / nbk_), c1 = (int)((long long)(bid_ + 1) * nsuper / nbk_);
+  long long before = 0, C = 0;
+  int last = -1;
+  for (int S = threadIdx.x; S < nsuper; S += kRunsBlock) {
+    const int c = cost[S];
+    C += c;
+    before += S < c0 ? c : 0;
     if (c > 0) last = S;
-    s_e[tid] = c;
-    s_c[tid] = w;
-    __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {
-      const int ve = tid >= off ? s_e[tid - off] : 0;
-      const long long vc = tid >= off ? s_c[tid - off] : 0;
-      __syncthreads();
-      s_e[tid] += ve;
-      s_c[tid] += vc;
-      __syncthreads();
-    }
-    if (S < nsuper) {
-      ep[S] = ecarry + s_e[tid] - c;
-      cp[S] = ccarry + s_c[tid] - w;
-    }
-    ecarry += s_e[1023];
-    ccarry += s_c[1023];
-    __syncthreads();
   }
+  before = wave_sum(before);
+  C = wave_sum(C);
   last = wave_max(last);
-  if ((tid & 63) == 0) s_last[tid >> 6] = last;
+  if (lane == 0) {
+    s_c[0][wv] = before;
+    s_c[1][wv] = C;
+    s_last[wv] = last;
+  }
   __syncthreads();
-  int lastS = -1;
-  for (int k = 0; k < 1024 / kWave; ++k) lastS = max(lastS, s_last[k]);
+  before = C = 0;
+  for (int k = 0; k < NW; ++k) {
+    before += s_c[0][k];
+    C += s_c[1][k];
+    last = max(last, s_last[k]);
+  }
   const long long per = (long long)kMinRuns * kRunCost;
-  const long long k = (ccarry + per - 1) / per;
+  const long long k = (C + per - 1) / per;
   int nruns = kMinRuns * (int)(k < 1 ? 1 : (k > kMaxRuns / kMinRuns ? kMaxRuns / kMinRuns : k));
   if (min_run_cost > 0) {
     // runs of at least min_run_cost units, in whole waves' worth of 64 runs:
     // a small list's runs would otherwise hold an entry or two each, and the
     // wave would spend its time on the i-force flush at every tile end
-    const long long r = (ccarry + min_run_cost - 1) / min_run_cost;
+    const long long r = (C + min_run_cost - 1) / min_run_cost;
     nruns = (int)min((long long)nruns, max(64ll, (r + 63) / 64 * 64));
   }
-  if (tid == 0) {
-    ep[nsuper] = ecarry;
-    cp[nsuper] = ccarry;
-    *nruns_p = nruns;
+  if (bid_ == 0) {
+    // an empty list: every run is empty
+    for (int w = C > 0 ? nruns + threadIdx.x : threadIdx.x; w < nruns; w += kRunsBlock) runs[w] = make_int2(0, 0);
+    if (threadIdx.x == 0) {
+      runs[0] = make_int2(0, 0);
+      runs[nruns] = make_int2(last + 1, 0);
+      ntiles[0] = nruns + last + 1;
+      ntiles[2] = nruns;
+    }
   }
-  // every boundary starts at the end (k_runs_cut moves those that fall in
-  // the list); run 0 starts at the beginning
-  for (int w = tid; w <= nruns; w += 1024) {
-    pos[w] = w == 0 ? 0 : ecarry;
-    posS[w] = w == 0 ? 0 : lastS + 1;
-  }
-}
-
-static __global__ void k_runs_prefix(int nsuper, const int *__restrict__ count, const int *__restrict__ cost,
-                              int *__restrict__ nruns_p, int *__restrict__ ep, long long *__restrict__ cp,
-                              int *__restrict__ pos, int *__restrict__ posS) {
-  runs_prefix_body(blockIdx.x, gridDim.x, nsuper, count, cost, nruns_p, ep, cp, pos, posS);
-}
-
-__device__ __forceinline__ void runs_cut_body(const int bid_, const int nbk_, int nsuper, const int *__restrict__ count,
-                                              const int *__restrict__ ecost, int cap, const int *__restrict__ nruns_p,
-                                              const int *__restrict__ ep, const long long *__restrict__ cp,
-                                              int *__restrict__ pos, int *__restrict__ posS) {
-  const int S = bid_;
-  const int nruns = *nruns_p;
-  const int n = count[S];
-  const long long C = cp[nsuper], base = cp[S];
   if (C <= 0) return;
-  const int *ec = ecost + (size_t)S * cap;
-  for (int e = threadIdx.x; e < n; e += blockDim.x) {
-    const long long lo = base + (e > 0 ? ec[e - 1] : 0), hi = base + ec[e];
-    // runs w in [1, nruns) with lo <= floor(w C / nruns) < hi
-    long long w0 = (lo * nruns + C - 1) / C, w1 = (hi * nruns + C - 1) / C;
-    w0 = max(w0, 1ll);
-    w1 = min(w1, (long long)nruns);
-    for (long long w = w0; w < w1; ++w) {
-      pos[w] = ep[S] + (e & ~1);  // runs hold whole pair-kernel groups
-      posS[w] = S;
-    }
-  }
-}
-
-static __global__ void k_runs_cut(int nsuper, const int *__restrict__ count, const int *__restrict__ ecost, int cap,
-                           const int *__restrict__ nruns_p, const int *__restrict__ ep,
-                           const long long *__restrict__ cp, int *__restrict__ pos, int *__restrict__ posS) {
-  runs_cut_body(blockIdx.x, gridDim.x, nsuper, count, ecost, cap, nruns_p, ep, cp, pos, posS);
-}
-
-__device__ __forceinline__ void runs_tiles_body(const int bid_, const int nbk_, const int *__restrict__ count,
-                                                const int *__restrict__ ep, const int *__restrict__ pos,
-                                                const int *__restrict__ posS, int *__restrict__ wstart,
-                                                int4 *__restrict__ tiles, int *__restrict__ ntiles, int ntiles_cap) {
-  __shared__ int s_n[1024];
-  const int tid = threadIdx.x;
-  const int nruns = ntiles[2];  // from k_runs_prefix
-  // run w: entries [pos[w], pos[w+1]), superclusters S0 .. S1
-  auto span = [&](int w, int &S0, int &S1) {
-    const int p0 = pos[w], p1 = pos[w + 1];
-    S0 = posS[w];
-    S1 = posS[w + 1] - (p1 == ep[posS[w + 1]] ? 1 : 0);
-    return p1 > p0 ? S1 - S0 + 1 : 0;
+  const int w0 = c0 + (int)((long long)wv * (c1 - c0) / NW), w1 = c0 + (int)((long long)(wv + 1) * (c1 - c0) / NW);
+  long long base = 0;
+  for (int S = c0 + lane; S < w0; S += kWave) base += cost[S];
+  base = before + wave_sum(base);
+  const double inv = 1.0 / (double)C;
+  // first run w with floor(w C / nruns) >= x, i.e. ceil(x nruns / C)
+  auto first_run = [&](long long x) {
+    // q is off by one at most (the product stays below 2^53)
+    const long long y = x * nruns, q = (long long)((double)y * inv), r = y - q * C;
+    return (int)min(q + (r > 0 ? 1 : 0) + (r > C ? 1 : 0) - (r <= -C ? 1 : 0), (long long)nruns);
   };
-  int carry = 0;
-  for (int base = 0; base < nruns; base += 1024) {
-    const int w = base + tid;
-    int S0, S1;
-    const int n = w < nruns ? span(w, S0, S1) : 0;
-    s_n[tid] = n;
-    __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {
-      const int v = tid >= off ? s_n[tid - off] : 0;
-      __syncthreads();
-      s_n[tid] += v;
-      __syncthreads();
-    }
-    if (w < nruns) {
-      int t = carry + s_n[tid] - n;
-      wstart[w] = min(t, ntiles_cap);
-      for (int S = S0; S < S0 + n && t < ntiles_cap; ++S, ++t) {
-        const int e0 = S == S0 ? pos[w] - ep[S] : 0;
-        const int e1 = S == S1 ? pos[w + 1] - ep[S] : count[S];
-        tiles[t] = make_int4(S, e0, e1, 0);
+  for (int S = w0; S < w1; ++S) {
+    const int n = count[S];
+    const int *ec = ecost + (size_t)S * cap;
+    int carry = first_run(base);
+    constexpr int AHEAD = 8;  // rounds whose loads are in flight together
+    for (int e0 = 0; e0 < n; e0 += AHEAD * kWave) {
+      int hi[AHEAD];
+#pragma unroll
+      for (int u = 0; u < AHEAD; ++u) {
+        const int e = e0 + u * kWave + lane;
+        hi[u] = e < n ? ec[e] : 0;
+      }
+#pragma unroll
+      for (int u = 0; u < AHEAD; ++u) {
+        const int e = e0 + u * kWave + lane;
+        if (e0 + u * kWave >= n) break;
+        const int rb = first_run(base + hi[u]);
+        int ra = __shfl_up(rb, 1);
+        if (lane == 0) ra = carry;
+        carry = __shfl(rb, kWave - 1);
+        // runs w in [1, nruns) with lo <= floor(w C / nruns) < hi
+        if (e < n)
+          for (int w = max(ra, 1); w < rb; ++w) runs[w] = make_int2(S, e & ~1);
       }
     }
-    carry += s_n[1023];
-    __syncthreads();
-  }
-  if (tid == 0) {
-    wstart[nruns] = min(carry, ntiles_cap);
-    ntiles[0] = min(carry, ntiles_cap);
+    base += cost[S];
   }
 }
 
-static __global__ void k_runs_tiles(const int *__restrict__ count, const int *__restrict__ ep, const int *__restrict__ pos,
-                             const int *__restrict__ posS, int *__restrict__ wstart, int4 *__restrict__ tiles,
-                             int *__restrict__ ntiles, int ntiles_cap) {
-  runs_tiles_body(blockIdx.x, gridDim.x, count, ep, pos, posS, wstart, tiles, ntiles, ntiles_cap);
+static __global__ void __launch_bounds__(kRunsBlock) k_runs(int nsuper, const int *__restrict__ count,
+                                                            const int *__restrict__ cost,
+                                                            const int *__restrict__ ecost, int cap,
+                                                            int2 *__restrict__ runs, int *__restrict__ ntiles) {
+  runs_body(blockIdx.x, gridDim.x, nsuper, count, cost, ecost, cap, 0, runs, ntiles);
 }
 
 // ---------------------------------------------------------------------------
 // 3. Pair kernel: LJ + Coulomb (cutoff or PME real space) with switching.
 //
-// Wavefront layout: lane = 8*tj + ti.  A work tile is (i-supercluster S,
-// up to kTileEntries list entries).  Each entry names one j-cluster (8 atoms,
+// Wavefront layout: lane = 8*tj + ti.  A work tile is the part of a run in
+// one i-supercluster S.  Each entry names one j-cluster (8 atoms,
 // lane tj holds atom tj) and an 8-bit mask of the i-clusters of S it is in
 // range of; for every set i-cluster c the 64 lanes evaluate the 8x8 atom
 // pairs (8c+ti, tj).  i-forces stay in registers for the whole tile, j-forces
@@ -1400,14 +1355,47 @@ __device__ inline double group8_sum(double v) {
   return v;
 }
 struct PairOut {
-  double *energy;            // [2 * ntiles_max]: per tile (coulomb, lj); int64 fixed point 2^-32 in the mixed form
-  long long *npairs;         // [ntiles_max] when stats
-  unsigned long long *hash;  // [ntiles_max]
+  double *energy;            // [2 * ntiles]: per tile (coulomb, lj); int64 fixed point 2^-32 in the mixed form
+  long long *npairs;         // [ntiles] when stats
+  unsigned long long *hash;  // [ntiles]
   int2 *border;              // recorded boundary pairs (sorted slots i, j)
   int *nborder;
   int maxborder;
   int *overflow;
   unsigned long long *border_acc;  // [4] boundary-pair energies and stats, cleared here
+  __device__ void clear(int t, bool stats) const {
+    energy[2 * t] = energy[2 * t + 1] = 0.0;
+    if (stats) {
+      npairs[t] = 0;
+      hash[t] = 0;
+    }
+  }
+};
+
+// A wave's way through runs w .. wstop - 1, tile by tile (wave-uniform).
+struct RunWalk {
+  int w, wstop, t = 0;    // next run; the tile's number
+  int S = 0, e0 = 0;      // the tile: supercluster, first entry
+  int Send = -1, eend = 0;  // the run's end
+  __device__ RunWalk(int r0, int r1) : w(r0), wstop(r1) {}
+  __device__ bool run_done() const { return S > Send; }
+  __device__ void next_run(const int2 *__restrict__ runs) {
+    const int2 a = runs[w], b = runs[w + 1];
+    S = __builtin_amdgcn_readfirstlane(a.x);
+    e0 = __builtin_amdgcn_readfirstlane(a.y);
+    Send = __builtin_amdgcn_readfirstlane(b.x);
+    eend = __builtin_amdgcn_readfirstlane(b.y);
+    t = w + S;
+    ++w;
+  }
+  __device__ int tile_end(const int *__restrict__ count) const {
+    return S == Send ? eend : __builtin_amdgcn_readfirstlane(count[S]);
+  }
+  __device__ void next_tile() {
+    ++S;
+    ++t;
+    e0 = 0;
+  }
 };
 
 // Queue entry of the compacted pair kernel: one in-cutoff pair awaiting its
@@ -1535,7 +1523,7 @@ __device__ inline void pair_delta(const R4 &xi, const R4 &xj, const EdgesR<R> &E
 // counts the in-cutoff pairs and sums their hashes.
 template <bool MIXED, int COUL, int LJSW, int CSW, bool BIGLJ, int MODE>
 __device__ __forceinline__ void pair_body(const int bid_, const int nbk_, PairParams pp, int dynamic,
-    const int4 *__restrict__ tiles, const int *__restrict__ ntiles_p, const int *__restrict__ wstart,
+    const int2 *__restrict__ runs, const int *__restrict__ ntiles_p, const int *__restrict__ count,
     int *__restrict__ tile_counter, const int4 *__restrict__ entries, int4 *entries_w, int cap,
     const unsigned short *__restrict__ masks,
     const typename Real4<typename std::conditional<MIXED, float, double>::type>::type *__restrict__ xs,
@@ -1600,30 +1588,34 @@ __device__ __forceinline__ void pair_body(const int bid_, const int nbk_, PairPa
   // (dynamic == 0: consecutive tiles often share a supercluster, whose
   // i-atoms then stay loaded), or
   // run w and then runs in order from a device-wide counter (dynamic == 1).
-  // Run r is tiles [wstart[r], wstart[r + 1]).  Which wave takes a run
+  // A tile is the part of a run in one supercluster.  Which wave takes a run
   // changes no result.
   const int nwaves = nbk_ * W;
   const int gw = bid_ * W + wv;
   const int nruns = ntiles_p[2];
   const int r0 = dynamic ? gw : (int)((long long)gw * nruns / nwaves);
   const int r1 = dynamic ? min(gw + 1, nruns) : (int)((long long)(gw + 1) * nruns / nwaves);
-  int t = r0 < r1 ? wstart[r0] : 0, tstop = r0 < r1 ? wstart[r1] : 0;
+  RunWalk walk(r0, r1);
   int curS = -1;      // supercluster whose i-atoms are loaded
   bool ireal = false;  // slot `lane` of curS holds an atom
   while (true) {
-    if (t >= tstop) {
-      if (!dynamic) break;
-      int rn = 0;
-      if (lane == 0) rn = nwaves + atomicAdd(tile_counter, 1);
-      const int r = __builtin_amdgcn_readfirstlane(__shfl(rn, 0));
-      if (r >= nruns) break;
-      t = wstart[r];
-      tstop = wstart[r + 1];
+    if (walk.run_done()) {
+      if (walk.w >= walk.wstop) {
+        if (!dynamic) break;
+        int rn = 0;
+        if (lane == 0) rn = nwaves + atomicAdd(tile_counter, 1);
+        const int r = __builtin_amdgcn_readfirstlane(__shfl(rn, 0));
+        if (r >= nruns) break;
+        walk = RunWalk(r, r + 1);
+      }
+      walk.next_run(runs);
+    }
+    const int S = walk.S, t = walk.t, e0 = walk.e0, e1 = walk.tile_end(count);
+    walk.next_tile();
+    if (e0 >= e1) {
+      if (lane == 0) out.clear(t, STATS);
       continue;
     }
-    const int4 tile = tiles[t];
-    const int S = __builtin_amdgcn_readfirstlane(tile.x);
-    const int e0 = __builtin_amdgcn_readfirstlane(tile.y);
     const float4 oS = sorg[S];
     if (S != curS) {
       curS = S;
@@ -1697,9 +1689,8 @@ __device__ __forceinline__ void pair_body(const int bid_, const int nbk_, PairPa
       __builtin_amdgcn_wave_barrier();
     };
 
-    const int eend = __builtin_amdgcn_readfirstlane(tile.z);
-    for (int eg = e0; eg < eend; eg += kGroup) {
-      const int ng = eend - eg < kGroup ? eend - eg : kGroup;
+    for (int eg = e0; eg < e1; eg += kGroup) {
+      const int ng = e1 - eg < kGroup ? e1 - eg : kGroup;
       int cjv[kGroup], emv[kGroup], mov[kGroup], shv[kGroup], tyj0[kGroup];
       unsigned mbv[kGroup];  // this lane's exclusion bits (candidate per i-cluster, MODIFIED << 8)
       R4 xj[kGroup];
@@ -1894,7 +1885,6 @@ __device__ __forceinline__ void pair_body(const int bid_, const int nbk_, PairPa
       }
     }
     __builtin_amdgcn_wave_barrier();
-    ++t;
   }
 }
 
@@ -1992,8 +1982,8 @@ __device__ inline float swap8_sum(float a, float b, bool hi) {
 
 template <int COUL, int LJSW, int CSW, bool BIGLJ, int MODE>
 __device__ __forceinline__ void pair_direct_body(
-    const int bid_, const int nbk_, const PairParams &pp, int dynamic, const int4 *__restrict__ tiles,
-    const int *__restrict__ ntiles_p, const int *__restrict__ wstart, int *__restrict__ tile_counter,
+    const int bid_, const int nbk_, const PairParams &pp, int dynamic, const int2 *__restrict__ runs,
+    const int *__restrict__ ntiles_p, const int *__restrict__ count, int *__restrict__ tile_counter,
     const int4 *__restrict__ entries, int4 *entries_w, int cap, const unsigned short *__restrict__ masks,
     const float4 *__restrict__ xs, const float4 *__restrict__ sorg, const int *__restrict__ ts,
     const int *__restrict__ perm, const double *__restrict__ ljtab, const float4 *__restrict__ ljt,
@@ -2026,21 +2016,25 @@ __device__ __forceinline__ void pair_direct_body(
   const int nruns = ntiles_p[2];
   const int r0 = dynamic ? gw : (int)((long long)gw * nruns / nwaves);
   const int r1 = dynamic ? min(gw + 1, nruns) : (int)((long long)(gw + 1) * nruns / nwaves);
-  int t = r0 < r1 ? wstart[r0] : 0, tstop = r0 < r1 ? wstart[r1] : 0;
+  RunWalk walk(r0, r1);
   while (true) {
-    if (t >= tstop) {
-      if (!dynamic) break;
-      int rn = 0;
-      if (lane == 0) rn = nwaves + atomicAdd(tile_counter, 1);
-      const int r = __builtin_amdgcn_readfirstlane(__shfl(rn, 0));
-      if (r >= nruns) break;
-      t = wstart[r];
-      tstop = wstart[r + 1];
+    if (walk.run_done()) {
+      if (walk.w >= walk.wstop) {
+        if (!dynamic) break;
+        int rn = 0;
+        if (lane == 0) rn = nwaves + atomicAdd(tile_counter, 1);
+        const int r = __builtin_amdgcn_readfirstlane(__shfl(rn, 0));
+        if (r >= nruns) break;
+        walk = RunWalk(r, r + 1);
+      }
+      walk.next_run(runs);
+    }
+    const int S = walk.S, t = walk.t, e0 = walk.e0, e1 = walk.tile_end(count);
+    walk.next_tile();
+    if (e0 >= e1) {
+      if (lane == 0) out.clear(t, STATS);
       continue;
     }
-    const int4 tile = tiles[t];
-    const int S = __builtin_amdgcn_readfirstlane(tile.x);
-    const int e0 = __builtin_amdgcn_readfirstlane(tile.y), e1 = __builtin_amdgcn_readfirstlane(tile.z);
     const float4 oS = sorg[S];
     // i-atoms, and the rows of the LJ table of this lane's (8 c + ti), 8 bits each
     __builtin_amdgcn_wave_barrier();
@@ -2060,7 +2054,7 @@ __device__ __forceinline__ void pair_direct_body(
     const int4 *const ep = entries + (size_t)S * cap;
     // the next entry is read while the current one is evaluated
     auto entry = [&](int e) {
-      int4 v = ep[max(0, min(e, e1 - 1))];  // (an empty tile has e1 = 0)
+      int4 v = ep[min(e, e1 - 1)];
       v.x = __builtin_amdgcn_readfirstlane(v.x);
       v.y = __builtin_amdgcn_readfirstlane(v.y);
       v.z = __builtin_amdgcn_readfirstlane(v.z);
@@ -2238,14 +2232,13 @@ __device__ __forceinline__ void pair_direct_body(
         out.hash[t] = hsum;
       }
     }
-    ++t;
   }
 }
 
 template <bool MIXED, int COUL, int LJSW, int CSW, bool BIGLJ, int MODE>
 __global__ void __launch_bounds__(kPairBlock, 4) k_pair(
-    PairParams pp, int dynamic, const int4 *__restrict__ tiles, const int *__restrict__ ntiles_p,
-    const int *__restrict__ wstart, int *__restrict__ tile_counter, const int4 *__restrict__ entries, int4 *entries_w,
+    PairParams pp, int dynamic, const int2 *__restrict__ runs, const int *__restrict__ ntiles_p,
+    const int *__restrict__ count, int *__restrict__ tile_counter, const int4 *__restrict__ entries, int4 *entries_w,
     int cap,
     const unsigned short *__restrict__ masks,
     const typename Real4<typename std::conditional<MIXED, float, double>::type>::type *__restrict__ xs,
@@ -2256,11 +2249,11 @@ __global__ void __launch_bounds__(kPairBlock, 4) k_pair(
   // the blocks of one XCD take a contiguous range of runs
   const int bid = xcd_block(blockIdx.x, gridDim.x);
   if constexpr (MIXED)
-    pair_direct_body<COUL, LJSW, CSW, BIGLJ, MODE>(bid, gridDim.x, pp, dynamic, tiles, ntiles_p, wstart, tile_counter,
+    pair_direct_body<COUL, LJSW, CSW, BIGLJ, MODE>(bid, gridDim.x, pp, dynamic, runs, ntiles_p, count, tile_counter,
                                                    entries, entries_w, cap, masks, xs, sorg, ts, perm, ljtab, ljt,
                                                    facc, out);
   else
-    pair_body<MIXED, COUL, LJSW, CSW, BIGLJ, MODE>(bid, gridDim.x, pp, dynamic, tiles, ntiles_p, wstart, tile_counter,
+    pair_body<MIXED, COUL, LJSW, CSW, BIGLJ, MODE>(bid, gridDim.x, pp, dynamic, runs, ntiles_p, count, tile_counter,
                                                    entries, entries_w, cap, masks, xs, sorg, ts, perm, ljtab, ljt,
                                                    facc, out);
 }

@@ -28,7 +28,7 @@ namespace pmx {
 
 #define PMX_PAIR_KERNEL(EXT, C, LJ, CS, BIG, MODE)                                                                   \
   EXT template __global__ void k_pair<true, C, LJ, CS, BIG, MODE>(                                                   \
-      PairParams, int, const int4 *__restrict__, const int *__restrict__, const int *__restrict__,                   \
+      PairParams, int, const int2 *__restrict__, const int *__restrict__, const int *__restrict__,                   \
       int *__restrict__, const int4 *__restrict__, int4 *, int, const unsigned short *__restrict__,                  \
       const float4 *__restrict__, const float4 *__restrict__, const int *__restrict__, const int *__restrict__,      \
       const double *__restrict__, const float4 *__restrict__, unsigned long long *__restrict__, PairOut);
