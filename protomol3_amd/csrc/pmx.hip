@@ -60,6 +60,12 @@ struct DevBuf {
   bool listed = false;  // registered in Sys::all (freed by pmx_sys_destroy)
 };
 
+// A pinned host block (host_get, host_put).
+struct HostBuf {
+  void *p = nullptr;
+  size_t bytes = 0;
+};
+
 // Timed stages: sort (+ integrate), list (+ accumulator zeroing), pair,
 // spread, fft (+ convolution), gather, fixups (exclusion correction, bonded
 // terms), finalize (boundary pairs, force unsort).  Events: 0 start, 1 sorted,
@@ -70,6 +76,14 @@ struct DevBuf {
 constexpr int kStages = 8;
 constexpr int kStageEv[kStages][2] = {{0, 1}, {1, 2}, {4, 3}, {2, 4}, {4, 5}, {5, 6}, {6, 7}, {7, 8}};
 static_assert(kStages == PMX_STAGES, "stage count of the C ABI");
+
+// Results of a force pass, in device memory (Sys::eout).
+struct PassResults {
+  double e[4];  // Coulomb, LJ, reciprocal, correction
+  long long np[1];
+  unsigned long long hash[1];
+  int overflow[2];
+};
 
 struct Sys {
   pmx_ctx *ctx = nullptr;
@@ -117,6 +131,7 @@ struct Sys {
   DevBuf xorig, xwrap, q_d, type_d, key, hist, start, cursor, scansum, perm, permp, slot, refcell, xs, xs64, ts,
       sc_info, sc_col, colsc, sctr, shalf, sorg, ctr, half, entries, count, ecost, lcost, runs, nmaskwork, masks, overflow, ntiles, tilectr, ljtab, ljt32, facc, fout,
       pair_e, npairs, hash, eptr_d, elist_d, cptr_d, clist_d, corr_e, recip_e, eout, np_out, hash_out, pmw, pmb, tcol, spec, theta, twx, twy, twz, border, nborder, border_acc;
+  // (overflow, np_out and hash_out are parts of eout: one copy brings a pass's results)
   int maxborder = 65536;
   // results
   long long last_np = 0;
@@ -133,7 +148,10 @@ struct Sys {
   bool acc_clean = false;              // force accumulators and pass counters are zero
   bool dry = false;                    // size only: allocations are counted, nothing runs
   unsigned long long dry_bytes = 0;
-  double eout_h[4] = {0, 0, 0, 0};
+  // pinned staging of this system's copies to and from the host, in chunks
+  // beyond kStageChunks x kStageChunk bytes (stage_ev: a chunk's copy is done)
+  HostBuf stage;
+  hipEvent_t stage_ev[4] = {nullptr, nullptr, nullptr, nullptr};
   // device-resident MD state
   struct Md {
     bool on = false;
@@ -225,6 +243,47 @@ void block_put(int device, void *p, size_t cls) {
   }
   g_block_cache[device].emplace(cls, p);
   g_cached_bytes += cls;
+}
+
+// Pinned host blocks, cached the same way (size classes, guarded by g_rt_mu):
+// a copy between device and pageable memory goes through the runtime's own
+// staging, about 20 us each and one after the other; copies to a pinned block
+// are queued together and waited for once.  The cache is bounded and goes
+// back to the system with the last context.
+std::multimap<size_t, void *> g_host_cache;
+size_t g_host_cached = 0;
+int g_contexts = 0;
+constexpr size_t kHostCacheMax = 256ull << 20;
+
+void host_put(HostBuf &b) {
+  if (!b.p) return;
+  RtLock lk(g_rt_mu);
+  if (g_host_cached + b.bytes > kHostCacheMax || g_contexts == 0) {
+    hipHostFree(b.p);
+  } else {
+    g_host_cache.emplace(b.bytes, b.p);
+    g_host_cached += b.bytes;
+  }
+  b = HostBuf{};
+}
+
+// At least `bytes`; a large enough block is kept (no copy may be in flight).
+bool host_get(HostBuf &b, size_t bytes) {
+  if (b.p && b.bytes >= bytes) return true;
+  host_put(b);
+  RtLock lk(g_rt_mu);
+  const size_t c = size_class(std::max<size_t>(bytes, 4096));
+  const auto it = g_host_cache.find(c);
+  if (it != g_host_cache.end()) {
+    b.p = it->second;
+    g_host_cache.erase(it);
+    g_host_cached -= c;
+  } else if (hipHostMalloc(&b.p, c, hipHostMallocDefault) != hipSuccess) {
+    b.p = nullptr;
+    return false;
+  }
+  b.bytes = c;
+  return true;
 }
 
 int dalloc(Sys *s, DevBuf &b, size_t bytes) {
@@ -700,16 +759,20 @@ int setup(Sys *s) {
       (rc = A(s->ecost, 4 * (size_t)s->nsuper * s->cap)) ||
       (rc = A(s->runs, 8 * ((size_t)kMaxRuns + 1))) ||
       (rc = A(s->nmaskwork, 8)) || (rc = A(s->masks, 16 * 8 * (size_t)s->maxmaskwork)) ||
-      (rc = A(s->overflow, 8)) || (rc = A(s->ntiles, 16)) ||
+      (rc = A(s->ntiles, 16)) ||
       (rc = A(s->tilectr, 8)) || (rc = A(s->ljtab, 8 * s->lj.size())) ||
       (rc = A(s->ljt32, 4 * s->lj.size())) || (rc = A(s->facc, 24 * NP)) ||
       (rc = A(s->fout, 24 * N)) || (rc = A(s->pair_e, 16 * (size_t)s->ntiles_cap)) ||
       (rc = A(s->npairs, 8 * (size_t)s->ntiles_cap)) || (rc = A(s->hash, 8 * (size_t)s->ntiles_cap)) ||
       (rc = A(s->eptr_d, 4 * (N + 1))) || (rc = A(s->elist_d, 8 * s->elist.size())) ||
-      (rc = A(s->eout, 64)) || (rc = A(s->np_out, 8)) ||
-      (rc = A(s->hash_out, 8)) || (rc = A(s->border, 8 * (size_t)s->maxborder)) ||
+      (rc = A(s->eout, 64)) || (rc = A(s->border, 8 * (size_t)s->maxborder)) ||
       (rc = A(s->nborder, 8)) || (rc = A(s->border_acc, 32)))
     return rc;
+  if (s->eout.p) {
+    s->np_out.p = P<PassResults>(s->eout)->np;
+    s->hash_out.p = P<PassResults>(s->eout)->hash;
+    s->overflow.p = P<PassResults>(s->eout)->overflow;
+  }
   s->term_blocks = (int)nblk((long long)NP, 256);
   // the correction table by atom (each entry listed for both of its atoms)
   std::vector<int> cptr;
@@ -1309,30 +1372,96 @@ int compute(Sys *s, unsigned flags) {
   return forces(s, flags, true);
 }
 
+constexpr size_t kStageChunk = 1 << 20;
+constexpr int kStageChunks = 4;
+constexpr size_t kStageBytes = kStageChunk * kStageChunks;
+
+int stage_get(Sys *s, size_t bytes) {
+  if (!host_get(s->stage, bytes)) return fail(s->ctx, PMX_ERR_OOM, "pinned host memory");
+  if (bytes < kStageBytes || s->stage_ev[0]) return PMX_OK;
+  RtLock lk(g_rt_mu);
+  for (auto &e : s->stage_ev) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  return PMX_OK;
+}
+
+// Device memory larger than the stage to the host: use(offset, data, bytes)
+// for each chunk in order while the copies of the next ones run.
+template <class F>
+int fetch(Sys *s, const void *src, size_t bytes, F use) {
+  hipStream_t st = s->ctx->stream;
+  if (int rc = stage_get(s, kStageBytes)) return rc;
+  unsigned char *const h = static_cast<unsigned char *>(s->stage.p);
+  const size_t nc = (bytes + kStageChunk - 1) / kStageChunk;
+  for (size_t k = 0; k < nc + kStageChunks - 1; ++k) {
+    if (k < nc) {
+      const size_t o = k * kStageChunk;
+      HIPCHK(hipMemcpyAsync(h + k % kStageChunks * kStageChunk, static_cast<const unsigned char *>(src) + o,
+                            std::min(kStageChunk, bytes - o), hipMemcpyDeviceToHost, st));
+      HIPCHK(hipEventRecord(s->stage_ev[k % kStageChunks], st));
+    }
+    if (k + 1 < (size_t)kStageChunks) continue;
+    const size_t c = k + 1 - kStageChunks, o = c * kStageChunk;
+    HIPCHK(hipEventSynchronize(s->stage_ev[c % kStageChunks]));
+    use(o, h + c % kStageChunks * kStageChunk, std::min(kStageChunk, bytes - o));
+  }
+  return PMX_OK;
+}
+
+// Host memory to the device in the stream's order; the source is free on
+// return.  Large sources go through the stage in chunks (the runtime copies
+// pageable memory one chunk after the other).
+int send(Sys *s, void *dst, const void *src, size_t bytes) {
+  hipStream_t st = s->ctx->stream;
+  if (bytes <= kStageBytes) {
+    HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st));
+    return PMX_OK;
+  }
+  if (int rc = stage_get(s, kStageBytes)) return rc;
+  unsigned char *const h = static_cast<unsigned char *>(s->stage.p);
+  const size_t nc = (bytes + kStageChunk - 1) / kStageChunk;
+  for (size_t k = 0; k < nc; ++k) {
+    const size_t o = k * kStageChunk, len = std::min(kStageChunk, bytes - o);
+    unsigned char *const c = h + k % kStageChunks * kStageChunk;
+    if (k >= (size_t)kStageChunks) HIPCHK(hipEventSynchronize(s->stage_ev[k % kStageChunks]));
+    std::memcpy(c, static_cast<const unsigned char *>(src) + o, len);
+    HIPCHK(hipMemcpyAsync(static_cast<unsigned char *>(dst) + o, c, len, hipMemcpyHostToDevice, st));
+    HIPCHK(hipEventRecord(s->stage_ev[k % kStageChunks], st));
+  }
+  for (auto &e : s->stage_ev) HIPCHK(hipEventSynchronize(e));
+  return PMX_OK;
+}
+
 int finish(Sys *s, unsigned flags, double *f_aos, double *energies) {
   hipStream_t st = s->ctx->stream;
-  int ovf = 0;
-  HIPCHK(hipMemcpyAsync(&ovf, s->overflow.p, 4, hipMemcpyDeviceToHost, st));
-  HIPCHK(hipMemcpyAsync(s->eout_h, s->eout.p, 32, hipMemcpyDeviceToHost, st));
-  HIPCHK(hipMemcpyAsync(&s->last_np, s->np_out.p, 8, hipMemcpyDeviceToHost, st));
-  HIPCHK(hipMemcpyAsync(&s->last_hash, s->hash_out.p, 8, hipMemcpyDeviceToHost, st));
-  std::vector<double> f;
-  if (f_aos) {
-    f.resize(3 * (size_t)s->n);
-    HIPCHK(hipMemcpyAsync(f.data(), s->fout.p, 24 * (size_t)s->n, hipMemcpyDeviceToHost, st));
-  }
+  const size_t fb = f_aos ? 24 * (size_t)s->n : 0;
+  const bool once = sizeof(PassResults) + fb <= kStageBytes;
+  if (int rc = stage_get(s, once ? sizeof(PassResults) + fb : kStageBytes)) return rc;
+  unsigned char *const h = static_cast<unsigned char *>(s->stage.p);
+  HIPCHK(hipMemcpyAsync(h, s->eout.p, sizeof(PassResults), hipMemcpyDeviceToHost, st));
+  if (once && fb) HIPCHK(hipMemcpyAsync(h + sizeof(PassResults), s->fout.p, fb, hipMemcpyDeviceToHost, st));
   HIPCHK(hipStreamSynchronize(st));
-  if (ovf) return fail(s->ctx, PMX_ERR_OVERFLOW, "cluster pair list capacity exceeded");
+  PassResults r;
+  std::memcpy(&r, h, sizeof r);
+  s->last_np = r.np[0];
+  s->last_hash = r.hash[0];
+  if (r.overflow[0]) return fail(s->ctx, PMX_ERR_OVERFLOW, "cluster pair list capacity exceeded");
   if ((flags & PMX_EVAL_TIMING) && s->ev)
     for (int k = 0; k < kStages; ++k)
       hipEventElapsedTime(&s->stage_ms[k], s->ev[kStageEv[k][0]], s->ev[kStageEv[k][1]]);
-  if (f_aos)
-    for (size_t k = 0; k < f.size(); ++k) f_aos[k] += f[k];
+  auto add = [&](size_t o, const void *data, size_t bytes) {
+    double *const to = f_aos + o / 8;
+    const double *const from = static_cast<const double *>(data);
+    for (size_t k = 0; k < bytes / 8; ++k) to[k] += from[k];
+  };
+  if (once && fb)
+    add(0, h + sizeof(PassResults), fb);
+  else if (fb)
+    if (int rc = fetch(s, s->fout.p, fb, add)) return rc;
   if (energies) {
-    double ec = s->eout_h[0];
-    if (s->pme_on) ec += s->eout_h[2] + s->eout_h[3] + s->self_e + s->charged_e;
+    double ec = r.e[0];
+    if (s->pme_on) ec += r.e[2] + r.e[3] + s->self_e + s->charged_e;
     energies[PMX_E_COULOMB] += ec;
-    energies[PMX_E_LENNARDJONES] += s->eout_h[1];
+    energies[PMX_E_LENNARDJONES] += r.e[1];
   }
   return PMX_OK;
 }
@@ -1406,6 +1535,7 @@ int pmx_ctx_create(int device, pmx_ctx **out) {
     delete c;
     return PMX_ERR_HIP;
   }
+  ++g_contexts;
   *out = c;
   return PMX_OK;
 }
@@ -1417,6 +1547,11 @@ int pmx_ctx_destroy(pmx_ctx *ctx) {
   if (ctx->stream) hipStreamDestroy(ctx->stream);
   if (ctx->stream2) hipStreamDestroy(ctx->stream2);
   if (ctx->batch_host) hipHostFree(ctx->batch_host);
+  if (--g_contexts == 0) {
+    for (auto &kv : g_host_cache) hipHostFree(kv.second);
+    g_host_cache.clear();
+    g_host_cached = 0;
+  }
   if (ctx->batch_fork) hipEventDestroy(ctx->batch_fork);
   if (ctx->batch_join) hipEventDestroy(ctx->batch_join);
   delete ctx;
@@ -1461,6 +1596,9 @@ int pmx_sys_destroy(pmx_sys *sys) {
   for (auto &e : s->md.chunk_ev)
     if (e) hipEventDestroy(e);
   if (s->md.host) hipHostFree(s->md.host);
+  for (auto &e : s->stage_ev)
+    if (e) hipEventDestroy(e);
+  host_put(s->stage);
   for (auto &set : s->evsets)
     for (auto &e : set) hipEventDestroy(e);
   delete sys;
@@ -1477,9 +1615,15 @@ int pmx_sys_set_positions(pmx_sys *sys, const double *x_aos) {
   if (!sys || !x_aos) return PMX_ERR_ARG;
   Sys *s = &sys->s;
   hipSetDevice(s->ctx->device);
-  for (size_t k = 0; k < 3 * (size_t)s->n; ++k)
-    if (!std::isfinite(x_aos[k])) return fail(s->ctx, PMX_ERR_ARG, "non-finite position");
-  HIPCHK(hipMemcpyAsync(s->xorig.p, x_aos, 24 * (size_t)s->n, hipMemcpyHostToDevice, s->ctx->stream));
+  // an exponent of all ones carries into the sign bit (one branch in all: the loop vectorizes)
+  unsigned long long bad = 0;
+  for (size_t k = 0; k < 3 * (size_t)s->n; ++k) {
+    unsigned long long u;
+    std::memcpy(&u, x_aos + k, 8);
+    bad |= (u & 0x7fffffffffffffffull) + 0x0010000000000000ull;
+  }
+  if (bad >> 63) return fail(s->ctx, PMX_ERR_ARG, "non-finite position");
+  if (int rc = send(s, s->xorig.p, x_aos, 24 * (size_t)s->n)) return rc;
   s->have_positions = true;
   return PMX_OK;
 }
@@ -1835,7 +1979,7 @@ int pmx_md_set_state(pmx_sys *sys, const double *x, const double *v) {
   if (!s->md.on) return fail(s->ctx, PMX_ERR_ARG, "pmx_md_init first");
   int rc = pmx_sys_set_positions(sys, x);
   if (rc) return rc;
-  HIPCHK(hipMemcpyAsync(s->md.v.p, v, 24 * (size_t)s->n, hipMemcpyHostToDevice, s->ctx->stream));
+  if ((rc = send(s, s->md.v.p, v, 24 * (size_t)s->n))) return rc;
   s->md.forces_valid = false;
   return PMX_OK;
 }
@@ -2216,7 +2360,9 @@ constexpr long long kBatchRunCost = 2048;
 // One batched launch: the argument table, each system's first block and the
 // system of each block.
 struct BatchLaunch {
-  BatchBuf tab, first, b2s;
+  size_t tab_at = 0, first_at = 0, b2s_at = 0;  // in the batch's tables
+  const void *tab = nullptr;
+  const int *first = nullptr, *b2s = nullptr;
   unsigned blocks = 0;
   size_t lds = 0;
   int threads = 0;  // block size (0: the op's kBlock)
@@ -2226,10 +2372,13 @@ struct Batch {
   pmx_ctx *ctx = nullptr;
   std::vector<Sys *> sys;
   int nsys = 0;
+  bool first_forces = false;  // MD: the forces at the set positions come first, for every system
   BatchLaunch bin, scan, scatter, split, list, runs;
   BatchLaunch kick, spread, pair, yfwd, xconv, yinv, plane, gather, fixups, ukd, unsort, begin, half;
   BatchLaunch energy;
-  BatchBuf bsys, need, base, flags, rebuilds;
+  BatchBuf tables, bsys, need, base, flags, rebuilds;
+  std::vector<unsigned char> image;    // the tables of every launch, uploaded in one copy
+  std::vector<BatchLaunch *> launches;
   // slices of the context's pinned staging, and its events
   BatchSys *bsys_h = nullptr;
   unsigned long long *base_h = nullptr;
@@ -2237,27 +2386,47 @@ struct Batch {
   hipEvent_t fork = nullptr, join = nullptr;
 };
 
-// Uploads the table of one batched launch (args[s], nblocks[s] blocks of
-// system s; dynamic LDS `lds`).
+// Adds the table of one batched launch (args[s], nblocks[s] blocks of system
+// s; dynamic LDS `lds`) to the batch's tables.
 template <class Op>
 int batch_table(Batch &b, BatchLaunch &L, const std::vector<typename Op::Args> &args,
                 const std::vector<int> &nblocks, size_t lds = 0, int threads = 0) {
-  std::vector<int> first(b.nsys + 1, 0);
-  for (int i = 0; i < b.nsys; ++i) first[i + 1] = first[i] + nblocks[i];
-  std::vector<int> b2s(std::max(1, first[b.nsys]));
-  for (int i = 0; i < b.nsys; ++i)
-    for (int k = first[i]; k < first[i + 1]; ++k) b2s[k] = i;
-  L.blocks = (unsigned)first[b.nsys];
   L.lds = lds;
   L.threads = threads ? threads : Op::kBlock;
-  const int dev = b.ctx->device;
-  if (!L.tab.get(dev, sizeof(typename Op::Args) * args.size()) || !L.first.get(dev, 4 * first.size()) ||
-      !L.b2s.get(dev, 4 * b2s.size()))
-    return fail(b.ctx, PMX_ERR_OOM, "batch tables");
-  RtLock lk(g_rt_mu);
-  BHIPCHK(hipMemcpy(L.tab.p, args.data(), sizeof(typename Op::Args) * args.size(), hipMemcpyHostToDevice));
-  BHIPCHK(hipMemcpy(L.first.p, first.data(), 4 * first.size(), hipMemcpyHostToDevice));
-  BHIPCHK(hipMemcpy(L.b2s.p, b2s.data(), 4 * b2s.size(), hipMemcpyHostToDevice));
+  auto room = [&](size_t bytes) {
+    const size_t at = (b.image.size() + 255) / 256 * 256;
+    b.image.resize(at + std::max<size_t>(bytes, 4));
+    return at;
+  };
+  L.tab_at = room(sizeof(typename Op::Args) * args.size());
+  std::memcpy(b.image.data() + L.tab_at, args.data(), sizeof(typename Op::Args) * args.size());
+  L.first_at = room(4 * ((size_t)b.nsys + 1));
+  int *first = reinterpret_cast<int *>(b.image.data() + L.first_at);
+  first[0] = 0;
+  for (int i = 0; i < b.nsys; ++i) first[i + 1] = first[i] + nblocks[i];
+  L.blocks = (unsigned)first[b.nsys];
+  L.b2s_at = room(4 * (size_t)L.blocks);
+  int *b2s = reinterpret_cast<int *>(b.image.data() + L.b2s_at);
+  for (int i = 0; i < b.nsys; ++i) b2s = std::fill_n(b2s, nblocks[i], i);
+  b.launches.push_back(&L);
+  return PMX_OK;
+}
+
+// Uploads the tables (nothing of an earlier upload may be in use).
+int batch_upload(Batch &b) {
+  if (!b.tables.get(b.ctx->device, b.image.size())) return fail(b.ctx, PMX_ERR_OOM, "batch tables");
+  {
+    RtLock lk(g_rt_mu);
+    BHIPCHK(hipMemcpy(b.tables.p, b.image.data(), b.image.size(), hipMemcpyHostToDevice));
+  }
+  const unsigned char *d = static_cast<const unsigned char *>(b.tables.p);
+  for (BatchLaunch *L : b.launches) {
+    L->tab = d + L->tab_at;
+    L->first = reinterpret_cast<const int *>(d + L->first_at);
+    L->b2s = reinterpret_cast<const int *>(d + L->b2s_at);
+  }
+  b.image.clear();
+  b.launches.clear();
   return PMX_OK;
 }
 
@@ -2265,8 +2434,7 @@ template <class Op>
 void batch_go(const BatchLaunch &L, hipStream_t st, const BatchStep &bs) {
   if (!L.blocks) return;
   hipLaunchKernelGGL(k_batch<Op>, dim3(L.blocks), dim3(L.threads), L.lds, st,
-                     reinterpret_cast<const typename Op::Args *>(L.tab.p), reinterpret_cast<const int *>(L.b2s.p),
-                     reinterpret_cast<const int *>(L.first.p), bs);
+                     static_cast<const typename Op::Args *>(L.tab), L.b2s, L.first, bs);
 }
 
 // The batch's kernel case: the pair kernel's cases of run_pair_phase for PME
@@ -2471,7 +2639,7 @@ int batch_tables(Batch &b) {
                            P<unsigned long long>(s->md.step_dev), P<int>(s->overflow),
                            reinterpret_cast<long long *>(b.rebuilds.p) + i};
   }
-  return PMX_OK;
+  return batch_upload(b);
 }
 
 // Queues one chunk of K steps of every system of the batch (the first step
@@ -2536,22 +2704,21 @@ int batch_chunk(Batch &b, int K, bool opening) {
 // One force pass of every system of the batch at its set positions (list
 // rebuilt for all), with the energies reduced: the work of compute() for
 // each.  Systems whose list outgrew its buffers are grown and computed again
-// alone.
+// alone (*grown: the tables hold their old buffers).
 template <bool MIXED, int C, int LJ, int CS, bool BIGLJ, int ORDER>
-int batch_forces(Batch &b) {
+int batch_forces(Batch &b, bool *grown) {
   using R = typename std::conditional<MIXED, float, double>::type;
   using T = R;
   hipStream_t st = b.ctx->stream, st2 = b.ctx->stream2;
   const int ns = b.nsys;
-  int rc = batch_tables<MIXED, C, LJ, CS, BIGLJ, ORDER>(b);
-  if (rc) return rc;
-  for (Sys *s : b.sys) {
+  int rc;
+  for (Sys *s : b.sys)
     if (!s->acc_clean) launch_zero(s);
-    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, P<int>(s->overflow), 0, 2ll);
-  }
   std::vector<unsigned char> all(ns, 1);
   BHIPCHK(hipMemcpyAsync(b.need.p, all.data(), ns, hipMemcpyHostToDevice, st));
   BHIPCHK(hipMemcpyAsync(b.bsys.p, b.bsys_h, sizeof(BatchSys) * ns, hipMemcpyHostToDevice, st));
+  hipLaunchKernelGGL(k_batch_clear, dim3(nblk(ns, 256)), dim3(256), 0, st, ns,
+                     reinterpret_cast<const BatchSys *>(b.bsys.p));
   const BatchStep bk{0, 0, reinterpret_cast<unsigned char *>(b.need.p)};
   batch_go<OpBin>(b.bin, st, bk);
   batch_go<OpScanColumns>(b.scan, st, bk);
@@ -2584,6 +2751,7 @@ int batch_forces(Batch &b) {
     s->prune_pending = false;
     s->acc_clean = true;
     for (int attempt = 0; b.flags_h[i] && attempt < 6; ++attempt) {
+      *grown = true;
       if ((rc = grow_and_retry(s)) || (rc = compute(s, 0))) return rc;
       int ovf = 0;
       if (hipMemcpyAsync(&ovf, s->overflow.p, 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
@@ -2606,6 +2774,19 @@ int batch_run(Batch &b, int nsteps) {
   hipStream_t st = b.ctx->stream;
   int rc = batch_tables<MIXED, C, LJ, CS, BIGLJ, ORDER>(b);
   if (rc) return rc;
+  if (b.first_forces) {
+    bool outgrew = false;
+    if ((rc = batch_forces<MIXED, C, LJ, CS, BIGLJ, ORDER>(b, &outgrew))) return rc;
+    for (int i = 0; i < b.nsys; ++i) {
+      if (b.flags_h[i]) return fail(b.ctx, PMX_ERR_OVERFLOW, "pair list capacity exceeded");
+      ++b.sys[i]->md.rebuilds;
+      b.sys[i]->md.forces_valid = true;
+    }
+    if (outgrew) {
+      BHIPCHK(hipStreamSynchronize(st));
+      if ((rc = batch_tables<MIXED, C, LJ, CS, BIGLJ, ORDER>(b))) return rc;
+    }
+  }
   BHIPCHK(hipMemsetAsync(b.rebuilds.p, 0, 8 * (size_t)b.nsys, st));
   int done = 0, retries = 0, last = 0;
   while (done < nsteps) {
@@ -2748,7 +2929,10 @@ namespace {
 // nsteps < 0: one force pass (batch_forces), else nsteps MD steps.
 template <bool MIXED, int C, int LJ, int CS, bool BIG, int ORDER>
 int batch_exec(Batch &b, int nsteps) {
-  return nsteps < 0 ? batch_forces<MIXED, C, LJ, CS, BIG, ORDER>(b) : batch_run<MIXED, C, LJ, CS, BIG, ORDER>(b, nsteps);
+  if (nsteps >= 0) return batch_run<MIXED, C, LJ, CS, BIG, ORDER>(b, nsteps);
+  if (int rc = batch_tables<MIXED, C, LJ, CS, BIG, ORDER>(b)) return rc;
+  bool grown = false;
+  return batch_forces<MIXED, C, LJ, CS, BIG, ORDER>(b, &grown);
 }
 
 template <bool MIXED, int CASE>
@@ -2799,13 +2983,18 @@ int batch_entry(pmx_sys *const *systems, int nsys, int nsteps) {
   Batch b;
   b.ctx = ctx;
   b.nsys = nsys;
+  // the first forces of a run: in one batched pass when every system needs
+  // them, one by one where only some do
+  b.first_forces = md;
+  for (int i = 0; i < nsys; ++i) b.first_forces &= !systems[i]->s.md.forces_valid;
   for (int i = 0; i < nsys; ++i) {
     Sys *s = &systems[i]->s;
     b.sys.push_back(s);
     if (!s->cached)
       if (int rc = setup(s)) return rc;
     if (md) {
-      if (int rc = md_ensure_forces(s)) return rc;
+      if (!b.first_forces)
+        if (int rc = md_ensure_forces(s)) return rc;
       if (!s->acc_clean) {
         launch_zero(s);
         s->acc_clean = true;
@@ -2870,8 +3059,8 @@ int pmx_md_get_state(pmx_sys *sys, double *x, double *v, double *energies) {
   hipSetDevice(s->ctx->device);
   hipStream_t st = s->ctx->stream;
   const int n = s->n;
-  if (x) HIPCHK(hipMemcpyAsync(x, s->xorig.p, 24 * (size_t)n, hipMemcpyDeviceToHost, st));
-  if (v) HIPCHK(hipMemcpyAsync(v, m.v.p, 24 * (size_t)n, hipMemcpyDeviceToHost, st));
+  const bool bonded = m.nb + m.na > 0;
+  const size_t nke = nblk(n, 256), nbe = bonded ? 2 * (size_t)s->term_blocks : 0, vec = 3 * (size_t)n;
   if (energies) {
     // potential energies at the current positions (computed first if the
     // state was just set) and kinetic energy of v
@@ -2879,27 +3068,56 @@ int pmx_md_get_state(pmx_sys *sys, double *x, double *v, double *energies) {
     reduce_energies(s, false);
     hipLaunchKernelGGL(k_kinetic, dim3(nblk(n, 256)), dim3(256), 0, st, n, P<double>(m.v), P<double>(m.minv),
                        P<double>(m.ke_e));
-    const int nbb = s->term_blocks;
-    std::vector<double> be(2 * nbb, 0.0), ke(nblk(n, 256));
-    if (m.nb + m.na > 0) HIPCHK(hipMemcpyAsync(be.data(), m.bond_e.p, 16 * (size_t)nbb, hipMemcpyDeviceToHost, st));
-    HIPCHK(hipMemcpyAsync(ke.data(), m.ke_e.p, 8 * ke.size(), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipMemcpyAsync(s->eout_h, s->eout.p, 32, hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
+  }
+  // everything in one go when it fits the stage, else positions and
+  // velocities in chunks first
+  size_t words = energies ? 4 + nke + nbe : 0;
+  const bool once = 8 * (words + (x ? vec : 0) + (v ? vec : 0)) <= kStageBytes;
+  for (int k = 0; k < 2 && !once; ++k) {
+    double *const to = k ? v : x;
+    if (!to) continue;
+    const int rc = fetch(s, k ? m.v.p : s->xorig.p, 8 * vec, [&](size_t o, const void *data, size_t bytes) {
+      std::memcpy(reinterpret_cast<unsigned char *>(to) + o, data, bytes);
+    });
+    if (rc) return rc;
+  }
+  if (once) words += (x ? vec : 0) + (v ? vec : 0);
+  if (int rc = stage_get(s, 8 * words)) return rc;
+  double *const h = static_cast<double *>(s->stage.p);
+  double *at = h;
+  auto take = [&](const void *src, size_t count) {
+    const hipError_t e = count ? hipMemcpyAsync(at, src, 8 * count, hipMemcpyDeviceToHost, st) : hipSuccess;
+    at += count;
+    return e;
+  };
+  if (energies) {
+    HIPCHK(take(s->eout.p, 4));
+    HIPCHK(take(m.ke_e.p, nke));
+    HIPCHK(take(m.bond_e.p, nbe));
+  }
+  double *const hx = at;
+  if (once && x) HIPCHK(take(s->xorig.p, vec));
+  double *const hv = at;
+  if (once && v) HIPCHK(take(m.v.p, vec));
+  HIPCHK(hipStreamSynchronize(st));
+  if (once && x) std::memcpy(x, hx, 8 * vec);
+  if (once && v) std::memcpy(v, hv, 8 * vec);
+  if (energies) {
+    const double *const ke = h + 4, *const be = ke + nke;
     double eb = 0, ea = 0, ek = 0;
-    for (int i = 0; i < nbb; ++i) {
-      eb += be[2 * i];
-      ea += be[2 * i + 1];
+    for (size_t i = 0; i < nbe; i += 2) {
+      eb += be[i];
+      ea += be[i + 1];
     }
-    for (double e : ke) ek += e;
-    double ec = s->eout_h[0];
-    if (s->pme_on) ec += s->eout_h[2] + s->eout_h[3] + s->self_e + s->charged_e;
+    for (size_t i = 0; i < nke; ++i) ek += ke[i];
+    double ec = h[0];
+    if (s->pme_on) ec += h[2] + h[3] + s->self_e + s->charged_e;
     energies[PMX_MD_E_COULOMB] = ec;
-    energies[PMX_MD_E_LJ] = s->eout_h[1];
+    energies[PMX_MD_E_LJ] = h[1];
     energies[PMX_MD_E_BOND] = eb;
     energies[PMX_MD_E_ANGLE] = ea;
     energies[PMX_MD_E_KINETIC] = ek;
   }
-  HIPCHK(hipStreamSynchronize(st));
   return PMX_OK;
 }
 

@@ -436,7 +436,7 @@ struct BatchSys {
   float lim2;                    // (skin / 2)^2
   int force;                     // rebuild at step 0 of the chunk whatever the displacement
   unsigned long long *step_dev;  // first step of the chunk
-  const int *overflow;
+  int *overflow;
   long long *rebuilds;           // device count of the builds in the batch
 };
 
@@ -457,6 +457,11 @@ static __global__ void k_batch_need(int nsys, const BatchSys *__restrict__ bs, i
 static __global__ void k_batch_steps(int nsys, const BatchSys *__restrict__ bs, const unsigned long long *__restrict__ base) {
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s < nsys) *bs[s].step_dev = base[s];
+}
+
+static __global__ void k_batch_clear(int nsys, const BatchSys *__restrict__ bs) {
+  const int s = blockIdx.x * blockDim.x + threadIdx.x;
+  if (s < nsys) bs[s].overflow[0] = bs[s].overflow[1] = 0;
 }
 
 static __global__ void k_batch_flags(int nsys, const BatchSys *__restrict__ bs, int *__restrict__ out) {
