@@ -956,16 +956,25 @@ int setup(Sys *s) {
 template <bool MIXED>
 FixupArgs<MIXED> fixup_args(Sys *s, bool stats, bool border_here, bool rest_here, int *nblocks);
 
-// Resident blocks per CU of a pair-kernel launch: at least 1, at most those
-// of kMinRuns waves on the device (the static schedule's runs are cut for
-// them; more would also leave the PME chain no room beside).  Each caller keeps its
+// The least number of runs of a system's list, and with it the pair kernel's
+// waves (kMinRuns).
+int min_runs(const Sys *s) {
+  const bool grid = s->pme_on && (s->d.pme_terms & PMX_PME_RECIP);
+  return s->mixed && !grid ? kMinRunsAlone : kMinRuns;
+}
+
+// Blocks per CU of a pair-kernel launch of `runs` least runs: at least 1, at
+// most those of as many waves on the device.
+int pair_blocks_of(int per_cu, int runs) { return std::min(per_cu, runs / (kPairBlock / kWave) / 256); }
+
+// Resident blocks per CU of a pair kernel, at least 1.  Each caller keeps its
 // kernel's value in a function-local static, initialized once even under
 // concurrent first calls.
 int pair_blocks_per_cu(const void *kernel) {
   int per_cu = 0;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kPairBlock, 0) != hipSuccess || per_cu < 1)
     per_cu = 1;
-  return std::min(per_cu, kMinRuns / (kPairBlock / kWave) / 256);
+  return per_cu;
 }
 
 template <bool MIXED, int C, int LJ, int CS, bool BIGLJ = false>
@@ -977,8 +986,9 @@ void launch_pair_phase(Sys *s, bool stats, int phase) {
   if (phase < 0) {
     // as many blocks as are resident at once (the schedules assign each
     // wave its first tile, or its whole run, statically)
-    static const int per_cu =
+    static const int fit =
         pair_blocks_per_cu(reinterpret_cast<const void *>(k_pair<MIXED, C, LJ, CS, BIGLJ, kPairPlain>));
+    const int per_cu = pair_blocks_of(fit, min_runs(s));
     // knob > 0: blocks per CU; 0: as many as fit; < 0: that many fewer
     const int bpc = s->tune_pair_blocks > 0 ? std::min(s->tune_pair_blocks, per_cu)
                                             : std::max(1, per_cu + s->tune_pair_blocks);
@@ -1193,7 +1203,7 @@ void timing_begin_call(Sys *s, bool timing) {
 unsigned runs_blocks(Sys *s) { return (unsigned)std::min<long long>(256, nblk(s->nsuper, kRunsBlock / kWave)); }
 void make_runs(Sys *s, hipStream_t st) {
   hipLaunchKernelGGL(k_runs, dim3(runs_blocks(s)), dim3(kRunsBlock), 0, st, s->nsuper, P<int>(s->count),
-                     P<int>(s->lcost), P<int>(s->ecost), s->cap, P<int2>(s->runs), P<int>(s->ntiles));
+                     P<int>(s->lcost), P<int>(s->ecost), s->cap, min_runs(s), P<int2>(s->runs), P<int>(s->ntiles));
 }
 
 SortedBins sorted_bins(Sys *s) {
@@ -2605,9 +2615,9 @@ int batch_tables(Batch &b) {
     // pair-kernel blocks in proportion to the atoms (a run's share of a
     // system's waves changes no result), about the device's resident blocks
     // in all
-    static const int per_cu =
+    static const int fit =
         pair_blocks_per_cu(reinterpret_cast<const void *>(k_batch<PairOp<MIXED, C, LJ, CS, BIGLJ, ORDER>>));
-    const double pair_blocks = (double)b.ctx->cus * per_cu;
+    const double pair_blocks = (double)b.ctx->cus * pair_blocks_of(fit, kMinRuns);
     for (int i = 0; i < ns; ++i)
       nb[i] = std::max(1, (int)std::lround(pair_blocks * b.sys[i]->n / (double)natoms));
     if ((rc = batch_table<PairOp<MIXED, C, LJ, CS, BIGLJ, ORDER>>(b, b.pair, args_pair, nb, 0))) return rc;

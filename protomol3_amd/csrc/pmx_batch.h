@@ -158,7 +158,7 @@ struct OpRuns {
   static constexpr int kBlock = kRunsBlock, kMinBlocks = 1;
   static constexpr bool kGated = true;
   __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &) {
-    runs_body(bid, nbk, a.nsuper, a.count, a.cost, a.ecost, a.cap, a.min_run_cost, a.runs, a.ntiles);
+    runs_body(bid, nbk, a.nsuper, a.count, a.cost, a.ecost, a.cap, kMinRuns, a.min_run_cost, a.runs, a.ntiles);
   }
 };
 

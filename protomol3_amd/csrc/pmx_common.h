@@ -19,7 +19,13 @@ constexpr int kTileEntries = 16;   // granularity of the per-supercluster list c
 // MI355X (256 CUs x 4 blocks of 4 waves): the static schedule gives every
 // wave k equal runs there (one for systems up to about 10^5 atoms: a run
 // boundary costs a flush of the i-forces, so runs are long).
+// A mixed system without the PME grid has the device to itself and takes six
+// blocks per CU, as many as its registers allow, and kMinRunsAlone for
+// kMinRuns: 46,000 atoms, unequal cutoffs, 97 -> 89 us a launch.  Beside
+// the PME chain six would leave its passes no room (26,000 atoms: a step of
+// 124 us becomes 136).
 constexpr int kMinRuns = 4096;
+constexpr int kMinRunsAlone = 6144;
 constexpr int kMaxRuns = 5 * kMinRuns;
 constexpr int kRunCost = 8192;     // work units (list cost model) per run, at least
 constexpr int kWave = 64;

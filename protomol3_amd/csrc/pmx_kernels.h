@@ -360,7 +360,8 @@ static __global__ void __launch_bounds__(kScanBlock) k_columns(int ncols, int nz
 // Exclusive scan of m <= kScanSingleMax counts and the columns'
 // superclusters, in one block: bound by latency, so each wave owns a
 // contiguous segment, four counts a lane and round, and every round is loaded
-// before the first is summed; segment totals are combined across the block.
+// before the first is summed; segment totals are combined across the block (13,000
+// bins: 12.3 and 4.8 us in two launches, 6.5 in one).
 // Counts and starts are padded to whole groups of four.  The counts are cleared for the next histogram.
 constexpr long long kScanSingleMax = 1 << 16;
 __device__ __forceinline__ void scan_columns_body(uint32_t *__restrict__ in, int m, uint32_t *out,
@@ -844,7 +845,12 @@ inline size_t list_lds_bytes(int cap) { return 8 * (size_t)((cap + 31) / 32); }
 // cluster, and the pair is not FULL-excluded; bit 8 + c marks MODIFIED.  The
 // entry's mask field becomes w.  The excluded pairs of the supercluster's
 // atoms look up their entry (sorted by j-cluster); a pair whose clusters are
-// not listed is beyond the list radius and never evaluated.
+// not listed is beyond the list radius and never evaluated.  Bound by the
+// chains of dependent loads of a block, of which eight fit a CU.  With the
+// masks in launches of their own (a thread per excluded pair that claimed its
+// entry by compare-and-swap, a wave per mask that searched every pair's
+// exclusions) 26,000 atoms took 30 + 12 + 20 us and 1,000,000 atoms 283 + 174 +
+// 387; in one 36 to 45 and 287.
 __device__ __forceinline__ void build_list_body(const int bid_, const int nbk_, const ListParams &q,
                                                 const int *__restrict__ sc_col, const int *__restrict__ colsc,
                                                 const float4 *__restrict__ sctr, const float4 *__restrict__ shalf,
@@ -1096,7 +1102,7 @@ __device__ inline int excl_class(const int *__restrict__ eptr, const int2 *__res
 // Run schedule: the list entries of all superclusters, in supercluster
 // order, are cut into nruns contiguous runs of equal estimated work (the
 // work estimates of k_build_list: per supercluster, and as an inclusive
-// prefix over its entries); nruns, a multiple of kMinRuns set by C, the
+// prefix over its entries); nruns, a multiple of min_runs set by C, the
 // total, depends only on the list.  Run w starts in supercluster runs[w].x
 // at entry runs[w].y (even: runs hold whole pair-kernel groups), where the
 // global work prefix first exceeds b_w = floor(w C / nruns), and ends where
@@ -1107,11 +1113,12 @@ __device__ inline int excl_class(const int *__restrict__ eptr, const int2 *__res
 // One launch: each block adds up the work ahead of its superclusters and in
 // total for itself (a table of 4 bytes per supercluster), its waves take one
 // supercluster after the other, and each entry places the run boundaries
-// that fall in its work interval.
+// that fall in its work interval.  26,000 atoms 23 us in three launches (two of
+// them one block), 9.7 in one; 1,000,000 atoms 130 and 28.
 constexpr int kRunsBlock = 1024;
 __device__ __forceinline__ void runs_body(const int bid_, const int nbk_, int nsuper, const int *__restrict__ count,
                                           const int *__restrict__ cost, const int *__restrict__ ecost, int cap,
-                                          long long min_run_cost, int2 *__restrict__ runs,
+                                          int min_runs, long long min_run_cost, int2 *__restrict__ runs,
                                           int *__restrict__ ntiles) {
   constexpr int NW = kRunsBlock / kWave;
   __shared__ long long s_c[2][NW];
@@ -1141,9 +1148,9 @@ __device__ __forceinline__ void runs_body(const int bid_, const int nbk_, int ns
     C += s_c[1][k];
     last = max(last, s_last[k]);
   }
-  const long long per = (long long)kMinRuns * kRunCost;
+  const long long per = (long long)min_runs * kRunCost;
   const long long k = (C + per - 1) / per;
-  int nruns = kMinRuns * (int)(k < 1 ? 1 : (k > kMaxRuns / kMinRuns ? kMaxRuns / kMinRuns : k));
+  int nruns = min_runs * (int)(k < 1 ? 1 : (k > kMaxRuns / min_runs ? kMaxRuns / min_runs : k));
   if (min_run_cost > 0) {
     // runs of at least min_run_cost units, in whole waves' worth of 64 runs:
     // a small list's runs would otherwise hold an entry or two each, and the
@@ -1204,9 +1211,9 @@ __device__ __forceinline__ void runs_body(const int bid_, const int nbk_, int ns
 
 static __global__ void __launch_bounds__(kRunsBlock) k_runs(int nsuper, const int *__restrict__ count,
                                                             const int *__restrict__ cost,
-                                                            const int *__restrict__ ecost, int cap,
+                                                            const int *__restrict__ ecost, int cap, int min_runs,
                                                             int2 *__restrict__ runs, int *__restrict__ ntiles) {
-  runs_body(blockIdx.x, gridDim.x, nsuper, count, cost, ecost, cap, 0, runs, ntiles);
+  runs_body(blockIdx.x, gridDim.x, nsuper, count, cost, ecost, cap, min_runs, 0, runs, ntiles);
 }
 
 // ---------------------------------------------------------------------------
