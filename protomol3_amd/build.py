@@ -7,12 +7,13 @@ import subprocess
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 LIB = os.path.join(HERE, "lib", "libpmx.so")
-SOURCES = [os.path.join(HERE, "csrc", f) for f in ("pmx.hip", "pmx_pair.hip", "pmx_pair.h", "pmx_kernels.h",
-                                                   "pmx_batch.h", "pmx_common.h")]
+SOURCES = [os.path.join(HERE, "csrc", f) for f in ("pmx.hip", "pmx_pair.hip", "pmx_pair64.hip", "pmx_pair.h",
+                                                   "pmx_kernels.h", "pmx_batch.h", "pmx_common.h")]
 # options of single files
 FILE_FLAGS = {
     # see the head of the file
     "pmx_pair.hip": ["-mllvm", "-structurizecfg-skip-uniform-regions"],
+    "pmx_pair64.hip": ["-mllvm", "-structurizecfg-skip-uniform-regions"],
 }
 
 HIPCC_FLAGS = [

@@ -120,6 +120,7 @@ struct Sys {
   int tune_prune = 1;          // 1: the first pair pass after a list build prunes the list's cluster pairs
   bool prune_pending = false;  // a list was built and its first pair pass has not run
   int pair_grid = 0;           // blocks of the pair-kernel launch
+  RunCut cut = kCutBeside;     // how the list is cut into runs
   long long nbins = 0;
   int nscanblocks = 0;
   int recip_blocks = 0, term_blocks = 0;  // blocks of the x pass and of the atoms' terms
@@ -692,28 +693,30 @@ int setup(Sys *s) {
   lp.skin = (float)s->md.skin;
   lp.rlist2 = (float)((rcmax + margin + s->md.skin) * (rcmax + margin + s->md.skin));
   s->pp.prune_r2 = (double)lp.rlist2 * (1.0 + 1e-5);
-  {
-    DirectC &c = s->pp.dc;
-    c = DirectC{};
+  auto direct = [&](auto &c) {
+    using R = std::decay_t<decltype(c.guard)>;
+    c = std::decay_t<decltype(c)>{};
     c.lj.load(pp.lj);
     c.co.load(pp.co);
     c.ljkind = pp.lj.kind;
     c.cokind = pp.co.kind;
     c.rmax2 = !pp.has_lj ? c.co.rc2 : (pp.coul == COUL_NONE ? c.lj.rc2 : std::max(c.lj.rc2, c.co.rc2));
-    c.guard = (float)pp.guard;
-    c.near2 = std::nextafter(c.rmax2 + c.guard, INFINITY);
-    c.in2 = std::nextafter(c.rmax2 - c.guard, 0.f);
-    c.pa = (float)(0.3275911 * pp.alpha);
-    c.ke = (float)(-1.4426950408889634 * pp.alpha * pp.alpha);
-    c.a2pi = (float)pp.a2pi;
-    c.csf = (float)pp.csf;
-    c.prune_r2 = (float)pp.prune_r2;
+    c.guard = (R)pp.guard;
+    c.near2 = std::nextafter(c.rmax2 + c.guard, (R)INFINITY);
+    c.in2 = std::nextafter(c.rmax2 - c.guard, (R)0);
+    c.pa = (R)(0.3275911 * pp.alpha);
+    c.ke = (R)((sizeof(R) == 4 ? -1.4426950408889634 : -1.0) * pp.alpha * pp.alpha);
+    c.a2pi = (R)pp.a2pi;
+    c.csf = (R)pp.csf;
+    c.prune_r2 = (R)pp.prune_r2;
     for (int k = 0; k < 3; ++k) {
-      c.hi[k] = (float)pp.Lhi[k];
-      c.lo[k] = (float)pp.Llo[k];
-      c.inv[k] = (float)bx.Linv[k];
+      c.hi[k] = (R)pp.Lhi[k];
+      c.lo[k] = (R)pp.Llo[k];
+      c.inv[k] = (R)bx.Linv[k];
     }
-  }
+  };
+  direct(s->pp.dc);
+  direct(s->pp.dd);
   lp.rc = (float)rcmax;
   lp.ncl = s->ncl;
   lp.nsuper = s->nsuper;
@@ -956,13 +959,6 @@ int setup(Sys *s) {
 template <bool MIXED>
 FixupArgs<MIXED> fixup_args(Sys *s, bool stats, bool border_here, bool rest_here, int *nblocks);
 
-// The least number of runs of a system's list, and with it the pair kernel's
-// waves (kMinRuns).
-int min_runs(const Sys *s) {
-  const bool grid = s->pme_on && (s->d.pme_terms & PMX_PME_RECIP);
-  return s->mixed && !grid ? kMinRunsAlone : kMinRuns;
-}
-
 // Blocks per CU of a pair-kernel launch of `runs` least runs: at least 1, at
 // most those of as many waves on the device.
 int pair_blocks_of(int per_cu, int runs) { return std::min(per_cu, runs / (kPairBlock / kWave) / 256); }
@@ -988,7 +984,12 @@ void launch_pair_phase(Sys *s, bool stats, int phase) {
     // wave its first tile, or its whole run, statically)
     static const int fit =
         pair_blocks_per_cu(reinterpret_cast<const void *>(k_pair<MIXED, C, LJ, CS, BIGLJ, kPairPlain>));
-    const int per_cu = pair_blocks_of(fit, min_runs(s));
+    // the least number of the list's runs is that of the waves: of the mixed
+    // form for the device it is cut for, whatever this one is
+    const bool grid = s->pme_on && (s->d.pme_terms & PMX_PME_RECIP);
+    s->cut = !MIXED ? kCut64 : grid ? kCutBeside : kCutAlone;
+    const int per_cu = pair_blocks_of(fit, s->cut.min_runs);
+    if (!MIXED) s->cut.min_runs = per_cu * (kPairBlock / kWave) * 256;
     // knob > 0: blocks per CU; 0: as many as fit; < 0: that many fewer
     const int bpc = s->tune_pair_blocks > 0 ? std::min(s->tune_pair_blocks, per_cu)
                                             : std::max(1, per_cu + s->tune_pair_blocks);
@@ -1203,7 +1204,7 @@ void timing_begin_call(Sys *s, bool timing) {
 unsigned runs_blocks(Sys *s) { return (unsigned)std::min<long long>(256, nblk(s->nsuper, kRunsBlock / kWave)); }
 void make_runs(Sys *s, hipStream_t st) {
   hipLaunchKernelGGL(k_runs, dim3(runs_blocks(s)), dim3(kRunsBlock), 0, st, s->nsuper, P<int>(s->count),
-                     P<int>(s->lcost), P<int>(s->ecost), s->cap, min_runs(s), P<int2>(s->runs), P<int>(s->ntiles));
+                     P<int>(s->lcost), P<int>(s->ecost), s->cap, s->cut, P<int2>(s->runs), P<int>(s->ntiles));
 }
 
 SortedBins sorted_bins(Sys *s) {
@@ -2359,14 +2360,6 @@ struct BatchBuf {
   }
 };
 
-// Smallest run of a list built in batched launches, in list-cost units (about
-// 35 ns of wave time each): a system's runs share the batch's waves with
-// every other system's, so its list is cut into runs of real work rather than
-// into as many runs as the device has resident waves (the single-system cut,
-// which keeps a small system's pass short alone).  The runs, and so a mixed
-// result, are those of the same list in any batch.
-constexpr long long kBatchRunCost = 2048;
-
 // One batched launch: the argument table, each system's first block and the
 // system of each block.
 struct BatchLaunch {
@@ -2514,7 +2507,7 @@ int batch_tables(Batch &b) {
                       P<float4>(s->ctr), P<float4>(s->half), P<int4>(s->entries), P<int>(s->count),
                       P<int>(s->ecost), P<int>(s->lcost), mask_args(s), P<int>(s->nmaskwork), P<int>(s->overflow)};
       list_lds = std::max(list_lds, list_lds_bytes(s->cap));
-      args_runs[i] = {s->nsuper, s->cap, P<int>(s->count), P<int>(s->lcost), P<int>(s->ecost), kBatchRunCost,
+      args_runs[i] = {s->nsuper, s->cap, P<int>(s->count), P<int>(s->lcost), P<int>(s->ecost),
                       P<int2>(s->runs), P<int>(s->ntiles)};
     }
     for (int i = 0; i < ns; ++i) nb[i] = (int)nblk(b.sys[i]->n, 256);

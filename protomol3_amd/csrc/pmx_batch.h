@@ -151,14 +151,13 @@ struct OpRuns {
   struct Args {
     int nsuper, cap;
     const int *count, *cost, *ecost;
-    long long min_run_cost;
     int2 *runs;
     int *ntiles;
   };
   static constexpr int kBlock = kRunsBlock, kMinBlocks = 1;
   static constexpr bool kGated = true;
   __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &) {
-    runs_body(bid, nbk, a.nsuper, a.count, a.cost, a.ecost, a.cap, kMinRuns, a.min_run_cost, a.runs, a.ntiles);
+    runs_body(bid, nbk, a.nsuper, a.count, a.cost, a.ecost, a.cap, kCutBatch, a.runs, a.ntiles);
   }
 };
 
@@ -227,18 +226,13 @@ struct OpPair {
     typename AccT<MIXED>::type *facc;
     PairOut out;
   };
-  static constexpr int kBlock = kPairBlock, kMinBlocks = 4;
+  static constexpr int kBlock = kPairBlock, kMinBlocks = MIXED ? 4 : 3;
   static constexpr bool kGated = false;
   // the runs in contiguous shares per wave (schedule 0)
   __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &) {
-    if constexpr (MIXED)
-      pair_direct_body<COUL, LJSW, CSW, BIGLJ, kPairPlain>(bid, nbk, a.pp, 0, a.runs, a.ntiles, a.count, a.tilectr,
-                                                           a.entries, a.entries, a.cap, a.masks, a.xs, a.sorg, a.ts,
-                                                           a.perm, a.ljtab, a.ljt, a.facc, a.out);
-    else
-      pair_body<MIXED, COUL, LJSW, CSW, BIGLJ, kPairPlain>(bid, nbk, a.pp, 0, a.runs, a.ntiles, a.count, a.tilectr,
-                                                           a.entries, a.entries, a.cap, a.masks, a.xs, a.sorg, a.ts,
-                                                           a.perm, a.ljtab, a.ljt, a.facc, a.out);
+    pair_body<MIXED, COUL, LJSW, CSW, BIGLJ, kPairPlain>(bid, nbk, a.pp, 0, a.runs, a.ntiles, a.count, a.tilectr,
+                                                         a.entries, a.entries, a.cap, a.masks, a.xs, a.sorg, a.ts,
+                                                         a.perm, a.ljtab, a.ljt, a.facc, a.out);
   }
 };
 

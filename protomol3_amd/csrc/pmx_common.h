@@ -28,6 +28,27 @@ constexpr int kMinRuns = 4096;
 constexpr int kMinRunsAlone = 6144;
 constexpr int kMaxRuns = 5 * kMinRuns;
 constexpr int kRunCost = 8192;     // work units (list cost model) per run, at least
+// How a list is cut.  A small list's runs would hold an entry or two each, and
+// a wave would spend its time on the i-force flush at every tile's end: runs of
+// at least `least` units (of about 35 ns of a wave each, in FP64 twice that),
+// and where that makes more than `few` runs, of at least least_many units,
+// which leaves registers to the PME passes.
+// Mixed, a launch alone with runs of 1 entry / 300 / 400 / 600 / 900 units: 1,500 atoms
+// 18.7 / 12.5 / 14.4 / 18.2 / 24.7 us, 4,000 atoms 26.1 / 21.0 / 19.5 / 20.5 /
+// 25.3; FP64, 1,500 atoms 18.9 / 14.9 / 17.6 / 23.0 / 29.9.  Steps with
+// the PME chain beside, 400 / 600 / 900: 9,400 atoms 90.4 / 83.3 / 82.9 us;
+// 4,096 / 3,072 / 2,048 runs: 13,800 atoms 97 / 94 / 91 us, 26,000 atoms 109 /
+// 107 / 130.
+struct RunCut {
+  int min_runs, least, least_many, few;
+};
+constexpr RunCut kCutBeside = {kMinRuns, 600, 1500, 1536};         // mixed, PME beside
+constexpr RunCut kCutAlone = {kMinRunsAlone, 400, 400, kMaxRuns};  // mixed, without the grid
+constexpr RunCut kCut64 = {kMinRuns, 300, 300, kMaxRuns};          // FP64 (min_runs: of the waves that fit)
+// A list built in batched launches: a system's runs share the batch's waves
+// with every other system's, so they hold real work.  The runs, and so a mixed
+// result, are those of the same list in any batch.
+constexpr RunCut kCutBatch = {kMinRuns, 2048, 2048, kMaxRuns};
 constexpr int kWave = 64;
 constexpr int kPairBlock = 256;    // 4 waves
 constexpr double kForceScale = 4294967296.0;      // 2^32: int64 fixed-point forces
@@ -66,28 +87,32 @@ struct SwR {
   }
 };
 
-// Constants of the mixed pair kernel, in FP32 from the host: kernel arguments
+// Constants of the pair kernel in its type, from the host: kernel arguments
 // stay in scalar registers (conversions in the kernel would hold thirty
 // vector registers).
+template <class R>
 struct DirectC {
-  SwR<float> lj, co;
+  SwR<R> lj, co;
   int ljkind, cokind;
   // membership radius^2, guard band; with one cutoff a candidate below in2 is a
   // member and one from in2 to near2 a boundary pair (rounded outwards: a pair
   // that is in doubt is re-tested)
-  float rmax2, guard, in2, near2;
-  float pa, ke, a2pi, csf;        // 0.3275911 alpha, -alpha^2 log2(e), 2 alpha/sqrt(pi), 1-4 scaling
-  float prune_r2;
-  float hi[3], lo[3], inv[3];     // box edges (see PairParams::Lhi) and their reciprocals
+  R rmax2, guard, in2, near2;
+  // 0.3275911 alpha, -alpha^2 (times log2(e) in FP32, whose exponential is the
+  // hardware's 2^x), 2 alpha/sqrt(pi), 1-4 scaling
+  R pa, ke, a2pi, csf;
+  R prune_r2;
+  R hi[3], lo[3], inv[3];  // box edges (see PairParams::Lhi) and their reciprocals
   // image k of a difference: d - k (hi + lo), hi exact
-  __device__ float image(float d, int ax) const {
-    const float k = rintf(d * inv[ax]);
+  __device__ R image(R d, int ax) const {
+    const R k = rint(d * inv[ax]);
     return (d - k * hi[ax]) - k * lo[ax];
   }
 };
 
 struct PairParams {
-  DirectC dc;
+  DirectC<float> dc;
+  DirectC<double> dd;
   Box box;
   SwitchC lj, co;
   double rc2max;     // membership radius^2 (max of the two cutoffs)
@@ -104,6 +129,9 @@ struct PairParams {
   // pair inside it, which no later pass before the next build can need
   double prune_r2;
 };
+
+__host__ __device__ inline const DirectC<float> &direct_of(const PairParams &pp, float) { return pp.dc; }
+__host__ __device__ inline const DirectC<double> &direct_of(const PairParams &pp, double) { return pp.dd; }
 
 // Sorted coordinates are stored relative to the origin of their supercluster
 // (the position of its first atom rounded to a multiple of kOriginQuantum),

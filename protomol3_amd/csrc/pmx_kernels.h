@@ -1102,10 +1102,9 @@ __device__ inline int excl_class(const int *__restrict__ eptr, const int2 *__res
 // Run schedule: the list entries of all superclusters, in supercluster
 // order, are cut into nruns contiguous runs of equal estimated work (the
 // work estimates of k_build_list: per supercluster, and as an inclusive
-// prefix over its entries); nruns, a multiple of min_runs set by C, the
-// total, depends only on the list.  Run w starts in supercluster runs[w].x
-// at entry runs[w].y (even: runs hold whole pair-kernel groups), where the
-// global work prefix first exceeds b_w = floor(w C / nruns), and ends where
+// prefix over its entries); nruns, a multiple of cut.min_runs set by C, the
+// total, or fewer (RunCut), depends only on the list.  Run w starts in supercluster runs[w].x
+// at entry runs[w].y, where the global work prefix first exceeds b_w = floor(w C / nruns), and ends where
 // run w + 1 starts; runs[nruns] is the end of the last supercluster with
 // entries.  The tile of run w in supercluster S, which may be empty at the
 // run's end, is number w + S: numbers rise by one from tile to tile, also from a
@@ -1118,7 +1117,7 @@ __device__ inline int excl_class(const int *__restrict__ eptr, const int2 *__res
 constexpr int kRunsBlock = 1024;
 __device__ __forceinline__ void runs_body(const int bid_, const int nbk_, int nsuper, const int *__restrict__ count,
                                           const int *__restrict__ cost, const int *__restrict__ ecost, int cap,
-                                          int min_runs, long long min_run_cost, int2 *__restrict__ runs,
+                                          RunCut cut, int2 *__restrict__ runs,
                                           int *__restrict__ ntiles) {
   constexpr int NW = kRunsBlock / kWave;
   __shared__ long long s_c[2][NW];
@@ -1148,14 +1147,14 @@ __device__ __forceinline__ void runs_body(const int bid_, const int nbk_, int ns
     C += s_c[1][k];
     last = max(last, s_last[k]);
   }
+  const int min_runs = cut.min_runs;
   const long long per = (long long)min_runs * kRunCost;
   const long long k = (C + per - 1) / per;
   int nruns = min_runs * (int)(k < 1 ? 1 : (k > kMaxRuns / min_runs ? kMaxRuns / min_runs : k));
-  if (min_run_cost > 0) {
-    // runs of at least min_run_cost units, in whole waves' worth of 64 runs:
-    // a small list's runs would otherwise hold an entry or two each, and the
-    // wave would spend its time on the i-force flush at every tile end
-    const long long r = (C + min_run_cost - 1) / min_run_cost;
+  {
+    // whole waves' worth of 64 runs of at least cut.least units
+    long long r = (C + cut.least - 1) / cut.least;
+    if (r > cut.few) r = max((long long)cut.few, (C + cut.least_many - 1) / cut.least_many);
     nruns = (int)min((long long)nruns, max(64ll, (r + 63) / 64 * 64));
   }
   if (bid_ == 0) {
@@ -1202,7 +1201,7 @@ __device__ __forceinline__ void runs_body(const int bid_, const int nbk_, int ns
         carry = __shfl(rb, kWave - 1);
         // runs w in [1, nruns) with lo <= floor(w C / nruns) < hi
         if (e < n)
-          for (int w = max(ra, 1); w < rb; ++w) runs[w] = make_int2(S, e & ~1);
+          for (int w = max(ra, 1); w < rb; ++w) runs[w] = make_int2(S, e);
       }
     }
     base += cost[S];
@@ -1211,9 +1210,9 @@ __device__ __forceinline__ void runs_body(const int bid_, const int nbk_, int ns
 
 static __global__ void __launch_bounds__(kRunsBlock) k_runs(int nsuper, const int *__restrict__ count,
                                                             const int *__restrict__ cost,
-                                                            const int *__restrict__ ecost, int cap, int min_runs,
+                                                            const int *__restrict__ ecost, int cap, RunCut cut,
                                                             int2 *__restrict__ runs, int *__restrict__ ntiles) {
-  runs_body(blockIdx.x, gridDim.x, nsuper, count, cost, ecost, cap, min_runs, 0, runs, ntiles);
+  runs_body(blockIdx.x, gridDim.x, nsuper, count, cost, ecost, cap, cut, runs, ntiles);
 }
 
 // ---------------------------------------------------------------------------
@@ -1232,11 +1231,46 @@ static __global__ void __launch_bounds__(kRunsBlock) k_runs(int nsuper, const in
 // operation order on the original coordinates before evaluating it.
 
 __device__ inline float fast_rsqrt(float x) { return __builtin_amdgcn_rsqf(x); }
-__device__ inline double fast_rsqrt(double x) { return 1.0 / sqrt(x); }
+// FP64: the unit's estimate (about 23 bits) and one step of third order, the
+// rounding of x y included.  Errors over 4 M arguments from 2^-8 to 2^8, in
+// units of the last place (1 / sqrt(x), 1 / x and exp in brackets): 0.5005
+// (1.4907), fast_rcp 0.5000 (0.5000), fast_exp 0.880 (0.879).  With the three
+// 26,000 atoms took 221 -> 210 us a launch, 93,000 with cutoffs 375 -> 364.
+__device__ inline double fast_rsqrt(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double h = x * y, l = fma(x, y, -h);
+  const double e = fma(-l, y, fma(-h, y, 1.0));
+  const double r = fma(y * e, fma(0.375, e, 0.5), y);
+  return x > 0.0 ? r : y;  // (coincident atoms: infinite, as before)
+}
 __device__ inline float fast_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
-__device__ inline double fast_rcp(double x) { return 1.0 / x; }
+__device__ inline double fast_rcp(double x) {  // 0 < x < infinity, normal
+  const double y = __builtin_amdgcn_rcp(x), e = fma(-x, y, 1.0);
+  return fma(y, fma(e, e, e), y);
+}
 __device__ inline float fast_exp(float x) { return __expf(x); }
-__device__ inline double fast_exp(double x) { return exp(x); }
+// x <= 0: x = n ln 2 + r (Cody and Waite's reduction), the Taylor series of
+// e^r to r^13 (|r| <= 0.35: the rest is below 5e-18), scaled by 2^n.
+__device__ inline double fast_exp(double x) {
+  const double n = rint(x * 1.4426950408889634);
+  double r = fma(n, -0x1.62e42fefa39efp-1, x);
+  r = fma(n, -0x1.abc9e3b39803fp-56, r);
+  double p = 1.0 / 6227020800.0;
+  p = fma(p, r, 1.0 / 479001600.0);
+  p = fma(p, r, 1.0 / 39916800.0);
+  p = fma(p, r, 1.0 / 3628800.0);
+  p = fma(p, r, 1.0 / 362880.0);
+  p = fma(p, r, 1.0 / 40320.0);
+  p = fma(p, r, 1.0 / 5040.0);
+  p = fma(p, r, 1.0 / 720.0);
+  p = fma(p, r, 1.0 / 120.0);
+  p = fma(p, r, 1.0 / 24.0);
+  p = fma(p, r, 1.0 / 6.0);
+  p = fma(p, r, 0.5);
+  p = fma(p, r, 1.0);
+  p = fma(p, r, 1.0);
+  return ldexp(p, (int)n);
+}
 __device__ inline float fast_rint(float x) { return rintf(x); }
 __device__ inline double fast_rint(double x) { return rint(x); }
 
@@ -1355,10 +1389,15 @@ __device__ inline float group8_sum(float v) {
   v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xF, 0xF, true));
   return v;
 }
+template <int CTRL>
+__device__ inline double dpp_of(double v) {
+  return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xF, 0xF, true),
+                          __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xF, 0xF, true));
+}
 __device__ inline double group8_sum(double v) {
-  v += __shfl_xor(v, 1);
-  v += __shfl_xor(v, 2);
-  v += __shfl_xor(v, 4);
+  v += dpp_of<0xB1>(v);
+  v += dpp_of<0x4E>(v);
+  v += dpp_of<0x141>(v);
   return v;
 }
 struct PairOut {
@@ -1405,47 +1444,11 @@ struct RunWalk {
   }
 };
 
-// Queue entry of the compacted pair kernel: one in-cutoff pair awaiting its
-// force.  info packs its force slot (bits 0..9: entry of the group, i-cluster
-// and lane, kGroup * 8 * 64 slots), MODIFIED (bit 10), the i-atom of the
-// supercluster (bits 11..16) and the group's j-atom (bits 17..20); the
-// evaluating lane reads the atoms' charges and types from LDS.
-template <class R>
-struct PairQ {
-  R r2;
-  int info;
-};
-constexpr int kSlotBits = 10;
 // r^2 given to an excluded candidate pair: beyond every cutoff, band and
 // list radius
 template <class R>
 constexpr R kFarR2 = (R)1e30;
 constexpr int kPairPlain = 0, kPairPrune = 1, kPairStats = 2;  // k_pair MODE
-
-// Charge and LJ type (clamped to 0 for padding) of a j-atom of the group.
-template <class R>
-struct JAtom {
-  R q;
-  int ty;
-};
-
-constexpr int kGroup = 2;    // list entries whose pairs share one queue flush
-constexpr int kQueue = 128;  // queue ring per wave (holds < 64 + 64 pairs)
-static_assert(kGroup == 2, "runs are cut at even entries (k_runs_cut)");
-
-// Wave-private LDS area of the pair kernel: the force slots of a group and
-// the queue; at a segment end, when both are empty, it holds the transpose of
-// one component of the i-force partial sums (8 values per lane).  (Kept
-// small: an FFT block of the PME chain must fit on a CU beside the pair
-// kernel's blocks.)
-template <class R>
-struct PairArea {
-  static constexpr int kSlotBytes = (int)sizeof(R) * kGroup * 8 * kWave;
-  static constexpr int kQueueBytes = (int)sizeof(PairQ<R>) * kQueue;
-  static constexpr int kTransBytes = (int)sizeof(R) * 8 * kWave;
-  static constexpr int kBytes =
-      kSlotBytes + kQueueBytes > kTransBytes ? kSlotBytes + kQueueBytes : kTransBytes;
-};
 
 // Fixed-point (mixed form) or FP64 sums of a wave's own i-atom forces and of
 // its pair energies.
@@ -1485,460 +1488,70 @@ struct EdgesR {
   }
 };
 
-// Minimum-image difference j - i in the kernel's arithmetic type.  Sorted
-// coordinates are relative to supercluster origins; xj has already been
-// moved by the entry offset (origin of j's supercluster - origin of i's,
-// plus the entry's image shift unless the entry needs the per-pair image,
-// per_pair, wave-uniform).  Phase A and phase C of k_pair call it with the
-// same operands.
-template <class R, class R4>
-__device__ inline void pair_delta(const R4 &xi, const R4 &xj, const EdgesR<R> &E, int per_pair, R &dx, R &dy,
-                                  R &dz) {
-  dx = xj.x - xi.x;
-  dy = xj.y - xi.y;
-  dz = xj.z - xi.z;
-  if (per_pair) {
-    dx = E.image(dx, 0);
-    dy = E.image(dy, 1);
-    dz = E.image(dz, 2);
-  }
-}
-
-// Cluster-pair kernel with compaction.  For a group of kGroup list entries:
-//   A. every candidate lane (i = 8c+ti of the supercluster, j = lane tj of
-//      the entry's j-cluster) computes r^2 and its membership; members are
-//      appended to a per-wave LDS queue (ballot + mbcnt), and every full
-//      64-pair batch of the queue is evaluated at once, all lanes busy;
-//   B. the last partial batch is evaluated; each pair's scalar force lands in
-//      its slot of an LDS array (zero for non-members);
-//   C. the candidate lanes read their slot and accumulate F = f d into the
-//      i-forces (registers) and j-forces (summed over the 8 i-lanes with DPP,
-//      one fixed-point atomic add per j-atom component and entry).
-// Only phase B does the expensive math (rsqrt, exp, erfc polynomial,
-// switches), on members only, which are about a quarter of the candidates.
+// Cluster-pair kernel.  Every lane of a cluster pair (i = 8c+ti of the
+// supercluster, j = lane tj of the entry's j-cluster) computes r^2 and its
+// membership; where any lane is a member all are evaluated and the others'
+// results selected away: no queue, no force slots.  A tile's i-atoms sit in
+// LDS, its i-forces in registers, the constants in scalar registers; the
+// j-forces are summed over the 8 i-lanes with DPP and added once per entry.
 // Deterministic sums: a tile (a run's part of one supercluster's list) is the
-// same whichever wave takes it, and at its end the i-force partial sums are
-// transposed through LDS, lane 8 c + ti sums its i-atom's eight partials in
-// a fixed order and adds the sum to the force array in fixed point; the
-// tile's FP32 pair-energy sums go to fixed point too.  So the mixed form's forces and energies do not depend
-// on the schedule, the grid or the device.
+// same whichever wave takes it, and at its end lane 8 c + ti sums its i-atom's
+// eight partials in a fixed order and adds the sum to the force array, in
+// fixed point in the mixed form, whose FP32 pair energies of a tile go to
+// fixed point too.  So the mixed form's forces and energies do not depend on
+// the schedule, the grid or the device.
 //
 // MODE kPairPrune (the first pass after a list build): cluster pairs without
 // a candidate pair inside the list radius are dropped from the entries'
 // masks (through entries_w, which aliases entries; each entry is read and
 // written by the one wave that takes it).  MODE kPairStats: the pass also
 // counts the in-cutoff pairs and sums their hashes.
-template <bool MIXED, int COUL, int LJSW, int CSW, bool BIGLJ, int MODE>
-__device__ __forceinline__ void pair_body(const int bid_, const int nbk_, PairParams pp, int dynamic,
-    const int2 *__restrict__ runs, const int *__restrict__ ntiles_p, const int *__restrict__ count,
-    int *__restrict__ tile_counter, const int4 *__restrict__ entries, int4 *entries_w, int cap,
-    const unsigned short *__restrict__ masks,
-    const typename Real4<typename std::conditional<MIXED, float, double>::type>::type *__restrict__ xs,
-    const float4 *__restrict__ sorg, const int *__restrict__ ts, const int *__restrict__ perm,
-    const double *__restrict__ ljtab,
-    const typename Real4<typename std::conditional<MIXED, float, double>::type>::type *__restrict__ ljt,
-    typename AccT<MIXED>::type *__restrict__ facc, PairOut out) {
-  using R = typename std::conditional<MIXED, float, double>::type;
-  using R4 = typename Real4<R>::type;
-  using Acc = AccT<MIXED>;
-  using WA = WaveAcc<MIXED>;
-  using AT = typename WA::T;
-  constexpr int W = kPairBlock / kWave;
-  constexpr bool PRUNE = MODE == kPairPrune, STATS = MODE == kPairStats;
-  __shared__ R4 s_i[W][kSuperSize];
-  __shared__ int s_ty[W][kSuperSize];
-  __shared__ R4 s_lj[kMaxTypes * kMaxTypes];  // {A, B, A14, B14}
-  __shared__ __align__(16) unsigned char s_area[W][PairArea<R>::kBytes];
-  __shared__ JAtom<R> s_j[W][kGroup * kClusterSize];
-
-  const int nt = pp.ntypes;
-  // up to kMaxTypes LJ types the table sits in LDS; beyond that (BIGLJ) the
-  // typed copy ljt is read through the caches
-  for (int k = threadIdx.x; !BIGLJ && k < nt * nt; k += blockDim.x) {
-    R4 v;
-    v.x = (R)ljtab[4 * k];
-    v.y = (R)ljtab[4 * k + 1];
-    v.z = (R)ljtab[4 * k + 2];
-    v.w = (R)ljtab[4 * k + 3];
-    s_lj[k] = v;
-  }
-  __syncthreads();
-
-  const int lane = threadIdx.x & 63;
-  const int wv = threadIdx.x >> 6;
-  const int ti = lane & 7, tj = lane >> 3;
-  // queue info of this lane's pairs: force slot (bits 0..9, with the group
-  // entry and i-cluster added), MODIFIED (bit 10), i-atom c * 8 + ti (bits
-  // 11..16, c added), j-atom g * 8 + tj (bits 17..20, g added)
-  const int info_lane = lane | (ti << 11) | (tj << 17);
-  EdgesR<R> E;
-  E.load(pp);
-  SwR<R> sl, sc;
-  sl.load(pp.lj);
-  sc.load(pp.co);
-  const R guard = (R)pp.guard;
-  const R alpha = (R)pp.alpha, a2pi = (R)pp.a2pi, csf = (R)pp.csf;
-  const bool one_cut = sl.rc2 == sc.rc2;  // one guard band serves both cutoffs
-  const bool same_cut = LJSW == SW_NONE || COUL == COUL_NONE || one_cut;
-  // membership: r^2 within the larger cutoff of the kinds present
-  const R rmax2 = LJSW == SW_NONE ? sc.rc2 : (COUL == COUL_NONE ? sl.rc2 : (sl.rc2 > sc.rc2 ? sl.rc2 : sc.rc2));
-  const R prune_r2 = (R)pp.prune_r2;
-  // the boundary-pair sums are filled after this kernel (same stream)
-  if (bid_ == 0 && threadIdx.x < 4) out.border_acc[threadIdx.x] = 0ull;
-  R4 *const si = s_i[wv];
-  R *const fr_slot = reinterpret_cast<R *>(s_area[wv]);
-  PairQ<R> *const q = reinterpret_cast<PairQ<R> *>(s_area[wv] + PairArea<R>::kSlotBytes);
-  R *const tr = reinterpret_cast<R *>(s_area[wv]);
-
-  // Runs (the grid holds the waves that fit on the device at once): wave w
-  // takes the contiguous runs [w nruns / nwaves, (w + 1) nruns / nwaves)
-  // (dynamic == 0: consecutive tiles often share a supercluster, whose
-  // i-atoms then stay loaded), or
-  // run w and then runs in order from a device-wide counter (dynamic == 1).
-  // A tile is the part of a run in one supercluster.  Which wave takes a run
-  // changes no result.
-  const int nwaves = nbk_ * W;
-  const int gw = bid_ * W + wv;
-  const int nruns = ntiles_p[2];
-  const int r0 = dynamic ? gw : (int)((long long)gw * nruns / nwaves);
-  const int r1 = dynamic ? min(gw + 1, nruns) : (int)((long long)(gw + 1) * nruns / nwaves);
-  RunWalk walk(r0, r1);
-  int curS = -1;      // supercluster whose i-atoms are loaded
-  bool ireal = false;  // slot `lane` of curS holds an atom
-  while (true) {
-    if (walk.run_done()) {
-      if (walk.w >= walk.wstop) {
-        if (!dynamic) break;
-        int rn = 0;
-        if (lane == 0) rn = nwaves + atomicAdd(tile_counter, 1);
-        const int r = __builtin_amdgcn_readfirstlane(__shfl(rn, 0));
-        if (r >= nruns) break;
-        walk = RunWalk(r, r + 1);
-      }
-      walk.next_run(runs);
-    }
-    const int S = walk.S, t = walk.t, e0 = walk.e0, e1 = walk.tile_end(count);
-    walk.next_tile();
-    if (e0 >= e1) {
-      if (lane == 0) out.clear(t, STATS);
-      continue;
-    }
-    const float4 oS = sorg[S];
-    if (S != curS) {
-      curS = S;
-      si[lane] = xs[S * kSuperSize + lane];
-      const int v = ts[S * kSuperSize + lane];
-      ireal = v >= 0;
-      s_ty[wv][lane] = (v < 0 ? 0 : v) * nt;  // row of the LJ table
-      __builtin_amdgcn_wave_barrier();
-    }
-
-    R fi[8][3];
-#pragma unroll
-    for (int c = 0; c < 8; ++c) fi[c][0] = fi[c][1] = fi[c][2] = (R)0;
-    R elT = 0, ecT = 0;  // this lane's pair energies over the tile
-    int npair = 0;
-    unsigned long long hsum = 0;
-    int qhead = 0, qtail = 0;  // wave-uniform queue positions
-
-    // Evaluates queue pairs [qhead, qhead + cnt) with lane l on pair qhead + l.
-    // A queued pair passed the membership test: it is in range of at least
-    // one of the two cutoffs, and not within the guard band of either.
-    // `inside` is std::true_type when every queued pair is inside the cutoff
-    // of each kind present (one cutoff for both kinds), so no per-pair test
-    // or select is needed.
-    auto eval_batch = [&](auto inside, int cnt, R &qel, R &qec) {
-      __builtin_amdgcn_wave_barrier();
-      if (lane < cnt) {
-        const PairQ<R> e = q[(qhead + lane) & (kQueue - 1)];
-        const int slot = e.info & ((1 << kSlotBits) - 1);
-        const bool mod = (e.info >> kSlotBits) & 1;
-        const int ia = (e.info >> 11) & 63;  // c * 8 + ti
-        const int ja = (e.info >> 17) & 15;  // g * 8 + tj
-        const JAtom<R> jd = s_j[wv][ja];
-        R qq = si[ia].w * jd.q;
-        if (mod) qq *= csf;
-        const bool il = LJSW != SW_NONE && (decltype(inside)::value || e.r2 <= sl.rc2);
-        const bool ic = COUL != COUL_NONE && (decltype(inside)::value || e.r2 <= sc.rc2);
-        R A = 0, B = 0;
-        if (LJSW != SW_NONE) {
-          const int li = s_ty[wv][ia] + jd.ty;
-          const R4 lj = BIGLJ ? ljt[li] : s_lj[li];
-          A = mod ? lj.z : lj.x;
-          B = mod ? lj.w : lj.y;
-        }
-        R e1, e2, f;
-        pair_eval<COUL, LJSW, CSW, R>(pp, sl, sc, alpha, a2pi, csf, e.r2, qq, A, B, il, ic, e1, e2, f);
-        qel += e1;
-        qec += e2;
-        fr_slot[slot] = f;
-      }
-      qhead += cnt;
-    };
-
-    // Tile end (queue empty, slots free): the tile's FP32 i-force partial
-    // sums go through LDS one component at a time so that lane 8 c + ti sums
-    // the eight partials of its i-atom (from lanes (ti, tj'), tj' = 0..7 in
-    // order) and adds the sum, in fixed point, to the atom's force.
-    auto flush = [&]() {
-      const int sidx = S * kSuperSize + lane;
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int c = 0; c < 8; ++c) tr[lane * 8 + c] = fi[c][k];
-        __builtin_amdgcn_wave_barrier();
-        R sk = 0;
-#pragma unroll
-        for (int tq = 0; tq < 8; ++tq) sk += tr[(8 * tq + ti) * 8 + tj];
-        if (ireal) WA::add(&facc[3 * sidx + k], WA::of(sk));
-      }
-      __builtin_amdgcn_wave_barrier();
-    };
-
-    for (int eg = e0; eg < e1; eg += kGroup) {
-      const int ng = e1 - eg < kGroup ? e1 - eg : kGroup;
-      int cjv[kGroup], emv[kGroup], mov[kGroup], shv[kGroup], tyj0[kGroup];
-      unsigned mbv[kGroup];  // this lane's exclusion bits (candidate per i-cluster, MODIFIED << 8)
-      R4 xj[kGroup];
-#pragma unroll
-      for (int g = 0; g < kGroup; ++g) {
-        int4 ent = make_int4(0, 0, -1, 0);
-        if (g < ng) ent = entries[(size_t)S * cap + eg + g];
-        cjv[g] = __builtin_amdgcn_readfirstlane(ent.x);
-        emv[g] = __builtin_amdgcn_readfirstlane(ent.y) & 0xff;
-        mov[g] = __builtin_amdgcn_readfirstlane(ent.z);
-        shv[g] = __builtin_amdgcn_readfirstlane(ent.w);
-        const int sj = cjv[g] * kClusterSize + tj;
-        xj[g] = xs[sj];
-        {
-          // j-cluster into the frame of S: origin difference (exact) plus
-          // the entry's image shift (hi part exact, lo part rounded once)
-          const float4 oJ = sorg[cjv[g] / (kSuperSize / kClusterSize)];
-          R ox = (R)(oJ.x - oS.x), oy = (R)(oJ.y - oS.y), oz = (R)(oJ.z - oS.z);
-          if (!(shv[g] & kShiftPerPair)) {
-            const R sx = (R)((shv[g] & 3) - 1), sy = (R)(((shv[g] >> 2) & 3) - 1), sz = (R)(((shv[g] >> 4) & 3) - 1);
-            ox = (ox + sx * E.hi[0]) + sx * E.lo[0];
-            oy = (oy + sy * E.hi[1]) + sy * E.lo[1];
-            oz = (oz + sz * E.hi[2]) + sz * E.lo[2];
-          }
-          xj[g].x += ox;
-          xj[g].y += oy;
-          xj[g].z += oz;
-        }
-        tyj0[g] = ts[sj];
-        mbv[g] = mov[g] >= 0 ? (unsigned)masks[(size_t)mov[g] * kWave + lane] : 0xffu;
-        if (ti == 0) s_j[wv][g * kClusterSize + tj] = JAtom<R>{xj[g].w, tyj0[g] < 0 ? 0 : tyj0[g]};
-      }
-      // every force slot of the group starts at zero (phase B fills the
-      // members' slots, phase C reads the slots of the entries' masks)
-#pragma unroll
-      for (int k = 0; k < kGroup * 8 / 4; ++k) {
-        R4 z;
-        z.x = z.y = z.z = z.w = (R)0;
-        reinterpret_cast<R4 *>(fr_slot)[k * kWave + lane] = z;
-      }
-      __builtin_amdgcn_wave_barrier();
-
-      // ---- phase A: membership, queue, full batches
-      R qel = 0, qec = 0;
-      unsigned used = 0;  // bit g * 8 + c: the cluster pair has a member
-      unsigned kept = 0;  // bit g * 8 + c: (prune pass) a candidate pair within the list radius
-      // Candidate scan of entry g, specialised on one cutoff for both kinds
-      // (SAME) and on the entry carrying an exclusion mask (MASKED), so that
-      // each membership flag is a single compare whose ballot is its lane
-      // mask.  An excluded candidate's r^2 becomes kFarR2, which fails every
-      // range and band test.  The flags are those of the plain form: with one
-      // cutoff, "outside the band and within range" is d < -guard.
-      auto scan = [&](auto same, auto masked, const int g) {
-        constexpr bool SAME = decltype(same)::value, MASKED = decltype(masked)::value;
-        const int sj = cjv[g] * kClusterSize + tj;
-        unsigned mrem = emv[g];
-        while (mrem) {
-          const int c = __builtin_ctz(mrem);
-          mrem &= mrem - 1;
-          const R4 xi = si[c * 8 + ti];
-          R dx, dy, dz;
-          pair_delta<R, R4>(xi, xj[g], E, shv[g] & kShiftPerPair, dx, dy, dz);
-          R r2 = dx * dx + dy * dy + dz * dz;
-          if (MASKED && !(mbv[g] & (1u << c))) r2 = kFarR2<R>;
-          // a pair within the guard band of a cutoff is left to the FP64
-          // boundary pass; a member is in range of a cutoff and outside
-          // every band
-          bool border, in;
-          if (SAME) {
-            const R d = r2 - rmax2;
-            border = fabs(d) <= guard;
-            in = d < -guard;
-          } else {
-            border = fmin(fabs(r2 - sl.rc2), fabs(r2 - sc.rc2)) <= guard;
-            in = (border ? kFarR2<R> : r2) <= rmax2;
-          }
-          const unsigned long long bm = __builtin_amdgcn_ballot_w64(in);
-          if (PRUNE && __builtin_amdgcn_ballot_w64(r2 <= prune_r2)) kept |= 1u << (g * 8 + c);
-          if (__builtin_amdgcn_ballot_w64(border) && border) {
-            const int b = atomicAdd(out.nborder, 1);
-            if (b < out.maxborder)
-              out.border[b] = make_int2(S * kSuperSize + c * 8 + ti, sj);
-            else
-              atomicExch(out.overflow, 1);
-          }
-          if (STATS && in) {
-            const int ai = perm[S * kSuperSize + c * 8 + ti], aj = perm[sj];
-            ++npair;
-            hsum += pair_hash(ai < aj ? ai : aj, ai < aj ? aj : ai);
-          }
-          if (bm) {
-            used |= 1u << (g * 8 + c);
-            if (in) {
-              // queue position: qtail + members in lower lanes
-              const unsigned pos = __builtin_amdgcn_mbcnt_hi((unsigned)(bm >> 32),
-                                                             __builtin_amdgcn_mbcnt_lo((unsigned)bm, (unsigned)qtail));
-              const int modified = MASKED ? (int)((mbv[g] >> (8 + c)) & 1u) : 0;
-              PairQ<R> e;
-              e.r2 = r2;
-              e.info = info_lane | (((g * 8 + c) << 6) | (c << 14) | (g << 20)) | (modified << kSlotBits);
-              q[pos & (kQueue - 1)] = e;
-            }
-            qtail += __popcll(bm);
-            while (qtail - qhead >= kWave) eval_batch(same, kWave, qel, qec);
-          }
-        }
-      };
-#pragma unroll
-      for (int g = 0; g < kGroup; ++g) {
-        if (same_cut) {
-          if (mov[g] >= 0)
-            scan(std::true_type{}, std::true_type{}, g);
-          else
-            scan(std::true_type{}, std::false_type{}, g);
-        } else {
-          if (mov[g] >= 0)
-            scan(std::false_type{}, std::true_type{}, g);
-          else
-            scan(std::false_type{}, std::false_type{}, g);
-        }
-      }
-      // prune pass: cluster pairs without a candidate pair inside the list
-      // radius cannot have a member before the next list build (every atom
-      // stays within half the skin of its build position); later passes skip
-      // them.  They have no member now either, so no result changes.
-      if (PRUNE) {
-#pragma unroll
-        for (int g = 0; g < kGroup; ++g) {
-          const int km = (kept >> (g * 8)) & 0xff;
-          if (g < ng && lane == 0 && km != emv[g]) entries_w[(size_t)S * cap + eg + g].y = km;
-        }
-      }
-      // ---- phase B: the rest of the queue
-      if (qtail > qhead) {
-        if (same_cut)
-          eval_batch(std::true_type{}, qtail - qhead, qel, qec);
-        else
-          eval_batch(std::false_type{}, qtail - qhead, qel, qec);
-      }
-      elT += qel;
-      ecT += qec;
-      __builtin_amdgcn_wave_barrier();
-
-      // ---- phase C: forces from the slots
-#pragma unroll
-      for (int g = 0; g < kGroup; ++g) {
-        if (g >= ng) break;
-        // cluster pairs without members add nothing (their slots are zero)
-        const int em = (used >> (g * 8)) & 0xff;
-        if (em == 0) continue;
-        const int sj = cjv[g] * kClusterSize + tj;
-        R fj0 = 0, fj1 = 0, fj2 = 0;
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-          if (!(em & (1 << c))) continue;
-          const R4 xi = si[c * 8 + ti];
-          R dx, dy, dz;
-          pair_delta<R, R4>(xi, xj[g], E, shv[g] & kShiftPerPair, dx, dy, dz);
-          const R f = fr_slot[(g * 8 + c) * kWave + lane];
-          const R fx = dx * f, fy = dy * f, fz = dz * f;
-          fi[c][0] -= fx;
-          fi[c][1] -= fy;
-          fi[c][2] -= fz;
-          fj0 += fx;
-          fj1 += fy;
-          fj2 += fz;
-        }
-        fj0 = group8_sum(fj0);
-        fj1 = group8_sum(fj1);
-        fj2 = group8_sum(fj2);
-        if (ti < 3 && tyj0[g] >= 0) {
-          const R v = ti == 0 ? fj0 : (ti == 1 ? fj1 : fj2);
-          Acc::add(&facc[3 * sj + ti], v);
-        }
-      }
-      __builtin_amdgcn_wave_barrier();
-    }
-    flush();
-    const AT eljA = wave_sum(WA::of(elT));
-    const AT ecoA = wave_sum(WA::of(ecT));
-    long long np = 0;
-    if (STATS) {
-      np = wave_sum((long long)npair);
-      hsum = wave_sum(hsum);
-    }
-    if (lane == 0) {
-      out.energy[2 * t] = WA::energy_bits(ecoA);
-      out.energy[2 * t + 1] = WA::energy_bits(eljA);
-      if (STATS) {
-        out.npairs[t] = np;
-        out.hash[t] = hsum;
-      }
-    }
-    __builtin_amdgcn_wave_barrier();
-  }
-}
-
-// ---- mixed form: direct evaluation --------------------------------------
 //
-// The mixed kernel evaluates the member lanes of a cluster pair where they
-// stand: no queue, no force slots.  Its FP32 math is short (about 60 issue
-// slots a cluster pair), so packing members first (about two fifths of the
-// lanes) cost as much issue time as it saved, and LDS round trips and scalar
-// work on top; FP64 math is several times longer and keeps the queue
-// (pair_body).  i-atoms sit in LDS, i-forces in registers for a whole tile,
-// constants in scalar registers.  Bound by VALU issue.
-// One launch alone, before (the queue) and after, skin 1.5 / 1.0 / 1.2 A:
-// 26,000 atoms 78.8 -> 60.1 us (VALU instructions 29.0 -> 25.1 M, scalar 16.0
-// -> 6.5 M, LDS 3.0 -> 0.8 M), 9,400 atoms 31.0 -> 27.3, 1,000,000 atoms 1.63
-// -> 1.07 ms; unequal cutoffs, 46,000 atoms 126 -> 97 us.
-// 72 VGPRs and 8 KB of LDS a block would take six blocks per CU (55.7 us and
-// 0.93 ms alone), but then the PME passes beside it starve and a step takes
+// Bound by VALU issue.  Before, the member pairs (about two fifths of the lanes)
+// were packed into an LDS queue and evaluated in full batches, which cost as
+// much issue time as it saved, and LDS round trips and scalar work on top; in
+// FP64 its 59 KB of LDS a block also left two waves per SIMD.
+// One launch alone, before and after, skin 1.5 / 1.0 / 1.2 A.  Mixed: 26,000
+// atoms 78.8 -> 60.1 us (VALU instructions 29.0 -> 25.1 M, scalar 16.0 -> 6.5 M,
+// LDS 3.0 -> 0.8 M), 9,400 atoms 31.0 -> 27.3, 1,000,000 atoms 1.63 -> 1.07 ms;
+// unequal cutoffs, 46,000 atoms 126 -> 97 us.  FP64: 26,000 atoms
+// with PME 210 -> 109 us, 93,000 with cutoffs 364 -> 173; three blocks per CU
+// (151 VGPRs; at 128 the PME form spills 118), with cutoffs four.
+// Mixed, 72 VGPRs and 8 KB of LDS a block would take six blocks per CU (55.7 us
+// and 0.93 ms alone), but then the PME passes beside it starve and a step takes
 // longer (26,000 atoms 124 -> 136 us): four, which leave them half the
 // registers.
 
+// e^(-alpha^2 r^2) from DirectC::ke r^2.
+__device__ inline float gauss(float x) { return __builtin_amdgcn_exp2f(x); }
+__device__ inline double gauss(double x) { return fast_exp(x); }
+
 // Energies and scalar force (F = f d) of one member pair; il, ic: in range of
 // the LJ and the Coulomb cutoff.
-template <int COUL, int LJSW, int CSW>
-__device__ __forceinline__ void direct_eval(const DirectC &k, float r2, float qq, float A, float B, float &elj,
-                                            float &eco, float &flj, float &fco) {
-  const float rinv = fast_rsqrt(r2);
-  const float rinv2 = rinv * rinv;
+template <int COUL, int LJSW, int CSW, class R>
+__device__ __forceinline__ void direct_eval(const DirectC<R> &k, R r2, R qq, R A, R B, R &elj, R &eco, R &flj,
+                                            R &fco) {
+  const R rinv = fast_rsqrt(r2);
+  const R rinv2 = rinv * rinv;
   if (LJSW != SW_NONE) {
     // LennardJonesForce.h:28-60
-    const float r6 = rinv2 * rinv2 * rinv2;
-    const float t = A * r6 - B;
-    float e = t * r6;                               // A r^-12 - B r^-6
-    float f = (A * r6 + t) * (r6 * (6.f * rinv2));  // (12 A r^-12 - 6 B r^-6) / r^2
+    const R r6 = rinv2 * rinv2 * rinv2;
+    const R t = A * r6 - B;
+    R e = t * r6;                               // A r^-12 - B r^-6
+    R f = (A * r6 + t) * (r6 * ((R)6 * rinv2));  // (12 A r^-12 - 6 B r^-6) / r^2
     if (LJSW == SW_C2) {
       // C2SwitchingFunction.h:42-53: 1 below r_on, the polynomial up to rc
       const bool on = r2 >= k.lj.on2;
       if (__builtin_amdgcn_ballot_w64(on)) {
-        const float c2 = k.lj.rc2 - r2, c4 = c2 * (k.lj.s2 + 2.f * r2);
-        const float sv = k.lj.s1 * (c2 * c4);
-        const float fs = f * sv - e * (k.lj.s3 * (c2 * c2 - c4)), es = e * sv;
+        const R c2 = k.lj.rc2 - r2, c4 = c2 * (k.lj.s2 + (R)2 * r2);
+        const R sv = k.lj.s1 * (c2 * c4);
+        const R fs = f * sv - e * (k.lj.s3 * (c2 * c2 - c4)), es = e * sv;
         f = on ? fs : f;
         e = on ? es : e;
       }
     } else {
-      float sv, sd;
-      switch_val<LJSW, float>(k.ljkind, k.lj, r2, rinv, sv, sd);
+      R sv, sd;
+      switch_val<LJSW, R>(k.ljkind, k.lj, r2, rinv, sv, sd);
       f = f * sv - e * sd;
       e = e * sv;
     }
@@ -1946,23 +1559,23 @@ __device__ __forceinline__ void direct_eval(const DirectC &k, float r2, float qq
     elj = e;
   }
   if (COUL != COUL_NONE) {
-    float e, f;
+    R e, f;
     if (COUL == COUL_CUTOFF) {
       // CoulombForce.h:29-40
       e = qq * rinv;
       f = e * rinv2;
     } else {
       // NonbondedPMEwaldSystemForce.h:657-683 (poly5 form)
-      const float t = fast_rcp(1.f + k.pa * (r2 * rinv));
-      const float ex = qq * __builtin_amdgcn_exp2f(k.ke * r2);
-      const float p = t * (0.254829592f +
-                           t * (-0.284496736f + t * (1.421413741f + t * (-1.453152027f + t * 1.061405429f))));
+      const R t = fast_rcp((R)1 + k.pa * (r2 * rinv));
+      const R ex = qq * gauss(k.ke * r2);
+      const R p = t * ((R)0.254829592 +
+                           t * ((R)-0.284496736 + t * ((R)1.421413741 + t * ((R)-1.453152027 + t * (R)1.061405429))));
       e = p * ex * rinv;
       f = (e + k.a2pi * ex) * rinv2;
     }
     if constexpr (CSW != SW_CUTOFF) {
-      float sv, sd;
-      switch_val<CSW, float>(k.cokind, k.co, r2, rinv, sv, sd);
+      R sv, sd;
+      switch_val<CSW, R>(k.cokind, k.co, r2, rinv, sv, sd);
       f = f * sv - e * sd;
       e = e * sv;
     }
@@ -1987,37 +1600,63 @@ __device__ inline float swap8_sum(float a, float b, bool hi) {
   return keep + __uint_as_float((unsigned)__builtin_amdgcn_update_dpp(0, __float_as_int(give), 0x128, 0xF, 0xF, true));
 }
 
-template <int COUL, int LJSW, int CSW, bool BIGLJ, int MODE>
-__device__ __forceinline__ void pair_direct_body(
+__device__ inline double double_of(unsigned lo, unsigned hi) { return __hiloint2double((int)hi, (int)lo); }
+__device__ inline double swap32_sum(double a, double b) {
+  const auto l = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
+  const auto h = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
+  return double_of(l[0], h[0]) + double_of(l[1], h[1]);
+}
+__device__ inline double swap16_sum(double a, double b) {
+  const auto l = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(b), false, false);
+  const auto h = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(b), false, false);
+  return double_of(l[0], h[0]) + double_of(l[1], h[1]);
+}
+__device__ inline double swap8_sum(double a, double b, bool hi) {
+  const double keep = hi ? b : a, give = hi ? a : b;
+  return keep + double_of((unsigned)__builtin_amdgcn_update_dpp(0, __double2loint(give), 0x128, 0xF, 0xF, true),
+                          (unsigned)__builtin_amdgcn_update_dpp(0, __double2hiint(give), 0x128, 0xF, 0xF, true));
+}
+
+template <bool MIXED, int COUL, int LJSW, int CSW, bool BIGLJ, int MODE>
+__device__ __forceinline__ void pair_body(
     const int bid_, const int nbk_, const PairParams &pp, int dynamic, const int2 *__restrict__ runs,
     const int *__restrict__ ntiles_p, const int *__restrict__ count, int *__restrict__ tile_counter,
     const int4 *__restrict__ entries, int4 *entries_w, int cap, const unsigned short *__restrict__ masks,
-    const float4 *__restrict__ xs, const float4 *__restrict__ sorg, const int *__restrict__ ts,
-    const int *__restrict__ perm, const double *__restrict__ ljtab, const float4 *__restrict__ ljt,
-    unsigned long long *__restrict__ facc, PairOut out) {
-  using WA = WaveAcc<true>;
+    const typename Real4<typename std::conditional<MIXED, float, double>::type>::type *__restrict__ xs,
+    const float4 *__restrict__ sorg, const int *__restrict__ ts, const int *__restrict__ perm,
+    const double *__restrict__ ljtab,
+    const typename Real4<typename std::conditional<MIXED, float, double>::type>::type *__restrict__ ljt,
+    typename AccT<MIXED>::type *__restrict__ facc, PairOut out) {
+  using R = typename std::conditional<MIXED, float, double>::type;
+  using R2 = typename std::conditional<MIXED, float2, double2>::type;
+  using R4 = typename Real4<R>::type;
+  using WA = WaveAcc<MIXED>;
   constexpr int W = kPairBlock / kWave;
   constexpr bool PRUNE = MODE == kPairPrune, STATS = MODE == kPairStats;
   constexpr bool LJ = LJSW != SW_NONE;
   // {A, B} of the plain and of the 1-4 pairs
-  __shared__ float2 s_lj[2][kMaxTypes * kMaxTypes];
-  __shared__ float4 s_i[W][kSuperSize];  // the tile's i-atoms
+  __shared__ R2 s_lj[2][kMaxTypes * kMaxTypes];
+  __shared__ R4 s_i[W][kSuperSize];  // the tile's i-atoms
   const int nt = pp.ntypes;
   for (int k = threadIdx.x; LJ && !BIGLJ && k < nt * nt; k += blockDim.x) {
-    s_lj[0][k] = make_float2((float)ljtab[4 * k], (float)ljtab[4 * k + 1]);
-    s_lj[1][k] = make_float2((float)ljtab[4 * k + 2], (float)ljtab[4 * k + 3]);
+    s_lj[0][k] = R2{(R)ljtab[4 * k], (R)ljtab[4 * k + 1]};
+    s_lj[1][k] = R2{(R)ljtab[4 * k + 2], (R)ljtab[4 * k + 3]};
   }
   __syncthreads();
 
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int ti = lane & 7, tj = lane >> 3;
-  const DirectC &kc = pp.dc;
+  const DirectC<R> &kc = direct_of(pp, R());
   const bool same_cut = !LJ || COUL == COUL_NONE || kc.lj.rc2 == kc.co.rc2;
   // the boundary-pair sums are filled after this kernel (same stream)
   if (bid_ == 0 && threadIdx.x < 4) out.border_acc[threadIdx.x] = 0ull;
 
-  // Runs: see pair_body.
+  // Runs (the grid holds the waves that fit on the device at once): wave w
+  // takes the contiguous runs [w nruns / nwaves, (w + 1) nruns / nwaves)
+  // (dynamic == 0), or run w and then runs in order from a device-wide counter
+  // (dynamic == 1).  A tile is the part of a run in one supercluster.  Which
+  // wave takes a run changes no result.
   const int nwaves = nbk_ * W;
   const int gw = bid_ * W + wv;
   const int nruns = ntiles_p[2];
@@ -2051,10 +1690,10 @@ __device__ __forceinline__ void pair_direct_body(
 #pragma unroll
     for (int c = 0; LJ && !BIGLJ && c < 8; ++c)
       irow[c >> 2] |= (unsigned)(max(0, ts[S * kSuperSize + c * kClusterSize + ti]) * nt) << (8 * (c & 3));
-    float fi[8][3];
+    R fi[8][3];
 #pragma unroll
-    for (int c = 0; c < 8; ++c) fi[c][0] = fi[c][1] = fi[c][2] = 0.f;
-    float elT = 0.f, ecT = 0.f;  // this lane's pair energies over the tile
+    for (int c = 0; c < 8; ++c) fi[c][0] = fi[c][1] = fi[c][2] = (R)0;
+    R elT = 0, ecT = 0;  // this lane's pair energies over the tile
     int npair = 0;
     unsigned long long hsum = 0;
 
@@ -2077,7 +1716,7 @@ __device__ __forceinline__ void pair_direct_body(
       const int sj = ent.x * kClusterSize + tj;
       const unsigned em = ent.y & 0xff;
       const int sh = ent.w, masked = ent.z >= 0;
-      float4 xj = xs[sj];
+      R4 xj = xs[sj];
       const int tyj = ts[sj];
       const float4 oJ = sorg[ent.x / (kSuperSize / kClusterSize)];
       const unsigned mb = mask_of(ent);
@@ -2085,9 +1724,9 @@ __device__ __forceinline__ void pair_direct_body(
       // j-cluster into the frame of S: origin difference (exact) plus the
       // entry's image shift (hi part exact, lo part rounded once)
       {
-        float ox = oJ.x - oS.x, oy = oJ.y - oS.y, oz = oJ.z - oS.z;
+        R ox = (R)(oJ.x - oS.x), oy = (R)(oJ.y - oS.y), oz = (R)(oJ.z - oS.z);
         if (!(sh & kShiftPerPair) && sh != 21) {  // 21: no shift
-          const float sx = (float)((sh & 3) - 1), sy = (float)(((sh >> 2) & 3) - 1), sz = (float)(((sh >> 4) & 3) - 1);
+          const R sx = (R)((sh & 3) - 1), sy = (R)(((sh >> 2) & 3) - 1), sz = (R)(((sh >> 4) & 3) - 1);
           ox = (ox + sx * kc.hi[0]) + sx * kc.lo[0];
           oy = (oy + sy * kc.hi[1]) + sy * kc.lo[1];
           oz = (oz + sz * kc.hi[2]) + sz * kc.lo[2];
@@ -2098,7 +1737,7 @@ __device__ __forceinline__ void pair_direct_body(
       }
       const int tyc = max(0, tyj);
       if (LJ && !BIGLJ) asm volatile("" : "+v"(irow[0]), "+v"(irow[1]));  // unpacked where used, not ahead of the loop
-      float fj0 = 0.f, fj1 = 0.f, fj2 = 0.f;
+      R fj0 = 0, fj1 = 0, fj2 = 0;
       unsigned used = 0, kept = 0;  // cluster pairs with a member; with a candidate within the list radius
 
       // GENERAL: the entry carries an exclusion mask or takes the per-pair
@@ -2108,15 +1747,15 @@ __device__ __forceinline__ void pair_direct_body(
 #pragma unroll
         for (int c = 0; c < 8; ++c) {
           if (!(em & (1u << c))) continue;
-          const float4 xi = s_i[wv][c * kClusterSize + ti];
-          float dx = xj.x - xi.x, dy = xj.y - xi.y, dz = xj.z - xi.z;
+          const R4 xi = s_i[wv][c * kClusterSize + ti];
+          R dx = xj.x - xi.x, dy = xj.y - xi.y, dz = xj.z - xi.z;
           if (GENERAL && (sh & kShiftPerPair)) {
             dx = kc.image(dx, 0);
             dy = kc.image(dy, 1);
             dz = kc.image(dz, 2);
           }
-          float r2 = dx * dx + dy * dy + dz * dz;
-          if (GENERAL && !(mb & (1u << c))) r2 = kFarR2<float>;
+          R r2 = dx * dx + dy * dy + dz * dz;
+          if (GENERAL && !(mb & (1u << c))) r2 = kFarR2<R>;
           if (PRUNE && __builtin_amdgcn_ballot_w64(r2 <= kc.prune_r2)) kept |= 1u << c;
           const bool near = r2 <= kc.near2;
           const unsigned long long nm = __builtin_amdgcn_ballot_w64(near);
@@ -2129,7 +1768,7 @@ __device__ __forceinline__ void pair_direct_body(
             in = r2 < kc.in2;
             border = near && !in;
           } else {
-            const float d = fminf(fabsf(r2 - kc.lj.rc2), fabsf(r2 - kc.co.rc2));
+            const R d = fmin(fabs(r2 - kc.lj.rc2), fabs(r2 - kc.co.rc2));
             in = r2 <= kc.rmax2 && d > kc.guard;
             border = near && d <= kc.guard;
           }
@@ -2152,30 +1791,30 @@ __device__ __forceinline__ void pair_direct_body(
           }
           // lanes without a member are evaluated too and selected away
           const bool mod = GENERAL && ((mb >> (8 + c)) & 1u);
-          float A = 0.f, B = 0.f;
+          R A = 0, B = 0;
           if (LJ && BIGLJ) {
             const int tyi = max(0, ts[S * kSuperSize + c * kClusterSize + ti]);
-            const float4 v = ljt[(size_t)tyi * nt + tyc];
+            const R4 v = ljt[(size_t)tyi * nt + tyc];
             A = mod ? v.z : v.x;
             B = mod ? v.w : v.y;
           } else if (LJ) {
-            const float2 v = s_lj[GENERAL ? (mod ? 1 : 0) : 0][((irow[c >> 2] >> (8 * (c & 3))) & 255u) + tyc];
+            const R2 v = s_lj[GENERAL ? (mod ? 1 : 0) : 0][((irow[c >> 2] >> (8 * (c & 3))) & 255u) + tyc];
             A = v.x;
             B = v.y;
           }
-          float qq = xi.w * xj.w;
+          R qq = xi.w * xj.w;
           if (GENERAL && mod) qq *= kc.csf;
-          float el = 0.f, ec = 0.f, fl = 0.f, fc = 0.f, f;
-          direct_eval<COUL, LJSW, CSW>(kc, r2, qq, A, B, el, ec, fl, fc);
+          R el = 0, ec = 0, fl = 0, fc = 0, f;
+          direct_eval<COUL, LJSW, CSW, R>(kc, r2, qq, A, B, el, ec, fl, fc);
           if (SAME) {
-            f = in ? fl + fc : 0.f;
-            elT += in ? el : 0.f;
-            ecT += in ? ec : 0.f;
+            f = in ? fl + fc : (R)0;
+            elT += in ? el : (R)0;
+            ecT += in ? ec : (R)0;
           } else {
             const bool il = in && r2 <= kc.lj.rc2, ic = in && r2 <= kc.co.rc2;
-            f = (il ? fl : 0.f) + (ic ? fc : 0.f);
-            elT += il ? el : 0.f;
-            ecT += ic ? ec : 0.f;
+            f = (il ? fl : (R)0) + (ic ? fc : (R)0);
+            elT += il ? el : (R)0;
+            ecT += ic ? ec : (R)0;
           }
           fi[c][0] += f * dx;  // of the opposite sign
           fi[c][1] += f * dy;
@@ -2205,8 +1844,8 @@ __device__ __forceinline__ void pair_direct_body(
         fj1 = group8_sum(fj1);
         fj2 = group8_sum(fj2);
         if (ti < 3 && tyj >= 0) {
-          const float v = ti == 0 ? fj0 : (ti == 1 ? fj1 : fj2);
-          AccT<true>::add(&facc[3 * sj + ti], v);
+          const R v = ti == 0 ? fj0 : (ti == 1 ? fj1 : fj2);
+          AccT<MIXED>::add(&facc[3 * sj + ti], v);
         }
       }
     }
@@ -2216,16 +1855,16 @@ __device__ __forceinline__ void pair_direct_body(
       const bool real = ts[s] >= 0, hi8 = lane & 8;
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
-        float a[4];
+        R a[4];
 #pragma unroll
         for (int c = 0; c < 4; ++c) a[c] = swap32_sum(fi[c][k], fi[c + 4][k]);
-        const float b0 = swap16_sum(a[0], a[2]), b1 = swap16_sum(a[1], a[3]);
-        const float v = swap8_sum(b0, b1, hi8);
+        const R b0 = swap16_sum(a[0], a[2]), b1 = swap16_sum(a[1], a[3]);
+        const R v = swap8_sum(b0, b1, hi8);
         if (real) WA::add(&facc[3 * s + k], WA::of(-v));
       }
     }
-    const long long eljA = wave_sum(WA::of(elT));
-    const long long ecoA = wave_sum(WA::of(ecT));
+    const typename WA::T eljA = wave_sum(WA::of(elT));
+    const typename WA::T ecoA = wave_sum(WA::of(ecT));
     long long np = 0;
     if (STATS) {
       np = wave_sum((long long)npair);
@@ -2243,7 +1882,7 @@ __device__ __forceinline__ void pair_direct_body(
 }
 
 template <bool MIXED, int COUL, int LJSW, int CSW, bool BIGLJ, int MODE>
-__global__ void __launch_bounds__(kPairBlock, 4) k_pair(
+__global__ void __launch_bounds__(kPairBlock, MIXED ? 4 : 3) k_pair(
     PairParams pp, int dynamic, const int2 *__restrict__ runs, const int *__restrict__ ntiles_p,
     const int *__restrict__ count, int *__restrict__ tile_counter, const int4 *__restrict__ entries, int4 *entries_w,
     int cap,
@@ -2255,14 +1894,9 @@ __global__ void __launch_bounds__(kPairBlock, 4) k_pair(
     typename AccT<MIXED>::type *__restrict__ facc, PairOut out) {
   // the blocks of one XCD take a contiguous range of runs
   const int bid = xcd_block(blockIdx.x, gridDim.x);
-  if constexpr (MIXED)
-    pair_direct_body<COUL, LJSW, CSW, BIGLJ, MODE>(bid, gridDim.x, pp, dynamic, runs, ntiles_p, count, tile_counter,
-                                                   entries, entries_w, cap, masks, xs, sorg, ts, perm, ljtab, ljt,
-                                                   facc, out);
-  else
-    pair_body<MIXED, COUL, LJSW, CSW, BIGLJ, MODE>(bid, gridDim.x, pp, dynamic, runs, ntiles_p, count, tile_counter,
-                                                   entries, entries_w, cap, masks, xs, sorg, ts, perm, ljtab, ljt,
-                                                   facc, out);
+  pair_body<MIXED, COUL, LJSW, CSW, BIGLJ, MODE>(bid, gridDim.x, pp, dynamic, runs, ntiles_p, count, tile_counter,
+                                                 entries, entries_w, cap, masks, xs, sorg, ts, perm, ljtab, ljt, facc,
+                                                 out);
 }
 
 // Boundary pairs: exact FP64 membership on the original coordinates

@@ -10,13 +10,10 @@
 
 namespace pmx {
 
-#define PMX_X(C, LJ, CS, BIG)                   \
-  PMX_PAIR_KERNEL(, C, LJ, CS, BIG, kPairPlain) \
-  PMX_PAIR_KERNEL(, C, LJ, CS, BIG, kPairPrune) \
-  PMX_PAIR_KERNEL(, C, LJ, CS, BIG, kPairStats)
+#define PMX_X(C, LJ, CS, BIG) PMX_PAIR_MODES(, true, C, LJ, CS, BIG)
 PMX_PAIR_CASES(PMX_X)
 #undef PMX_X
-#define PMX_X(C, LJ, CS, BIG) PMX_BATCH_PAIR_KERNEL(, C, LJ, CS, BIG)
+#define PMX_X(C, LJ, CS, BIG) PMX_BATCH_PAIR_KERNEL(, true, C, LJ, CS, BIG)
 PMX_BATCH_PAIR_CASES(PMX_X)
 #undef PMX_X
 
