@@ -152,6 +152,7 @@ struct Sys {
   // pinned staging of this system's copies to and from the host, in chunks
   // beyond kStageChunks x kStageChunk bytes (stage_ev: a chunk's copy is done)
   HostBuf stage;
+  bool staged = false;  // the stage holds the last pass's results and forces (batched passes)
   hipEvent_t stage_ev[4] = {nullptr, nullptr, nullptr, nullptr};
   // device-resident MD state
   struct Md {
@@ -1174,15 +1175,14 @@ int run_pme(Sys *s, bool timing) {
   return PMX_OK;
 }
 
-void reduce_energies(Sys *s, bool stats) {
+EnergyArgs energy_args(Sys *s, bool stats) {
   const bool recip = s->pme_on && (s->d.pme_terms & PMX_PME_RECIP);
   const bool corr = s->pme_on && (s->d.pme_terms & PMX_PME_CORR) && !s->etab.empty();
-  hipLaunchKernelGGL(k_reduce_energy, dim3(1), dim3(1024), 0, s->ctx->stream, s->ntiles_cap, P<int>(s->ntiles),
-                     P<double>(s->pair_e), s->mixed ? 1 : 0, recip ? s->recip_blocks : 0, P<double>(s->recip_e),
-                     corr ? s->term_blocks : 0, P<double>(s->corr_e), P<long long>(s->npairs),
-                     P<unsigned long long>(s->hash), stats ? 1 : 0, P<unsigned long long>(s->border_acc),
-                     P<unsigned long long>(s->border_acc) + 2, P<double>(s->eout), P<long long>(s->np_out),
-                     P<unsigned long long>(s->hash_out));
+  return {s->ntiles_cap, P<int>(s->ntiles), P<double>(s->pair_e), s->mixed ? 1 : 0, recip ? s->recip_blocks : 0,
+          P<double>(s->recip_e), corr ? s->term_blocks : 0, P<double>(s->corr_e), P<long long>(s->npairs),
+          P<unsigned long long>(s->hash), stats ? 1 : 0, P<unsigned long long>(s->border_acc),
+          P<unsigned long long>(s->border_acc) + 2, P<double>(s->eout), P<long long>(s->np_out),
+          P<unsigned long long>(s->hash_out)};
 }
 
 void timing_begin_call(Sys *s, bool timing) {
@@ -1216,12 +1216,14 @@ MaskArgs mask_args(Sys *s) {
           P<unsigned short>(s->masks), s->maxmaskwork};
 }
 
-int rebuild(Sys *s, bool timing) {
+// clear: a pass begins, with its overflow flag cleared.
+int rebuild(Sys *s, bool timing, bool clear) {
   hipStream_t st = s->ctx->stream;
   const int n = s->n;
   // the histogram starts cleared (set-up, then each scan clears it)
   hipLaunchKernelGGL(k_bin, dim3(nblk(n, 256)), dim3(256), 0, st, n, P<double>(s->xorig), s->bin, P<uint32_t>(s->key),
-                     P<double>(s->xwrap), P<int>(s->refcell), P<uint32_t>(s->hist));
+                     P<double>(s->xwrap), P<int>(s->refcell), P<uint32_t>(s->hist),
+                     clear ? P<int>(s->overflow) : nullptr);
   if (s->nbins <= kScanSingleMax) {
     hipLaunchKernelGGL(k_scan_columns, dim3(1), dim3(kScanBlock), 0, st, P<uint32_t>(s->hist), (int)s->nbins,
                        P<uint32_t>(s->start), P<uint32_t>(s->cursor), s->ncols, s->bin.nzb, n, s->nsuper,
@@ -1294,6 +1296,7 @@ int forces(Sys *s, unsigned flags, bool energies, const Kick *next = nullptr, un
   // after an interrupted pass clears them here.
   if (!s->acc_clean) launch_zero(s);
   s->acc_clean = false;
+  s->staged = false;
   if (timing) hipEventRecord(s->ev[2], st);
   // fork: FFT, gather, exclusion correction and bonded terms on the second
   // stream beside the pair kernel; all add into the zeroed accumulators.
@@ -1360,6 +1363,14 @@ int forces(Sys *s, unsigned flags, bool energies, const Kick *next = nullptr, un
                        P<int>(s->nborder), P<double>(s->md.minv), P<double>(s->md.v), P<double>(s->xorig),
                        P<double>(s->md.xbuild), P<double4>(s->xs), P<double4>(s->xs64), P<float4>(s->sorg),
                        next_dmax, s->pme, pme_slots<double>(s));
+  else if (energies && s->mixed)
+    hipLaunchKernelGGL(k_unsort_energy<true>, dim3(1 + nblk(n, kEndBlock)), dim3(kEndBlock), 0, st, n, P<int>(s->slot),
+                       P<unsigned long long>(s->facc), P<double>(s->fout), P<int>(s->tilectr), P<int>(s->nborder),
+                       energy_args(s, stats));
+  else if (energies)
+    hipLaunchKernelGGL(k_unsort_energy<false>, dim3(1 + nblk(n, kEndBlock)), dim3(kEndBlock), 0, st, n,
+                       P<int>(s->slot), P<double>(s->facc), P<double>(s->fout), P<int>(s->tilectr),
+                       P<int>(s->nborder), energy_args(s, stats));
   else if (s->mixed)
     hipLaunchKernelGGL(k_unsort_forces<true>, dim3(nblk(n, 256)), dim3(256), 0, st, n, P<int>(s->slot),
                        P<unsigned long long>(s->facc), P<double>(s->fout), P<int>(s->tilectr),
@@ -1368,7 +1379,6 @@ int forces(Sys *s, unsigned flags, bool energies, const Kick *next = nullptr, un
     hipLaunchKernelGGL(k_unsort_forces<false>, dim3(nblk(n, 256)), dim3(256), 0, st, n, P<int>(s->slot),
                        P<double>(s->facc), P<double>(s->fout), P<int>(s->tilectr), P<int>(s->nborder));
   s->acc_clean = true;
-  if (energies) reduce_energies(s, stats);
   if (timing) hipEventRecord(s->ev[8], st);
   HIPCHK(hipGetLastError());
   return PMX_OK;
@@ -1377,8 +1387,7 @@ int forces(Sys *s, unsigned flags, bool energies, const Kick *next = nullptr, un
 int compute(Sys *s, unsigned flags) {
   const bool timing = flags & PMX_EVAL_TIMING;
   timing_begin_call(s, timing);
-  hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, s->ctx->stream, P<int>(s->overflow), 0, 2ll);
-  int rc = rebuild(s, timing);
+  int rc = rebuild(s, timing, true);
   if (rc) return rc;
   return forces(s, flags, true);
 }
@@ -1388,6 +1397,7 @@ constexpr int kStageChunks = 4;
 constexpr size_t kStageBytes = kStageChunk * kStageChunks;
 
 int stage_get(Sys *s, size_t bytes) {
+  s->staged = false;
   if (!host_get(s->stage, bytes)) return fail(s->ctx, PMX_ERR_OOM, "pinned host memory");
   if (bytes < kStageBytes || s->stage_ev[0]) return PMX_OK;
   RtLock lk(g_rt_mu);
@@ -1442,15 +1452,41 @@ int send(Sys *s, void *dst, const void *src, size_t bytes) {
   return PMX_OK;
 }
 
+// The results of a pass, and then its forces, in the stage.
+constexpr size_t kResultWords = sizeof(PassResults) / 8;
+bool results_fit(const Sys *s) { return 8 * (kResultWords + 3 * (size_t)s->n) <= kStageBytes; }
+
+struct OutList {
+  OutArgs a{};
+  int k = 0;
+  explicit OutList(void *dst) { a.dst = static_cast<unsigned long long *>(dst); }
+  // words of 8 bytes from src on; returns where they arrive
+  double *add(const void *src, size_t words) {
+    const long long at = k ? a.end[k - 1] : 0;
+    for (int i = k; i < 5; ++i) {
+      a.src[i] = static_cast<const unsigned long long *>(src);
+      a.end[i] = at + (long long)words;
+    }
+    if (words) ++k;
+    return reinterpret_cast<double *>(a.dst + at);
+  }
+  unsigned blocks() const { return (unsigned)std::min<long long>(1024, std::max<long long>(1, (a.end[4] + 255) / 256)); }
+  void launch(hipStream_t st) const { hipLaunchKernelGGL(k_out, dim3(blocks()), dim3(256), 0, st, a); }
+};
+
 int finish(Sys *s, unsigned flags, double *f_aos, double *energies) {
   hipStream_t st = s->ctx->stream;
   const size_t fb = f_aos ? 24 * (size_t)s->n : 0;
-  const bool once = sizeof(PassResults) + fb <= kStageBytes;
-  if (int rc = stage_get(s, once ? sizeof(PassResults) + fb : kStageBytes)) return rc;
-  unsigned char *const h = static_cast<unsigned char *>(s->stage.p);
-  HIPCHK(hipMemcpyAsync(h, s->eout.p, sizeof(PassResults), hipMemcpyDeviceToHost, st));
-  if (once && fb) HIPCHK(hipMemcpyAsync(h + sizeof(PassResults), s->fout.p, fb, hipMemcpyDeviceToHost, st));
+  const bool once = s->staged || !fb || results_fit(s);
+  if (!s->staged) {
+    if (int rc = stage_get(s, once ? sizeof(PassResults) + fb : kStageBytes)) return rc;
+    OutList out(s->stage.p);
+    out.add(s->eout.p, kResultWords);
+    if (once) out.add(s->fout.p, fb / 8);
+    out.launch(st);
+  }
   HIPCHK(hipStreamSynchronize(st));
+  const unsigned char *const h = static_cast<const unsigned char *>(s->stage.p);
   PassResults r;
   std::memcpy(&r, h, sizeof r);
   s->last_np = r.np[0];
@@ -2005,8 +2041,7 @@ int md_ensure_forces(Sys *s) {
   if (m.forces_valid) return PMX_OK;
   hipStream_t st = s->ctx->stream;
   for (int tries = 0;; ++tries) {
-    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, P<int>(s->overflow), 0, 2ll);
-    int rc = rebuild(s, false);
+    int rc = rebuild(s, false, true);
     if (rc) return rc;
     ++m.rebuilds;
     if ((rc = forces(s, 0, false))) return rc;
@@ -2075,7 +2110,7 @@ int md_step(Sys *s, double kick, long long step, bool rebuild_here, int dslot,
                        P<double>(m.xbuild), P<double4>(s->xs), P<double4>(s->xs64),
                        P<float4>(s->sorg), P<unsigned>(m.dmax) + dslot, s->pme, pme_slots<double>(s));
   if (rebuild_here) {
-    int rc = rebuild(s, timing);
+    int rc = rebuild(s, timing, false);
     if (rc) return rc;
   } else if (timing) {
     hipEventRecord(s->ev[1], st);
@@ -2375,10 +2410,11 @@ struct Batch {
   pmx_ctx *ctx = nullptr;
   std::vector<Sys *> sys;
   int nsys = 0;
+  bool results = false;       // a force pass alone: its results go to the systems' stages with it
   bool first_forces = false;  // MD: the forces at the set positions come first, for every system
   BatchLaunch bin, scan, scatter, split, list, runs;
   BatchLaunch kick, spread, pair, yfwd, xconv, yinv, plane, gather, fixups, ukd, unsort, begin, half;
-  BatchLaunch energy;
+  BatchLaunch energy, out;
   BatchBuf tables, bsys, need, base, flags, rebuilds;
   std::vector<unsigned char> image;    // the tables of every launch, uploaded in one copy
   std::vector<BatchLaunch *> launches;
@@ -2535,7 +2571,9 @@ int batch_tables(Batch &b) {
     std::vector<typename OpUnsortForces<MIXED>::Args> args_unsort(ns);
     std::vector<OpChunkBegin::Args> args_begin(ns);
     std::vector<OpHalfKick::Args> args_half(ns);
-    std::vector<OpReduceEnergy::Args> args_energy(ns);
+    std::vector<typename OpUnsortEnergy<MIXED>::Args> args_energy(ns);
+    std::vector<OutArgs> args_out(ns, OutArgs{});
+    std::vector<int> nout(ns, 0);
     std::vector<int> nfix(ns);
     long long natoms = 0;
     size_t lds_z = 0, lds_g = 0, lds_y = 0, lds_x = 0, lds_p = 0;
@@ -2575,13 +2613,16 @@ int batch_tables(Batch &b) {
       args_begin[i] = {3ll * s->n, P<double>(s->xorig), P<double>(m.v), P<double>(s->fout), P<double>(m.xbak),
                        P<double>(m.vbak), P<double>(m.fbak), P<int>(s->overflow), P<unsigned>(m.dmax), kMaxChunk};
       args_half[i] = {s->n, kk, m.h, P<double>(s->fout), P<double>(m.minv), P<double>(m.v)};
-      const bool recip = s->pme_on && (s->d.pme_terms & PMX_PME_RECIP);
-      const bool corr = s->pme_on && (s->d.pme_terms & PMX_PME_CORR) && !s->etab.empty();
-      args_energy[i] = {s->ntiles_cap, P<int>(s->ntiles), P<double>(s->pair_e), s->mixed ? 1 : 0,
-                        recip ? s->recip_blocks : 0, corr ? s->term_blocks : 0, P<double>(s->recip_e),
-                        P<double>(s->corr_e), P<long long>(s->npairs), P<unsigned long long>(s->hash),
-                        P<unsigned long long>(s->border_acc), P<unsigned long long>(s->border_acc) + 2,
-                        P<double>(s->eout), P<long long>(s->np_out), P<unsigned long long>(s->hash_out)};
+      args_energy[i] = {s->n, P<int>(s->slot), facc, P<double>(s->fout), P<int>(s->tilectr), P<int>(s->nborder),
+                        energy_args(s, false)};
+      if (b.results && results_fit(s)) {
+        if ((rc = stage_get(s, 8 * (kResultWords + 3 * (size_t)s->n)))) return rc;
+        OutList out(s->stage.p);
+        out.add(s->eout.p, kResultWords);
+        out.add(s->fout.p, 3 * (size_t)s->n);
+        args_out[i] = out.a;
+        nout[i] = (int)out.blocks();
+      }
       // dynamic LDS and block size of each launch: the largest of the
       // systems it serves
       thr_z = std::max(thr_z, s->thr_z);
@@ -2630,8 +2671,9 @@ int batch_tables(Batch &b) {
     for (int i = 0; i < ns; ++i) nb[i] = (int)nblk(b.sys[i]->n, 256);
     if ((rc = batch_table<OpUnsortForces<MIXED>>(b, b.unsort, args_unsort, nb, 0))) return rc;
     if ((rc = batch_table<OpHalfKick>(b, b.half, args_half, nb, 0))) return rc;
-    for (int i = 0; i < ns; ++i) nb[i] = 1;
-    if ((rc = batch_table<OpReduceEnergy>(b, b.energy, args_energy, nb, 0))) return rc;
+    for (int i = 0; i < ns; ++i) nb[i] = 1 + (int)nblk(b.sys[i]->n, kEndBlock);
+    if ((rc = batch_table<OpUnsortEnergy<MIXED>>(b, b.energy, args_energy, nb, 0))) return rc;
+    if ((rc = batch_table<OpOut>(b, b.out, args_out, nout, 0))) return rc;
     for (int i = 0; i < ns; ++i) nb[i] = (int)nblk(std::max<long long>(3ll * b.sys[i]->n, kMaxChunk), 256);
     if ((rc = batch_table<OpChunkBegin>(b, b.begin, args_begin, nb, 0))) return rc;
   }
@@ -2741,8 +2783,8 @@ int batch_forces(Batch &b, bool *grown) {
   BHIPCHK(hipEventRecord(b.join, st2));
   batch_go<OpFixups<MIXED, C, LJ, CS>>(b.fixups, st, bk);
   BHIPCHK(hipStreamWaitEvent(st, b.join, 0));
-  batch_go<OpUnsortForces<MIXED>>(b.unsort, st, bk);
-  batch_go<OpReduceEnergy>(b.energy, st, bk);
+  batch_go<OpUnsortEnergy<MIXED>>(b.energy, st, bk);
+  batch_go<OpOut>(b.out, st, bk);
   hipLaunchKernelGGL(k_batch_flags, dim3(nblk(ns, 256)), dim3(256), 0, st, ns,
                      reinterpret_cast<const BatchSys *>(b.bsys.p), reinterpret_cast<int *>(b.flags.p));
   BHIPCHK(hipMemcpyAsync(b.flags_h, b.flags.p, 4 * (size_t)ns, hipMemcpyDeviceToHost, st));
@@ -2753,6 +2795,7 @@ int batch_forces(Batch &b, bool *grown) {
     s->list_valid = true;
     s->prune_pending = false;
     s->acc_clean = true;
+    s->staged = b.results && results_fit(s);
     for (int attempt = 0; b.flags_h[i] && attempt < 6; ++attempt) {
       *grown = true;
       if ((rc = grow_and_retry(s)) || (rc = compute(s, 0))) return rc;
@@ -2988,6 +3031,7 @@ int batch_entry(pmx_sys *const *systems, int nsys, int nsteps) {
   b.nsys = nsys;
   // the first forces of a run: in one batched pass when every system needs
   // them, one by one where only some do
+  b.results = !md;
   b.first_forces = md;
   for (int i = 0; i < nsys; ++i) b.first_forces &= !systems[i]->s.md.forces_valid;
   for (int i = 0; i < nsys; ++i) {
@@ -3068,7 +3112,7 @@ int pmx_md_get_state(pmx_sys *sys, double *x, double *v, double *energies) {
     // potential energies at the current positions (computed first if the
     // state was just set) and kinetic energy of v
     if (int rc = md_ensure_forces(s)) return rc;
-    reduce_energies(s, false);
+    hipLaunchKernelGGL(k_reduce_energy, dim3(1), dim3(kEndBlock), 0, st, energy_args(s, false));
     hipLaunchKernelGGL(k_kinetic, dim3(nblk(n, 256)), dim3(256), 0, st, n, P<double>(m.v), P<double>(m.minv),
                        P<double>(m.ke_e));
   }
@@ -3086,27 +3130,21 @@ int pmx_md_get_state(pmx_sys *sys, double *x, double *v, double *energies) {
   }
   if (once) words += (x ? vec : 0) + (v ? vec : 0);
   if (int rc = stage_get(s, 8 * words)) return rc;
-  double *const h = static_cast<double *>(s->stage.p);
-  double *at = h;
-  auto take = [&](const void *src, size_t count) {
-    const hipError_t e = count ? hipMemcpyAsync(at, src, 8 * count, hipMemcpyDeviceToHost, st) : hipSuccess;
-    at += count;
-    return e;
-  };
+  OutList out(s->stage.p);
+  const double *const h = static_cast<double *>(s->stage.p);
+  const double *ke = h, *be = h;
   if (energies) {
-    HIPCHK(take(s->eout.p, 4));
-    HIPCHK(take(m.ke_e.p, nke));
-    HIPCHK(take(m.bond_e.p, nbe));
+    out.add(s->eout.p, 4);
+    ke = out.add(m.ke_e.p, nke);
+    be = out.add(m.bond_e.p, nbe);
   }
-  double *const hx = at;
-  if (once && x) HIPCHK(take(s->xorig.p, vec));
-  double *const hv = at;
-  if (once && v) HIPCHK(take(m.v.p, vec));
+  const double *const hx = out.add(s->xorig.p, once && x ? vec : 0);
+  const double *const hv = out.add(m.v.p, once && v ? vec : 0);
+  if (out.a.end[4]) out.launch(st);
   HIPCHK(hipStreamSynchronize(st));
   if (once && x) std::memcpy(x, hx, 8 * vec);
   if (once && v) std::memcpy(v, hv, 8 * vec);
   if (energies) {
-    const double *const ke = h + 4, *const be = ke + nke;
     double eb = 0, ea = 0, ek = 0;
     for (size_t i = 0; i < nbe; i += 2) {
       eb += be[i];

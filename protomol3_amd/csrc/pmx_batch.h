@@ -67,7 +67,7 @@ struct OpBin {
   static constexpr int kBlock = 256, kMinBlocks = 1;
   static constexpr bool kGated = true;
   __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &) {
-    bin_body(bid, nbk, a.n, a.xorig, a.p, a.key, a.xwrap, a.refcell, a.hist);
+    bin_body(bid, nbk, a.n, a.xorig, a.p, a.key, a.xwrap, a.refcell, a.hist, nullptr);
   }
 };
 
@@ -365,25 +365,29 @@ struct OpUnsortForces {
 };
 
 // a force pass's energy partials into the system's energy slots (one block)
-struct OpReduceEnergy {
+// The end of a force pass with energies, one more block a system than the forces take.
+template <bool MIXED>
+struct OpUnsortEnergy {
   struct Args {
-    int ntiles_cap;
-    const int *ntiles;
-    const double *pair_e;
-    int pair_fixed, nrecip, ncorr;
-    const double *recip_e, *corr_e;
-    const long long *npairs;
-    const unsigned long long *hash, *border_e, *border_stat;
-    double *out;
-    long long *out_np;
-    unsigned long long *out_hash;
+    int n;
+    const int *slot;
+    typename AccT<MIXED>::type *facc;
+    double *fout;
+    int *tilectr, *nborder;
+    EnergyArgs e;
   };
-  static constexpr int kBlock = 1024, kMinBlocks = 1;
+  static constexpr int kBlock = kEndBlock, kMinBlocks = 1;
   static constexpr bool kGated = false;
   __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &) {
-    reduce_energy_body(bid, nbk, a.ntiles_cap, a.ntiles, a.pair_e, a.pair_fixed, a.nrecip, a.recip_e, a.ncorr,
-                       a.corr_e, a.npairs, a.hash, 0, a.border_e, a.border_stat, a.out, a.out_np, a.out_hash);
+    unsort_energy_body<MIXED>(bid, a.n, a.slot, a.facc, a.fout, a.tilectr, a.nborder, a.e);
   }
+};
+
+struct OpOut {
+  using Args = OutArgs;
+  static constexpr int kBlock = 256, kMinBlocks = 1;
+  static constexpr bool kGated = false;
+  __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &) { out_body(bid, nbk, a); }
 };
 
 // backups for a restore, cleared overflow flags and displacement record

@@ -182,8 +182,9 @@ __device__ inline int xcd_block(int bx, int nb) {
 
 __device__ __forceinline__ void bin_body(const int bid_, const int nbk_, int n, const double *__restrict__ xorig,
                                          BinParams p, uint32_t *__restrict__ key, double *__restrict__ xwrap,
-                                         int *__restrict__ refcell, uint32_t *__restrict__ hist) {
+                                         int *__restrict__ refcell, uint32_t *__restrict__ hist, int *clear) {
   int a = bid_ * blockDim.x + threadIdx.x;
+  if (clear && a < 2) clear[a] = 0;  // the overflow flag of the pass that begins here
   if (a >= n) return;
   double w[3];
 #pragma unroll
@@ -224,8 +225,8 @@ __device__ __forceinline__ void bin_body(const int bid_, const int nbk_, int n, 
 }
 
 static __global__ void k_bin(int n, const double *__restrict__ xorig, BinParams p, uint32_t *__restrict__ key,
-                      double *__restrict__ xwrap, int *__restrict__ refcell, uint32_t *__restrict__ hist) {
-  bin_body(blockIdx.x, gridDim.x, n, xorig, p, key, xwrap, refcell, hist);
+                      double *__restrict__ xwrap, int *__restrict__ refcell, uint32_t *__restrict__ hist, int *clear) {
+  bin_body(blockIdx.x, gridDim.x, n, xorig, p, key, xwrap, refcell, hist, clear);
 }
 
 // Counting sort by key (one radix digit spanning the key range): histogram,
@@ -2720,39 +2721,47 @@ __global__ void k_unsort_forces(int n, const int *__restrict__ slot, typename Ac
 // Pair energies per tile are int64 fixed point (2^-32) when pair_fixed (the
 // mixed form: their sum is exact, whatever tiles the schedule made), FP64
 // otherwise.
-__device__ __forceinline__ void reduce_energy_body(const int bid_, const int nbk_, int ntiles_cap,
-                                                   const int *__restrict__ ntiles_p, const double *__restrict__ pair_e,
-                                                   int pair_fixed, int nrecip, const double *__restrict__ recip_e,
-                                                   int ncorr, const double *__restrict__ corr_e,
-                                                   const long long *__restrict__ npairs,
-                                                   const unsigned long long *__restrict__ hash, int stats,
-                                                   const unsigned long long *__restrict__ border_e,
-                                                   const unsigned long long *__restrict__ border_stat,
-                                                   double *__restrict__ out, long long *__restrict__ out_np,
-                                                   unsigned long long *__restrict__ out_hash) {
+struct EnergyArgs {
+  int ntiles_cap;
+  const int *ntiles;
+  const double *pair_e;
+  int pair_fixed, nrecip;
+  const double *recip_e;
+  int ncorr;
+  const double *corr_e;
+  const long long *npairs;
+  const unsigned long long *hash;
+  int stats;
+  const unsigned long long *border_e, *border_stat;
+  double *out;
+  long long *out_np;
+  unsigned long long *out_hash;
+};
+
+__device__ __forceinline__ void reduce_energy_body(const EnergyArgs &a) {
   __shared__ double sd[4][1024 / kWave];
   __shared__ long long sn[1024 / kWave];
   __shared__ unsigned long long sh[1024 / kWave];
   __shared__ long long sf[2][1024 / kWave];
-  const int nt = min(*ntiles_p, ntiles_cap);
+  const int nt = min(*a.ntiles, a.ntiles_cap);
   double c = 0, l = 0, r = 0, k = 0;
   long long np = 0, cf = 0, lf = 0;
   unsigned long long h = 0;
   for (int i = threadIdx.x; i < nt; i += blockDim.x) {
-    if (pair_fixed) {
-      cf += __double_as_longlong(pair_e[2 * i]);
-      lf += __double_as_longlong(pair_e[2 * i + 1]);
+    if (a.pair_fixed) {
+      cf += __double_as_longlong(a.pair_e[2 * i]);
+      lf += __double_as_longlong(a.pair_e[2 * i + 1]);
     } else {
-      c += pair_e[2 * i];
-      l += pair_e[2 * i + 1];
+      c += a.pair_e[2 * i];
+      l += a.pair_e[2 * i + 1];
     }
-    if (stats) {
-      np += npairs[i];
-      h += hash[i];
+    if (a.stats) {
+      np += a.npairs[i];
+      h += a.hash[i];
     }
   }
-  for (int i = threadIdx.x; i < nrecip; i += blockDim.x) r += recip_e[i];
-  for (int i = threadIdx.x; i < ncorr; i += blockDim.x) k += corr_e[i];
+  for (int i = threadIdx.x; i < a.nrecip; i += blockDim.x) r += a.recip_e[i];
+  for (int i = threadIdx.x; i < a.ncorr; i += blockDim.x) k += a.corr_e[i];
   c = wave_sum(c);
   l = wave_sum(l);
   cf = wave_sum(cf);
@@ -2787,25 +2796,57 @@ __device__ __forceinline__ void reduce_energy_body(const int bid_, const int nbk
       N += sn[i];
       H += sh[i];
     }
-    out[0] = C + (double)(CF + (long long)border_e[0]) * (1.0 / kForceScale);
-    out[1] = Lj + (double)(LF + (long long)border_e[1]) * (1.0 / kForceScale);
-    out[2] = 0.5 * Rr;
-    out[3] = K;
-    *out_np = N + (long long)border_stat[0];
-    *out_hash = H + border_stat[1];
+    a.out[0] = C + (double)(CF + (long long)a.border_e[0]) * (1.0 / kForceScale);
+    a.out[1] = Lj + (double)(LF + (long long)a.border_e[1]) * (1.0 / kForceScale);
+    a.out[2] = 0.5 * Rr;
+    a.out[3] = K;
+    *a.out_np = N + (long long)a.border_stat[0];
+    *a.out_hash = H + a.border_stat[1];
   }
 }
 
-static __global__ void k_reduce_energy(int ntiles_cap, const int *__restrict__ ntiles_p, const double *__restrict__ pair_e,
-                                int pair_fixed, int nrecip, const double *__restrict__ recip_e, int ncorr,
-                                const double *__restrict__ corr_e, const long long *__restrict__ npairs,
-                                const unsigned long long *__restrict__ hash, int stats,
-                                const unsigned long long *__restrict__ border_e,
-                                const unsigned long long *__restrict__ border_stat, double *__restrict__ out,
-                                long long *__restrict__ out_np, unsigned long long *__restrict__ out_hash) {
-  reduce_energy_body(blockIdx.x, gridDim.x, ntiles_cap, ntiles_p, pair_e, pair_fixed, nrecip, recip_e, ncorr, corr_e,
-                     npairs, hash, stats, border_e, border_stat, out, out_np, out_hash);
+static __global__ void k_reduce_energy(EnergyArgs a) { reduce_energy_body(a); }
+
+// The end of a pass whose energies are wanted: block 0 reduces them, the others
+// bring the forces into the caller's order (the two in turn took 6 + 11 us at
+// 26,000 atoms, and a launch).
+constexpr int kEndBlock = 1024;
+template <bool MIXED>
+__device__ __forceinline__ void unsort_energy_body(const int bid_, int n, const int *__restrict__ slot,
+                                                   typename AccT<MIXED>::type *__restrict__ facc,
+                                                   double *__restrict__ fout, int *__restrict__ tilectr,
+                                                   int *__restrict__ nborder, const EnergyArgs &a) {
+  if (bid_ == 0)
+    reduce_energy_body(a);
+  else
+    unsort_forces_body<MIXED>(bid_ - 1, 0, n, slot, facc, fout, tilectr, nborder);
 }
+
+template <bool MIXED>
+__global__ void __launch_bounds__(kEndBlock) k_unsort_energy(int n, const int *__restrict__ slot,
+                                                             typename AccT<MIXED>::type *__restrict__ facc,
+                                                             double *__restrict__ fout, int *__restrict__ tilectr,
+                                                             int *__restrict__ nborder, EnergyArgs a) {
+  unsort_energy_body<MIXED>(blockIdx.x, n, slot, facc, fout, tilectr, nborder, a);
+}
+
+// Results to the host: up to five arrays of 8-byte words one after the other
+// into pinned memory, in one launch instead of a copy each.
+struct OutArgs {
+  const unsigned long long *src[5];
+  long long end[5];  // running ends (unused: the last end again)
+  unsigned long long *dst;
+};
+__device__ __forceinline__ void out_body(int bid, int nbk, const OutArgs &a) {
+  for (long long i = (long long)bid * blockDim.x + threadIdx.x; i < a.end[4]; i += (long long)nbk * blockDim.x) {
+    const unsigned long long *p = a.src[0] + i;
+#pragma unroll
+    for (int k = 1; k < 5; ++k)
+      if (i >= a.end[k - 1]) p = a.src[k] + (i - a.end[k - 1]);
+    a.dst[i] = *p;
+  }
+}
+static __global__ void __launch_bounds__(256) k_out(OutArgs a) { out_body(blockIdx.x, gridDim.x, a); }
 
 // ---------------------------------------------------------------------------
 // 7. Device-resident MD: bonded terms, leapfrog kick/drift, kinetic energy.
