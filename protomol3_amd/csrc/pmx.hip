@@ -1239,18 +1239,18 @@ int rebuild(Sys *s, bool timing, bool clear) {
   }
   hipLaunchKernelGGL(k_scatter, dim3(nblk(n, 256)), dim3(256), 0, st, n, P<uint32_t>(s->key), P<uint32_t>(s->cursor),
                      P<int>(s->perm));
-  double *xbuild = s->md.on ? P<double>(s->md.xbuild) : nullptr;
+  double4 *xbuild = s->md.on ? P<double4>(s->md.xbuild) : nullptr;
   if (s->mixed)
     hipLaunchKernelGGL(k_split_fill<float>, dim3(nblk((long long)s->nsuper * 64, 256)), dim3(256), 0, st, s->nsuper,
                        P<int2>(s->sc_info), sorted_bins(s), P<double>(s->xwrap), P<int>(s->permp), P<int>(s->slot),
                        P<double>(s->q_d), P<int>(s->type_d), P<float4>(s->xs), P<double4>(s->xs64), P<int>(s->ts),
-                       P<double>(s->xorig), xbuild, P<float4>(s->sorg), P<float4>(s->ctr), P<float4>(s->half),
+                       P<double>(s->xorig), P<double>(s->md.minv), xbuild, P<float4>(s->sorg), P<float4>(s->ctr), P<float4>(s->half),
                        P<float4>(s->sctr), P<float4>(s->shalf), P<int>(s->nmaskwork), s->qpair, s->pme, pme_slots<float>(s));
   else
     hipLaunchKernelGGL(k_split_fill<double>, dim3(nblk((long long)s->nsuper * 64, 256)), dim3(256), 0, st, s->nsuper,
                        P<int2>(s->sc_info), sorted_bins(s), P<double>(s->xwrap), P<int>(s->permp), P<int>(s->slot),
                        P<double>(s->q_d), P<int>(s->type_d), P<double4>(s->xs), P<double4>(s->xs64), P<int>(s->ts),
-                       P<double>(s->xorig), xbuild, P<float4>(s->sorg), P<float4>(s->ctr), P<float4>(s->half),
+                       P<double>(s->xorig), P<double>(s->md.minv), xbuild, P<float4>(s->sorg), P<float4>(s->ctr), P<float4>(s->half),
                        P<float4>(s->sctr), P<float4>(s->shalf), P<int>(s->nmaskwork), s->qpair, s->pme, pme_slots<double>(s));
   if (timing) hipEventRecord(s->ev[1], st);
   hipLaunchKernelGGL(k_build_list, dim3(s->nsuper), dim3(kListBlock), list_lds_bytes(s->cap), st, s->lp,
@@ -1286,7 +1286,8 @@ void launch_zero(Sys *s) {
   hipLaunchKernelGGL(k_zero, dim3(std::max(1u, nblk(3ll * npad, 256)), nr), dim3(256), 0, s->ctx->stream, z);
 }
 
-int forces(Sys *s, unsigned flags, bool energies, const Kick *next = nullptr, unsigned *next_dmax = nullptr) {
+int forces(Sys *s, unsigned flags, bool energies, const Kick *next = nullptr, unsigned *next_dmax = nullptr,
+           const ChunkEnd &end = {}) {
   hipStream_t st = s->ctx->stream;
   const bool timing = flags & PMX_EVAL_TIMING;
   const bool stats = flags & PMX_EVAL_PAIRSTATS;
@@ -1353,15 +1354,14 @@ int forces(Sys *s, unsigned flags, bool energies, const Kick *next = nullptr, un
   HIPCHK(hipStreamWaitEvent(st, s->join_ev, 0));
   if (next && s->mixed)
     hipLaunchKernelGGL((k_unsort_kick_drift<true, float>), dim3(nblk(npad, 256)), dim3(256), 0, st, npad, *next,
-                       s->md.h, P<int>(s->permp), P<unsigned long long>(s->facc), P<double>(s->fout),
-                       P<int>(s->tilectr), P<int>(s->nborder), P<double>(s->md.minv), P<double>(s->md.v),
-                       P<double>(s->xorig), P<double>(s->md.xbuild), P<float4>(s->xs), P<double4>(s->xs64),
+                       s->md.h, P<int>(s->permp), P<unsigned long long>(s->facc), P<int>(s->tilectr),
+                       P<int>(s->nborder), P<double>(s->md.v), P<double>(s->xorig), P<double4>(s->md.xbuild),
+                        P<float4>(s->xs), P<double4>(s->xs64),
                        P<float4>(s->sorg), next_dmax, s->pme, pme_slots<float>(s));
   else if (next)
     hipLaunchKernelGGL((k_unsort_kick_drift<false, double>), dim3(nblk(npad, 256)), dim3(256), 0, st, npad, *next,
-                       s->md.h, P<int>(s->permp), P<double>(s->facc), P<double>(s->fout), P<int>(s->tilectr),
-                       P<int>(s->nborder), P<double>(s->md.minv), P<double>(s->md.v), P<double>(s->xorig),
-                       P<double>(s->md.xbuild), P<double4>(s->xs), P<double4>(s->xs64), P<float4>(s->sorg),
+                       s->md.h, P<int>(s->permp), P<double>(s->facc), P<int>(s->tilectr), P<int>(s->nborder),
+                       P<double>(s->md.v), P<double>(s->xorig), P<double4>(s->md.xbuild), P<double4>(s->xs), P<double4>(s->xs64), P<float4>(s->sorg),
                        next_dmax, s->pme, pme_slots<double>(s));
   else if (energies && s->mixed)
     hipLaunchKernelGGL(k_unsort_energy<true>, dim3(1 + nblk(n, kEndBlock)), dim3(kEndBlock), 0, st, n, P<int>(s->slot),
@@ -1374,10 +1374,10 @@ int forces(Sys *s, unsigned flags, bool energies, const Kick *next = nullptr, un
   else if (s->mixed)
     hipLaunchKernelGGL(k_unsort_forces<true>, dim3(nblk(n, 256)), dim3(256), 0, st, n, P<int>(s->slot),
                        P<unsigned long long>(s->facc), P<double>(s->fout), P<int>(s->tilectr),
-                       P<int>(s->nborder));
+                       P<int>(s->nborder), end);
   else
     hipLaunchKernelGGL(k_unsort_forces<false>, dim3(nblk(n, 256)), dim3(256), 0, st, n, P<int>(s->slot),
-                       P<double>(s->facc), P<double>(s->fout), P<int>(s->tilectr), P<int>(s->nborder));
+                       P<double>(s->facc), P<double>(s->fout), P<int>(s->tilectr), P<int>(s->nborder), end);
   s->acc_clean = true;
   if (timing) hipEventRecord(s->ev[8], st);
   HIPCHK(hipGetLastError());
@@ -1996,7 +1996,7 @@ int pmx_md_init(pmx_sys *sys, const pmx_md_desc *d) {
   int rc;
   if ((rc = dalloc(s, m.mptr, 8 * mp.size())) || (rc = dalloc(s, m.bonds, 4 * b.size())) || (rc = dalloc(s, m.bpar, 16 * bp.size())) ||
       (rc = dalloc(s, m.angles, 16 * a.size())) || (rc = dalloc(s, m.apar, 16 * ap.size())) ||
-      (rc = dalloc(s, m.minv, 8 * N)) || (rc = dalloc(s, m.v, 24 * N)) || (rc = dalloc(s, m.xbuild, 24 * N)) ||
+      (rc = dalloc(s, m.minv, 8 * N)) || (rc = dalloc(s, m.v, 24 * N)) || (rc = dalloc(s, m.xbuild, 32 * (size_t)s->npad)) ||
       (rc = dalloc(s, m.xbak, 2 * 24 * N)) || (rc = dalloc(s, m.vbak, 2 * 24 * N)) ||
       (rc = dalloc(s, m.fbak, 2 * 24 * N)) || (rc = dalloc(s, m.dmax, 4 * 2 * kMaxChunk)) ||
       (rc = dalloc(s, m.step_dev, 8)) || (rc = dalloc(s, m.bond_e, 16 * (size_t)s->term_blocks)) ||
@@ -2090,7 +2090,7 @@ Kick make_kick(const Sys::Md &m, double kick, long long step, const unsigned lon
 // drift; next (with next_dslot): fuse the following step's into this one's.
 int md_step(Sys *s, double kick, long long step, bool rebuild_here, int dslot,
             const unsigned long long *step_dev = nullptr, bool kicked = false, const Kick *next = nullptr,
-            int next_dslot = 0) {
+            int next_dslot = 0, const ChunkEnd &end = {}) {
   hipStream_t st = s->ctx->stream;
   Sys::Md &m = s->md;
   const bool timing = s->timing_active;
@@ -2101,13 +2101,13 @@ int md_step(Sys *s, double kick, long long step, bool rebuild_here, int dslot,
     ;
   else if (s->mixed)
     hipLaunchKernelGGL(k_kick_drift<float>, dim3(nblk(s->npad, 256)), dim3(256), 0, st, s->npad, kk, m.h,
-                       P<int>(s->permp), P<double>(s->fout), P<double>(m.minv), P<double>(m.v), P<double>(s->xorig),
-                       P<double>(m.xbuild), P<float4>(s->xs), P<double4>(s->xs64),
+                       P<int>(s->permp), P<double>(s->fout), P<double>(m.v), P<double>(s->xorig),
+                       P<double4>(m.xbuild), P<float4>(s->xs), P<double4>(s->xs64),
                        P<float4>(s->sorg), P<unsigned>(m.dmax) + dslot, s->pme, pme_slots<float>(s));
   else
     hipLaunchKernelGGL(k_kick_drift<double>, dim3(nblk(s->npad, 256)), dim3(256), 0, st, s->npad, kk, m.h,
-                       P<int>(s->permp), P<double>(s->fout), P<double>(m.minv), P<double>(m.v), P<double>(s->xorig),
-                       P<double>(m.xbuild), P<double4>(s->xs), P<double4>(s->xs64),
+                       P<int>(s->permp), P<double>(s->fout), P<double>(m.v), P<double>(s->xorig),
+                       P<double4>(m.xbuild), P<double4>(s->xs), P<double4>(s->xs64),
                        P<float4>(s->sorg), P<unsigned>(m.dmax) + dslot, s->pme, pme_slots<double>(s));
   if (rebuild_here) {
     int rc = rebuild(s, timing, false);
@@ -2116,13 +2116,14 @@ int md_step(Sys *s, double kick, long long step, bool rebuild_here, int dslot,
     hipEventRecord(s->ev[1], st);
     hipEventRecord(s->ev[2], st);
   }
-  return forces(s, timing ? PMX_EVAL_TIMING : 0u, false, next, next ? P<unsigned>(m.dmax) + next_dslot : nullptr);
+  return forces(s, timing ? PMX_EVAL_TIMING : 0u, false, next, next ? P<unsigned>(m.dmax) + next_dslot : nullptr,
+                end);
 }
 
 // A chunk of K steps from the committed state: its state is backed up in
-// slot `slot`, step 0 rebuilds the list, and the per-step displacements and
-// the overflow flag are copied to the slot's pinned host record, after which
-// the slot's event fires.
+// slot `slot`, step 0 rebuilds the list, and the last pass writes the per-step
+// displacements and the overflow flag to the slot's pinned host record, after
+// which the slot's event fires.
 struct Chunk {
   int K;
   long long step0;
@@ -2146,17 +2147,17 @@ int chunk_body(Sys *s, const Chunk &c, bool rel) {
   // inside the chunk each force pass ends with the next step's kick and
   // drift (one launch instead of two); timed steps keep them apart
   const bool fuse = !s->timing_active;
+  unsigned *const h = m.host + c.slot * (kMaxChunk + 1);
+  const ChunkEnd end{P<unsigned>(m.dmax) + c.slot * kMaxChunk, c.K, P<int>(s->overflow), h, h + kMaxChunk};
   for (int k = 0; k < c.K; ++k) {
     Kick nk{};
     const bool nx = fuse && k + 1 < c.K;
     if (nx) nk = make_kick(m, 1.0, rel ? k + 1 : c.step0 + k + 1, sd);
     int rc = md_step(s, (c.first && k == 0) ? 0.5 : 1.0, rel ? k : c.step0 + k, k == 0 || m.skin == 0.0,
-                     c.slot * kMaxChunk + k, sd, fuse && k > 0, nx ? &nk : nullptr, c.slot * kMaxChunk + k + 1);
+                     c.slot * kMaxChunk + k, sd, fuse && k > 0, nx ? &nk : nullptr, c.slot * kMaxChunk + k + 1,
+                     k + 1 < c.K ? ChunkEnd{} : end);
     if (rc) return rc;
   }
-  unsigned *h = m.host + c.slot * (kMaxChunk + 1);
-  HIPCHK(hipMemcpyAsync(h, P<uint32_t>(m.dmax) + c.slot * kMaxChunk, 4 * (size_t)c.K, hipMemcpyDeviceToHost, st));
-  HIPCHK(hipMemcpyAsync(h + kMaxChunk, s->overflow.p, 4, hipMemcpyDeviceToHost, st));
   return PMX_OK;
 }
 
@@ -2529,7 +2530,8 @@ int batch_tables(Batch &b) {
       sp.xs64 = P<double4>(s->xs64);
       sp.ts = P<int>(s->ts);
       sp.xorig = P<double>(s->xorig);
-      sp.xbuild = P<double>(s->md.xbuild);
+      sp.minv = P<double>(s->md.minv);
+      sp.xbuild = P<double4>(s->md.xbuild);
       sp.sorg = P<float4>(s->sorg);
       sp.ctr = P<float4>(s->ctr);
       sp.half = P<float4>(s->half);
@@ -2584,7 +2586,7 @@ int batch_tables(Batch &b) {
       natoms += s->n;
       const Kick kk = make_kick(m, 1.0, 0, P<unsigned long long>(m.step_dev));
       Acc *facc = P<Acc>(s->facc);
-      args_kick[i] = {s->npad, kk, m.h, P<int>(s->permp), P<double>(s->fout), P<double>(m.minv), P<double>(m.xbuild),
+      args_kick[i] = {s->npad, kk, m.h, P<int>(s->permp), P<double>(s->fout), P<double4>(m.xbuild),
                       P<double>(m.v), P<double>(s->xorig), P<R4>(s->xs), P<double4>(s->xs64), P<float4>(s->sorg),
                       P<unsigned>(m.dmax), s->pme, pme_slots<R>(s)};
       args_spread[i] = {s->pme, s->plz, P<int2>(s->tcol), P<int>(s->colsc), P<R4>(s->pmw), P<int2>(s->pmb),
@@ -2606,8 +2608,8 @@ int batch_tables(Batch &b) {
       args_gather[i] = {s->pme_g, s->plz, P<int2>(s->tcol) + pm.ntx + pm.nty, P<int>(s->colsc), P<R4>(s->pmw), P<int2>(s->pmb),
                         P<Cx<T>>(s->twz), P<Cx<T>>(s->spec), facc};
       args_fixups[i] = fixup_args<MIXED>(s, false, true, true, &nfix[i]);
-      args_ukd[i] = {s->npad, kk, m.h, P<int>(s->permp), facc, P<double>(s->fout), P<int>(s->tilectr),
-                     P<int>(s->nborder), P<double>(m.minv), P<double>(m.xbuild), P<double>(m.v), P<double>(s->xorig),
+      args_ukd[i] = {s->npad, kk, m.h, P<int>(s->permp), facc, P<int>(s->tilectr), P<int>(s->nborder),
+                     P<double4>(m.xbuild), P<double>(m.v), P<double>(s->xorig),
                      P<R4>(s->xs), P<double4>(s->xs64), P<float4>(s->sorg), P<unsigned>(m.dmax), pm, pme_slots<R>(s)};
       args_unsort[i] = {s->n, P<int>(s->slot), facc, P<double>(s->fout), P<int>(s->tilectr), P<int>(s->nborder)};
       args_begin[i] = {3ll * s->n, P<double>(s->xorig), P<double>(m.v), P<double>(s->fout), P<double>(m.xbak),
@@ -3170,10 +3172,11 @@ unsigned long long pmx_estimate_bytes(const pmx_sys_desc *desc, int kind) {
   s->dry = true;
   if (setup(s) != PMX_OK) return 0;
   unsigned long long b = s->dry_bytes;
-  // device MD state: velocities, masses, build positions, two chunk backups
+  // device MD state: velocities, masses, build positions by slot, two chunk backups
   // of x, v and f, bonded tables (bonds and angles about one per atom in the
   // systems served)
-  if (kind == 1) b += 200ull * (unsigned long long)desc->n + 132ull * (unsigned long long)desc->n + 8192;
+  if (kind == 1)
+    b += 176ull * (unsigned long long)desc->n + 32ull * (unsigned long long)s->npad + 132ull * (unsigned long long)desc->n + 8192;
   return b;
 }
 

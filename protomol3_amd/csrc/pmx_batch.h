@@ -113,7 +113,8 @@ struct OpSplitFill {
     double4 *xs64;
     int *ts;
     const double *xorig;
-    double *xbuild;
+    const double *minv;
+    double4 *xbuild;
     float4 *sorg, *ctr, *half, *sctr, *shalf;
     int *nmaskwork;
     double qpair;
@@ -124,7 +125,7 @@ struct OpSplitFill {
   static constexpr bool kGated = true;
   __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &) {
     split_fill_body<R>(bid, nbk, a.nsuper, a.sc_info, a.sb, a.xwrap, a.permp, a.slot, a.q, a.type, a.xs, a.xs64,
-                       a.ts, a.xorig, a.xbuild, a.sorg, a.ctr, a.half, a.sctr, a.shalf, a.nmaskwork, a.qpair, a.pme,
+                       a.ts, a.xorig, a.minv, a.xbuild, a.sorg, a.ctr, a.half, a.sctr, a.shalf, a.nmaskwork, a.qpair, a.pme,
                        a.rec);
   }
 };
@@ -170,7 +171,8 @@ struct OpKickDrift {
     Kick kick;
     double h;
     const int *perm;
-    const double *fout, *minv, *xbuild;
+    const double *fout;
+    const double4 *xbuild;
     double *v, *x;
     typename Real4<R>::type *xs;
     const double4 *xs64;
@@ -182,8 +184,8 @@ struct OpKickDrift {
   static constexpr int kBlock = 256, kMinBlocks = 1;
   static constexpr bool kGated = false;
   __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &st) {
-    kick_drift_body<R>(bid, nbk, a.n, batch_kick(a.kick, a.h, st.k, st.opening), a.h, a.perm, a.fout, a.minv, a.v,
-                       a.x, a.xbuild, a.xs, a.xs64, a.sorg, a.dmax + st.k, a.pme, a.rec);
+    kick_drift_body<R>(bid, nbk, a.n, batch_kick(a.kick, a.h, st.k, st.opening), a.h, a.perm, a.fout, a.v, a.x,
+                       a.xbuild, a.xs, a.xs64, a.sorg, a.dmax + st.k, a.pme, a.rec);
   }
 };
 
@@ -328,9 +330,8 @@ struct OpUnsortKickDrift {
     double h;
     const int *perm;
     typename AccT<MIXED>::type *facc;
-    double *fout;
     int *tilectr, *nborder;
-    const double *minv, *xbuild;
+    const double4 *xbuild;
     double *v, *x;
     typename Real4<R>::type *xs;
     const double4 *xs64;
@@ -343,7 +344,7 @@ struct OpUnsortKickDrift {
   static constexpr bool kGated = false;
   __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &st) {
     unsort_kick_drift_body<MIXED, R>(bid, nbk, a.n, batch_kick(a.kick, a.h, st.k + 1, false), a.h, a.perm, a.facc,
-                                     a.fout, a.tilectr, a.nborder, a.minv, a.v, a.x, a.xbuild, a.xs, a.xs64, a.sorg,
+                                     a.tilectr, a.nborder, a.v, a.x, a.xbuild, a.xs, a.xs64, a.sorg,
                                      a.dmax + st.k + 1, a.pme, a.rec);
   }
 };

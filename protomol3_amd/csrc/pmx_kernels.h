@@ -478,12 +478,12 @@ constexpr float kScSlack = 1e-3f;
 //    position of the first slot's atom rounded to 1/16 A, in sorg) + charge
 //    times qpair (0 when the pair pass carries no Coulomb term),
 //    FP64 copy in xs64, LJ type (padding: type -1); xbuild (MD only, else
-//    null) receives the positions the list is built from;
+//    null) receives the positions the list is built from and the inverse masses;
 //  - with PME, the atoms' grid records (rec);
 //  - bounding boxes (FP32, list building only): per cluster (8-lane groups;
 //    ctr.w = real atoms, empty clusters get negative half extents), and per
 //    supercluster (the whole wave, widened by kScSlack).
-// Thread 0 also clears the mask work counter of the list build that follows.
+// Thread 0 also clears the mask slot counter for the list build that follows.
 // The atoms by bin (in any order within a bin) and the bins' first positions.
 struct SortedBins {
   int n;
@@ -500,7 +500,8 @@ __device__ __forceinline__ void split_fill_body(const int bid_, const int nbk_, 
                                                 int *__restrict__ slot, const double *__restrict__ q,
                                                 const int *__restrict__ type, typename Real4<R>::type *__restrict__ xs,
                                                 double4 *__restrict__ xs64, int *__restrict__ ts,
-                                                const double *__restrict__ xorig, double *__restrict__ xbuild,
+                                                const double *__restrict__ xorig, const double *__restrict__ minv,
+                                                double4 *__restrict__ xbuild,
                                                 float4 *__restrict__ sorg, float4 *__restrict__ ctr,
                                                 float4 *__restrict__ half, float4 *__restrict__ sctr,
                                                 float4 *__restrict__ shalf, int *__restrict__ nmaskwork, double qpair,
@@ -553,11 +554,7 @@ __device__ __forceinline__ void split_fill_body(const int bid_, const int nbk_, 
   if (lane == 0) sorg[sc] = make_float4((float)o[0], (float)o[1], (float)o[2], 0.f);
   typename Real4<R>::type v;
   if (a >= 0) {
-    if (xbuild) {
-      xbuild[3 * a] = xorig[3 * a];
-      xbuild[3 * a + 1] = xorig[3 * a + 1];
-      xbuild[3 * a + 2] = xorig[3 * a + 2];
-    }
+    if (xbuild) xbuild[s] = make_double4(xorig[3 * a], xorig[3 * a + 1], xorig[3 * a + 2], minv[a]);
     v.x = (R)(p[0] - o[0]);
     v.y = (R)(p[1] - o[1]);
     v.z = (R)(p[2] - o[2]);
@@ -630,13 +627,14 @@ __global__ void __launch_bounds__(256) k_split_fill(int nsuper_max, const int2 *
                                                     const double *__restrict__ q, const int *__restrict__ type,
                                                     typename Real4<R>::type *__restrict__ xs,
                                                     double4 *__restrict__ xs64, int *__restrict__ ts,
-                                                    const double *__restrict__ xorig, double *__restrict__ xbuild,
+                                                    const double *__restrict__ xorig, const double *__restrict__ minv,
+                                                double4 *__restrict__ xbuild,
                                                     float4 *__restrict__ sorg, float4 *__restrict__ ctr,
                                                     float4 *__restrict__ half, float4 *__restrict__ sctr,
                                                     float4 *__restrict__ shalf, int *__restrict__ nmaskwork,
                                                     double qpair, PmeParams pme, PmeSlots<R> rec) {
   split_fill_body<R>(blockIdx.x, gridDim.x, nsuper_max, sc_info, sb, xwrap, permp, slot, q, type, xs, xs64, ts,
-                     xorig, xbuild, sorg, ctr, half, sctr, shalf, nmaskwork, qpair, pme, rec);
+                     xorig, minv, xbuild, sorg, ctr, half, sctr, shalf, nmaskwork, qpair, pme, rec);
 }
 
 
@@ -2690,15 +2688,30 @@ __global__ void __launch_bounds__(kPmeBlock, MIXED ? 8 : 4) k_pme_z_gather(
 // kernel's tile counter and the boundary-pair count, so the next force pass
 // starts from zero without a separate clearing launch (padding slots are
 // never accumulated into).
+// What the last pass of a chunk of MD steps hands to the host: the chunk's
+// displacement record (at most 256 steps) and the overflow flag, both complete
+// by then, into pinned memory.
+struct ChunkEnd {
+  const unsigned *record;
+  int steps;  // 0: none
+  const int *overflow;
+  unsigned *host_record, *host_overflow;
+};
+
 template <bool MIXED>
 __device__ __forceinline__ void unsort_forces_body(const int bid_, const int nbk_, int n, const int *__restrict__ slot,
                                                    typename AccT<MIXED>::type *__restrict__ facc,
                                                    double *__restrict__ fout, int *__restrict__ tilectr,
-                                                   int *__restrict__ nborder) {
+                                                   int *__restrict__ nborder, const ChunkEnd &end = {}) {
   int a = bid_ * blockDim.x + threadIdx.x;
   if (a == 0) {
     *tilectr = 0;
     *nborder = 0;
+  }
+  if (a < end.steps) {
+    end.host_record[a] = end.record[a];
+    if (a == 0) *end.host_overflow = (unsigned)*end.overflow;
+    __threadfence_system();
   }
   if (a >= n) return;
   const int s = slot[a];
@@ -2713,8 +2726,9 @@ __device__ __forceinline__ void unsort_forces_body(const int bid_, const int nbk
 
 template <bool MIXED>
 __global__ void k_unsort_forces(int n, const int *__restrict__ slot, typename AccT<MIXED>::type *__restrict__ facc,
-                                double *__restrict__ fout, int *__restrict__ tilectr, int *__restrict__ nborder) {
-  unsort_forces_body<MIXED>(blockIdx.x, gridDim.x, n, slot, facc, fout, tilectr, nborder);
+                                double *__restrict__ fout, int *__restrict__ tilectr, int *__restrict__ nborder,
+                                ChunkEnd end) {
+  unsort_forces_body<MIXED>(blockIdx.x, gridDim.x, n, slot, facc, fout, tilectr, nborder, end);
 }
 
 // Deterministic energy/pair-stat reduction in one block, in index order.
@@ -3074,6 +3088,22 @@ __device__ inline void apply_kick(const Kick &kk, int a, const double f[3], doub
   }
 }
 
+// The largest of a block's values (>= 0) folded into *dmax: one atomic a block.
+// Adds to one address take about 12 ns each whatever the grid; one per wave
+// bound the kick and drift: 1,000,000 atoms 185 -> 55 us, 26,000 atoms 8.1 -> 5.1.
+__device__ __forceinline__ void record_max(float d, unsigned *__restrict__ dmax) {
+  __shared__ float s_d[256 / kWave];
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) d = fmaxf(d, __shfl_xor(d, m));
+  if ((threadIdx.x & 63) == 0) s_d[threadIdx.x >> 6] = d;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int w = 1; w < 256 / kWave; ++w) d = fmaxf(d, s_d[w]);
+    if (d > 0.f) atomicMax(dmax, __float_as_uint(d));
+  }
+}
+
 // Kick (v += F kick h / m) and drift (x += v h) of every atom, FP64
 // (LeapfrogIntegrator.cpp:33-87).  The pair kernel's sorted coordinates then
 // follow each atom continuously from its wrapped position at the last list
@@ -3082,8 +3112,8 @@ __device__ inline void apply_kick(const Kick &kk, int a, const double f[3], doub
 template <class R>
 __device__ __forceinline__ void kick_drift_body(const int bid_, const int nbk_, int n, Kick kk, double h,
                                                 const int *__restrict__ perm, const double *__restrict__ fout,
-                                                const double *__restrict__ minv, double *__restrict__ v,
-                                                double *__restrict__ x, const double *__restrict__ xbuild,
+                                                double *__restrict__ v, double *__restrict__ x,
+                                                const double4 *__restrict__ xbuild,
                                                 typename Real4<R>::type *__restrict__ xs,
                                                 const double4 *__restrict__ xs64, const float4 *__restrict__ sorg,
                                                 unsigned int *__restrict__ dmax, const PmeParams &pme,
@@ -3094,13 +3124,14 @@ __device__ __forceinline__ void kick_drift_body(const int bid_, const int nbk_, 
   if (a >= 0) {
     double dd[3], xn[3], vv[3] = {v[3 * a], v[3 * a + 1], v[3 * a + 2]};
     const double ff[3] = {fout[3 * a], fout[3 * a + 1], fout[3 * a + 2]};
-    apply_kick(kk, a, ff, minv[a], vv);
+    const double4 xb = xbuild[s];
+    apply_kick(kk, a, ff, xb.w, vv);
     double d2 = 0;
     for (int k = 0; k < 3; ++k) {
       v[3 * a + k] = vv[k];
       const double xk = x[3 * a + k] + vv[k] * h;
       x[3 * a + k] = xn[k] = xk;
-      dd[k] = xk - xbuild[3 * a + k];
+      dd[k] = xk - (k == 0 ? xb.x : k == 1 ? xb.y : xb.z);
       d2 += dd[k] * dd[k];
     }
     d2f = (float)d2;
@@ -3113,34 +3144,33 @@ __device__ __forceinline__ void kick_drift_body(const int bid_, const int nbk_, 
     xs[s] = r;
     if (rec.w) pme_record<R>(pme, rec, s, true, xn, b.w);
   }
-  // wave max, one atomic per wave
-  for (int m = 32; m >= 1; m >>= 1) d2f = fmaxf(d2f, __shfl_xor(d2f, m));
-  if ((threadIdx.x & 63) == 0) atomicMax(dmax, __float_as_uint(d2f));
+  record_max(d2f, dmax);
 }
 
 template <class R>
 __global__ void k_kick_drift(int n, Kick kk, double h, const int *__restrict__ perm,
-                             const double *__restrict__ fout, const double *__restrict__ minv, double *__restrict__ v,
-                             double *__restrict__ x, const double *__restrict__ xbuild,
+                             const double *__restrict__ fout, double *__restrict__ v, double *__restrict__ x,
+                             const double4 *__restrict__ xbuild,
                              typename Real4<R>::type *__restrict__ xs, const double4 *__restrict__ xs64,
                              const float4 *__restrict__ sorg, unsigned int *__restrict__ dmax, PmeParams pme,
                              PmeSlots<R> rec) {
-  kick_drift_body<R>(blockIdx.x, gridDim.x, n, kk, h, perm, fout, minv, v, x, xbuild, xs, xs64, sorg, dmax, pme,
+  kick_drift_body<R>(blockIdx.x, gridDim.x, n, kk, h, perm, fout, v, x, xbuild, xs, xs64, sorg, dmax, pme,
                      rec);
 }
 
 // The end of one MD step and the start of the next in one pass over the
 // sorted slots: the step's forces leave the accumulators (cleared, with the
-// pass counters) for the caller's atom order, and the next step's kick and
-// drift use them at once (k_unsort_forces followed by k_kick_drift).
+// pass counters) for the next step's kick and drift (the force array is
+// written only where a chunk of steps ends).  Bound by memory: positions and
+// velocities are in the caller's order, each 24 bytes of one or two lines;
+// build positions and inverse masses lie by slot.
 template <bool MIXED, class R>
 __device__ __forceinline__ void unsort_kick_drift_body(const int bid_, const int nbk_, int n, const Kick &kk, double h,
                                                        const int *__restrict__ perm,
                                                        typename AccT<MIXED>::type *__restrict__ facc,
-                                                       double *__restrict__ fout, int *__restrict__ tilectr,
-                                                       int *__restrict__ nborder, const double *__restrict__ minv,
+                                                       int *__restrict__ tilectr, int *__restrict__ nborder,
                                                        double *__restrict__ v, double *__restrict__ x,
-                                                       const double *__restrict__ xbuild,
+                                                       const double4 *__restrict__ xbuild,
                                                        typename Real4<R>::type *__restrict__ xs,
                                                        const double4 *__restrict__ xs64,
                                                        const float4 *__restrict__ sorg,
@@ -3162,16 +3192,16 @@ __device__ __forceinline__ void unsort_kick_drift_body(const int bid_, const int
       else
         ff[k] = ((const double *)facc)[3 * s + k];
       facc[3 * s + k] = 0;
-      fout[3 * a + k] = ff[k];
     }
     double dd[3], xn[3], vv[3] = {v[3 * a], v[3 * a + 1], v[3 * a + 2]};
-    apply_kick(kk, a, ff, minv[a], vv);
+    const double4 xb = xbuild[s];
+    apply_kick(kk, a, ff, xb.w, vv);
     double d2 = 0;
     for (int k = 0; k < 3; ++k) {
       v[3 * a + k] = vv[k];
       const double xk = x[3 * a + k] + vv[k] * h;
       x[3 * a + k] = xn[k] = xk;
-      dd[k] = xk - xbuild[3 * a + k];
+      dd[k] = xk - (k == 0 ? xb.x : k == 1 ? xb.y : xb.z);
       d2 += dd[k] * dd[k];
     }
     d2f = (float)d2;
@@ -3184,20 +3214,17 @@ __device__ __forceinline__ void unsort_kick_drift_body(const int bid_, const int
     xs[s] = r;
     if (rec.w) pme_record<R>(pme, rec, s, true, xn, b.w);
   }
-  for (int m = 32; m >= 1; m >>= 1) d2f = fmaxf(d2f, __shfl_xor(d2f, m));
-  if ((threadIdx.x & 63) == 0) atomicMax(dmax, __float_as_uint(d2f));
+  record_max(d2f, dmax);
 }
 
 template <bool MIXED, class R>
 __global__ void k_unsort_kick_drift(int n, Kick kk, double h, const int *__restrict__ perm,
-                                    typename AccT<MIXED>::type *__restrict__ facc, double *__restrict__ fout,
-                                    int *__restrict__ tilectr, int *__restrict__ nborder,
-                                    const double *__restrict__ minv, double *__restrict__ v,
-                                    double *__restrict__ x, const double *__restrict__ xbuild,
+                                    typename AccT<MIXED>::type *__restrict__ facc, int *__restrict__ tilectr,
+                                    int *__restrict__ nborder, double *__restrict__ v, double *__restrict__ x, const double4 *__restrict__ xbuild,
                                     typename Real4<R>::type *__restrict__ xs, const double4 *__restrict__ xs64,
                                     const float4 *__restrict__ sorg, unsigned int *__restrict__ dmax, PmeParams pme,
                                     PmeSlots<R> rec) {
-  unsort_kick_drift_body<MIXED, R>(blockIdx.x, gridDim.x, n, kk, h, perm, facc, fout, tilectr, nborder, minv, v, x,
+  unsort_kick_drift_body<MIXED, R>(blockIdx.x, gridDim.x, n, kk, h, perm, facc, tilectr, nborder, v, x,
                                    xbuild, xs, xs64, sorg, dmax, pme, rec);
 }
 
