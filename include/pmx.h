@@ -202,7 +202,8 @@ int pmx_sys_time_pair(pmx_sys *sys, int reps, float *ms_per_launch);
  * PMX_TUNE_FIXUP_STREAM  0 (default from 100,000 atoms): the exclusion
  *                        correction and the bonded terms run on the second
  *                        stream after the PME chain; 1 (default below 100,000
- *                        atoms): on the main stream, in one launch with the
+ *                        atoms): on the main stream, with the charge spread
+ *                        where that runs there too, else in one launch with the
  *                        boundary pairs after the pair kernel (better where
  *                        the PME chain is the longer branch);
  * PMX_TUNE_FUSED_SPREAD  0 or 1, no effect: the charge spread is one launch

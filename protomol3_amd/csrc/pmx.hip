@@ -1117,15 +1117,24 @@ PmeSlots<R> pme_slots(Sys *s) {
   return PmeSlots<R>{P<typename Real4<R>::type>(s->pmw), P<int2>(s->pmb)};
 }
 
-// Charge spread with the z transform (order: even, 2..8).
+// Charge spread with the z transform (order: even, 2..8); with: the atoms'
+// terms in the same launch (blocks of 256 threads).
 template <bool MIXED>
-void run_spread(Sys *s, hipStream_t st) {
+void run_spread(Sys *s, hipStream_t st, bool with = false) {
   using T = typename std::conditional<MIXED, float, double>::type;
   using T4 = typename Real4<T>::type;
-#define PMX_SPREAD(ORD)                                                                                              \
-  hipLaunchKernelGGL((k_pme_spread_z<MIXED, ORD>), dim3(s->pme.ntx * s->pme.nty), dim3(s->thr_z), s->lds_z, st,      \
-                     s->pme, s->plz, P<int2>(s->tcol), P<int>(s->colsc), P<T4>(s->pmw), P<int2>(s->pmb),              \
-                     P<Cx<T>>(s->twz), P<Cx<T>>(s->spec))
+  int nterms = 0;
+  FixupArgs<MIXED> terms{};
+  if (with) terms = fixup_args<MIXED>(s, false, false, true, &nterms);
+#define PMX_SPREAD_ARGS \
+  s->pme, s->plz, P<int2>(s->tcol), P<int>(s->colsc), P<T4>(s->pmw), P<int2>(s->pmb), P<Cx<T>>(s->twz), P<Cx<T>>(s->spec)
+#define PMX_SPREAD(ORD)                                                                                             \
+  if (nterms)                                                                                                       \
+    hipLaunchKernelGGL((k_pme_spread_terms<MIXED, ORD>), dim3(s->pme.ntx * s->pme.nty + nterms), dim3(s->thr_z),    \
+                       s->lds_z, st, PMX_SPREAD_ARGS, terms);                                                       \
+  else                                                                                                              \
+    hipLaunchKernelGGL((k_pme_spread_z<MIXED, ORD>), dim3(s->pme.ntx * s->pme.nty), dim3(s->thr_z), s->lds_z, st,   \
+                       PMX_SPREAD_ARGS)
   switch (s->pme.order) {
     case 2: PMX_SPREAD(2); break;
     case 4: PMX_SPREAD(4); break;
@@ -1133,6 +1142,7 @@ void run_spread(Sys *s, hipStream_t st) {
     default: PMX_SPREAD(8); break;
   }
 #undef PMX_SPREAD
+#undef PMX_SPREAD_ARGS
 }
 
 // The transforms and the force gather on the second stream.
@@ -1307,11 +1317,14 @@ int forces(Sys *s, unsigned flags, bool energies, const Kick *next = nullptr, un
   hipStream_t st2 = s->ctx->stream2;
   const bool spread = s->pme_on && (s->d.pme_terms & PMX_PME_RECIP);
   const bool spread2 = spread && s->tune_spread_stream2;
+  // with the spread on the main stream go the correction and the bonded terms
+  // that would follow the pair kernel there
+  const bool terms_early = spread && !spread2 && s->tune_fixup_main && s->thr_z == 256;
   if (spread && !spread2) {
     if (s->mixed)
-      run_spread<true>(s, st);
+      run_spread<true>(s, st, terms_early);
     else
-      run_spread<false>(s, st);
+      run_spread<false>(s, st, terms_early);
   }
   HIPCHK(hipEventRecord(s->fork_ev, st));
   HIPCHK(hipStreamWaitEvent(st2, s->fork_ev, 0));
@@ -1334,10 +1347,10 @@ int forces(Sys *s, unsigned flags, bool energies, const Kick *next = nullptr, un
     hipEventRecord(s->ev[5], st2);
     hipEventRecord(s->ev[6], st2);
   }
-  // the exclusion correction and bonded terms on the second stream (after
-  // the PME chain), or with the boundary pairs on the main stream after the
-  // pair kernel (tuning knob)
-  const int fix_phase = s->tune_fixup_main ? 3 : 1;
+  // the exclusion correction and bonded terms (unless they went with the
+  // spread) on the second stream (after the PME chain), or with the boundary
+  // pairs on the main stream after the pair kernel (tuning knob)
+  const int fix_phase = s->tune_fixup_main && !terms_early ? 3 : 1;
   if (!s->tune_fixup_main) {
     if (s->mixed)
       run_pair_phase<true>(s, stats, 2);

@@ -3056,6 +3056,24 @@ __global__ void __launch_bounds__(256) k_fixups(FixupArgs<MIXED> a) {
   fixups_body<MIXED, COUL, LJSW, CSW>(blockIdx.x, gridDim.x, a);
 }
 
+// Charge spread and the atoms' terms in one launch, where the spread has the
+// device to itself: its blocks leave most CUs idle, and the terms, a chain of
+// dependent FP64 operations of 9 us, no longer follow the pair kernel.  A step of
+// 1,500 atoms 61.6 -> 60.2 us, 9,400 atoms 81.7 -> 80.5.
+template <bool MIXED, int P>
+__global__ void __launch_bounds__(kPmeBlock, 4) k_pme_spread_terms(
+    PmeParams p, FftPlan pl, const int2 *__restrict__ tcol, const int *__restrict__ colsc,
+    const typename Real4<typename std::conditional<MIXED, float, double>::type>::type *__restrict__ pmw,
+    const int2 *__restrict__ pmb, const Cx<typename std::conditional<MIXED, float, double>::type> *__restrict__ tw,
+    Cx<typename std::conditional<MIXED, float, double>::type> *__restrict__ spec, FixupArgs<MIXED> a) {
+  const int tiles = p.ntx * p.nty, b = blockIdx.x;
+  if (b < tiles)
+    pme_spread_z_body<MIXED, P>(xcd_block(b, tiles), tiles, p, pl, tcol, colsc, pmw, pmb, tw, spec);
+  else
+    atom_terms_block<MIXED>(b - tiles, a.npad, a.perm, a.xorig, a.q, a.pp.box, a.alpha, a.csf, a.at, a.facc, a.corr_e,
+                            a.bond_e);
+}
+
 // Velocity kicks of one leapfrog step.  Leapfrog (LeapfrogIntegrator.cpp):
 // v += F h_kick / m.  Langevin leapfrog (LangevinLeapfrogIntegrator.cpp:
 // 44-71): nhalf half kicks v = v vdt + F fdt / m + g sqrt(fc / m) ndt, g a
