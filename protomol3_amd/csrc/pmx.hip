@@ -127,6 +127,7 @@ struct Sys {
   int xlog = 0, ylog = 0;              // lines of a block of the x and y passes (log2)
   size_t lds_z = 0, lds_g = 0, lds_y = 0, lds_x = 0, lds_p = 0;  // dynamic LDS of the PME launches
   int thr_z = 256, thr_g = 256, thr_y = 256, thr_x = 256, thr_p = 256;  // and their block sizes
+  int thr_gb = 256, thr_pb = 256;  // gather and plane in batched launches
   // device buffers
   std::vector<DevBuf *> all;
   DevBuf xorig, xwrap, q_d, type_d, key, hist, start, cursor, scansum, perm, permp, slot, refcell, xs, xs64, ts,
@@ -504,13 +505,22 @@ int fft_blocking(Sys *s) {
   s->lds_x = cx * (((size_t)(pm.nx | 1) << s->xlog) + pm.nx);
   s->lds_p = cx * ((size_t)(pm.nx | 1) * pm.ny + pm.nx + pm.ny);
   // threads: a line needs n / kFftPerThread; the tiles and planes transform
-  // as many lines at a time as the block has threads for
+  // as many lines at a time as the block has threads for.  Planes and the
+  // gather take 512, which finds room beside the pair kernel's four blocks of 80
+  // registers: a step of 4,000 / 9,400 / 13,800 / 26,000 / 1,000,000 atoms
+  // 65.9 / 80.5 / 87.1 / 105.5 / 1,501 us with 256, 63.7 / 75.7 / 78.0 /
+  // 97.3 / 1,465 with 512.  The spread and the line passes on large grids do
+  // better with two blocks of 256 (1,000,000 atoms 1,465 -> 1,592 and 1,527), and
+  // so do planes and gather in batches, which fill the device (64 systems 24.0
+  // ms with 256, 24.8 with 512; 16 in FP64 14.0 and 14.9).
   auto threads = [&](int n, int l) { return ((long long)n << l) > small ? 512 : 256; };
   s->thr_z = alone && wide ? 512 : threads(pm.nz, 0);
-  s->thr_g = threads(pm.nz, 0);
+  s->thr_g = kPmeBlock;
+  s->thr_gb = threads(pm.nz, 0);
   s->thr_y = threads(pm.ny, s->ylog);
   s->thr_x = threads(pm.nx, s->xlog);
-  s->thr_p = threads(std::max(pm.nx, pm.ny), 0);
+  s->thr_p = kPmeBlock;
+  s->thr_pb = threads(std::max(pm.nx, pm.ny), 0);
   s->fft_plane = s->tune_fft_planes && pm.nx * pm.ny <= kFftPlanePoints && s->lds_p <= 36864;
   s->recip_blocks = s->fft_plane ? pm.nzh : pm.nzh * ((pm.ny + (1 << s->xlog) - 1) >> s->xlog);
   // the columns of the sort that can hold atoms whose stencils touch a row or
@@ -2616,7 +2626,7 @@ int batch_tables(Batch &b) {
       args_xconv[i] = {pm, s->plx, s->xlog, s->thr_x, P<Cx<T>>(s->twx), P<T>(s->theta), P<Cx<T>>(s->spec),
                        P<double>(s->recip_e)};
       args_yinv[i] = {pm, s->ply, s->ylog, true, P<Cx<T>>(s->twy), P<Cx<T>>(s->spec)};
-      args_plane[i] = {pm, s->ply, s->plx, s->thr_p, P<Cx<T>>(s->twy), P<Cx<T>>(s->twx), P<T>(s->theta), P<Cx<T>>(s->spec),
+      args_plane[i] = {pm, s->ply, s->plx, s->thr_pb, P<Cx<T>>(s->twy), P<Cx<T>>(s->twx), P<T>(s->theta), P<Cx<T>>(s->spec),
                        P<double>(s->recip_e)};
       args_gather[i] = {s->pme_g, s->plz, P<int2>(s->tcol) + pm.ntx + pm.nty, P<int>(s->colsc), P<R4>(s->pmw), P<int2>(s->pmb),
                         P<Cx<T>>(s->twz), P<Cx<T>>(s->spec), facc};
@@ -2641,12 +2651,12 @@ int batch_tables(Batch &b) {
       // dynamic LDS and block size of each launch: the largest of the
       // systems it serves
       thr_z = std::max(thr_z, s->thr_z);
-      thr_g = std::max(thr_g, s->thr_g);
+      thr_g = std::max(thr_g, s->thr_gb);
       lds_g = std::max(lds_g, s->lds_g);
       lds_z = std::max(lds_z, s->lds_z);
       if (s->fft_plane) {
         lds_p = std::max(lds_p, s->lds_p);
-        thr_p = std::max(thr_p, s->thr_p);
+        thr_p = std::max(thr_p, s->thr_pb);
       } else {
         lds_y = std::max(lds_y, s->lds_y);
         lds_x = std::max(lds_x, s->lds_x);
