@@ -153,7 +153,9 @@ struct Sys {
   // pinned staging of this system's copies to and from the host, in chunks
   // beyond kStageChunks x kStageChunk bytes (stage_ev: a chunk's copy is done)
   HostBuf stage;
-  bool staged = false;  // the stage holds the last pass's results and forces (batched passes)
+  bool staged = false;  // the stage holds the last pass's results and forces (batched passes); cleared by
+                        // whatever may write new ones
+  bool recorded = false;  // a pass was recorded into a graph, whose replays the host does not see: never staged
   hipEvent_t stage_ev[4] = {nullptr, nullptr, nullptr, nullptr};
   // device-resident MD state
   struct Md {
@@ -1409,6 +1411,8 @@ int forces(Sys *s, unsigned flags, bool energies, const Kick *next = nullptr, un
 
 int compute(Sys *s, unsigned flags) {
   const bool timing = flags & PMX_EVAL_TIMING;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s->ctx->stream, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone) s->recorded = true;
   timing_begin_call(s, timing);
   int rc = rebuild(s, timing, true);
   if (rc) return rc;
@@ -1478,6 +1482,8 @@ int send(Sys *s, void *dst, const void *src, size_t bytes) {
 // The results of a pass, and then its forces, in the stage.
 constexpr size_t kResultWords = sizeof(PassResults) / 8;
 bool results_fit(const Sys *s) { return 8 * (kResultWords + 3 * (size_t)s->n) <= kStageBytes; }
+// A batched pass brings this system's results to the host.
+bool batch_stages(const Sys *s) { return results_fit(s) && !s->recorded; }
 
 struct OutList {
   OutArgs a{};
@@ -2225,6 +2231,7 @@ int enqueue_chunk(Sys *s, const Chunk &c) {
       }
     }
   }
+  s->staged = false;  // a replay runs no host code of the passes in it
   if (x) {
     hipLaunchKernelGGL(k_set_u64, dim3(1), dim3(1), 0, st, P<unsigned long long>(m.step_dev),
                        (unsigned long long)c.step0);
@@ -2640,7 +2647,7 @@ int batch_tables(Batch &b) {
       args_half[i] = {s->n, kk, m.h, P<double>(s->fout), P<double>(m.minv), P<double>(m.v)};
       args_energy[i] = {s->n, P<int>(s->slot), facc, P<double>(s->fout), P<int>(s->tilectr), P<int>(s->nborder),
                         energy_args(s, false)};
-      if (b.results && results_fit(s)) {
+      if (b.results && batch_stages(s)) {
         if ((rc = stage_get(s, 8 * (kResultWords + 3 * (size_t)s->n)))) return rc;
         OutList out(s->stage.p);
         out.add(s->eout.p, kResultWords);
@@ -2820,7 +2827,7 @@ int batch_forces(Batch &b, bool *grown) {
     s->list_valid = true;
     s->prune_pending = false;
     s->acc_clean = true;
-    s->staged = b.results && results_fit(s);
+    s->staged = b.results && batch_stages(s);
     for (int attempt = 0; b.flags_h[i] && attempt < 6; ++attempt) {
       *grown = true;
       if ((rc = grow_and_retry(s)) || (rc = compute(s, 0))) return rc;
@@ -3061,6 +3068,7 @@ int batch_entry(pmx_sys *const *systems, int nsys, int nsteps) {
   for (int i = 0; i < nsys; ++i) b.first_forces &= !systems[i]->s.md.forces_valid;
   for (int i = 0; i < nsys; ++i) {
     Sys *s = &systems[i]->s;
+    s->staged = false;
     b.sys.push_back(s);
     if (!s->cached)
       if (int rc = setup(s)) return rc;
