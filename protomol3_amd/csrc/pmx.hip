@@ -147,6 +147,7 @@ struct Sys {
   bool have_positions = false;
   bool cached = false;
   bool list_valid = false;             // entries, counts and work of a built list are in place
+  bool reduced = false;                // eout holds the energies of the last pass (whose partials may be gone)
   bool acc_clean = false;              // force accumulators and pass counters are zero
   bool dry = false;                    // size only: allocations are counted, nothing runs
   unsigned long long dry_bytes = 0;
@@ -1207,6 +1208,13 @@ EnergyArgs energy_args(Sys *s, bool stats) {
           P<unsigned long long>(s->hash_out)};
 }
 
+// The energies of the last pass into eout, unless they are there.
+void reduce_energies(Sys *s) {
+  if (!s->reduced)
+    hipLaunchKernelGGL(k_reduce_energy, dim3(1), dim3(kEndBlock), 0, s->ctx->stream, energy_args(s, false));
+  s->reduced = true;
+}
+
 void timing_begin_call(Sys *s, bool timing) {
   if (!timing) return;
   RtLock lk(g_rt_mu);
@@ -1320,6 +1328,7 @@ int forces(Sys *s, unsigned flags, bool energies, const Kick *next = nullptr, un
   if (!s->acc_clean) launch_zero(s);
   s->acc_clean = false;
   s->staged = false;
+  s->reduced = energies;
   if (timing) hipEventRecord(s->ev[2], st);
   // fork: FFT, gather, exclusion correction and bonded terms on the second
   // stream beside the pair kernel; all add into the zeroed accumulators.
@@ -1921,9 +1930,11 @@ int pmx_sys_set_tuning(pmx_sys *sys, int knob, int value) {
     default:
       return fail(s->ctx, PMX_ERR_ARG, "unknown tuning knob");
   }
-  // captured chunks hold the old launch shapes; the energy partials of the
-  // x pass may be reallocated, and the tile windows change
+  // captured chunks hold the old launch shapes; the tiles of the list and
+  // the blocks of the x pass change, and with them the places of the energy
+  // partials: those of the state at hand are added up before
   hipSetDevice(s->ctx->device);
+  if (s->md.on && s->md.forces_valid) reduce_energies(s);
   HIPCHK(hipStreamSynchronize(s->ctx->stream));
   HIPCHK(hipStreamSynchronize(s->ctx->stream2));
   {
@@ -2231,7 +2242,7 @@ int enqueue_chunk(Sys *s, const Chunk &c) {
       }
     }
   }
-  s->staged = false;  // a replay runs no host code of the passes in it
+  s->staged = s->reduced = false;  // a replay runs no host code of the passes in it
   if (x) {
     hipLaunchKernelGGL(k_set_u64, dim3(1), dim3(1), 0, st, P<unsigned long long>(m.step_dev),
                        (unsigned long long)c.step0);
@@ -2828,6 +2839,7 @@ int batch_forces(Batch &b, bool *grown) {
     s->prune_pending = false;
     s->acc_clean = true;
     s->staged = b.results && batch_stages(s);
+    s->reduced = b.results;
     for (int attempt = 0; b.flags_h[i] && attempt < 6; ++attempt) {
       *grown = true;
       if ((rc = grow_and_retry(s)) || (rc = compute(s, 0))) return rc;
@@ -3068,7 +3080,7 @@ int batch_entry(pmx_sys *const *systems, int nsys, int nsteps) {
   for (int i = 0; i < nsys; ++i) b.first_forces &= !systems[i]->s.md.forces_valid;
   for (int i = 0; i < nsys; ++i) {
     Sys *s = &systems[i]->s;
-    s->staged = false;
+    s->staged = s->reduced = false;
     b.sys.push_back(s);
     if (!s->cached)
       if (int rc = setup(s)) return rc;
@@ -3145,7 +3157,7 @@ int pmx_md_get_state(pmx_sys *sys, double *x, double *v, double *energies) {
     // potential energies at the current positions (computed first if the
     // state was just set) and kinetic energy of v
     if (int rc = md_ensure_forces(s)) return rc;
-    hipLaunchKernelGGL(k_reduce_energy, dim3(1), dim3(kEndBlock), 0, st, energy_args(s, false));
+    reduce_energies(s);
     hipLaunchKernelGGL(k_kinetic, dim3(nblk(n, 256)), dim3(256), 0, st, n, P<double>(m.v), P<double>(m.minv),
                        P<double>(m.ke_e));
   }

@@ -54,3 +54,48 @@ def test_forces_of_a_run_after_a_batched_evaluation(ctx, how, graphs):
         scale = np.abs(f).max()
         assert np.abs(f - f_old).max() > 1e-3 * scale
         assert np.abs(f - g).max() <= 1e-8 * scale
+
+
+@pytest.mark.parametrize("precision", [pmx.MIXED, pmx.FP64])
+@pytest.mark.parametrize("how", ["batch", "run"])
+def test_energies_of_the_state_under_new_launch_shapes(ctx, how, precision):
+    """The energies of the state at hand do not change with the launch shapes
+    set after the run (the list is cut into other runs, the x pass into other
+    blocks), nor with a force pass that keeps its partials elsewhere."""
+    sys_ = [_make(ctx, n, 40 + n, precision) for n in (900, 4000)]
+    try:
+        if how == "batch":
+            pmx.run_batch(sys_, 16)
+        else:
+            for sy in sys_:
+                sy.md_run(16)
+        for sy, first in zip(sys_, (False, True)):
+            e0 = sy.md_get_state()[2] if first else None
+            for knob, value in ((pmx.TUNE_PAIR_BLOCKS_PER_CU, 1), (pmx.TUNE_FFT_PLANES, 0), (pmx.TUNE_FFT_LINES, 1),
+                                (pmx.TUNE_FFT_PLANES, 1)):
+                sy.set_tuning(knob, value)
+                e = sy.md_get_state()[2]
+                if e0 is None:
+                    e0 = e
+                assert e == e0, (knob, value)
+            x, _, _ = sy.md_get_state()
+            _, ec, elj = sy.evaluate(x)
+            # FP32 pair energies summed over other runs: 1e-6 of their magnitudes
+            tol = 1e-9 if precision == pmx.FP64 else 1e-6
+            size = abs(ec) + abs(elj)
+            assert abs(e0["coulomb"] - ec) <= tol * size + (1e-3 if precision == pmx.MIXED else 0.0)
+            assert abs(e0["lj"] - elj) <= tol * size + (1e-3 if precision == pmx.MIXED else 0.0)
+        if how == "batch":
+            pmx.run_batch(sys_, 16)
+        for sy in sys_:
+            if how == "run":
+                sy.md_run(16)
+            sy.compute_noalloc()
+            e = sy.md_get_state()[2]
+            _, ec, elj = sy.evaluate(sy.md_get_state()[0])
+            size = abs(ec) + abs(elj)
+            tol = (1e-9 if precision == pmx.FP64 else 1e-6) * size + (1e-3 if precision == pmx.MIXED else 0.0)
+            assert abs(e["coulomb"] - ec) <= tol and abs(e["lj"] - elj) <= tol
+    finally:
+        for sy in sys_:
+            sy.close()
