@@ -2453,7 +2453,7 @@ struct Batch {
   std::vector<Sys *> sys;
   int nsys = 0;
   bool results = false;       // a force pass alone: its results go to the systems' stages with it
-  bool first_forces = false;  // MD: the forces at the set positions come first, for every system
+  bool first_forces = false;  // MD: the forces at the set positions come first, for every system; no energies
   BatchLaunch bin, scan, scatter, split, list, runs;
   BatchLaunch kick, spread, pair, yfwd, xconv, yinv, plane, gather, fixups, ukd, unsort, begin, half;
   BatchLaunch energy, out;
@@ -2790,8 +2790,8 @@ int batch_chunk(Batch &b, int K, bool opening) {
 }
 
 // One force pass of every system of the batch at its set positions (list
-// rebuilt for all), with the energies reduced: the work of compute() for
-// each.  Systems whose list outgrew its buffers are grown and computed again
+// rebuilt for all): the work of compute() for each, or of md_ensure_forces
+// (first_forces), which leaves the last evaluation's energies.  Systems whose list outgrew its buffers are grown and computed again
 // alone (*grown: the tables hold their old buffers).
 template <bool MIXED, int C, int LJ, int CS, bool BIGLJ, int ORDER>
 int batch_forces(Batch &b, bool *grown) {
@@ -2826,7 +2826,10 @@ int batch_forces(Batch &b, bool *grown) {
   BHIPCHK(hipEventRecord(b.join, st2));
   batch_go<OpFixups<MIXED, C, LJ, CS>>(b.fixups, st, bk);
   BHIPCHK(hipStreamWaitEvent(st, b.join, 0));
-  batch_go<OpUnsortEnergy<MIXED>>(b.energy, st, bk);
+  if (b.first_forces)
+    batch_go<OpUnsortForces<MIXED>>(b.unsort, st, bk);
+  else
+    batch_go<OpUnsortEnergy<MIXED>>(b.energy, st, bk);
   batch_go<OpOut>(b.out, st, bk);
   hipLaunchKernelGGL(k_batch_flags, dim3(nblk(ns, 256)), dim3(256), 0, st, ns,
                      reinterpret_cast<const BatchSys *>(b.bsys.p), reinterpret_cast<int *>(b.flags.p));
@@ -2917,6 +2920,7 @@ int batch_run(Batch &b, int nsteps) {
     s->md.steps += nsteps;
     s->md.rebuilds += nreb[i];
     s->list_valid = true;
+    s->reduced = false;
     s->prune_pending = false;
     s->acc_clean = true;
   }

@@ -99,3 +99,30 @@ def test_energies_of_the_state_under_new_launch_shapes(ctx, how, precision):
     finally:
         for sy in sys_:
             sy.close()
+
+
+def _mixed(ctx, s, spec):
+    sy = pmx.System(ctx, s, spec, pmx.MIXED)
+    sy.md_init(s, 1.0, skin=1.0)
+    sy.md_set_state(s.pos, s.vel)
+    return sy
+
+
+@pytest.mark.parametrize("how", ["batch", "run"])
+def test_a_run_leaves_the_energies_of_the_last_evaluation(ctx, how):
+    """pmx_sys_get_forces gives the last step's forces and the energies and
+    pair statistics of the last evaluation, in either kind of run."""
+    s = systems.replica_box(900, 13).with_velocities(300.0, seed=14)
+    sy = _mixed(ctx, s, serve.request_spec(s))
+    try:
+        _, ec, elj = sy.evaluate(s.pos + 0.05 * np.sin(np.arange(3 * s.n).reshape(-1, 3)), pmx.EVAL_PAIRSTATS)
+        stats = sy.pair_stats()
+        sy.md_set_state(s.pos, s.vel)
+        if how == "batch":
+            pmx.run_batch([sy], 10)
+        else:
+            sy.md_run(10)
+        _, ec2, elj2 = sy.get_forces()
+        assert (ec2, elj2) == (ec, elj) and sy.pair_stats() == stats
+    finally:
+        sy.close()
