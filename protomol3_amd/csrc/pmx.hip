@@ -2791,67 +2791,68 @@ int batch_chunk(Batch &b, int K, bool opening) {
 
 // One force pass of every system of the batch at its set positions (list
 // rebuilt for all): the work of compute() for each, or of md_ensure_forces
-// (first_forces), which leaves the last evaluation's energies.  Systems whose list outgrew its buffers are grown and computed again
-// alone (*grown: the tables hold their old buffers).
+// (first_forces), which leaves the last evaluation's energies.  Where a list
+// outgrew its buffers they are grown and the batch computed again: a system
+// computed alone would get another cut of its list, and in the mixed form
+// other last bits than without the growth.
 template <bool MIXED, int C, int LJ, int CS, bool BIGLJ, int ORDER>
-int batch_forces(Batch &b, bool *grown) {
+int batch_forces(Batch &b) {
   using R = typename std::conditional<MIXED, float, double>::type;
   using T = R;
   hipStream_t st = b.ctx->stream, st2 = b.ctx->stream2;
   const int ns = b.nsys;
-  int rc;
-  for (Sys *s : b.sys)
-    if (!s->acc_clean) launch_zero(s);
   std::vector<unsigned char> all(ns, 1);
-  BHIPCHK(hipMemcpyAsync(b.need.p, all.data(), ns, hipMemcpyHostToDevice, st));
-  BHIPCHK(hipMemcpyAsync(b.bsys.p, b.bsys_h, sizeof(BatchSys) * ns, hipMemcpyHostToDevice, st));
-  hipLaunchKernelGGL(k_batch_clear, dim3(nblk(ns, 256)), dim3(256), 0, st, ns,
-                     reinterpret_cast<const BatchSys *>(b.bsys.p));
-  const BatchStep bk{0, 0, reinterpret_cast<unsigned char *>(b.need.p)};
-  batch_go<OpBin>(b.bin, st, bk);
-  batch_go<OpScanColumns>(b.scan, st, bk);
-  batch_go<OpScatter>(b.scatter, st, bk);
-  batch_go<OpSplitFill<R>>(b.split, st, bk);
-  batch_go<OpBuildList>(b.list, st, bk);
-  batch_go<OpRuns>(b.runs, st, bk);
-  batch_go<OpPmeSpreadZ<MIXED, ORDER>>(b.spread, st, bk);
-  BHIPCHK(hipEventRecord(b.fork, st));
-  BHIPCHK(hipStreamWaitEvent(st2, b.fork, 0));
-  batch_go<PairOp<MIXED, C, LJ, CS, BIGLJ, ORDER>>(b.pair, st, bk);
-  batch_go<OpFftPlane<T>>(b.plane, st2, bk);
-  batch_go<OpFftY<T>>(b.yfwd, st2, bk);
-  batch_go<OpFftXConv<T>>(b.xconv, st2, bk);
-  batch_go<OpFftY<T>>(b.yinv, st2, bk);
-  batch_go<OpPmeZGather<MIXED, ORDER>>(b.gather, st2, bk);
-  BHIPCHK(hipEventRecord(b.join, st2));
-  batch_go<OpFixups<MIXED, C, LJ, CS>>(b.fixups, st, bk);
-  BHIPCHK(hipStreamWaitEvent(st, b.join, 0));
-  if (b.first_forces)
-    batch_go<OpUnsortForces<MIXED>>(b.unsort, st, bk);
-  else
-    batch_go<OpUnsortEnergy<MIXED>>(b.energy, st, bk);
-  batch_go<OpOut>(b.out, st, bk);
-  hipLaunchKernelGGL(k_batch_flags, dim3(nblk(ns, 256)), dim3(256), 0, st, ns,
-                     reinterpret_cast<const BatchSys *>(b.bsys.p), reinterpret_cast<int *>(b.flags.p));
-  BHIPCHK(hipMemcpyAsync(b.flags_h, b.flags.p, 4 * (size_t)ns, hipMemcpyDeviceToHost, st));
-  BHIPCHK(hipGetLastError());
-  BHIPCHK(hipStreamSynchronize(st));
-  for (int i = 0; i < ns; ++i) {
-    Sys *s = b.sys[i];
+  for (int attempt = 0;; ++attempt) {
+    for (Sys *s : b.sys)
+      if (!s->acc_clean) launch_zero(s);
+    BHIPCHK(hipMemcpyAsync(b.need.p, all.data(), ns, hipMemcpyHostToDevice, st));
+    BHIPCHK(hipMemcpyAsync(b.bsys.p, b.bsys_h, sizeof(BatchSys) * ns, hipMemcpyHostToDevice, st));
+    hipLaunchKernelGGL(k_batch_clear, dim3(nblk(ns, 256)), dim3(256), 0, st, ns,
+                       reinterpret_cast<const BatchSys *>(b.bsys.p));
+    const BatchStep bk{0, 0, reinterpret_cast<unsigned char *>(b.need.p)};
+    batch_go<OpBin>(b.bin, st, bk);
+    batch_go<OpScanColumns>(b.scan, st, bk);
+    batch_go<OpScatter>(b.scatter, st, bk);
+    batch_go<OpSplitFill<R>>(b.split, st, bk);
+    batch_go<OpBuildList>(b.list, st, bk);
+    batch_go<OpRuns>(b.runs, st, bk);
+    batch_go<OpPmeSpreadZ<MIXED, ORDER>>(b.spread, st, bk);
+    BHIPCHK(hipEventRecord(b.fork, st));
+    BHIPCHK(hipStreamWaitEvent(st2, b.fork, 0));
+    batch_go<PairOp<MIXED, C, LJ, CS, BIGLJ, ORDER>>(b.pair, st, bk);
+    batch_go<OpFftPlane<T>>(b.plane, st2, bk);
+    batch_go<OpFftY<T>>(b.yfwd, st2, bk);
+    batch_go<OpFftXConv<T>>(b.xconv, st2, bk);
+    batch_go<OpFftY<T>>(b.yinv, st2, bk);
+    batch_go<OpPmeZGather<MIXED, ORDER>>(b.gather, st2, bk);
+    BHIPCHK(hipEventRecord(b.join, st2));
+    batch_go<OpFixups<MIXED, C, LJ, CS>>(b.fixups, st, bk);
+    BHIPCHK(hipStreamWaitEvent(st, b.join, 0));
+    if (b.first_forces)
+      batch_go<OpUnsortForces<MIXED>>(b.unsort, st, bk);
+    else
+      batch_go<OpUnsortEnergy<MIXED>>(b.energy, st, bk);
+    batch_go<OpOut>(b.out, st, bk);
+    hipLaunchKernelGGL(k_batch_flags, dim3(nblk(ns, 256)), dim3(256), 0, st, ns,
+                       reinterpret_cast<const BatchSys *>(b.bsys.p), reinterpret_cast<int *>(b.flags.p));
+    BHIPCHK(hipMemcpyAsync(b.flags_h, b.flags.p, 4 * (size_t)ns, hipMemcpyDeviceToHost, st));
+    BHIPCHK(hipGetLastError());
+    BHIPCHK(hipStreamSynchronize(st));
+    bool grown = false;
+    for (int i = 0; i < ns; ++i) {
+      b.sys[i]->acc_clean = true;
+      if (!b.flags_h[i] || attempt >= 6) continue;
+      grown = true;
+      if (int rc = grow_and_retry(b.sys[i])) return rc;
+    }
+    if (!grown) break;
+    if (int rc = batch_tables<MIXED, C, LJ, CS, BIGLJ, ORDER>(b)) return rc;
+  }
+  for (Sys *s : b.sys) {
     s->list_valid = true;
     s->prune_pending = false;
-    s->acc_clean = true;
     s->staged = b.results && batch_stages(s);
     s->reduced = b.results;
-    for (int attempt = 0; b.flags_h[i] && attempt < 6; ++attempt) {
-      *grown = true;
-      if ((rc = grow_and_retry(s)) || (rc = compute(s, 0))) return rc;
-      int ovf = 0;
-      if (hipMemcpyAsync(&ovf, s->overflow.p, 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
-          hipStreamSynchronize(st) != hipSuccess)
-        return fail(b.ctx, PMX_ERR_HIP, "overflow flag");
-      b.flags_h[i] = ovf;
-    }
   }
   return PMX_OK;
 }
@@ -2868,16 +2869,11 @@ int batch_run(Batch &b, int nsteps) {
   int rc = batch_tables<MIXED, C, LJ, CS, BIGLJ, ORDER>(b);
   if (rc) return rc;
   if (b.first_forces) {
-    bool outgrew = false;
-    if ((rc = batch_forces<MIXED, C, LJ, CS, BIGLJ, ORDER>(b, &outgrew))) return rc;
+    if ((rc = batch_forces<MIXED, C, LJ, CS, BIGLJ, ORDER>(b))) return rc;
     for (int i = 0; i < b.nsys; ++i) {
       if (b.flags_h[i]) return fail(b.ctx, PMX_ERR_OVERFLOW, "pair list capacity exceeded");
       ++b.sys[i]->md.rebuilds;
       b.sys[i]->md.forces_valid = true;
-    }
-    if (outgrew) {
-      BHIPCHK(hipStreamSynchronize(st));
-      if ((rc = batch_tables<MIXED, C, LJ, CS, BIGLJ, ORDER>(b))) return rc;
     }
   }
   BHIPCHK(hipMemsetAsync(b.rebuilds.p, 0, 8 * (size_t)b.nsys, st));
@@ -3025,8 +3021,7 @@ template <bool MIXED, int C, int LJ, int CS, bool BIG, int ORDER>
 int batch_exec(Batch &b, int nsteps) {
   if (nsteps >= 0) return batch_run<MIXED, C, LJ, CS, BIG, ORDER>(b, nsteps);
   if (int rc = batch_tables<MIXED, C, LJ, CS, BIG, ORDER>(b)) return rc;
-  bool grown = false;
-  return batch_forces<MIXED, C, LJ, CS, BIG, ORDER>(b, &grown);
+  return batch_forces<MIXED, C, LJ, CS, BIG, ORDER>(b);
 }
 
 template <bool MIXED, int CASE>

@@ -101,11 +101,58 @@ def test_energies_of_the_state_under_new_launch_shapes(ctx, how, precision):
             sy.close()
 
 
+def _droplet(n, seed):
+    """A water droplet in a box of four times its edge: its lists outgrow the
+    capacity set for the box's mean density."""
+    s = systems.replica_box(n, seed).with_velocities(300.0, seed=seed + 1)
+    first = s.pos[np.searchsorted(s.molecule, s.molecule)]
+    s.pos = s.pos - s.box * np.rint((s.pos - first) / s.box)
+    edge = float(s.box[0])
+    s.box = np.array([4 * edge] * 3)
+    spec = pmx.ForceSpec(4.5, lj=(pmx.SW_C2, 7.0, 9.0), pme=dict(rc=9.0, grid=(48, 48, 48), order=4, alpha=0.35))
+    return s, spec
+
+
 def _mixed(ctx, s, spec):
     sy = pmx.System(ctx, s, spec, pmx.MIXED)
     sy.md_init(s, 1.0, skin=1.0)
     sy.md_set_state(s.pos, s.vel)
     return sy
+
+
+def _states(sys_):
+    return [sy.md_get_state() for sy in sys_]
+
+
+def _equal(a, b):
+    return np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1]) and a[2] == b[2]
+
+
+def test_batched_results_where_a_list_outgrows_its_buffers(ctx):
+    """The first batched run or evaluation of a droplet, in which its buffers
+    grow, gives the results of the second, in which they fit."""
+    other = systems.replica_box(900, 3).with_velocities(300.0, seed=4)
+    drop = _droplet(3000, 8)
+    sys_ = [_mixed(ctx, *drop), _mixed(ctx, other, serve.request_spec(other))]
+    ev = [pmx.System(ctx, *drop, pmx.MIXED), pmx.System(ctx, other, serve.request_spec(other), pmx.MIXED)]
+    try:
+        before = ev[0].device_bytes()
+        e1 = pmx.evaluate_batch(ev, [drop[0].pos, other.pos])
+        assert ev[0].device_bytes() > before
+        e2 = pmx.evaluate_batch(ev, [drop[0].pos, other.pos])
+        pmx.run_batch(sys_, 20)
+        r1 = _states(sys_)
+        for sy, s in zip(sys_, (drop[0], other)):
+            sy.md_set_state(s.pos, s.vel)
+        pmx.run_batch(sys_, 20)
+        r2 = _states(sys_)
+    finally:
+        for sy in sys_ + ev:
+            sy.close()
+    for a, b in zip(e1, e2):
+        assert np.array_equal(a[0], b[0]) and a[1:] == b[1:]
+    for a, b in zip(r1, r2):
+        assert _equal(a, b)
 
 
 @pytest.mark.parametrize("how", ["batch", "run"])
