@@ -2453,7 +2453,8 @@ struct Batch {
   std::vector<Sys *> sys;
   int nsys = 0;
   bool results = false;       // a force pass alone: its results go to the systems' stages with it
-  bool first_forces = false;  // MD: the forces at the set positions come first, for every system; no energies
+  bool first_forces = false;  // a force pass of a run's new systems: no energies, no results
+  std::vector<Sys *> fresh;   // MD: systems that lack the forces at their positions
   BatchLaunch bin, scan, scatter, split, list, runs;
   BatchLaunch kick, spread, pair, yfwd, xconv, yinv, plane, gather, fixups, ukd, unsort, begin, half;
   BatchLaunch energy, out;
@@ -2466,6 +2467,39 @@ struct Batch {
   int *flags_h = nullptr;
   hipEvent_t fork = nullptr, join = nullptr;
 };
+
+// The batch's device buffers, and its slices of the context's pinned staging
+// (a batch that comes before another of the context shares them).
+int batch_buffers(Batch &b) {
+  pmx_ctx *ctx = b.ctx;
+  const int dev = ctx->device, nsys = b.nsys;
+  if (!b.bsys.get(dev, sizeof(BatchSys) * nsys) || !b.need.get(dev, nsys) || !b.base.get(dev, 8 * (size_t)nsys) ||
+      !b.flags.get(dev, 4 * (size_t)nsys) || !b.rebuilds.get(dev, 8 * (size_t)nsys))
+    return fail(ctx, PMX_ERR_OOM, "batch buffers");
+  {
+    RtLock lk(g_rt_mu);
+    const size_t need = (sizeof(BatchSys) + 16) * (size_t)nsys;
+    if (ctx->batch_host_bytes < need) {
+      if (ctx->batch_host) hipHostFree(ctx->batch_host);
+      ctx->batch_host = nullptr;
+      ctx->batch_host_bytes = 0;
+      if (hipHostMalloc(&ctx->batch_host, need, hipHostMallocDefault) != hipSuccess)
+        return fail(ctx, PMX_ERR_HIP, "batch host buffers");
+      ctx->batch_host_bytes = need;
+    }
+    if ((!ctx->batch_fork &&
+         hipEventCreateWithFlags(&ctx->batch_fork, hipEventDisableTiming | hipEventDisableSystemFence) != hipSuccess) ||
+        (!ctx->batch_join &&
+         hipEventCreateWithFlags(&ctx->batch_join, hipEventDisableTiming | hipEventDisableSystemFence) != hipSuccess))
+      return fail(ctx, PMX_ERR_HIP, "batch events");
+  }
+  b.bsys_h = static_cast<BatchSys *>(ctx->batch_host);
+  b.base_h = reinterpret_cast<unsigned long long *>(b.bsys_h + nsys);
+  b.flags_h = reinterpret_cast<int *>(b.base_h + nsys);
+  b.fork = ctx->batch_fork;
+  b.join = ctx->batch_join;
+  return PMX_OK;
+}
 
 // Adds the table of one batched launch (args[s], nblocks[s] blocks of system
 // s; dynamic LDS `lds`) to the batch's tables.
@@ -2866,16 +2900,29 @@ constexpr int kBatchChunk = 64;  // steps between the host's checks of a batch
 template <bool MIXED, int C, int LJ, int CS, bool BIGLJ, int ORDER>
 int batch_run(Batch &b, int nsteps) {
   hipStream_t st = b.ctx->stream;
-  int rc = batch_tables<MIXED, C, LJ, CS, BIGLJ, ORDER>(b);
-  if (rc) return rc;
-  if (b.first_forces) {
-    if ((rc = batch_forces<MIXED, C, LJ, CS, BIGLJ, ORDER>(b))) return rc;
-    for (int i = 0; i < b.nsys; ++i) {
-      if (b.flags_h[i]) return fail(b.ctx, PMX_ERR_OVERFLOW, "pair list capacity exceeded");
-      ++b.sys[i]->md.rebuilds;
-      b.sys[i]->md.forces_valid = true;
+  int rc;
+  // the first forces of the systems that lack them, in a batched pass of
+  // their own: whatever the others of the batch, their lists get the same cut
+  if (!b.fresh.empty()) {
+    const bool every = b.fresh.size() == b.sys.size();
+    Batch some;
+    Batch &f = every ? b : some;
+    if (!every) {
+      some.ctx = b.ctx;
+      some.sys = b.fresh;
+      some.nsys = (int)b.fresh.size();
+      if ((rc = batch_buffers(some))) return rc;
+    }
+    f.first_forces = true;
+    if ((rc = batch_tables<MIXED, C, LJ, CS, BIGLJ, ORDER>(f)) || (rc = batch_forces<MIXED, C, LJ, CS, BIGLJ, ORDER>(f)))
+      return rc;
+    for (int i = 0; i < f.nsys; ++i) {
+      if (f.flags_h[i]) return fail(b.ctx, PMX_ERR_OVERFLOW, "pair list capacity exceeded");
+      ++f.sys[i]->md.rebuilds;
+      f.sys[i]->md.forces_valid = true;
     }
   }
+  if (b.fresh.size() < b.sys.size() && (rc = batch_tables<MIXED, C, LJ, CS, BIGLJ, ORDER>(b))) return rc;
   BHIPCHK(hipMemsetAsync(b.rebuilds.p, 0, 8 * (size_t)b.nsys, st));
   int done = 0, retries = 0, last = 0;
   while (done < nsteps) {
@@ -3072,52 +3119,20 @@ int batch_entry(pmx_sys *const *systems, int nsys, int nsteps) {
   Batch b;
   b.ctx = ctx;
   b.nsys = nsys;
-  // the first forces of a run: in one batched pass when every system needs
-  // them, one by one where only some do
   b.results = !md;
-  b.first_forces = md;
-  for (int i = 0; i < nsys; ++i) b.first_forces &= !systems[i]->s.md.forces_valid;
   for (int i = 0; i < nsys; ++i) {
     Sys *s = &systems[i]->s;
     s->staged = s->reduced = false;
     b.sys.push_back(s);
     if (!s->cached)
       if (int rc = setup(s)) return rc;
-    if (md) {
-      if (!b.first_forces)
-        if (int rc = md_ensure_forces(s)) return rc;
-      if (!s->acc_clean) {
-        launch_zero(s);
-        s->acc_clean = true;
-      }
+    if (md && !s->md.forces_valid) b.fresh.push_back(s);
+    if (md && !s->acc_clean) {
+      launch_zero(s);
+      s->acc_clean = true;
     }
   }
-  const int dev = ctx->device;
-  if (!b.bsys.get(dev, sizeof(BatchSys) * nsys) || !b.need.get(dev, nsys) || !b.base.get(dev, 8 * (size_t)nsys) ||
-      !b.flags.get(dev, 4 * (size_t)nsys) || !b.rebuilds.get(dev, 8 * (size_t)nsys))
-    return fail(ctx, PMX_ERR_OOM, "batch buffers");
-  {
-    RtLock lk(g_rt_mu);
-    const size_t need = (sizeof(BatchSys) + 16) * (size_t)nsys;
-    if (ctx->batch_host_bytes < need) {
-      if (ctx->batch_host) hipHostFree(ctx->batch_host);
-      ctx->batch_host = nullptr;
-      ctx->batch_host_bytes = 0;
-      if (hipHostMalloc(&ctx->batch_host, need, hipHostMallocDefault) != hipSuccess)
-        return fail(ctx, PMX_ERR_HIP, "batch host buffers");
-      ctx->batch_host_bytes = need;
-    }
-    if ((!ctx->batch_fork &&
-         hipEventCreateWithFlags(&ctx->batch_fork, hipEventDisableTiming | hipEventDisableSystemFence) != hipSuccess) ||
-        (!ctx->batch_join &&
-         hipEventCreateWithFlags(&ctx->batch_join, hipEventDisableTiming | hipEventDisableSystemFence) != hipSuccess))
-      return fail(ctx, PMX_ERR_HIP, "batch events");
-  }
-  b.bsys_h = static_cast<BatchSys *>(ctx->batch_host);
-  b.base_h = reinterpret_cast<unsigned long long *>(b.bsys_h + nsys);
-  b.flags_h = reinterpret_cast<int *>(b.base_h + nsys);
-  b.fork = ctx->batch_fork;
-  b.join = ctx->batch_join;
+  if (int rc = batch_buffers(b)) return rc;
   // the batch runs on the context's two streams, idle from here on
   if (hipStreamSynchronize(ctx->stream) != hipSuccess || hipStreamSynchronize(ctx->stream2) != hipSuccess)
     return fail(ctx, PMX_ERR_HIP, "stream synchronize");

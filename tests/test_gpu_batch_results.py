@@ -173,3 +173,25 @@ def test_a_run_leaves_the_energies_of_the_last_evaluation(ctx, how):
         assert (ec2, elj2) == (ec, elj) and sy.pair_stats() == stats
     finally:
         sy.close()
+
+
+def test_first_forces_do_not_depend_on_the_partners(ctx):
+    """A new system's batched run is the same, to the last bit in the mixed
+    form, in a batch of its own, with new partners and with partners that
+    continue an earlier run."""
+    s, t = (systems.replica_box(n, seed).with_velocities(300.0, seed=seed + 1) for n, seed in ((1500, 31), (2400, 33)))
+    out = []
+    for partner in (None, "new", "continued"):
+        sys_ = [_mixed(ctx, s, serve.request_spec(s))]
+        try:
+            if partner:
+                sys_.append(_mixed(ctx, t, serve.request_spec(t)))
+            if partner == "continued":
+                pmx.run_batch(sys_[1:], 5)
+            pmx.run_batch(sys_, 12)
+            out.append(_states(sys_[:1])[0] + (sys_[0].md_stats(),))
+        finally:
+            for sy in sys_:
+                sy.close()
+    for o in out[1:]:
+        assert _equal(o, out[0]) and o[3] == out[0][3]
