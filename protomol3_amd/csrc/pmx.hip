@@ -375,6 +375,13 @@ bool make_plan(int n, FftPlan &pl) {
 }
 
 void bspline_host(int order, double w, double *th, double *dth) {
+  if (order == 2) {
+    th[0] = 1.0 - w;
+    th[1] = w;
+    dth[0] = -1.0;
+    dth[1] = 1.0;
+    return;
+  }
   th[order - 1] = 0.0;
   th[1] = w;
   th[0] = 1.0 - w;

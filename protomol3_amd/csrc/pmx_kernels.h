@@ -1988,6 +1988,13 @@ __device__ void border_pairs(int blk, int nblocks, const PairParams &pp, int sta
 // compile-time order P (2..8): weights th[0..P-1] and derivatives dth.
 template <int P, class R>
 __device__ inline void bspline_w(R w, R *th, R *dth) {
+  if constexpr (P == 2) {  // linear: the recursion starts from it
+    th[0] = (R)1 - w;
+    th[1] = w;
+    dth[0] = (R)-1;
+    dth[1] = (R)1;
+    return;
+  }
   th[P - 1] = 0;
   th[1] = w;
   th[0] = (R)1 - w;
