@@ -74,7 +74,7 @@ typedef struct {
   int coul_kind;          /* pmx_coulomb */
   int coul_switch;        /* cutoff Coulomb: CUTOFF/C1/C2; PME real: CUTOFF or C1 */
   double coul_on, coul_rc;
-  int pme_grid[3];        /* -gridsize nx ny nz */
+  int pme_grid[3];        /* -gridsize nx ny nz: products of 2, 3 and 5, at most 10,125 each (5,120 in FP64) */
   int pme_order;          /* -order (even, >= 2) */
   double pme_accuracy;    /* -accuracy */
   double pme_alpha;       /* -alpha (<= 0: chosen from accuracy and cutoff) */

@@ -477,9 +477,9 @@ int fft_blocking(Sys *s) {
   const size_t cx = s->mixed ? 8 : 16;
   const int small = 256 * kFftPerThread;  // points of a block of 256 threads
   // the larger of the charge sums (16 bytes a point of two lines) and the
-  // transforms (a complex number), and the twiddles
+  // transforms (a complex number), and the twiddles (of LONG passes in memory)
   auto lds = [&](const PmeParams &q, size_t per_point) {
-    return per_point * (size_t)(q.tx * q.ty / 2) * pme_line(q.nz, q.order) + cx * (q.nz + 1);
+    return per_point * (size_t)(q.tx * q.ty / 2) * pme_line(q.nz, q.order) + (q.nz > kFftMax ? 0 : cx * (q.nz + 1));
   };
   auto tiles = [&](PmeParams &q, int tx, size_t per_point, size_t most) {
     q.tx = tx;
@@ -511,8 +511,8 @@ int fft_blocking(Sys *s) {
   };
   s->ylog = lines(pm.ny, pm.nx);
   s->xlog = lines(pm.nx, pm.ny);
-  s->lds_y = cx * (((size_t)(pm.ny | 1) << s->ylog) + pm.ny);
-  s->lds_x = cx * (((size_t)(pm.nx | 1) << s->xlog) + pm.nx);
+  s->lds_y = cx * (((size_t)(pm.ny | 1) << s->ylog) + (pm.ny > kFftMax ? 0 : pm.ny));
+  s->lds_x = cx * (((size_t)(pm.nx | 1) << s->xlog) + (pm.nx > kFftMax ? 0 : pm.nx));
   s->lds_p = cx * ((size_t)(pm.nx | 1) * pm.ny + pm.nx + pm.ny);
   // threads: a line needs n / kFftPerThread; the tiles and planes transform
   // as many lines at a time as the block has threads for.  Planes and the
@@ -872,8 +872,8 @@ int setup(Sys *s) {
     pm.offz = -(pm.order - 1) / 2 + pm.nz;
     if (!make_plan(pm.nx, s->plx) || !make_plan(pm.ny, s->ply) || !make_plan(pm.nz, s->plz))
       return fail(s->ctx, PMX_ERR_UNSUPPORTED, "PME grid sizes must be products of 2, 3 and 5");
-    if (std::max(pm.nx, std::max(pm.ny, pm.nz)) > kFftMax)
-      return fail(s->ctx, PMX_ERR_UNSUPPORTED, "PME grid axes have at most 4096 points");
+    if (std::max(pm.nx, std::max(pm.ny, pm.nz)) > (s->mixed ? kFftMaxLong<float> : kFftMaxLong<double>))
+      return fail(s->ctx, PMX_ERR_UNSUPPORTED, "PME grid axes have at most 10125 points (5120 in FP64)");
     pm.ncx = bp.ncx;
     pm.ncy = bp.ncy;
     const size_t GH = (size_t)pm.nx * pm.ny * pm.nzh;
@@ -1152,6 +1152,9 @@ void run_spread(Sys *s, hipStream_t st, bool with = false) {
   if (nterms)                                                                                                       \
     hipLaunchKernelGGL((k_pme_spread_terms<MIXED, ORD>), dim3(s->pme.ntx * s->pme.nty + nterms), dim3(s->thr_z),    \
                        s->lds_z, st, PMX_SPREAD_ARGS, terms);                                                       \
+  else if (s->pme.nz > kFftMax)                                                                                     \
+    hipLaunchKernelGGL((k_pme_spread_z<MIXED, ORD, true>), dim3(s->pme.ntx * s->pme.nty), dim3(s->thr_z), s->lds_z, \
+                       st, PMX_SPREAD_ARGS);                                                                        \
   else                                                                                                              \
     hipLaunchKernelGGL((k_pme_spread_z<MIXED, ORD>), dim3(s->pme.ntx * s->pme.nty), dim3(s->thr_z), s->lds_z, st,   \
                        PMX_SPREAD_ARGS)
@@ -1179,18 +1182,36 @@ int run_pme(Sys *s, bool timing) {
                          P<Cx<T>>(s->twy), P<Cx<T>>(s->twx), P<T>(s->theta), P<Cx<T>>(s->spec), P<double>(s->recip_e));
     } else {
       const int yb = pm.nzh * ((pm.nx + (1 << s->ylog) - 1) >> s->ylog);
-      hipLaunchKernelGGL((k_fft_y<T>), dim3(yb), dim3(s->thr_y), s->lds_y, st, pm, s->ply, s->ylog, false,
-                         P<Cx<T>>(s->twy), P<Cx<T>>(s->spec));
-      hipLaunchKernelGGL((k_fft_x_conv<T>), dim3(s->recip_blocks), dim3(s->thr_x), s->lds_x, st, pm, s->plx, s->xlog,
-                         P<Cx<T>>(s->twx), P<T>(s->theta), P<Cx<T>>(s->spec), P<double>(s->recip_e));
-      hipLaunchKernelGGL((k_fft_y<T>), dim3(yb), dim3(s->thr_y), s->lds_y, st, pm, s->ply, s->ylog, true,
-                         P<Cx<T>>(s->twy), P<Cx<T>>(s->spec));
+      auto y = [&](bool inverse) {
+        auto go = [&](auto kernel) {
+          hipLaunchKernelGGL(kernel, dim3(yb), dim3(s->thr_y), s->lds_y, st, pm, s->ply, s->ylog, inverse,
+                             P<Cx<T>>(s->twy), P<Cx<T>>(s->spec));
+        };
+        if (pm.ny > kFftMax)
+          go(k_fft_y<T, true>);
+        else
+          go(k_fft_y<T>);
+      };
+      auto x = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(s->recip_blocks), dim3(s->thr_x), s->lds_x, st, pm, s->plx, s->xlog,
+                           P<Cx<T>>(s->twx), P<T>(s->theta), P<Cx<T>>(s->spec), P<double>(s->recip_e));
+      };
+      y(false);
+      if (pm.nx > kFftMax)
+        x(k_fft_x_conv<T, true>);
+      else
+        x(k_fft_x_conv<T>);
+      y(true);
     }
     if (timing) hipEventRecord(s->ev[5], st);
+#define PMX_GATHER_ARGS                                                                                              \
+  dim3(pg.ntx * pg.nty), dim3(s->thr_g), s->lds_g, st, pg, s->plz, P<int2>(s->tcol) + pm.ntx + pm.nty,               \
+      P<int>(s->colsc), P<T4>(s->pmw), P<int2>(s->pmb), P<Cx<T>>(s->twz), P<Cx<T>>(s->spec), P<Acc>(s->facc)
 #define PMX_GATHER(ORD)                                                                                              \
-  hipLaunchKernelGGL((k_pme_z_gather<MIXED, ORD>), dim3(pg.ntx * pg.nty), dim3(s->thr_g), s->lds_g, st, pg, s->plz, \
-                     P<int2>(s->tcol) + pm.ntx + pm.nty, P<int>(s->colsc), P<T4>(s->pmw), P<int2>(s->pmb), P<Cx<T>>(s->twz),           \
-                     P<Cx<T>>(s->spec), P<Acc>(s->facc))
+  if (pm.nz > kFftMax)                                                                                               \
+    hipLaunchKernelGGL((k_pme_z_gather<MIXED, ORD, true>), PMX_GATHER_ARGS);                                         \
+  else                                                                                                               \
+    hipLaunchKernelGGL((k_pme_z_gather<MIXED, ORD>), PMX_GATHER_ARGS)
     switch (pm.order) {
       case 2: PMX_GATHER(2); break;
       case 4: PMX_GATHER(4); break;
@@ -1198,6 +1219,7 @@ int run_pme(Sys *s, bool timing) {
       default: PMX_GATHER(8); break;
     }
 #undef PMX_GATHER
+#undef PMX_GATHER_ARGS
   } else if (timing) {
     hipEventRecord(s->ev[5], st);
   }
@@ -2465,6 +2487,7 @@ struct Batch {
   BatchLaunch bin, scan, scatter, split, list, runs;
   BatchLaunch kick, spread, pair, yfwd, xconv, yinv, plane, gather, fixups, ukd, unsort, begin, half;
   BatchLaunch energy, out;
+  BatchLaunch spreadL, yfwdL, xconvL, yinvL, gatherL;  // the systems with axes beyond kFftMax
   BatchBuf tables, bsys, need, base, flags, rebuilds;
   std::vector<unsigned char> image;    // the tables of every launch, uploaded in one copy
   std::vector<BatchLaunch *> launches;
@@ -2660,8 +2683,9 @@ int batch_tables(Batch &b) {
     std::vector<int> nout(ns, 0);
     std::vector<int> nfix(ns);
     long long natoms = 0;
-    size_t lds_z = 0, lds_g = 0, lds_y = 0, lds_x = 0, lds_p = 0;
-    int thr_z = 256, thr_g = 256, thr_y = 256, thr_x = 256, thr_p = 256;
+    // [1]: the LONG forms of the passes
+    size_t lds_z[2] = {0, 0}, lds_g[2] = {0, 0}, lds_y[2] = {0, 0}, lds_x[2] = {0, 0}, lds_p = 0;
+    int thr_z[2] = {256, 256}, thr_g[2] = {256, 256}, thr_y[2] = {256, 256}, thr_x[2] = {256, 256}, thr_p = 256;
     for (int i = 0; i < ns; ++i) {
       Sys *s = b.sys[i];
       Sys::Md &m = s->md;
@@ -2709,27 +2733,38 @@ int batch_tables(Batch &b) {
       }
       // dynamic LDS and block size of each launch: the largest of the
       // systems it serves
-      thr_z = std::max(thr_z, s->thr_z);
-      thr_g = std::max(thr_g, s->thr_gb);
-      lds_g = std::max(lds_g, s->lds_g);
-      lds_z = std::max(lds_z, s->lds_z);
+      auto most = [](auto &v, auto w) { v = std::max(v, w); };
+      const int zl = pm.nz > kFftMax, yl = pm.ny > kFftMax, xl = pm.nx > kFftMax;
+      most(thr_z[zl], s->thr_z);
+      most(thr_g[zl], s->thr_gb);
+      most(lds_g[zl], s->lds_g);
+      most(lds_z[zl], s->lds_z);
       if (s->fft_plane) {
-        lds_p = std::max(lds_p, s->lds_p);
-        thr_p = std::max(thr_p, s->thr_pb);
+        most(lds_p, s->lds_p);
+        most(thr_p, s->thr_pb);
       } else {
-        lds_y = std::max(lds_y, s->lds_y);
-        lds_x = std::max(lds_x, s->lds_x);
-        thr_y = std::max(thr_y, s->thr_y);
-        thr_x = std::max(thr_x, s->thr_x);
+        most(lds_y[yl], s->lds_y);
+        most(lds_x[xl], s->lds_x);
+        most(thr_y[yl], s->thr_y);
+        most(thr_x[xl], s->thr_x);
       }
     }
     for (int i = 0; i < ns; ++i) nb[i] = (int)nblk(b.sys[i]->npad, 256);
     if ((rc = batch_table<OpKickDrift<R>>(b, b.kick, args_kick, nb, 0))) return rc;
     if ((rc = batch_table<OpUnsortKickDrift<MIXED, R>>(b, b.ukd, args_ukd, nb, 0))) return rc;
-    for (int i = 0; i < ns; ++i) nb[i] = b.sys[i]->pme.ntx * b.sys[i]->pme.nty;
-    if ((rc = batch_table<OpPmeSpreadZ<MIXED, ORDER>>(b, b.spread, args_spread, nb, lds_z, thr_z))) return rc;
-    for (int i = 0; i < ns; ++i) nb[i] = b.sys[i]->pme_g.ntx * b.sys[i]->pme_g.nty;
-    if ((rc = batch_table<OpPmeZGather<MIXED, ORDER>>(b, b.gather, args_gather, nb, lds_g, thr_g))) return rc;
+    // blocks(s) of the systems of one form of a pass, none of the others
+    auto of = [&](bool form, auto is, auto blocks) -> const std::vector<int> & {
+      for (int i = 0; i < ns; ++i) nb[i] = (is(b.sys[i]) == form) ? blocks(b.sys[i]) : 0;
+      return nb;
+    };
+    auto zlong = [](const Sys *s) { return s->pme.nz > kFftMax; };
+    auto spread_blocks = [](const Sys *s) { return s->pme.ntx * s->pme.nty; };
+    auto gather_blocks = [](const Sys *s) { return s->pme_g.ntx * s->pme_g.nty; };
+    if ((rc = batch_table<OpPmeSpreadZ<MIXED, ORDER>>(b, b.spread, args_spread, of(false, zlong, spread_blocks),
+                                                      lds_z[0], thr_z[0])) ||
+        (rc = batch_table<OpPmeZGather<MIXED, ORDER>>(b, b.gather, args_gather, of(false, zlong, gather_blocks),
+                                                      lds_g[0], thr_g[0])))
+      return rc;
     // pair-kernel blocks in proportion to the atoms (a run's share of a
     // system's waves changes no result), about the device's resident blocks
     // in all
@@ -2741,14 +2776,29 @@ int batch_tables(Batch &b) {
     if ((rc = batch_table<PairOp<MIXED, C, LJ, CS, BIGLJ, ORDER>>(b, b.pair, args_pair, nb, 0))) return rc;
     // systems with small planes take the one-launch plane pass, the others
     // the three line passes
-    for (int i = 0; i < ns; ++i) {
-      const Sys *s = b.sys[i];
-      nb[i] = s->fft_plane ? 0 : s->pme.nzh * ((s->pme.nx + (1 << s->ylog) - 1) >> s->ylog);
+    auto ylong = [](const Sys *s) { return s->pme.ny > kFftMax; };
+    auto xlong = [](const Sys *s) { return s->pme.nx > kFftMax; };
+    auto y_blocks = [](const Sys *s) {
+      return s->fft_plane ? 0 : s->pme.nzh * ((s->pme.nx + (1 << s->ylog) - 1) >> s->ylog);
+    };
+    auto x_blocks = [](const Sys *s) { return s->fft_plane ? 0 : s->recip_blocks; };
+    of(false, ylong, y_blocks);
+    if ((rc = batch_table<OpFftY<T>>(b, b.yfwd, args_yfwd, nb, lds_y[0], thr_y[0])) ||
+        (rc = batch_table<OpFftY<T>>(b, b.yinv, args_yinv, nb, lds_y[0], thr_y[0])) ||
+        (rc = batch_table<OpFftXConv<T>>(b, b.xconv, args_xconv, of(false, xlong, x_blocks), lds_x[0], thr_x[0])))
+      return rc;
+    if (std::any_of(b.sys.begin(), b.sys.end(), [&](const Sys *s) { return xlong(s) || ylong(s) || zlong(s); })) {
+      if ((rc = batch_table<OpPmeSpreadZLong<MIXED, ORDER>>(b, b.spreadL, args_spread, of(true, zlong, spread_blocks),
+                                                            lds_z[1], thr_z[1])) ||
+          (rc = batch_table<OpPmeZGatherLong<MIXED, ORDER>>(b, b.gatherL, args_gather, of(true, zlong, gather_blocks),
+                                                            lds_g[1], thr_g[1])))
+        return rc;
+      of(true, ylong, y_blocks);
+      if ((rc = batch_table<OpFftYLong<T>>(b, b.yfwdL, args_yfwd, nb, lds_y[1], thr_y[1])) ||
+          (rc = batch_table<OpFftYLong<T>>(b, b.yinvL, args_yinv, nb, lds_y[1], thr_y[1])) ||
+          (rc = batch_table<OpFftXConvLong<T>>(b, b.xconvL, args_xconv, of(true, xlong, x_blocks), lds_x[1], thr_x[1])))
+        return rc;
     }
-    if ((rc = batch_table<OpFftY<T>>(b, b.yfwd, args_yfwd, nb, lds_y, thr_y))) return rc;
-    if ((rc = batch_table<OpFftY<T>>(b, b.yinv, args_yinv, nb, lds_y, thr_y))) return rc;
-    for (int i = 0; i < ns; ++i) nb[i] = b.sys[i]->fft_plane ? 0 : b.sys[i]->recip_blocks;
-    if ((rc = batch_table<OpFftXConv<T>>(b, b.xconv, args_xconv, nb, lds_x, thr_x))) return rc;
     for (int i = 0; i < ns; ++i) nb[i] = b.sys[i]->fft_plane ? b.sys[i]->pme.nzh : 0;
     if ((rc = batch_table<OpFftPlane<T>>(b, b.plane, args_plane, nb, lds_p, thr_p))) return rc;
     if ((rc = batch_table<OpFixups<MIXED, C, LJ, CS>>(b, b.fixups, args_fixups, nfix, 0))) return rc;
@@ -2805,14 +2855,19 @@ int batch_chunk(Batch &b, int K, bool opening) {
     // systems of 331,000 atoms); fork: the rest of the PME chain beside the
     // pair kernel
     batch_go<OpPmeSpreadZ<MIXED, ORDER>>(b.spread, st, bk);
+    batch_go<OpPmeSpreadZLong<MIXED, ORDER>>(b.spreadL, st, bk);
     BHIPCHK(hipEventRecord(b.fork, st));
     BHIPCHK(hipStreamWaitEvent(st2, b.fork, 0));
     batch_go<PairOp<MIXED, C, LJ, CS, BIGLJ, ORDER>>(b.pair, st, bk);
     batch_go<OpFftPlane<T>>(b.plane, st2, bk);
     batch_go<OpFftY<T>>(b.yfwd, st2, bk);
+    batch_go<OpFftYLong<T>>(b.yfwdL, st2, bk);
     batch_go<OpFftXConv<T>>(b.xconv, st2, bk);
+    batch_go<OpFftXConvLong<T>>(b.xconvL, st2, bk);
     batch_go<OpFftY<T>>(b.yinv, st2, bk);
+    batch_go<OpFftYLong<T>>(b.yinvL, st2, bk);
     batch_go<OpPmeZGather<MIXED, ORDER>>(b.gather, st2, bk);
+    batch_go<OpPmeZGatherLong<MIXED, ORDER>>(b.gatherL, st2, bk);
     BHIPCHK(hipEventRecord(b.join, st2));
     // boundary pairs, exclusion correction and bonded terms after the pair
     // kernel, then the join
@@ -2858,14 +2913,19 @@ int batch_forces(Batch &b) {
     batch_go<OpBuildList>(b.list, st, bk);
     batch_go<OpRuns>(b.runs, st, bk);
     batch_go<OpPmeSpreadZ<MIXED, ORDER>>(b.spread, st, bk);
+    batch_go<OpPmeSpreadZLong<MIXED, ORDER>>(b.spreadL, st, bk);
     BHIPCHK(hipEventRecord(b.fork, st));
     BHIPCHK(hipStreamWaitEvent(st2, b.fork, 0));
     batch_go<PairOp<MIXED, C, LJ, CS, BIGLJ, ORDER>>(b.pair, st, bk);
     batch_go<OpFftPlane<T>>(b.plane, st2, bk);
     batch_go<OpFftY<T>>(b.yfwd, st2, bk);
+    batch_go<OpFftYLong<T>>(b.yfwdL, st2, bk);
     batch_go<OpFftXConv<T>>(b.xconv, st2, bk);
+    batch_go<OpFftXConvLong<T>>(b.xconvL, st2, bk);
     batch_go<OpFftY<T>>(b.yinv, st2, bk);
+    batch_go<OpFftYLong<T>>(b.yinvL, st2, bk);
     batch_go<OpPmeZGather<MIXED, ORDER>>(b.gather, st2, bk);
+    batch_go<OpPmeZGatherLong<MIXED, ORDER>>(b.gatherL, st2, bk);
     BHIPCHK(hipEventRecord(b.join, st2));
     batch_go<OpFixups<MIXED, C, LJ, CS>>(b.fixups, st, bk);
     BHIPCHK(hipStreamWaitEvent(st, b.join, 0));

@@ -209,6 +209,15 @@ struct OpPmeSpreadZ {
   }
 };
 
+template <bool MIXED, int P>
+struct OpPmeSpreadZLong : OpPmeSpreadZ<MIXED, P> {
+  using typename OpPmeSpreadZ<MIXED, P>::Args;
+  static constexpr int kMinBlocks = 2;
+  __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &) {
+    pme_spread_z_body<MIXED, P, true>(bid, nbk, a.p, a.pl, a.tcol, a.colsc, a.pmw, a.pmb, a.tw, a.spec);
+  }
+};
+
 template <bool MIXED, int COUL, int LJSW, int CSW, bool BIGLJ>
 struct OpPair {
   using R4 = typename Real4<typename std::conditional<MIXED, float, double>::type>::type;
@@ -256,6 +265,15 @@ struct OpFftY {
 };
 
 template <class T>
+struct OpFftYLong : OpFftY<T> {
+  using typename OpFftY<T>::Args;
+  static constexpr int kMinBlocks = 2;
+  __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &) {
+    fft_y_body<T, true>(bid, nbk, a.p, a.pl, a.llog, a.inverse, a.tw, a.spec);
+  }
+};
+
+template <class T>
 struct OpFftXConv {
   struct Args {
     PmeParams p;
@@ -270,6 +288,15 @@ struct OpFftXConv {
   static constexpr bool kGated = false;
   __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &) {
     fft_x_conv_body<T>(bid, nbk, a.p, a.pl, a.llog, a.threads, a.tw, a.theta, a.spec, a.epart);
+  }
+};
+
+template <class T>
+struct OpFftXConvLong : OpFftXConv<T> {
+  using typename OpFftXConv<T>::Args;
+  static constexpr int kMinBlocks = 2;
+  __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &) {
+    fft_x_conv_body<T, true>(bid, nbk, a.p, a.pl, a.llog, a.threads, a.tw, a.theta, a.spec, a.epart);
   }
 };
 
@@ -308,6 +335,15 @@ struct OpPmeZGather {
   static constexpr bool kGated = false;
   __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &) {
     pme_z_gather_body<MIXED, P>(bid, nbk, a.p, a.pl, a.tcol, a.colsc, a.pmw, a.pmb, a.tw, a.spec, a.facc);
+  }
+};
+
+template <bool MIXED, int P>
+struct OpPmeZGatherLong : OpPmeZGather<MIXED, P> {
+  using typename OpPmeZGather<MIXED, P>::Args;
+  static constexpr int kMinBlocks = 2;
+  __device__ static void run(const Args &a, int bid, int nbk, const BatchStep &) {
+    pme_z_gather_body<MIXED, P, true>(bid, nbk, a.p, a.pl, a.tcol, a.colsc, a.pmw, a.pmb, a.tw, a.spec, a.facc);
   }
 };
 

@@ -2132,12 +2132,23 @@ __device__ __forceinline__ void dft_small(Cx<T> *v) {
 __host__ __device__ inline unsigned div_magic(unsigned d) { return (unsigned)(0x100000000ull / d) + 1u; }
 __device__ inline int div_by(int t, unsigned magic) { return (int)__umulhi((unsigned)t, magic); }
 
-constexpr int kFftMax = 4096;       // longest transform (points), and most points of a block
+constexpr int kFftMax = 4096;       // longest ordinary transform (points), and most points of a block
 constexpr int kFftPerThread = 8;    // points a thread holds in a pass, at least (8 keeps a pass within 64 VGPRs,
                                     // so that these kernels fit on a SIMD beside four pair-kernel waves)
 constexpr int kPmeBlock = kFftMax / kFftPerThread;  // threads of a PME block, at most
 template <class T>
 constexpr int kPmeWaves = sizeof(T) == 4 ? 8 : 4;   // resident waves per SIMD to compile for
+// Axes beyond kFftMax take passes of their own (LONG; a block per line, on z
+// per pair of lines) with more points per thread and the twiddles read from
+// memory: up to 10,125 points in the mixed form, whose FP64 charge sums of a
+// line pair then fill the 160 KB of LDS, half as many in FP64, whose
+// points take twice the registers.  A launch that asks for more LDS than a
+// CU has ends the queue.
+template <class T, bool LONG>
+constexpr int kFftPoints = !LONG ? kFftPerThread : sizeof(T) == 4 ? 20 : 10;
+template <class T>
+constexpr int kFftMaxLong = sizeof(T) == 4 ? 10125 : kPmeBlock * kFftPoints<T, true>;
+static_assert(kFftMaxLong<float> <= kPmeBlock * kFftPoints<float, true>);
 struct FftPlan {
   int n;
   int nrad;
@@ -2155,13 +2166,13 @@ struct FftLines {
 };
 
 // One Stockham pass of radix R in place: every thread holds its butterflies
-// (up to kFftPerThread points or the next multiple of R) in registers between the two
+// (up to PER points or the next multiple of R) in registers between the two
 // barriers.  Butterfly j reads elements j + r n/R, twiddles by
 // tw[k r n/(Ns R)] (k = j mod Ns), writes (j - k) R + k + r Ns.
-template <int R, class T>
+template <int R, class T, int PER>
 __device__ __forceinline__ void fft_pass(Cx<T> *buf, const FftLines &f, int n, int Ns, unsigned magic,
                                          const Cx<T> *tw) {
-  constexpr int NB = (kFftPerThread + R - 1) / R;
+  constexpr int NB = (PER + R - 1) / R;
   const int line = threadIdx.x & ((1 << f.llog) - 1), tb = threadIdx.x >> f.llog, step = blockDim.x >> f.llog;
   const int nbut = n / R, tstep = n / (Ns * R);
   Cx<T> v[NB][R];
@@ -2194,23 +2205,23 @@ __device__ __forceinline__ void fft_pass(Cx<T> *buf, const FftLines &f, int n, i
 }
 
 // Forward transforms of the lines in place (blockDim.x >> f.llog threads per
-// line, at least n / kFftPerThread; tw in LDS).  All threads of the block take part;
+// line, at least n / PER; tw in LDS, or in memory).  All threads of the block take part;
 // the data are in place before the call and after it.
-template <class T>
+template <class T, int PER = kFftPerThread>
 __device__ __forceinline__ void lds_fft(Cx<T> *buf, const FftLines &f, const FftPlan &pl, const Cx<T> *tw) {
   int Ns = 1;
   for (int s = 0; s < pl.nrad; ++s) {
     const unsigned mg = pl.magic[s];
     const int R = __builtin_amdgcn_readfirstlane(pl.rad[s]);
     switch (R) {
-      case 2: fft_pass<2, T>(buf, f, pl.n, Ns, mg, tw); break;
-      case 3: fft_pass<3, T>(buf, f, pl.n, Ns, mg, tw); break;
-      case 4: fft_pass<4, T>(buf, f, pl.n, Ns, mg, tw); break;
-      case 5: fft_pass<5, T>(buf, f, pl.n, Ns, mg, tw); break;
-      case 6: fft_pass<6, T>(buf, f, pl.n, Ns, mg, tw); break;
-      case 8: fft_pass<8, T>(buf, f, pl.n, Ns, mg, tw); break;
-      case 9: fft_pass<9, T>(buf, f, pl.n, Ns, mg, tw); break;
-      default: fft_pass<10, T>(buf, f, pl.n, Ns, mg, tw); break;
+      case 2: fft_pass<2, T, PER>(buf, f, pl.n, Ns, mg, tw); break;
+      case 3: fft_pass<3, T, PER>(buf, f, pl.n, Ns, mg, tw); break;
+      case 4: fft_pass<4, T, PER>(buf, f, pl.n, Ns, mg, tw); break;
+      case 5: fft_pass<5, T, PER>(buf, f, pl.n, Ns, mg, tw); break;
+      case 6: fft_pass<6, T, PER>(buf, f, pl.n, Ns, mg, tw); break;
+      case 8: fft_pass<8, T, PER>(buf, f, pl.n, Ns, mg, tw); break;
+      case 9: fft_pass<9, T, PER>(buf, f, pl.n, Ns, mg, tw); break;
+      default: fft_pass<10, T, PER>(buf, f, pl.n, Ns, mg, tw); break;
     }
     Ns *= R;
   }
@@ -2223,8 +2234,10 @@ __device__ __forceinline__ void lds_twiddles(Cx<T> *s_tw, const Cx<T> *__restric
 
 // Calls work(cnt, slot) for the atoms whose stencils touch the tile (i0, j0),
 // up to 64 of them at a time on one wave (lanes below cnt hold a slot).
-// Waves take the superclusters of the tile's columns in turn.
-template <int P, class WORK>
+// Waves take the superclusters of the tile's columns in turn.  LONG: without
+// the queue, whose LDS such lines leave no room for (cnt is 64 in the lanes
+// that hold a slot and 0 in the others).
+template <int P, bool LONG, class WORK>
 __device__ __forceinline__ void pme_tile_atoms(const PmeParams &p, const int2 *__restrict__ tcol, int tix, int tjy,
                                                const int *__restrict__ colsc, const int2 *__restrict__ pmb,
                                                int (*s_q)[128], WORK work) {
@@ -2232,7 +2245,7 @@ __device__ __forceinline__ void pme_tile_atoms(const PmeParams &p, const int2 *_
   const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int i0 = tix * p.tx, j0 = tjy * p.ty;
   const int2 cx = tcol[tix], cy = tcol[p.ntx + tjy];  // first column and column count
-  int *const q = s_q[wv];
+  int *const q = LONG ? nullptr : s_q[wv];
   int qn = 0;                   // queued slots
   int r = -1;                   // range of superclusters: column a = r / 2 of the x window, part r & 1 in y
   int sc = 0, s1 = 0;           // the range's next supercluster and its end
@@ -2263,6 +2276,10 @@ __device__ __forceinline__ void pme_tile_atoms(const PmeParams &p, const int2 *_
       ey -= ey >= p.ny ? p.ny : 0;
       ey += ey < 0 ? p.ny : 0;
       const bool hit = b != kNoGrid && ex < p.tx + P - 1 && ey < p.ty + P - 1;
+      if constexpr (LONG) {
+        work(hit ? kWave : 0, s);
+        continue;
+      }
       const unsigned long long m = __ballot(hit);
       if (hit) q[qn + __popcll(m & ((1ull << lane) - 1ull))] = s;
       qn += __popcll(m);
@@ -2286,8 +2303,12 @@ __host__ __device__ constexpr int pme_line(int nz, int order) { return (nz + ord
 
 // Transforms of all of a tile's np line pairs, as many at a time as the block
 // holds points for.
-template <class T>
+template <class T, bool LONG>
 __device__ __forceinline__ void pme_tile_fft(Cx<T> *buf, int np, int n, int ls, const FftPlan &pl, const Cx<T> *tw) {
+  if constexpr (LONG) {
+    for (int l = 0; l < np; ++l) lds_fft<T, kFftPoints<T, true>>(buf + l * ls, FftLines{0, 1, ls, 1}, pl, tw);
+    return;
+  }
   const int need = n > kFftPerThread ? 32 - __clz((n - 1) / kFftPerThread) : 0;  // log2 of a line's threads
   const int llog = min(31 - __clz(np), 31 - __clz((int)blockDim.x) - need);
   for (int l0 = 0; l0 < np; l0 += 1 << llog)
@@ -2306,7 +2327,7 @@ constexpr double kGridRound = 6144.0;  // 1.5 2^12: its last bit is 2^-40
 // block's own latency bounds it: 9.5 us at 30^3 points and 1,500 atoms, where
 // the spread (in the kick-drift launch) and the z transform took 7 + 5.6 us
 // and a launch gap.
-template <bool MIXED, int P>
+template <bool MIXED, int P, bool LONG = false>
 __device__ __forceinline__ void pme_spread_z_body(
     const int bid_, const int nbk_, const PmeParams &p, const FftPlan &pl, const int2 *__restrict__ tcol,
     const int *__restrict__ colsc,
@@ -2315,19 +2336,19 @@ __device__ __forceinline__ void pme_spread_z_body(
     Cx<typename std::conditional<MIXED, float, double>::type> *__restrict__ spec) {
   using T = typename std::conditional<MIXED, float, double>::type;
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  __shared__ int s_q[kPmeBlock / kWave][128];
+  __shared__ int s_q[LONG ? 1 : kPmeBlock / kWave][128];
   Cx<T> *const s_tw = reinterpret_cast<Cx<T> *>(smem_raw);
   // sums of lines 2 l and 2 l + 1 interleaved at l, in the order of the
   // complex lines they become
-  double *const acc = reinterpret_cast<double *>(s_tw + ((p.nz + 1) & ~1));
+  double *const acc = reinterpret_cast<double *>(s_tw + (LONG ? 0 : (p.nz + 1) & ~1));
   Cx<T> *const buf = reinterpret_cast<Cx<T> *>(acc);
   const int nzs = pme_line(p.nz, P), lines = p.tx * p.ty;
   const int tjy = bid_ / p.ntx, tix = bid_ - tjy * p.ntx;
   const int i0 = tix * p.tx, j0 = tjy * p.ty;
-  lds_twiddles(s_tw, tw, p.nz);
+  if (!LONG) lds_twiddles(s_tw, tw, p.nz);
   for (int t = threadIdx.x; t < lines * nzs; t += blockDim.x) acc[t] = 0.0;
   __syncthreads();
-  pme_tile_atoms<P>(p, tcol, tix, tjy, colsc, pmb, s_q, [&](int cnt, int slot) {
+  pme_tile_atoms<P, LONG>(p, tcol, tix, tjy, colsc, pmb, s_q, [&](int cnt, int slot) {
     if ((int)(threadIdx.x & 63) >= cnt) return;
     const auto a = pmw[slot];
     const int2 b = pmb[slot];
@@ -2388,7 +2409,7 @@ __device__ __forceinline__ void pme_spread_z_body(
     }
     __syncthreads();
   }
-  pme_tile_fft<T>(buf, np, p.nz, nzs, pl, s_tw);
+  pme_tile_fft<T, LONG>(buf, np, p.nz, nzs, pl, LONG ? tw : s_tw);
   const int hlog = 31 - __clz(p.tx) - 1;  // line pairs per row of the tile: tx / 2
   for (int t = threadIdx.x; t < p.nzh << nplog; t += blockDim.x) {
     const int l = t & (np - 1), k = t >> nplog;
@@ -2401,32 +2422,32 @@ __device__ __forceinline__ void pme_spread_z_body(
   }
 }
 
-template <bool MIXED, int P>
-__global__ void __launch_bounds__(kPmeBlock, MIXED ? 8 : 4) k_pme_spread_z(
+template <bool MIXED, int P, bool LONG = false>
+__global__ void __launch_bounds__(kPmeBlock, LONG ? 2 : MIXED ? 8 : 4) k_pme_spread_z(
     PmeParams p, FftPlan pl, const int2 *__restrict__ tcol, const int *__restrict__ colsc,
     const typename Real4<typename std::conditional<MIXED, float, double>::type>::type *__restrict__ pmw,
     const int2 *__restrict__ pmb, const Cx<typename std::conditional<MIXED, float, double>::type> *__restrict__ tw,
     Cx<typename std::conditional<MIXED, float, double>::type> *__restrict__ spec) {
   // the blocks of one XCD take a contiguous range of tiles
-  pme_spread_z_body<MIXED, P>(xcd_block(blockIdx.x, gridDim.x), gridDim.x, p, pl, tcol, colsc, pmw, pmb, tw, spec);
+  pme_spread_z_body<MIXED, P, LONG>(xcd_block(blockIdx.x, gridDim.x), gridDim.x, p, pl, tcol, colsc, pmw, pmb, tw, spec);
 }
 
 // y pass of the lines (k, i0 .. i0 + (1 << llog) - 1), in place: forward, or
 // inverse (conj-in / conj-out around the forward transform).  Bound by memory
 // on large grids: 0.21 -> 0.058 ms for 2 x 50 MB (216 x 240 x 240, beside the
 // pair kernel).
-template <class T>
+template <class T, bool LONG = false>
 __device__ __forceinline__ void fft_y_body(const int bid_, const int nbk_, const PmeParams &p, const FftPlan &pl,
                                            int llog, bool inverse, const Cx<T> *__restrict__ tw,
                                            Cx<T> *__restrict__ spec) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   Cx<T> *const s_tw = reinterpret_cast<Cx<T> *>(smem_raw);
-  Cx<T> *const buf = s_tw + p.ny;
+  Cx<T> *const buf = LONG ? s_tw : s_tw + p.ny;
   const int it = (p.nx + (1 << llog) - 1) >> llog;
   const int k = bid_ / it, i0 = (bid_ - k * it) << llog;
   const FftLines f{llog, min(1 << llog, p.nx - i0), p.ny | 1, 1};
   Cx<T> *const g = spec + (size_t)k * p.ny * p.nx + i0;
-  lds_twiddles(s_tw, tw, p.ny);
+  if (!LONG) lds_twiddles(s_tw, tw, p.ny);
   const int l = threadIdx.x & ((1 << llog) - 1);
   if (l < f.lines)
     for (int j = threadIdx.x >> llog; j < p.ny; j += blockDim.x >> llog) {
@@ -2435,7 +2456,7 @@ __device__ __forceinline__ void fft_y_body(const int bid_, const int nbk_, const
       buf[l * f.ls + j] = v;
     }
   __syncthreads();
-  lds_fft<T>(buf, f, pl, s_tw);
+  lds_fft<T, kFftPoints<T, LONG>>(buf, f, pl, LONG ? tw : s_tw);
   if (l < f.lines)
     for (int j = threadIdx.x >> llog; j < p.ny; j += blockDim.x >> llog) {
       Cx<T> v = buf[l * f.ls + j];
@@ -2444,10 +2465,10 @@ __device__ __forceinline__ void fft_y_body(const int bid_, const int nbk_, const
     }
 }
 
-template <class T>
-__global__ void __launch_bounds__(kPmeBlock, kPmeWaves<T>) k_fft_y(PmeParams p, FftPlan pl, int llog, bool inverse,
+template <class T, bool LONG = false>
+__global__ void __launch_bounds__(kPmeBlock, LONG ? 2 : kPmeWaves<T>) k_fft_y(PmeParams p, FftPlan pl, int llog, bool inverse,
                                                      const Cx<T> *__restrict__ tw, Cx<T> *__restrict__ spec) {
-  fft_y_body<T>(xcd_block(blockIdx.x, gridDim.x), gridDim.x, p, pl, llog, inverse, tw, spec);
+  fft_y_body<T, LONG>(xcd_block(blockIdx.x, gridDim.x), gridDim.x, p, pl, llog, inverse, tw, spec);
 }
 
 // Weight of plane k of the half spectrum in the energy.
@@ -2483,26 +2504,26 @@ __device__ inline double convolve(Cx<T> &v, T th) {
 // batched launch), so it does not depend on the batch.  0.49 -> 0.11 ms for
 // 125 MB on that grid: radices up to 10 in registers (three passes of LDS
 // instead of five), no division by a length, odd line strides.
-template <class T>
+template <class T, bool LONG = false>
 __device__ __forceinline__ void fft_x_conv_body(const int bid_, const int nbk_, const PmeParams &p, const FftPlan &pl,
                                                 int llog, int threads, const Cx<T> *__restrict__ tw,
                                                 const T *__restrict__ theta, Cx<T> *__restrict__ spec,
                                                 double *__restrict__ epart) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   Cx<T> *const s_tw = reinterpret_cast<Cx<T> *>(smem_raw);
-  Cx<T> *const buf = s_tw + p.nx;
+  Cx<T> *const buf = LONG ? s_tw : s_tw + p.nx;
   const int jt = (p.ny + (1 << llog) - 1) >> llog;
   const int k = bid_ / jt, j0 = (bid_ - k * jt) << llog;
   const FftLines f{llog, min(1 << llog, p.ny - j0), p.nx | 1, 1};
   const int pad = f.ls - p.nx;
   const size_t base = ((size_t)k * p.ny + j0) * p.nx;
-  lds_twiddles(s_tw, tw, p.nx);
+  if (!LONG) lds_twiddles(s_tw, tw, p.nx);
   for (int t = threadIdx.x; t < f.lines * p.nx; t += blockDim.x)
     buf[t + pad * div_by(t, pl.magic_n)] = spec[base + t];
   __syncthreads();
   double e = 0.0;
   for (int back = 0; back < 2; ++back) {
-    lds_fft<T>(buf, f, pl, s_tw);
+    lds_fft<T, kFftPoints<T, LONG>>(buf, f, pl, LONG ? tw : s_tw);
     if (back) break;
     for (int t = threadIdx.x; (int)threadIdx.x < threads && t < f.lines * p.nx; t += threads)
       e += convolve<T>(buf[t + pad * div_by(t, pl.magic_n)], theta[base + t]);
@@ -2516,11 +2537,11 @@ __device__ __forceinline__ void fft_x_conv_body(const int bid_, const int nbk_, 
   block_energy(plane_weight(p, k) * e, &epart[bid_]);
 }
 
-template <class T>
-__global__ void __launch_bounds__(kPmeBlock, kPmeWaves<T>) k_fft_x_conv(PmeParams p, FftPlan pl, int llog,
+template <class T, bool LONG = false>
+__global__ void __launch_bounds__(kPmeBlock, LONG ? 2 : kPmeWaves<T>) k_fft_x_conv(PmeParams p, FftPlan pl, int llog,
                                                           const Cx<T> *__restrict__ tw, const T *__restrict__ theta,
                                                           Cx<T> *__restrict__ spec, double *__restrict__ epart) {
-  fft_x_conv_body<T>(xcd_block(blockIdx.x, gridDim.x), gridDim.x, p, pl, llog, blockDim.x, tw, theta, spec, epart);
+  fft_x_conv_body<T, LONG>(xcd_block(blockIdx.x, gridDim.x), gridDim.x, p, pl, llog, blockDim.x, tw, theta, spec, epart);
 }
 
 // The y pass, the x pass with the convolution and the inverse y pass of one
@@ -2589,7 +2610,7 @@ __global__ void __launch_bounds__(kPmeBlock, kPmeWaves<T>) k_fft_plane_conv(
 // potential of lines 2 l and 2 l + 1 is the real and the (negated) imaginary
 // part of transform l; each lane takes one atom, sums the stencil rows
 // inside the tile and adds the atom's force.
-template <bool MIXED, int P>
+template <bool MIXED, int P, bool LONG = false>
 __device__ __forceinline__ void pme_z_gather_body(
     const int bid_, const int nbk_, const PmeParams &p, const FftPlan &pl, const int2 *__restrict__ tcol,
     const int *__restrict__ colsc,
@@ -2599,13 +2620,13 @@ __device__ __forceinline__ void pme_z_gather_body(
     typename AccT<MIXED>::type *__restrict__ facc) {
   using T = typename std::conditional<MIXED, float, double>::type;
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  __shared__ int s_q[kPmeBlock / kWave][128];
+  __shared__ int s_q[LONG ? 1 : kPmeBlock / kWave][128];
   Cx<T> *const s_tw = reinterpret_cast<Cx<T> *>(smem_raw);
-  Cx<T> *const buf = s_tw + p.nz;
+  Cx<T> *const buf = LONG ? s_tw : s_tw + p.nz;
   const int nzs = pme_line(p.nz, P), lines = p.tx * p.ty;
   const int tjy = bid_ / p.ntx, tix = bid_ - tjy * p.ntx;
   const int i0 = tix * p.tx, j0 = tjy * p.ty;
-  lds_twiddles(s_tw, tw, p.nz);
+  if (!LONG) lds_twiddles(s_tw, tw, p.nz);
   const int np = lines >> 1, nplog = 31 - __clz(np), hlog = 31 - __clz(p.tx) - 1;
   for (int t = threadIdx.x; t < p.nzh << nplog; t += blockDim.x) {
     const int l = t & (np - 1), k = t >> nplog;
@@ -2625,7 +2646,7 @@ __device__ __forceinline__ void pme_z_gather_body(
     if (!self) buf[l * nzs + p.nz - k] = Cx<T>{a.x + b.y, a.y - b.x};
   }
   __syncthreads();
-  pme_tile_fft<T>(buf, np, p.nz, nzs, pl, s_tw);
+  pme_tile_fft<T, LONG>(buf, np, p.nz, nzs, pl, LONG ? tw : s_tw);
   for (int t = threadIdx.x; t < np * (P - 1); t += blockDim.x) {
     const int l = t & (np - 1), k = t >> nplog;
     int g = k;
@@ -2634,7 +2655,7 @@ __device__ __forceinline__ void pme_z_gather_body(
   }
   __syncthreads();
   const T *const pot = reinterpret_cast<const T *>(buf);
-  pme_tile_atoms<P>(p, tcol, tix, tjy, colsc, pmb, s_q, [&](int cnt, int slot) {
+  pme_tile_atoms<P, LONG>(p, tcol, tix, tjy, colsc, pmb, s_q, [&](int cnt, int slot) {
     if ((int)(threadIdx.x & 63) >= cnt) return;
     const auto a = pmw[slot];
     const int2 b = pmb[slot];
@@ -2678,14 +2699,14 @@ __device__ __forceinline__ void pme_z_gather_body(
   });
 }
 
-template <bool MIXED, int P>
-__global__ void __launch_bounds__(kPmeBlock, MIXED ? 8 : 4) k_pme_z_gather(
+template <bool MIXED, int P, bool LONG = false>
+__global__ void __launch_bounds__(kPmeBlock, LONG ? 2 : MIXED ? 8 : 4) k_pme_z_gather(
     PmeParams p, FftPlan pl, const int2 *__restrict__ tcol, const int *__restrict__ colsc,
     const typename Real4<typename std::conditional<MIXED, float, double>::type>::type *__restrict__ pmw,
     const int2 *__restrict__ pmb, const Cx<typename std::conditional<MIXED, float, double>::type> *__restrict__ tw,
     const Cx<typename std::conditional<MIXED, float, double>::type> *__restrict__ spec,
     typename AccT<MIXED>::type *__restrict__ facc) {
-  pme_z_gather_body<MIXED, P>(xcd_block(blockIdx.x, gridDim.x), gridDim.x, p, pl, tcol, colsc, pmw, pmb, tw, spec,
+  pme_z_gather_body<MIXED, P, LONG>(xcd_block(blockIdx.x, gridDim.x), gridDim.x, p, pl, tcol, colsc, pmw, pmb, tw, spec,
                               facc);
 }
 
