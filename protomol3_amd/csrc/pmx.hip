@@ -472,6 +472,10 @@ int validate(pmx_ctx *c, const pmx_sys_desc *d) {
 //  - y pass: 8 neighbouring lines (64- or 128-byte segments), x pass: 8
 //    (contiguous anyway), fewer while that leaves fewer than two blocks per
 //    CU; at most tune_fft_lines.
+// The compute units are a constant, not the device's: the gather adds an FP32
+// partial per tile and the x pass an energy partial per block, so other tiles
+// or lines would give other last bits on a partition of the device.
+constexpr int kShapeCus = 256;
 int fft_blocking(Sys *s) {
   PmeParams &pm = s->pme, &pg = s->pme_g;
   const size_t cx = s->mixed ? 8 : 16;
@@ -496,7 +500,7 @@ int fft_blocking(Sys *s) {
     q.nty = (q.ny + q.ty - 1) / q.ty;
   };
   pg = pm;
-  const bool wide = (long long)pm.nx * pm.ny >= 32ll * 4 * s->ctx->cus;
+  const bool wide = (long long)pm.nx * pm.ny >= 32ll * 4 * kShapeCus;
   const bool alone = !s->tune_spread_stream2;
   tiles(pg, wide ? 8 : 4, cx, 36864);
   tiles(pm, wide ? 8 : 4, 16, alone ? 73728 : 36864);
@@ -506,7 +510,7 @@ int fft_blocking(Sys *s) {
     int l = 0;
     while (l < 3 && (2 << l) <= s->tune_fft_lines && ((long long)n << (l + 1)) <= small) ++l;
     while (l > 0 && (1 << l) >= 2 * other) --l;
-    while (l > 2 && (long long)pm.nzh * ((other + (1 << l) - 1) >> l) < 2 * s->ctx->cus) --l;
+    while (l > 2 && (long long)pm.nzh * ((other + (1 << l) - 1) >> l) < 2 * kShapeCus) --l;
     return l;
   };
   s->ylog = lines(pm.ny, pm.nx);
