@@ -459,16 +459,18 @@ int validate(pmx_ctx *c, const pmx_sys_desc *d) {
   return PMX_OK;
 }
 
-// Launch shapes of the PME passes.  Beside the pair kernel's four blocks a
-// CU has room for one more block of 256 threads (64 VGPRs a lane are left on
-// each SIMD) and about 38 KB of LDS, so the passes that run there stay within
-// that; a block of 512 threads would wait for the pair kernel's last blocks
-// (the y pass of a 216 x 240 x 240 grid took 0.70 ms that way, 0.1 ms so).
+// Launch shapes of the PME passes.  Beside the pair kernel's four blocks of
+// 80 registers a CU has 64 VGPRs a lane left on each SIMD, which is room for one
+// block of 512 threads or two of 256, and about 38 KB of LDS; the passes stay
+// within that (which take 512 threads: see below).
 //  - Tiles of the spread and gather passes: tx x ty lines along z.  Wider
 //    tiles repeat less of an atom's work (each tile that an atom's stencil
 //    touches visits it: (tx + p - 1)(ty + p - 1) / (tx ty) tiles) and write
-//    longer segments; the spread takes 8 x 4 where it has the device to
-//    itself and that still gives at least 4 tiles per CU.
+//    longer segments; 8 x 4 where that still gives at least 4 tiles per CU.
+//    Where the spread has the device to itself (main stream, batches) tiles of
+//    twice the LDS in blocks of 512 threads did no better: 9,000 atoms on 192 x
+//    192 x 48 points 104 us a step with, 103 without, on 256 x 256 x 64 at order
+//    8 196 and 185, in FP64 269 and 247; 200,000 atoms on 192^3 306 and 303.
 //  - y pass: 8 neighbouring lines (64- or 128-byte segments), x pass: 8
 //    (contiguous anyway), fewer while that leaves fewer than two blocks per
 //    CU; at most tune_fft_lines.
@@ -485,10 +487,10 @@ int fft_blocking(Sys *s) {
   auto lds = [&](const PmeParams &q, size_t per_point) {
     return per_point * (size_t)(q.tx * q.ty / 2) * pme_line(q.nz, q.order) + (q.nz > kFftMax ? 0 : cx * (q.nz + 1));
   };
-  auto tiles = [&](PmeParams &q, int tx, size_t per_point, size_t most) {
+  auto tiles = [&](PmeParams &q, int tx, size_t per_point) {
     q.tx = tx;
     q.ty = 4;
-    while (q.tx * q.ty > 2 && lds(q, per_point) > most) {
+    while (q.tx * q.ty > 2 && lds(q, per_point) > 36864) {
       if (q.tx > 4)
         q.tx /= 2;
       else if (q.ty > 1)
@@ -501,9 +503,8 @@ int fft_blocking(Sys *s) {
   };
   pg = pm;
   const bool wide = (long long)pm.nx * pm.ny >= 32ll * 4 * kShapeCus;
-  const bool alone = !s->tune_spread_stream2;
-  tiles(pg, wide ? 8 : 4, cx, 36864);
-  tiles(pm, wide ? 8 : 4, 16, alone ? 73728 : 36864);
+  tiles(pg, wide ? 8 : 4, cx);
+  tiles(pm, wide ? 8 : 4, 16);
   s->lds_z = lds(pm, 16);
   s->lds_g = lds(pg, cx);
   auto lines = [&](int n, int other) {
@@ -524,11 +525,13 @@ int fft_blocking(Sys *s) {
   // registers: a step of 4,000 / 9,400 / 13,800 / 26,000 / 1,000,000 atoms
   // 65.9 / 80.5 / 87.1 / 105.5 / 1,501 us with 256, 63.7 / 75.7 / 78.0 /
   // 97.3 / 1,465 with 512.  The spread and the line passes on large grids do
-  // better with two blocks of 256 (1,000,000 atoms 1,465 -> 1,592 and 1,527), and
+  // better with two blocks of 256 (1,000,000 atoms 1,465 -> 1,592 and 1,527; a y
+  // pass of 216 x 240 x 240 points whose blocks of 512 waited for the pair kernel's
+  // last ones took 0.70 ms instead of 0.1), and
   // so do planes and gather in batches, which fill the device (64 systems 24.0
   // ms with 256, 24.8 with 512; 16 in FP64 14.0 and 14.9).
   auto threads = [&](int n, int l) { return ((long long)n << l) > small ? 512 : 256; };
-  s->thr_z = alone && wide ? 512 : threads(pm.nz, 0);
+  s->thr_z = threads(pm.nz, 0);
   s->thr_g = kPmeBlock;
   s->thr_gb = threads(pm.nz, 0);
   s->thr_y = threads(pm.ny, s->ylog);
