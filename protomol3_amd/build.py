@@ -83,7 +83,23 @@ def build_serve(verbose: bool = False) -> str:
     return SERVE_LIB
 
 
+CHECK_LIB = os.path.join(ROOT, "tests", "native", "libpairfunctions.so")
+
+
+def build_checks(verbose: bool = False) -> str:
+    """Device functions of the pair kernel behind a C entry, for the tests."""
+    src = os.path.join(ROOT, "tests", "native", "pair_functions.hip")
+    r = subprocess.run(["hipcc", *HIPCC_FLAGS, "-shared", src, "-o", CHECK_LIB + ".tmp"], capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("hipcc failed:\n" + r.stderr[-4000:])
+    os.replace(CHECK_LIB + ".tmp", CHECK_LIB)
+    if verbose:
+        print("built", CHECK_LIB)
+    return CHECK_LIB
+
+
 if __name__ == "__main__":
     build_lib(verbose=True)
     build_host(verbose=True)
     build_serve(verbose=True)
+    build_checks(verbose=True)
