@@ -125,12 +125,16 @@ struct PmeSlots {
 };
 
 // Grid index of base + offset for base in [0, K), offset < K.
-__device__ inline int wrap_grid(int v, int K) { return v >= K ? v - K : v; }
+__host__ __device__ inline int wrap_grid(int v, int K) { return v >= K ? v - K : v; }
 
 // Grid coordinate of one axis: u = x K/L wrapped to [0, K) (Grid.h:111-120);
-// the base is wrapped too.
-__device__ inline void grid_coord(double x, double hr, int K, int off, int &base, double &w) {
+// the base is wrapped too.  Far from the box whole periods are taken off at
+// once, exactly (their number times K is below 2^53); from 2^40 points on (a run
+// that blew up, infinity) no fraction is left and the place is 0.  One period at
+// a time would take up to 2^40 turns of the loop there, or never end.
+__host__ __device__ inline void grid_coord(double x, double hr, int K, int off, int &base, double &w) {
   double u = x * hr;
+  if (fabs(u) >= 1024.0 * K) u = fabs(u) < 0x1p40 ? u - K * floor(u / K) : 0.0;
   while (u < 0.0) u += K;
   while (u >= K) u -= K;
   const int iu = (int)u;

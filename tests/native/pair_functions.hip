@@ -1,5 +1,7 @@
-// The FP64 functions of the pair kernel, one argument per thread, for
-// tests/test_gpu_pair_functions.py (built by protomol3_amd/build.py).
+// Device functions behind a C entry (built by protomol3_amd/build.py): the FP64
+// functions of the pair kernel, one argument per thread, for
+// tests/test_gpu_pair_functions.py, and the grid coordinate on the host, for
+// tests/test_grid_coord_cpu.py.
 #include <hip/hip_runtime.h>
 
 #include "../../protomol3_amd/csrc/pmx_kernels.h"
@@ -28,4 +30,8 @@ extern "C" int pair_function(int which, int n, const double *x, double *y) {
   if (e == hipSuccess) e = hipMemcpy(y, d + n, 8 * (size_t)n, hipMemcpyDeviceToHost);
   hipFree(d);
   return e;
+}
+
+extern "C" void grid_coordinate(double x, double hr, int points, int off, int *base, double *w) {
+  pmx::grid_coord(x, hr, points, off, *base, *w);
 }
