@@ -114,8 +114,10 @@ int pmx_sys_sync(pmx_sys *sys);
  * pmx_md_run_batch, with the same conditions on the systems; flags must be 0).
  * Each system's forces and energies are those it gets in a batch of its own
  * (the mixed form to the last bit) and pmx_sys_compute's to FP32 rounding
- * (a list built in batched launches is cut into coarser runs); fetch them
- * with pmx_sys_get_forces.  For many
+ * (a list built in batched launches is cut into coarser runs).  Unlike
+ * pmx_sys_compute the call waits for the pass and brings the results of each
+ * system of up to 174,000 atoms (4 MB) to pinned host memory, from which
+ * pmx_sys_get_forces adds them to the caller's arrays.  For many
  * small systems at once (a request loop's force requests, ensemble force
  * calls), whose passes alone are bound by launch latency. */
 int pmx_sys_compute_batch(pmx_sys *const *systems, int nsys, unsigned flags);
@@ -160,9 +162,13 @@ int pmx_sys_cells(pmx_sys *sys, int *cell_of_atom, int *dims);
 
 /* Device milliseconds of the last evaluate with PMX_EVAL_TIMING, in the
  * order: sort (+ MD integrate), list (+ accumulator zeroing), pair (the
- * cluster-pair kernel alone), spread, fft+convolve, gather, fixups (FP64
- * re-test of pairs at the cutoff, exclusion correction, bonded terms),
- * finalize.  ms must hold PMX_STAGES floats. */
+ * cluster-pair kernel alone), spread (with the z transform), fft+convolve,
+ * gather (with the inverse z transform), fixups (exclusion correction, bonded
+ * terms), finalize (FP64 re-test of pairs at the cutoff, force order).  Work
+ * counts where it runs: a charge spread on the second stream in fft, the
+ * correction and bonded terms on the main stream in spread or finalize
+ * (PMX_TUNE_SPREAD_STREAM, PMX_TUNE_FIXUP_STREAM).  ms must hold PMX_STAGES
+ * floats. */
 enum { PMX_STAGES = 8 };
 int pmx_sys_stage_times(const pmx_sys *sys, float *ms);
 /* Per-stage device times averaged over every pmx_sys_compute call made with
@@ -178,18 +184,18 @@ int pmx_sys_timing_end(pmx_sys *sys, float *avg_ms, int *ncalls);
 int pmx_sys_time_pair(pmx_sys *sys, int reps, float *ms_per_launch);
 /* Launch shapes for the autotuner (no counterpart in the reference):
  * PMX_TUNE_FFT_LINES     most lines per FFT block of the x and y transforms
- *                        (1..64, default 16; a block also holds at most 2,048
- *                        points);
+ *                        (1..64, default 16; a block takes at most 8, and at
+ *                        most 2,048 points unless one line has more);
  * PMX_TUNE_PAIR_BLOCKS_PER_CU  pair-kernel blocks per CU (0: as many as fit,
  *                        -k: k fewer than fit, at least 1; fewer leave room
  *                        for the PME chain beside it);
- * PMX_TUNE_PAIR_SCHEDULE 0 (default): the pair list's runs (a number fixed by
- *                        the list, a multiple of 4,096, of equal estimated
- *                        work each) are dealt to the resident waves in
+ * PMX_TUNE_PAIR_SCHEDULE 0 (default): the pair list's runs (of equal estimated
+ *                        work, their number fixed by the list and the form)
+ *                        are dealt to the resident waves in
  *                        contiguous shares; 1: each wave's first run is
  *                        static, later ones come one at a time from a
  *                        device-wide counter (better when fewer waves are
- *                        resident than the default launch's 4,096);
+ *                        resident than the list has runs for);
  * PMX_TUNE_SPREAD_STREAM 0 (default below 10,000 atoms): the PME charge spread
  *                        (with the z transform) runs on the main stream before
  *                        the pair kernel; 1 (default from 10,000 atoms): it
@@ -209,8 +215,8 @@ int pmx_sys_time_pair(pmx_sys *sys, int reps, float *ms_per_launch);
  * PMX_TUNE_FUSED_SPREAD  0 or 1, no effect: the charge spread is one launch
  *                        with the z transform (kept for callers that set it);
  * PMX_TUNE_FFT_PLANES    1 (default): on PME grids whose x-y planes have at
- *                        most 4,096 points (mixed form, 2,048 in FP64), the y
- *                        transform, the x transform
+ *                        most 4,096 points and fit 36 KB of LDS (about 2,200
+ *                        points in FP64), the y transform, the x transform
  *                        with the convolution and the inverse y transform run
  *                        as one launch with a block per plane; 0: three
  *                        launches over lines (also the only form on larger

@@ -67,8 +67,13 @@ struct HostBuf {
 };
 
 // Timed stages: sort (+ integrate), list (+ accumulator zeroing), pair,
-// spread, fft (+ convolution), gather, fixups (exclusion correction, bonded
-// terms), finalize (boundary pairs, force unsort).  Events: 0 start, 1 sorted,
+// spread (with the z transform, and with the exclusion correction and bonded
+// terms where these go with it; only where it runs on the main stream, by
+// default below kSpread2From atoms), fft (+ convolution, after the spread
+// where that runs on the second stream), gather (with the inverse z transform), fixups (exclusion
+// correction and bonded terms, where they run on the second stream), finalize
+// (boundary pairs, with them those terms where they follow the pair kernel, and
+// the force unsort).  Events: 0 start, 1 sorted,
 // 2 list built and accumulators zeroed, 4 spread done = fork (main stream), 3
 // pair done (main stream), 5 fft, 6 gather, 7 correction + bonded done
 // (second stream), 8 end.  The second stream's stages run beside the pair
@@ -2830,9 +2835,8 @@ int batch_tables(Batch &b) {
 
 // Queues one chunk of K steps of every system of the batch (the first step
 // of each system's run when `opening`), then the gathering of the overflow
-// flags into b.flags_h.  Step 0 kicks and drifts and spreads on its own;
-// every later step's kick, drift and spread run in the previous step's last
-// launch.
+// flags into b.flags_h.  Step 0 kicks and drifts in a launch of its own; every
+// later step's kick and drift run in the previous step's last launch.
 template <bool MIXED, int C, int LJ, int CS, bool BIGLJ, int ORDER>
 int batch_chunk(Batch &b, int K, bool opening) {
   using R = typename std::conditional<MIXED, float, double>::type;

@@ -401,7 +401,6 @@ struct OpUnsortForces {
   }
 };
 
-// a force pass's energy partials into the system's energy slots (one block)
 // The end of a force pass with energies, one more block a system than the forces take.
 template <bool MIXED>
 struct OpUnsortEnergy {

@@ -248,10 +248,6 @@ static __global__ void k_fill_u64(unsigned long long *p, unsigned long long v, l
   long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
 }
-static __global__ void k_fill_f64(double *p, double v, long long n) {
-  long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = v;
-}
 
 // Exclusive scan of m uint32 in 3 launches: per-block sums, scan of sums in
 // one block, then per-block rescan with the block offset.
@@ -1515,8 +1511,8 @@ struct EdgesR {
 // much issue time as it saved, and LDS round trips and scalar work on top; in
 // FP64 its 59 KB of LDS a block also left two waves per SIMD.
 // One launch alone, before and after, skin 1.5 / 1.0 / 1.2 A.  Mixed: 26,000
-// atoms 78.8 -> 60.1 us (VALU instructions 29.0 -> 25.1 M, scalar 16.0 -> 6.5 M,
-// LDS 3.0 -> 0.8 M), 9,400 atoms 31.0 -> 27.3, 1,000,000 atoms 1.63 -> 1.07 ms;
+// atoms 78.8 -> 60.1 us (VALU instructions 29.0 -> 26.6 M, scalar 16.0 -> 6.7 M,
+// LDS 3.0 -> 0.9 M), 9,400 atoms 31.0 -> 27.3, 1,000,000 atoms 1.63 -> 1.07 ms;
 // unequal cutoffs, 46,000 atoms 126 -> 97 us.  FP64: 26,000 atoms
 // with PME 210 -> 109 us, 93,000 with cutoffs 364 -> 173; three blocks per CU
 // (151 VGPRs; at 128 the PME form spills 118), with cutoffs four.
