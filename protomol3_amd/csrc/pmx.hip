@@ -152,7 +152,8 @@ struct Sys {
   bool have_positions = false;
   bool cached = false;
   bool list_valid = false;             // entries, counts and work of a built list are in place
-  bool reduced = false;                // eout holds the energies of the last pass (whose partials may be gone)
+  enum { kInPartials, kInResults, kInHeld } energies_at = kInPartials;  // where the last pass's energies are:
+                                       // its partials, eout, md.held (the partials may be gone)
   bool acc_clean = false;              // force accumulators and pass counters are zero
   bool dry = false;                    // size only: allocations are counted, nothing runs
   unsigned long long dry_bytes = 0;
@@ -168,7 +169,7 @@ struct Sys {
     bool on = false;
     int nb = 0, na = 0;
     double h = 0, skin = 0;
-    DevBuf mptr, bonds, bpar, angles, apar, minv, v, xbuild, xbak, vbak, fbak, dmax, bond_e, ke_e;
+    DevBuf mptr, bonds, bpar, angles, apar, minv, v, xbuild, xbak, vbak, fbak, dmax, bond_e, ke_e, held;
     int chunk = 16;
     long long steps = 0, rebuilds = 0, rollbacks = 0;
     bool forces_valid = false;
@@ -1249,11 +1250,19 @@ EnergyArgs energy_args(Sys *s, bool stats) {
           P<unsigned long long>(s->hash_out)};
 }
 
-// The energies of the last pass into eout, unless they are there.
-void reduce_energies(Sys *s) {
-  if (!s->reduced)
-    hipLaunchKernelGGL(k_reduce_energy, dim3(1), dim3(kEndBlock), 0, s->ctx->stream, energy_args(s, false));
-  s->reduced = true;
+// The energies of the last pass added up: into eout for pmx_md_get_state, or
+// aside before its partials go, where eout keeps the last evaluation's.
+void reduce_energies(Sys *s, bool aside) {
+  if (s->energies_at != Sys::kInPartials) return;
+  EnergyArgs a = energy_args(s, false);
+  if (aside) {
+    PassResults *const h = P<PassResults>(s->md.held);
+    a.out = h->e;
+    a.out_np = h->np;
+    a.out_hash = h->hash;
+  }
+  hipLaunchKernelGGL(k_reduce_energy, dim3(1), dim3(kEndBlock), 0, s->ctx->stream, a);
+  s->energies_at = aside ? Sys::kInHeld : Sys::kInResults;
 }
 
 void timing_begin_call(Sys *s, bool timing) {
@@ -1369,7 +1378,7 @@ int forces(Sys *s, unsigned flags, bool energies, const Kick *next = nullptr, un
   if (!s->acc_clean) launch_zero(s);
   s->acc_clean = false;
   s->staged = false;
-  s->reduced = energies;
+  s->energies_at = energies ? Sys::kInResults : Sys::kInPartials;
   if (timing) hipEventRecord(s->ev[2], st);
   // fork: FFT, gather, exclusion correction and bonded terms on the second
   // stream beside the pair kernel; all add into the zeroed accumulators.
@@ -1975,7 +1984,7 @@ int pmx_sys_set_tuning(pmx_sys *sys, int knob, int value) {
   // the blocks of the x pass change, and with them the places of the energy
   // partials: those of the state at hand are added up before
   hipSetDevice(s->ctx->device);
-  if (s->md.on && s->md.forces_valid) reduce_energies(s);
+  if (s->md.on && s->md.forces_valid) reduce_energies(s, true);
   HIPCHK(hipStreamSynchronize(s->ctx->stream));
   HIPCHK(hipStreamSynchronize(s->ctx->stream2));
   {
@@ -2081,7 +2090,7 @@ int pmx_md_init(pmx_sys *sys, const pmx_md_desc *d) {
       (rc = dalloc(s, m.xbak, 2 * 24 * N)) || (rc = dalloc(s, m.vbak, 2 * 24 * N)) ||
       (rc = dalloc(s, m.fbak, 2 * 24 * N)) || (rc = dalloc(s, m.dmax, 4 * 2 * kMaxChunk)) ||
       (rc = dalloc(s, m.step_dev, 8)) || (rc = dalloc(s, m.bond_e, 16 * (size_t)s->term_blocks)) ||
-      (rc = dalloc(s, m.ke_e, 8 * (size_t)nblk(N, 256))))
+      (rc = dalloc(s, m.ke_e, 8 * (size_t)nblk(N, 256))) || (rc = dalloc(s, m.held, sizeof(PassResults))))
     return rc;
   if (!m.host) {
     RtLock lk(g_rt_mu);
@@ -2283,7 +2292,8 @@ int enqueue_chunk(Sys *s, const Chunk &c) {
       }
     }
   }
-  s->staged = s->reduced = false;  // a replay runs no host code of the passes in it
+  s->staged = false;  // a replay runs no host code of the passes in it
+  s->energies_at = Sys::kInPartials;
   if (x) {
     hipLaunchKernelGGL(k_set_u64, dim3(1), dim3(1), 0, st, P<unsigned long long>(m.step_dev),
                        (unsigned long long)c.step0);
@@ -2964,7 +2974,7 @@ int batch_forces(Batch &b) {
     s->list_valid = true;
     s->prune_pending = false;
     s->staged = b.results && batch_stages(s);
-    s->reduced = b.results;
+    s->energies_at = b.results ? Sys::kInResults : Sys::kInPartials;
   }
   return PMX_OK;
 }
@@ -3041,7 +3051,7 @@ int batch_run(Batch &b, int nsteps) {
     s->md.steps += nsteps;
     s->md.rebuilds += nreb[i];
     s->list_valid = true;
-    s->reduced = false;
+    s->energies_at = Sys::kInPartials;
     s->prune_pending = false;
     s->acc_clean = true;
   }
@@ -3200,7 +3210,8 @@ int batch_entry(pmx_sys *const *systems, int nsys, int nsteps) {
   b.results = !md;
   for (int i = 0; i < nsys; ++i) {
     Sys *s = &systems[i]->s;
-    s->staged = s->reduced = false;
+    s->staged = false;
+    s->energies_at = Sys::kInPartials;
     b.sys.push_back(s);
     if (!s->cached)
       if (int rc = setup(s)) return rc;
@@ -3249,7 +3260,7 @@ int pmx_md_get_state(pmx_sys *sys, double *x, double *v, double *energies) {
     // potential energies at the current positions (computed first if the
     // state was just set) and kinetic energy of v
     if (int rc = md_ensure_forces(s)) return rc;
-    reduce_energies(s);
+    reduce_energies(s, false);
     hipLaunchKernelGGL(k_kinetic, dim3(nblk(n, 256)), dim3(256), 0, st, n, P<double>(m.v), P<double>(m.minv),
                        P<double>(m.ke_e));
   }
@@ -3271,7 +3282,7 @@ int pmx_md_get_state(pmx_sys *sys, double *x, double *v, double *energies) {
   const double *const h = static_cast<double *>(s->stage.p);
   const double *ke = h, *be = h;
   if (energies) {
-    out.add(s->eout.p, 4);
+    out.add(s->energies_at == Sys::kInHeld ? s->md.held.p : s->eout.p, 4);
     ke = out.add(m.ke_e.p, nke);
     be = out.add(m.bond_e.p, nbe);
   }

@@ -195,3 +195,29 @@ def test_first_forces_do_not_depend_on_the_partners(ctx):
                 sy.close()
     for o in out[1:]:
         assert _equal(o, out[0]) and o[3] == out[0][3]
+
+
+@pytest.mark.parametrize("how", ["batch", "run"])
+def test_launch_shapes_leave_the_energies_of_the_last_evaluation(ctx, how):
+    """Shapes set after a run change neither what pmx_sys_get_forces gives
+    (the last evaluation's energies and pair statistics) nor the energies of
+    the state."""
+    s = systems.replica_box(900, 13).with_velocities(300.0, seed=14)
+    sy, twin = _mixed(ctx, s, serve.request_spec(s)), _mixed(ctx, s, serve.request_spec(s))
+    try:
+        for t in (sy, twin):
+            _, ec, elj = t.evaluate(s.pos + 0.05 * np.sin(np.arange(3 * s.n).reshape(-1, 3)), pmx.EVAL_PAIRSTATS)
+            t.md_set_state(s.pos, s.vel)
+            if how == "batch":
+                pmx.run_batch([t], 10)
+            else:
+                t.md_run(10)
+        stats = sy.pair_stats()
+        for knob, value in ((pmx.TUNE_PAIR_BLOCKS_PER_CU, 1), (pmx.TUNE_FFT_PLANES, 0)):
+            sy.set_tuning(knob, value)
+            _, ec2, elj2 = sy.get_forces()
+            assert (ec2, elj2) == (ec, elj) and sy.pair_stats() == stats
+        assert sy.md_get_state()[2] == twin.md_get_state()[2]
+    finally:
+        sy.close()
+        twin.close()
